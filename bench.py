@@ -89,7 +89,7 @@ def profiled_traffic(root, workload, kernel_name):
 def roofline_of(root, shape, res, read_peak):
     """The roofline object of one workload's gate/up launch.  `read_peak`: the measured streaming-read rate."""
     kname = res["kernels"]["gate_up"]
-    bound = "mfma" if kname.startswith("expert_prefill") else "hbm"
+    bound = "mfma" if kname.startswith(("expert_prefill", "expert_tile")) else "hbm"
     traffic, source = profiled_traffic(root, shape.name, kname)
     ms, nbytes, flops, what = res["mlp1"]["ms"], res["mlp1"]["bytes"], res["mlp1"]["flops"], "gate/up GEMM + SwiGLU"
     if kname.startswith("expert_fused"):  # one launch holds both GEMMs; its time is reported as the gate/up stage

@@ -20,20 +20,27 @@ constexpr size_t kAlign = 256;
 inline size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 inline hipStream_t as_stream(moe_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 
-// Token-block sizes of the expert kernels' tile map: decode-sized buckets / prefill-sized buckets.
+// Token-block sizes of the expert kernels' tile map: decode-sized buckets / prefill-sized buckets of MXFP4 and of bf16
+// experts.
 constexpr int kStreamTileTokens = 64;
 constexpr int kPrefillTileTokens = 128;
+constexpr int kPrefillTileTokensBf16 = 256;
+inline int tile_tokens_of(bool prefill, int format) {
+    return !prefill ? kStreamTileTokens : format == MOE_WEIGHTS_BF16 ? kPrefillTileTokensBf16 : kPrefillTileTokens;
+}
 
 // Which family runs the expert GEMMs, by average bucket size T*K/E (measured crossovers, 20b
 // shapes, token counts 256..4096).  MXFP4: the 128-token-block kernels win as soon as buckets start
 // to overflow one 64-token block (the streaming kernel then reads an expert's weights once per
-// block of its bucket).  bf16: the same (E = 32: 350 against 428 us at 48 rows per expert, 572 against
-// 437 us at 64).
-inline bool use_prefill_kernels(int T, int K, int E, int format, unsigned flags) {
+// block of its bucket).  bf16, streaming kernels against 256-token blocks: E = 32, 302 : 340 us at 44 rows per expert,
+// 373 : 343 at 48, 455 : 347 at 56; E = 128, 1199 : 1228 at 44, 1329 : 1246 at 50.
+inline bool use_prefill_kernels(int T, int H, int I, int K, int E, int format, unsigned flags) {
     if (flags & MOE_FLAG_FORCE_STREAM) return false;
-    if (flags & MOE_FLAG_FORCE_TILED) return true;
     const long long rows = (long long)T * K;
-    return format == MOE_WEIGHTS_MXFP4_TILED ? rows >= 52LL * E : rows >= 56LL * E;
+    // activation tensors past 4 GiB: only the streaming kernels address them
+    if (format == MOE_WEIGHTS_BF16 && !(expert_tile_fits(T, 2 * I, H) && expert_tile_fits(rows, H, I))) return false;
+    if (flags & MOE_FLAG_FORCE_TILED) return true;
+    return format == MOE_WEIGHTS_MXFP4_TILED ? rows >= 52LL * E : rows >= 46LL * E;
 }
 
 // Bucketing inside the expert kernels instead of a launch of its own: for the weight-streaming
@@ -443,6 +450,7 @@ struct ExpertPlan {
         g.tile_row0 = ws.tile_row0;
         g.tile_rows = ws.tile_rows;
         g.n_tiles = ws.n_tiles;
+        g.expert_offsets = ws.expert_offsets;
         g.max_tiles = max_tiles;
         g.alpha = p->alpha;
         g.limit = p->swiglu_limit;
@@ -461,10 +469,7 @@ struct ExpertPlan {
     // 32 rows each.  Blocks run in rounds of one per CU, so the cheaper choice is the one with the
     // smaller rounds x rows-per-block product; more rows per block also re-read the activations less.
     int pick_kernel(int rows) const {
-        if (prefill) {  // bf16 weights, buckets of 80 rows and more on average: the one-block-a-CU kernel
-            const bool big = (long long)p->n_tokens * p->experts_per_token >= 80LL * p->n_experts;
-            return p->weight_format == MOE_WEIGHTS_BF16 && big ? 17 : 16;
-        }
+        if (prefill) return p->weight_format == MOE_WEIGHTS_BF16 ? 17 : 16;
         const int cost10 = ceil_div(ceil_div(rows / 32, 10) * est_tiles, n_cus) * 10;
         const int cost12 = ceil_div(ceil_div(rows / 32, 12) * est_tiles, n_cus) * 12;
         return cost12 <= cost10 ? 1 : 0;
@@ -539,6 +544,11 @@ struct ExpertPlan {
             a.s_expert_stride = (long long)sb;
         }
     }
+    void use_second_map(ExpertGemmArgs& a) const {
+        a.tile_expert += second_map;
+        a.tile_row0 += second_map;
+        a.tile_rows += second_map;
+    }
     // act: bf16 [T, H] rows gathered by token; out: bf16 SwiGLU rows [A, I]
     ExpertGemmArgs gate_up(const uint16_t* act, uint16_t* out) const {
         ExpertGemmArgs a = g;
@@ -551,6 +561,7 @@ struct ExpertPlan {
         // row blocks on one XCD takes 1 % off the bf16 launch (its token rows enter one L2 instead of eight) and
         // leaves the MXFP4 launch as it is; with token blocks from the tile map it cost up to 2 %
         a.xcd_tiles = direct ? 1 : 0;
+        if (a.waves_per_block == 17) use_second_map(a);  // places an expert's blocks by where its tiles begin
         return a;
     }
     // act: bf16 [A, I] rows (by slot, or by assignment when bucketing is done in the kernel); out: fp32 [A, H]
@@ -565,11 +576,7 @@ struct ExpertPlan {
         // (largest first: the launch's tail is made of short blocks); the down GEMM is 2 % faster in bucket
         // order, where a partial block runs next to full blocks of its expert and finds the expert's weights
         // on their way through the caches.
-        if (!direct) {
-            a.tile_expert += second_map;
-            a.tile_row0 += second_map;
-            a.tile_rows += second_map;
-        }
+        if (!direct) use_second_map(a);
         // measured: the down GEMM gains 4-10 % from keeping a token block on one XCD (its input rows were
         // written by the gate/up launch just before)
         a.xcd_tiles = 1;
@@ -640,9 +647,9 @@ static int block_forward_impl(const moe_block_params* caller, moe_stream_t strea
     // 2. bucketing + token-block map  (src/forward.cpp:329-376)
     // Small batches need no bucketing launch: each block of the expert kernels finds its expert's
     // bucket in topk_i itself and rows are addressed by assignment id (token * K + k).
-    const bool prefill = use_prefill_kernels(T, K, E, p->weight_format, p->flags);
+    const bool prefill = use_prefill_kernels(T, H, I, K, E, p->weight_format, p->flags);
     const bool direct = use_direct_bucketing(T, K, E, prefill, p->flags);
-    const int tile_tokens = prefill ? kPrefillTileTokens : kStreamTileTokens;
+    const int tile_tokens = tile_tokens_of(prefill, fmt);
     const int max_tiles = tile_map_capacity(T * K, E, tile_tokens);  // <= ws.max_tiles (sized for 64)
     if (!direct) {
         TileMap map{ws.tile_expert, ws.tile_row0, ws.tile_rows, ws.n_tiles, tile_tokens, max_tiles, ws.max_tiles};
@@ -729,9 +736,9 @@ int moe_block_describe(const moe_block_params* p, char* text, size_t text_bytes)
                              ? "router_screen_kernel + router_refine_kernel"
                              : (!strict && router_fused_fits(H)) ? "router_fused_kernel"
                                                                  : "router_partial_kernel + router_finalize_kernel";
-    const bool prefill = use_prefill_kernels(T, K, E, fmt, p->flags);
+    const bool prefill = use_prefill_kernels(T, H, I, K, E, fmt, p->flags);
     const bool direct = use_direct_bucketing(T, K, E, prefill, p->flags);
-    const int tile_tokens = prefill ? kPrefillTileTokens : kStreamTileTokens;
+    const int tile_tokens = tile_tokens_of(prefill, fmt);
     BlockWorkspace ws(nullptr, T, H, I, E, K);
     const ExpertPlan plan(p, ws, prefill, direct, tile_tokens, tile_map_capacity(T * K, E, tile_tokens));
     auto gemm_name = [&](int rows, int epi, char* out, size_t n) {
@@ -739,7 +746,7 @@ int moe_block_describe(const moe_block_params* p, char* text, size_t text_bytes)
         if (direct && fmt == MOE_WEIGHTS_MXFP4_TILED) plan.pick_two_pass(rows, &kernel, &row_blocks);
         const int cons = kernel == 1 ? 12 : 10;
         if (prefill && kernel == 17) {
-            snprintf(out, n, "expert_prefill_bf16_kernel<%d>", epi);
+            snprintf(out, n, "expert_tile_bf16_kernel<%d>", epi);
         } else if (prefill) {
             snprintf(out, n, "expert_prefill_kernel<%d, %d, 4>", fmt, epi);
         } else if (direct) {
@@ -794,9 +801,9 @@ int moe_block_down_gemm(const moe_block_params* caller, const moe_bf16_t* h_by_a
     BlockWorkspace ws(p->workspace, T, H, I, E, K);
     if (p->workspace_bytes < ws.bytes) return MOE_ERR_WORKSPACE;
     hipStream_t stream = as_stream(stream_);
-    const bool prefill = use_prefill_kernels(T, K, E, fmt, p->flags);
+    const bool prefill = use_prefill_kernels(T, H, I, K, E, fmt, p->flags);
     const bool direct = use_direct_bucketing(T, K, E, prefill, p->flags);
-    const int tile_tokens = prefill ? kPrefillTileTokens : kStreamTileTokens;
+    const int tile_tokens = tile_tokens_of(prefill, fmt);
     const int max_tiles = tile_map_capacity(T * K, E, tile_tokens);
     const ExpertPlan plan(p, ws, prefill, direct, tile_tokens, max_tiles);
     if (direct) return launch_expert_stream(plan.down(h_by_assignment, y_by_assignment), 1, stream);

@@ -83,6 +83,7 @@ struct ExpertGemmArgs {
     const int* tile_row0;
     const int* tile_rows;
     const int* n_tiles;
+    const int* expert_offsets;  // [E + 1] with the tile map: rows of the experts before each
     void* out;                  // see launch_expert_stream
     int rows;                   // weight rows per expert (2I or H)
     int K;                      // contraction length (H or I)
@@ -97,11 +98,14 @@ struct ExpertGemmArgs {
     int xcd_tiles;              // producer-consumer kernel: all row blocks of a token block on one XCD
     int waves_per_block;        // kernel choice of the fused block: 0 / 1 producer-consumer kernel with 10 / 12
                                 // consumer waves (+ 2 producers), 64-token blocks; 16 prefill kernel (4 waves,
-                                // 128-token blocks, two blocks a CU); 17 bf16 weights only: prefill kernel with
-                                // one block a CU and a register ring of weights (MXFP4: as 16).  Ignored by the
-                                // work-queue entries.
+                                // 128-token blocks, two blocks a CU; MXFP4 weights only); 17 tile kernel
+                                // (256-token blocks; bf16 weights only).  Ignored by the work-queue entries.
 };
 int launch_expert_stream(const ExpertGemmArgs& a, int epi, hipStream_t stream);
+
+// ---- experts_tile.hip: prefill-sized buckets of bf16 experts (token blocks of up to 256 rows) ----
+bool expert_tile_fits(long long act_rows, int rows, int K);
+int launch_expert_tile_bf16(const ExpertGemmArgs& a, int epi, hipStream_t stream);
 int expert_direct_max_assignments();
 
 // ---- experts_fused.hip: both expert GEMMs of a block in one launch (bucketing inside the kernel) --
