@@ -555,7 +555,7 @@ MOE_DEVICE void ws_consumer(const ExpertGemmArgs& a, const uint8_t* lds, int e, 
             __builtin_amdgcn_sched_barrier(0);  // the loads are issued here, three stages ahead of their use
             // In a ragged last stage the lane groups past the last MX block hold another tile's bytes (or zeros);
             // the tiled scale tensor has scale byte 0 in the slots of blocks that do not exist (moe_mxfp4_repack
-            // clears the tensor before it scatters), which converts to a factor of exactly 0: no select needed.
+            // writes it), which converts to a factor of exactly 0: no select needed.
             float sc[R];
 #pragma unroll
             for (int r = 0; r < R; ++r) sc[r] = mxfp4_scale_to_f32((sw_cur[r] >> (8 * i)) & 0xFFu);

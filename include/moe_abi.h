@@ -265,7 +265,7 @@ MOE_API int moe_dequant_mxfp4(const uint8_t* blocks, const uint8_t* scales, long
  * moe_mxfp4_tiled_bytes gives the sizes of the two destination buffers for ONE expert; experts
  * are stored back to back.  moe_mxfp4_unpack is the exact inverse.  The tiled scale tensor is
  * padded to whole groups of four 128-element stages per row tile; moe_mxfp4_repack writes scale
- * byte 0 into the slots of MX blocks that do not exist (it clears the tensor first), and the
+ * byte 0 into the slots of MX blocks that do not exist, and the
  * expert kernels rely on that byte: it converts to a factor of exactly 0 for whatever a lane past
  * the last block of a row has loaded.  A tiled tensor must therefore come from moe_mxfp4_repack
  * (or moe_ckpt_upload_layer, which calls it). */
