@@ -54,6 +54,18 @@ inline bool use_direct_bucketing(int T, int K, int E, bool prefill, unsigned fla
     return A <= 48LL * E;
 }
 
+// The kernels for a handful of rows per expert (experts_small.hip).  They keep every compute unit busy whatever share of the
+// experts has rows; the producer/consumer kernels have the better rate once all blocks of one round have work.  Whole
+// block, 20b / 120b shapes, small : streaming kernels, us.  Where these come in one round of blocks (E = 32, MXFP4), 7 tokens
+// 57 : 65, 10 tokens 62 : 67, 16 tokens 80 : 76; in several rounds, E = 32, bf16: 7 tokens 168 : 210, 24 tokens 255 : 254, 32
+// skewed 255 : 241; E = 128, MXFP4: 33 tokens 199 : 236, 96 tokens 281 : 285; E = 128, bf16: 33 tokens 650 : 808.
+inline bool use_small_kernels(int T, int H, int I, int K, int E, int format, bool direct, unsigned flags, int n_cus) {
+    if (!direct || (flags & (MOE_FLAG_FORCE_STREAM | MOE_FLAG_FORCE_DIRECT | MOE_FLAG_FUSED_GEMM_LAUNCH))) return false;
+    if (!expert_small_fits(T * K, 2 * I, H, format) || !expert_small_fits(T * K, H, I, format)) return false;
+    const long long blocks = (long long)E * ceil_div(2 * I / 32, format == MOE_WEIGHTS_MXFP4_TILED ? 24 : 12);
+    return 4LL * T * K <= (blocks > n_cus ? 12LL : 5LL) * E;
+}
+
 // Both expert GEMMs in one launch: on request, when the bucketing is done inside the expert kernels and
 // the experts fit the kernel's per-XCD tables.  Measured at the 20b decode shape it ties with the two
 // launches for bf16 weights (what it saves in launch boundaries it pays for emptying and refilling its
@@ -437,7 +449,7 @@ static int device_cu_count() {
 struct ExpertPlan {
     const moe_block_params* p;
     ExpertGemmArgs g{};
-    bool prefill, direct;
+    bool prefill, direct, small;
     int est_tiles, n_cus;
     int second_map;  // index of the token-block map in bucket order inside the map arrays
 
@@ -463,6 +475,7 @@ struct ExpertPlan {
         }
         est_tiles = direct ? E : std::max(ceil_div(T * K, tile_tokens), std::min(E, T * K));
         n_cus = device_cu_count();
+        small = use_small_kernels(T, p->hidden_dim, p->intermediate_dim, K, E, p->weight_format, direct, p->flags, n_cus);
         second_map = ws.max_tiles;
     }
     // Decode-sized buckets (producer/consumer kernel, one block per CU): 10 or 12 consumer waves of
@@ -529,7 +542,10 @@ struct ExpertPlan {
         a.rows = rows;
         a.K = Kdim;
         a.bias_expert_stride = rows;
-        if (direct && p->weight_format == MOE_WEIGHTS_MXFP4_TILED) {
+        if (small) {
+            a.waves_per_block = 18;
+            a.n_cus = n_cus;
+        } else if (direct && p->weight_format == MOE_WEIGHTS_MXFP4_TILED) {
             pick_two_pass(rows, &a.waves_per_block, &a.row_blocks);
         } else {
             a.waves_per_block = pick_kernel(rows);
@@ -749,6 +765,8 @@ int moe_block_describe(const moe_block_params* p, char* text, size_t text_bytes)
             snprintf(out, n, "expert_tile_bf16_kernel<%d>", epi);
         } else if (prefill) {
             snprintf(out, n, "expert_prefill_kernel<%d, %d, 4>", fmt, epi);
+        } else if (plan.small) {
+            snprintf(out, n, "expert_small_kernel<%d, %d>", fmt, epi);
         } else if (direct) {
             // as the launcher: at least enough row blocks for one (bf16) or two (MXFP4) passes of `cons` row units
             const int units = rows / 32;

@@ -1,0 +1,355 @@
+// Expert GEMMs of the MoE block for batches that give an expert a handful of rows: every wave streams 16 weight rows of
+// one expert over the whole contraction range on its own.  Replaces moe_mlp1_swiglu_mfma_kernel (src/hip/moe.hip:9-235)
+// and moe_mlp2_scatter_mfma_kernel (src/hip/moe.hip:261-512) at those sizes.
+//
+// What bounds it: the weights of the experts that got a row, and below that the launch's chain of latencies (expert ids,
+// then weights and activation rows, then the stores).  The producer/consumer kernels cut an expert into blocks of 320 to
+// 768 weight rows, one to a compute unit: one token's four experts occupy 32 of 256 compute units, and the 20 experts of
+// seven tokens are 320 blocks, i.e. two rounds for the work of 1.25.  Here the bucket's few rows are staged once, whole,
+// the stage barriers go, and the work is cut by MFMA tile.  Gate/up + down launch, us: one token, E = 32 MXFP4 25 + 15 -> 10 + 7
+// (2.1 TB/s in the larger: ids, rows and weights are a chain of three round trips), bf16 124 + 65 -> 25 + 14; 7 tokens, E = 32
+// bf16 138 + 66 -> 105 + 52 (6.2 TB/s); 33 tokens, E = 128 MXFP4 116 + 70 -> 108 + 59 (6.8).  Two tiles a wave, and three
+// blocks a compute unit instead of two: no faster.
+#include <type_traits>
+
+#include "expert_tiles.h"
+
+namespace moe {
+
+namespace {
+
+constexpr int kSmallWaves = 8;         // at most
+constexpr int kSmallMaxAssign = 512;   // one expert id per thread of a full block
+constexpr int kSmallRows = 32;         // bucket rows of one pass over the weights (two token tiles)
+constexpr int kSmallLds = 64 * 1024;   // of staged activations, so that two blocks fit a compute unit
+constexpr int kSmallGroup = 8;         // a phase (what is staged at once) is a multiple of so many stages
+
+// Tile `tile` (16 weight rows, order of tile_row_in_group) against the nrows <= 16 NT bucket rows starting at row0.  The
+// activations of `per_phase` stages of 128 contraction elements are staged at a time, rows_img (nrows rounded up to four)
+// rows to a stage, 256 bytes each, chunk c of row r at position ws_pos(c) ^ (r % 16).  All waves of the block call this
+// with the same bucket; those without a tile (active false) only stage.
+template <int FMT, int NT, int EPI>
+MOE_DEVICE void small_tile(const ExpertGemmArgs& a, uint8_t* lds, int e, const int* bucket, int row0, int nrows, int tile,
+                           bool active, int lds_bytes) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int waves = blockDim.x >> 6;
+    const int q = lane & 15;
+    const int g = lane >> 4;
+    const int K = a.K;
+    const int n_stages = ceil_div(K, kStageElems);
+    const int rows_img = (nrows + 3) & ~3;
+    const int stage_bytes = rows_img * 256;
+    const int per_phase = min(n_stages, lds_bytes / stage_bytes / kSmallGroup * kSmallGroup);
+    // token of assignment s = s / assign_div, as a float multiplication (exact for s < 4096, assign_div <= 8)
+    const float inv_div = 1.0f / (float)a.assign_div;
+    // stages [s0, s0 + per_phase) to LDS: instruction n moves four rows of one stage, whole 256-byte pieces; the waves
+    // take them in turn
+    auto stage_rows = [&](int s0) {
+        const int quads = rows_img >> 2;
+        const int n_instr = min(per_phase, n_stages - s0) * quads;
+        int st = wave / quads, rq = wave - st * quads;  // wave-uniform
+        const int dst_step = waves / quads, dq_step = waves - dst_step * quads;
+        for (int n = wave; n < n_instr; n += waves) {
+            const int r = rq * 4 + g;
+            const int s = bucket[row0 + min(r, nrows - 1)];
+            const int src = a.gather ? (int)(((float)s + 0.5f) * inv_div) : s;
+            const int k = (s0 + st) * kStageElems + 8 * ws_chunk_at<FMT>(q ^ (r & 15));
+            // a position past the row re-reads its start: its weights count as zero
+            dma16(reinterpret_cast<const uint8_t*>(a.act + (size_t)src * K + (k < K ? k : 0)),
+                  lds + (size_t)n * 1024);
+            st += dst_step;
+            rq += dq_step;
+            if (rq >= quads) {
+                rq -= quads;
+                ++st;
+            }
+        }
+    };
+    auto restage = [&](int s0) {  // all waves are past the reads of the stages before
+        stage_rows(s0);
+        wait_vmcnt<0>();
+        __syncthreads();
+    };
+    if (!active) {
+        restage(0);
+        for (int s0 = per_phase; s0 < n_stages; s0 += per_phase) {
+            __syncthreads();
+            restage(s0);
+        }
+        return;
+    }
+    const int group = tile >> 2;
+    const int r0 = tile & 3;
+    uint2 bias_raw[1];
+    load_bias<1>(a, e, group, r0, bias_raw);
+    // the columns past the bucket's end take its last staged row again; they are never stored.  MFMA step j of lane group g
+    // reads position 2g + (j & 1) + 8 (j >> 1) of its row in either format's image: the steps differ in address bits 4 and 7
+    uint32_t b_lane[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int row = min(t * 16 + q, rows_img - 1);
+        b_lane[t] = (uint32_t)(row * 256 + ((ws_pos<FMT>(ws_chunk<FMT>(0, g)) ^ (row & 15)) << 4));
+    }
+    int phase0 = 0;  // first stage that is staged now
+    uint32_t b_at[NT];
+    auto at_stage = [&](int s) {
+        uint32_t off = (uint32_t)(s - phase0) * (uint32_t)stage_bytes;
+        asm volatile("" : "+s"(off));  // kept a scalar: otherwise every stage's addresses are held in registers of their own
+#pragma unroll
+        for (int t = 0; t < NT; ++t) b_at[t] = b_lane[t] + off;
+    };
+    auto b_frag = [&](int j, int t) {
+        return *reinterpret_cast<const u32x4*>(lds + (b_at[t] ^ (uint32_t)((j & 1) * 16 + (j >> 1) * 128)));
+    };
+    auto next_phase = [&](int s) {  // stage s is the next to be computed
+        if (s == phase0 + per_phase) {
+            phase0 = s;
+            __syncthreads();
+            restage(s);
+        }
+    };
+    f32x4 acc[1][NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[0][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    if constexpr (FMT == FMT_BF16) {
+        // Weights as in ws_consumer: pairs of MFMA steps, each fetched by two non-temporal loads of whole 128-byte lines
+        // whose lane halves trade places at use; a ring of four pairs (two stages).
+        constexpr int D = 4;
+        const int n_pairs = K / 64;
+        const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint16_t*>(reinterpret_cast<const uint16_t*>(a.w) + (size_t)e * a.w_expert_stride), 0,
+            (int)((uint32_t)a.rows * (uint32_t)K * 2u), 0x00020000);
+        const uint32_t a_tile = (uint32_t)(group * 64 + tile_row_in_group(r0, 0)) * (uint32_t)K * 2u;
+        const uint32_t a_lane = (uint32_t)(tile_row_in_group(0, q & 7) * K + 8 * (2 * g + (q >> 3))) * 2u;
+        const uint32_t second_half = 32u * (uint32_t)K * 2u;  // tile row q + 8 is weight row + 32 (tile_row_in_group)
+        u32x4 ar[D][2];
+        auto load_a = [&](int slot, int pair) {
+            const uint32_t off = a_tile + (uint32_t)(pair < n_pairs ? pair : 0) * 128u;  // past the end: unused
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                ar[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, (int)a_lane, (int)(off + second_half * i), 2 /* nt */);
+        };
+#pragma unroll
+        for (int i = 0; i < D - 1; ++i) load_a(i, i);
+        restage(0);
+        auto pair_step = [&](int u, int pair) {
+            load_a((u + D - 1) % D, pair + D - 1);
+            __builtin_amdgcn_sched_barrier(0);  // the loads are issued here, three pairs ahead of their use
+            if ((u & 1) == 0) at_stage(pair >> 1);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                u32x4 av;
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+                    av[d] = h == 0 ? (uint32_t)__builtin_amdgcn_update_dpp((int)ar[u][0][d], (int)ar[u][1][d], 0x128, 0xF, 0xC, false)
+                                   : (uint32_t)__builtin_amdgcn_update_dpp((int)ar[u][1][d], (int)ar[u][0][d], 0x128, 0xF, 0x3, false);
+#pragma unroll
+                for (int t = 0; t < NT; ++t) acc[0][t] = mfma_16x16x32(av, b_frag(2 * (u & 1) + h, t), acc[0][t]);
+            }
+        };
+        const int full = n_pairs / D;
+        for (int i = 0; i < full; ++i) {
+            next_phase(2 * i);
+#pragma unroll
+            for (int u = 0; u < D; ++u) pair_step(u, D * i + u);
+        }
+        if (D * full < n_pairs) {
+            next_phase(2 * full);
+            pair_step(0, D * full);
+            if (D * full + 1 < n_pairs) pair_step(1, D * full + 1);
+            if (D * full + 2 < n_pairs) pair_step(2, D * full + 2);
+        }
+    } else {
+        // Weights as in ws_consumer: one 1 KiB chunk per stage, one scale dword per four stages, reads past the tile only
+        // where the scale byte is 0 or nobody looks; a ring of eight stages, scales one group of eight ahead.
+        constexpr int D = kSmallGroup;
+        const int G = K / 32;
+        const uint32_t wtile = (uint32_t)tile * (uint32_t)G * 256u;
+        const uint32_t stile = (uint32_t)tile * (uint32_t)ceil_div(ceil_div(G, 4), 4) * 256u;
+        const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint8_t*>(reinterpret_cast<const uint8_t*>(a.w) + (size_t)e * a.w_expert_stride), 0,
+            (int)a.w_expert_stride, 0x00020000);
+        const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint8_t*>(a.w_scales + (size_t)e * a.s_expert_stride), 0, (int)a.s_expert_stride, 0x00020000);
+        u32x4 araw[D];
+        uint32_t sw_cur[2], sw_nxt[2];
+        auto load_a = [&](int slot, int s) {
+            araw[slot] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, lane * 16, (int)(wtile + (uint32_t)s * 1024u), 2 /* nt */);
+        };
+        auto load_scales = [&](uint32_t (&dst)[2], int grp) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                dst[i] = __builtin_amdgcn_raw_buffer_load_b32(s_rsrc, lane * 4, (int)(stile + (uint32_t)(2 * grp + i) * 256u), 0);
+        };
+        load_scales(sw_cur, 0);
+#pragma unroll
+        for (int i = 0; i < D - 1; ++i) load_a(i, i);
+        restage(0);
+        auto stage = [&](auto i_tag, int s, auto more_tag) {
+            constexpr int i = decltype(i_tag)::value;
+            if constexpr (decltype(more_tag)::value) load_a((i + D - 1) % D, s + D - 1);
+            __builtin_amdgcn_sched_barrier(0);  // the load is issued here, seven stages ahead of its use
+            at_stage(s);
+            const float sc = mxfp4_scale_to_f32((sw_cur[i >> 2] >> (8 * (i & 3))) & 0xFFu);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                uint32_t d[4];
+                mxfp4_dword_to_bf16x8(araw[i][j], sc, d);
+                const u32x4 av = {d[0], d[1], d[2], d[3]};
+#pragma unroll
+                for (int t = 0; t < NT; ++t) acc[0][t] = mfma_16x16x32(av, b_frag(j, t), acc[0][t]);
+            }
+            // the stage's products are formed here: the compiler otherwise gathers the (dependent) MFMAs of all stages of
+            // the group behind their conversions and spills the operands
+#pragma unroll
+            for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(acc[0][t]));
+        };
+        const int full = n_stages / D;
+        for (int i = 0; i < full; ++i) {
+            next_phase(D * i);
+            load_scales(sw_nxt, i + 1);
+            const int s = D * i;
+            stage(std::integral_constant<int, 0>{}, s, std::true_type{});
+            stage(std::integral_constant<int, 1>{}, s + 1, std::true_type{});
+            stage(std::integral_constant<int, 2>{}, s + 2, std::true_type{});
+            stage(std::integral_constant<int, 3>{}, s + 3, std::true_type{});
+            stage(std::integral_constant<int, 4>{}, s + 4, std::true_type{});
+            stage(std::integral_constant<int, 5>{}, s + 5, std::true_type{});
+            stage(std::integral_constant<int, 6>{}, s + 6, std::true_type{});
+            stage(std::integral_constant<int, 7>{}, s + 7, std::true_type{});
+            sw_cur[0] = sw_nxt[0];
+            sw_cur[1] = sw_nxt[1];
+        }
+        const int s = D * full, tail = n_stages - s;  // all of the tail's weights are in the ring
+        if (tail > 0) {
+            next_phase(s);
+            auto last = [&](auto u) {
+                if (tail > decltype(u)::value) stage(u, s + decltype(u)::value, std::false_type{});
+            };
+            last(std::integral_constant<int, 0>{});
+            last(std::integral_constant<int, 1>{});
+            last(std::integral_constant<int, 2>{});
+            last(std::integral_constant<int, 3>{});
+            last(std::integral_constant<int, 4>{});
+            last(std::integral_constant<int, 5>{});
+            last(std::integral_constant<int, 6>{});
+        }
+    }
+    stream_epilogue<1, NT, EPI>(a, acc, e, [&](int i) { return bucket[row0 + i]; }, nrows, group, r0, bias_raw);
+}
+
+// Block index -> (i-th expert that has a row, row block).  Experts are counted off in the assignment list itself, so blocks
+// of experts without rows (most of them at one token) are neither launched nor scheduled between the others.
+// grid = min(E, assignments) x row blocks, block = 64 waves, one tile of 16 weight rows per wave.
+template <int FMT, int EPI>
+__global__ __launch_bounds__(64 * kSmallWaves, 4) void expert_small_kernel(ExpertGemmArgs a, int lds_bytes) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    __shared__ uint32_t present[32];
+    __shared__ int counts[8];
+    __shared__ int bucket[kSmallMaxAssign];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int waves = blockDim.x >> 6;
+    const int ordinal = blockIdx.x / a.row_blocks;
+    const int rb = blockIdx.x - ordinal * a.row_blocks;
+    // chunk c of 64 assignments: wave c % waves (a block of four waves takes two chunks each)
+    int ids[kSmallMaxAssign / 64 / 4];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const int s = (p * waves + wave) * 64 + lane;
+        ids[p] = s < a.n_assign ? a.topk_i[s] : -1;
+    }
+    if (threadIdx.x < 32) present[threadIdx.x] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+        if (ids[p] >= 0) atomicOr(&present[ids[p] >> 5], 1u << (ids[p] & 31));
+    __syncthreads();
+    int e;
+    {
+        uint32_t word = lane < 32 ? present[lane] : 0u;
+        uint32_t incl = __popc(word);
+#define MOE_STEP(C, M) incl += dpp_move<C, M>(0u, incl);
+        MOE_DPP_STEPS(MOE_STEP)
+#undef MOE_STEP
+        if (ordinal >= (int)__builtin_amdgcn_readlane(incl, 63)) return;  // block-uniform
+        const int w = __popcll(__ballot((int)incl <= ordinal));  // words whose experts all come before
+        word = __builtin_amdgcn_readlane(word, w);
+        int skip = ordinal - ((int)__builtin_amdgcn_readlane(incl, w) - __popc(word));
+        while (skip-- > 0) word &= word - 1u;
+        e = 32 * w + __builtin_ctz(word);
+    }
+    int n_bucket = 0;
+    {
+        unsigned long long match[2];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            match[p] = __ballot(ids[p] == e);
+            const int c = p * waves + wave;
+            if (lane == 0 && c < 8) counts[c] = __popcll(match[p]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            int base = 0;
+            for (int c = 0; c < 8; ++c) {
+                const int n = __builtin_amdgcn_readfirstlane(counts[c]);
+                if (c < p * waves + wave) base += n;
+                if (p == 0) n_bucket += n;
+            }
+            if (ids[p] == e) bucket[base + __popcll(match[p] & ((1ull << lane) - 1ull))] = (p * waves + wave) * 64 + lane;
+        }
+    }
+    __syncthreads();
+    const int tile = rb * waves + wave;
+    const bool active = tile < a.rows / 16;
+    for (int row0 = 0; row0 < n_bucket; row0 += kSmallRows) {
+        if (row0 > 0) __syncthreads();  // everyone is done with the staged rows
+        const int nrows = min(kSmallRows, n_bucket - row0);
+        if (nrows > 16) small_tile<FMT, 2, EPI>(a, lds, e, bucket, row0, nrows, tile, active, lds_bytes);
+        else small_tile<FMT, 1, EPI>(a, lds, e, bucket, row0, nrows, tile, active, lds_bytes);
+    }
+}
+
+}  // namespace
+
+// Assignments, and buffer descriptors that reach an expert's whole matrix (31-bit byte offsets).
+bool expert_small_fits(int n_assign, int rows, int K, int format) {
+    size_t bytes = 2ull * (size_t)rows * (size_t)K, scales = 0;
+    if (format == FMT_MXFP4) mxfp4_tiled_bytes(rows, K, &bytes, &scales);
+    return n_assign <= kSmallMaxAssign && bytes <= 0x7fffffffull;
+}
+
+int launch_expert_small(const ExpertGemmArgs& a, int epi, hipStream_t stream) {
+    if (!a.topk_i || a.rows % 64 != 0 || a.K % 64 != 0) return MOE_ERR_SHAPE;
+    if (!expert_small_fits(a.n_assign, a.rows, a.K, a.format) || a.assign_div <= 0 || a.assign_div > 8 || a.n_experts > 1024)
+        return MOE_ERR_LIMIT;
+    ExpertGemmArgs b = a;
+    const int items = min(a.n_assign, a.n_experts);
+    const int tiles = a.rows / 16;
+    // half-sized blocks while whole ones would not give every compute unit one
+    const int waves = items * ceil_div(tiles, kSmallWaves) < a.n_cus ? kSmallWaves / 2 : kSmallWaves;
+    b.row_blocks = ceil_div(tiles, waves);
+    // a bucket has at most one row per token; what a smaller batch does not stage leaves room for more blocks
+    const int max_rows = min(kSmallRows, (ceil_div(a.n_assign, a.assign_div) + 3) & ~3);
+    const int n_stages = ceil_div(a.K, kStageElems);
+    const int lds_bytes = (int)min((long long)kSmallLds, (long long)ceil_div(n_stages, kSmallGroup) * kSmallGroup * max_rows * 256);
+    const dim3 grid(items * b.row_blocks), block(64 * waves);
+    auto launch = [&](auto fmt, auto e) {
+        hipLaunchKernelGGL((expert_small_kernel<decltype(fmt)::value, decltype(e)::value>), grid, block, lds_bytes, stream, b,
+                           lds_bytes);
+        return launch_status();
+    };
+    auto by_epi = [&](auto fmt) {
+        if (epi == EPI_SWIGLU_BF16) return launch(fmt, std::integral_constant<int, EPI_SWIGLU_BF16>{});
+        if (epi == EPI_ROWS_F32) return launch(fmt, std::integral_constant<int, EPI_ROWS_F32>{});
+        return (int)MOE_ERR_FORMAT;
+    };
+    if (a.format == FMT_BF16) return by_epi(std::integral_constant<int, FMT_BF16>{});
+    if (a.format == FMT_MXFP4) return by_epi(std::integral_constant<int, FMT_MXFP4>{});
+    return MOE_ERR_FORMAT;
+}
+
+}  // namespace moe

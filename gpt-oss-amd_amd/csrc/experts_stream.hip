@@ -1290,6 +1290,7 @@ int expert_direct_max_assignments() { return kDirectMaxAssign; }
 // in/out, 3 down with fp32 in and atomic scatter.  Token blocks hold at most 64 rows.
 int launch_expert_stream(const ExpertGemmArgs& a, int epi, hipStream_t stream) {
     if (a.rows % 64 != 0 || a.K % 32 != 0) return MOE_ERR_SHAPE;
+    if (a.waves_per_block == 18) return launch_expert_small(a, epi, stream);
     const bool queue = a.work_queue != nullptr;
     if (queue != (epi == EPI_SWIGLU_F32 || epi == EPI_SCATTER)) return MOE_ERR_FORMAT;
     if (a.format == FMT_BF16) {

@@ -99,7 +99,9 @@ struct ExpertGemmArgs {
     int waves_per_block;        // kernel choice of the fused block: 0 / 1 producer-consumer kernel with 10 / 12
                                 // consumer waves (+ 2 producers), 64-token blocks; 16 prefill kernel (4 waves,
                                 // 128-token blocks, two blocks a CU; MXFP4 weights only); 17 tile kernel
-                                // (256-token blocks; bf16 weights only).  Ignored by the work-queue entries.
+                                // (256-token blocks; bf16 weights only); 18 a 16-row tile per wave, buckets of a
+                                // handful of rows.  Ignored by the work-queue entries.
+    int n_cus;                  // compute units to fill (18 only)
 };
 int launch_expert_stream(const ExpertGemmArgs& a, int epi, hipStream_t stream);
 
@@ -107,6 +109,10 @@ int launch_expert_stream(const ExpertGemmArgs& a, int epi, hipStream_t stream);
 bool expert_tile_fits(long long act_rows, int rows, int K);
 int launch_expert_tile_bf16(const ExpertGemmArgs& a, int epi, hipStream_t stream);
 int expert_direct_max_assignments();
+
+// ---- experts_small.hip: a handful of rows per expert (bucketing inside the kernel) ---------------
+bool expert_small_fits(int n_assign, int rows, int K, int format);
+int launch_expert_small(const ExpertGemmArgs& a, int epi, hipStream_t stream);
 
 // ---- experts_fused.hip: both expert GEMMs of a block in one launch (bucketing inside the kernel) --
 struct ExpertFusedArgs {
