@@ -643,7 +643,7 @@ static int block_forward_impl(const moe_block_params* caller, moe_stream_t strea
         rc = launch_router_two_pass(p->t, p->w_router, p->b_router, ws.router_partial, ws.t_bf16, p->topk_v, p->topk_i, T,
                                     H, E, K, 1, stream, timer ? timer->ev[stage++] : nullptr);
         if (rc) return rc;
-    } else if (!strict && router_fused_fits(H)) {
+    } else if (!strict && router_fused_fits(H) && !router_split(T, E)) {
         // one launch, block per token: the exact pass of the two-pass router applied to every expert
         rc = launch_router_fused(p->t, p->w_router, p->b_router, ws.t_bf16, p->router_score, p->topk_v, p->topk_i, T, H,
                                  E, K, 1, stream);
@@ -750,7 +750,8 @@ int moe_block_describe(const moe_block_params* p, char* text, size_t text_bytes)
     const bool strict = (p->flags & MOE_FLAG_ROUTER_STRICT_ORDER) != 0;
     const char* router = (!strict && !p->router_score && router_two_pass(T, E, H))
                              ? "router_screen_kernel + router_refine_kernel"
-                             : (!strict && router_fused_fits(H)) ? "router_fused_kernel"
+                             : (!strict && router_fused_fits(H) && !router_split(T, E))
+                                 ? "router_fused_kernel"
                                                                  : "router_partial_kernel + router_finalize_kernel";
     const bool prefill = use_prefill_kernels(T, H, I, K, E, fmt, p->flags);
     const bool direct = use_direct_bucketing(T, K, E, prefill, p->flags);

@@ -19,6 +19,7 @@ int launch_softmax_rows(float* x, int B, int size, hipStream_t stream);
 // Whole router in one launch (block per token): logits as the exact pass of the two-pass router,
 // top-k, softmax, the bf16 activation copy and, if scores_out is not NULL, the score matrix.
 bool router_fused_fits(int H);
+bool router_split(int T, int E);  // partial + finalize rather than the fused kernel
 int launch_router_fused(const float* x, const uint16_t* w, const uint16_t* bias, uint16_t* x_bf16, float* scores_out,
                         float* topk_v, int* topk_i, int T, int H, int E, int K, int do_softmax, hipStream_t stream);
 // Two-pass router (fp32 screening of all experts, exact scores of the candidates): same top-k and

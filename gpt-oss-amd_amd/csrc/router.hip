@@ -839,9 +839,19 @@ int launch_router_partial(const float* x, const uint16_t* w, double* partial, ui
 }
 
 // ---- two-pass router -----------------------------------------------------------------------------
-// Worth it once the exact pass is throughput bound (three vector instructions per term); small
-// batches are latency bound and keep the single exact pass.
-bool router_two_pass(int T, int E, int H) { return (long long)T * E >= 65536 && H % 32 == 0; }
+// Worth it once the exact pass is throughput bound (three vector instructions per term), or once the fused kernel (a block
+// per token) would need a second round of blocks over the 256 compute units.  Block of tiny experts, us, fused : two-pass:
+// E = 32, 512 tokens 75 : 80, 700 tokens 90 : 87, 1000 tokens 113 : 103, 1500 tokens 136 : 113; E = 96, 256 tokens 80 : 85,
+// 350 tokens 102 : 89; E = 128, 256 tokens 84 : 84, 350 tokens 109 : 90.
+bool router_two_pass(int T, int E, int H) {
+    return H % 32 == 0 && ((long long)T * E >= 65536 || T > (E <= 32 ? 640 : 256));
+}
+
+// Partial sums and finalize in two launches instead of the fused kernel: beyond 32 experts its eight waves score a token's
+// experts in passes of 32, a memory round trip each, while few tokens leave most compute units idle.  The same block, us, fused :
+// two launches: E = 64, 1 token 35 : 31, 128 tokens 63 : 61, 200 tokens 66 : 70; E = 128, 1 token 45 : 33, 33 tokens 65 : 53, 128
+// tokens 79 : 74; E = 1000, 16 tokens 199 : 92.  Up to 32 experts one launch is the faster one (256 tokens 59 : 63).
+bool router_split(int T, int E) { return E > 32 && T <= 128; }
 
 static int screen_tiles(int E) { return E <= 16 ? 1 : E <= 32 ? 2 : 4; }  // 16-expert tiles per wave
 
