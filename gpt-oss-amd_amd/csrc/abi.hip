@@ -274,6 +274,56 @@ int moe_build_work_queue(const int* expert_offsets, int E, int* work_queue, int*
     return launch_build_work_queue(expert_offsets, E, work_queue, work_count, as_stream(stream));
 }
 
+// Compute units of the current device, asked once per device (the kernel choices below count rounds
+// of blocks over them).
+static int device_cu_count() {
+    static std::atomic<int> cached[64];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    int n = cached[dev].load(std::memory_order_relaxed);
+    if (n <= 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+        cached[dev].store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
+
+// Decode-sized buckets (producer/consumer kernel, one block per CU): 10 or 12 consumer waves of
+// 32 rows each.  Blocks run in rounds of one per CU, so the cheaper choice is the one with the
+// smaller rounds x rows-per-block product; more rows per block also re-read the activations less.
+static int pick_stream_kernel(int rows, int tiles, int n_cus) {
+    const int cost10 = ceil_div(ceil_div(rows / 32, 10) * tiles, n_cus) * 10;
+    const int cost12 = ceil_div(ceil_div(rows / 32, 12) * tiles, n_cus) * 12;
+    return cost12 <= cost10 ? 1 : 0;
+}
+// one row block more than necessary when that makes the block count a whole number of rounds
+static int pick_stream_row_blocks(int rows, int kernel, int tiles, int n_cus) {
+    const int n = ceil_div(rows / 32, kernel == 1 ? 12 : 10);
+    return ((n * tiles) % n_cus != 0 && ((n + 1) * tiles) % n_cus == 0) ? n + 1 : n;
+}
+// MXFP4 blocks of one (expert, row block) pair each: a block may cover up to two passes of CONS row units
+// (the second pass starts with its weights already in flight), so fewer, longer blocks pay fewer
+// pipeline fills.  Time of a round of blocks ~ one fill + passes x stages x consumers / 12; all
+// (consumers, row blocks) choices that keep every compute unit busy are priced.
+static void pick_stream_two_pass(int rows, int tiles, int n_cus, int* kernel, int* row_blocks) {
+    const int units = rows / 32;
+    double best = 1e30;
+    for (int k = 0; k < 2; ++k) {
+        const int cons = k == 1 ? 12 : 10;
+        for (int n = ceil_div(units, 2 * cons); n <= ceil_div(units, cons); ++n) {
+            const int per_block = ceil_div(units, n);
+            const int passes = ceil_div(per_block, cons);
+            const int rounds = ceil_div(n * tiles, n_cus);
+            const double cost = rounds * (6.0 + passes * 25.0 * cons / 12.0);
+            if (cost < best - 1e-9) {
+                best = cost;
+                *kernel = k;
+                *row_blocks = n;
+            }
+        }
+    }
+}
+
 // ---- expert GEMMs, reference data flow ---------------------------------------------------------
 static int queue_gemm(int epi, int format, const int* work_queue, int work_start, int work_count,
                       const float* act, void* out, const int* tokens_flat, const float* weights_flat,
@@ -294,7 +344,7 @@ static int queue_gemm(int epi, int format, const int* work_queue, int work_start
     a.work_queue = work_queue;
     a.work_start = work_start;
     a.work_count = work_count;
-    a.max_rows_hint = maxNe < 64 ? 64 : (maxNe > 64 * 1024 ? 64 * 1024 : maxNe);
+    a.max_rows_hint = std::max(1, maxNe);
     a.out = out;
     a.rows = rows;
     a.K = Kdim;
@@ -304,7 +354,19 @@ static int queue_gemm(int epi, int format, const int* work_queue, int work_start
     a.alpha = alpha;
     a.limit = limit;
     a.format = format;
-    a.waves_per_block = 4;
+    a.n_cus = device_cu_count();
+    a.xcd_tiles = 1;
+    // Short entries: a tile of weight rows per wave (experts_small.hip).  The layer's calls with at most n rows an entry, us, that
+    // kernel : producers and consumers: E = 32, bf16, n = 1 92 : 158, 4 176 : 227, 16 294 : 288; MXFP4, 4 92 : 98, 16 124 : 120, 32
+    // 134 : 125; E = 128, bf16, 16 440 : 498, 32 675 : 658; MXFP4, 16 164 : 196.
+    if (maxNe <= 16 && expert_small_fits(0, rows, Kdim, format)) {
+        a.waves_per_block = 18;
+    } else if (format == MOE_WEIGHTS_MXFP4_TILED) {
+        pick_stream_two_pass(rows, work_count, a.n_cus, &a.waves_per_block, &a.row_blocks);
+    } else {
+        a.waves_per_block = pick_stream_kernel(rows, work_count, a.n_cus);
+        a.row_blocks = pick_stream_row_blocks(rows, a.waves_per_block, work_count, a.n_cus);
+    }
     return launch_expert_stream(a, epi, as_stream(stream));
 }
 
@@ -431,20 +493,6 @@ struct moe_stage_timer {
     hipEvent_t ev[MOE_N_STAGES + 1];
 };
 
-// Compute units of the current device, asked once per device (the kernel choices below count rounds
-// of blocks over them).
-static int device_cu_count() {
-    static std::atomic<int> cached[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    int n = cached[dev].load(std::memory_order_relaxed);
-    if (n <= 0) {
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        cached[dev].store(n, std::memory_order_relaxed);
-    }
-    return n;
-}
-
 // Launch parameters of the two expert GEMMs of one block.
 struct ExpertPlan {
     const moe_block_params* p;
@@ -478,42 +526,15 @@ struct ExpertPlan {
         small = use_small_kernels(T, p->hidden_dim, p->intermediate_dim, K, E, p->weight_format, direct, p->flags, n_cus);
         second_map = ws.max_tiles;
     }
-    // Decode-sized buckets (producer/consumer kernel, one block per CU): 10 or 12 consumer waves of
-    // 32 rows each.  Blocks run in rounds of one per CU, so the cheaper choice is the one with the
-    // smaller rounds x rows-per-block product; more rows per block also re-read the activations less.
     int pick_kernel(int rows) const {
         if (prefill) return p->weight_format == MOE_WEIGHTS_BF16 ? 17 : 16;
-        const int cost10 = ceil_div(ceil_div(rows / 32, 10) * est_tiles, n_cus) * 10;
-        const int cost12 = ceil_div(ceil_div(rows / 32, 12) * est_tiles, n_cus) * 12;
-        return cost12 <= cost10 ? 1 : 0;
+        return pick_stream_kernel(rows, est_tiles, n_cus);
     }
-    // one row block more than necessary when that makes the block count a whole number of rounds
     int pick_row_blocks(int rows, int kernel) const {
-        if (prefill) return 0;
-        const int n = ceil_div(rows / 32, kernel == 1 ? 12 : 10);
-        return ((n * est_tiles) % n_cus != 0 && ((n + 1) * est_tiles) % n_cus == 0) ? n + 1 : n;
+        return prefill ? 0 : pick_stream_row_blocks(rows, kernel, est_tiles, n_cus);
     }
-    // MXFP4 with the bucketing inside the kernel: a block may cover up to two passes of CONS row units
-    // (the second pass starts with its weights already in flight), so fewer, longer blocks pay fewer
-    // pipeline fills.  Time of a round of blocks ~ one fill + passes x stages x consumers / 12; all
-    // (consumers, row blocks) choices that keep every compute unit busy are priced.
     void pick_two_pass(int rows, int* kernel, int* row_blocks) const {
-        const int units = rows / 32;
-        double best = 1e30;
-        for (int k = 0; k < 2; ++k) {
-            const int cons = k == 1 ? 12 : 10;
-            for (int n = ceil_div(units, 2 * cons); n <= ceil_div(units, cons); ++n) {
-                const int per_block = ceil_div(units, n);
-                const int passes = ceil_div(per_block, cons);
-                const int rounds = ceil_div(n * est_tiles, n_cus);
-                const double cost = rounds * (6.0 + passes * 25.0 * cons / 12.0);
-                if (cost < best - 1e-9) {
-                    best = cost;
-                    *kernel = k;
-                    *row_blocks = n;
-                }
-            }
-        }
+        pick_stream_two_pass(rows, est_tiles, n_cus, kernel, row_blocks);
     }
     // One launch for both GEMMs: row blocks per expert (n1 gate/up, n2 down, at most the kernel's consumer
     // waves in row units each).  A block's time is its number of items (an item's ticks take about the same

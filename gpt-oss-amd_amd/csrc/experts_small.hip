@@ -28,9 +28,10 @@ constexpr int kSmallGroup = 8;         // a phase (what is staged at once) is a 
 // activations of `per_phase` stages of 128 contraction elements are staged at a time, rows_img (nrows rounded up to four)
 // rows to a stage, 256 bytes each, chunk c of row r at position ws_pos(c) ^ (r % 16).  All waves of the block call this
 // with the same bucket; those without a tile (active false) only stage.
-template <int FMT, int NT, int EPI>
-MOE_DEVICE void small_tile(const ExpertGemmArgs& a, uint8_t* lds, int e, const int* bucket, int row0, int nrows, int tile,
-                           bool active, int lds_bytes) {
+// ACT_F32: the rows are fp32 (rows slot_of_row(i) of a.act_f32), rounded to bf16 while they are staged.
+template <int FMT, int NT, int EPI, bool ACT_F32, class SlotFn>
+MOE_DEVICE void small_tile(const ExpertGemmArgs& a, uint8_t* lds, int e, SlotFn slot_of_row, int nrows, int tile, bool active,
+                           int lds_bytes) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int waves = blockDim.x >> 6;
@@ -50,19 +51,46 @@ MOE_DEVICE void small_tile(const ExpertGemmArgs& a, uint8_t* lds, int e, const i
         const int n_instr = min(per_phase, n_stages - s0) * quads;
         int st = wave / quads, rq = wave - st * quads;  // wave-uniform
         const int dst_step = waves / quads, dq_step = waves - dst_step * quads;
-        for (int n = wave; n < n_instr; n += waves) {
-            const int r = rq * 4 + g;
-            const int s = bucket[row0 + min(r, nrows - 1)];
-            const int src = a.gather ? (int)(((float)s + 0.5f) * inv_div) : s;
-            const int k = (s0 + st) * kStageElems + 8 * ws_chunk_at<FMT>(q ^ (r & 15));
-            // a position past the row re-reads its start: its weights count as zero
-            dma16(reinterpret_cast<const uint8_t*>(a.act + (size_t)src * K + (k < K ? k : 0)),
-                  lds + (size_t)n * 1024);
+        auto next = [&]() {
             st += dst_step;
             rq += dq_step;
             if (rq >= quads) {
                 rq -= quads;
                 ++st;
+            }
+        };
+        // the lane's row and contraction element; a position past the row re-reads its start: its weights count as zero
+        auto slot = [&]() { return slot_of_row(min(rq * 4 + g, nrows - 1)); };
+        auto elem = [&]() {
+            const int k = (s0 + st) * kStageElems + 8 * ws_chunk_at<FMT>(q ^ ((rq * 4 + g) & 15));
+            return k < K ? k : 0;
+        };
+        if constexpr (ACT_F32) {
+            constexpr int B = 4;  // loads of a batch are in flight together
+            for (int n = wave; n < n_instr; n += B * waves) {
+                float4 x[B][2];
+#pragma unroll
+                for (int i = 0; i < B; ++i) {
+                    if (n + i * waves < n_instr) {  // wave-uniform
+                        const float4* src = reinterpret_cast<const float4*>(a.act_f32 + (size_t)slot() * K + elem());
+                        x[i][0] = src[0];
+                        x[i][1] = src[1];
+                    }
+                    next();
+                }
+#pragma unroll
+                for (int i = 0; i < B; ++i)
+                    if (n + i * waves < n_instr)
+                        *reinterpret_cast<u32x4*>(lds + (size_t)(n + i * waves) * 1024 + lane * 16) =
+                            u32x4{pack_bf16x2(x[i][0].x, x[i][0].y), pack_bf16x2(x[i][0].z, x[i][0].w),
+                                  pack_bf16x2(x[i][1].x, x[i][1].y), pack_bf16x2(x[i][1].z, x[i][1].w)};
+            }
+        } else {
+            for (int n = wave; n < n_instr; n += waves) {
+                const int s = slot();
+                const int src = a.gather ? (int)(((float)s + 0.5f) * inv_div) : s;
+                dma16(reinterpret_cast<const uint8_t*>(a.act + (size_t)src * K + elem()), lds + (size_t)n * 1024);
+                next();
             }
         }
     };
@@ -237,14 +265,29 @@ MOE_DEVICE void small_tile(const ExpertGemmArgs& a, uint8_t* lds, int e, const i
             last(std::integral_constant<int, 6>{});
         }
     }
-    stream_epilogue<1, NT, EPI>(a, acc, e, [&](int i) { return bucket[row0 + i]; }, nrows, group, r0, bias_raw);
+    stream_epilogue<1, NT, EPI>(a, acc, e, slot_of_row, nrows, group, r0, bias_raw);
+}
+
+// All rows of a bucket, max_rows (a multiple of four that the LDS holds eight stages of) to a pass over the weights.
+template <int FMT, int EPI, bool ACT_F32, class SlotFn>
+MOE_DEVICE void small_rows(const ExpertGemmArgs& a, uint8_t* lds, int e, SlotFn slot_of_row, int n_rows, int rb, int max_rows,
+                           int lds_bytes) {
+    const int tile = rb * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool active = tile < a.rows / 16;
+    for (int row0 = 0; row0 < n_rows; row0 += max_rows) {
+        if (row0 > 0) __syncthreads();  // everyone is done with the staged rows
+        const int nrows = min(max_rows, n_rows - row0);
+        auto slot = [&](int i) { return slot_of_row(row0 + i); };
+        if (nrows > 16) small_tile<FMT, 2, EPI, ACT_F32>(a, lds, e, slot, nrows, tile, active, lds_bytes);
+        else small_tile<FMT, 1, EPI, ACT_F32>(a, lds, e, slot, nrows, tile, active, lds_bytes);
+    }
 }
 
 // Block index -> (i-th expert that has a row, row block).  Experts are counted off in the assignment list itself, so blocks
 // of experts without rows (most of them at one token) are neither launched nor scheduled between the others.
 // grid = min(E, assignments) x row blocks, block = 64 waves, one tile of 16 weight rows per wave.
 template <int FMT, int EPI>
-__global__ __launch_bounds__(64 * kSmallWaves, 4) void expert_small_kernel(ExpertGemmArgs a, int lds_bytes) {
+__global__ __launch_bounds__(64 * kSmallWaves, 4) void expert_small_kernel(ExpertGemmArgs a, int max_rows, int lds_bytes) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ uint32_t present[32];
     __shared__ int counts[8];
@@ -303,14 +346,19 @@ __global__ __launch_bounds__(64 * kSmallWaves, 4) void expert_small_kernel(Exper
         }
     }
     __syncthreads();
-    const int tile = rb * waves + wave;
-    const bool active = tile < a.rows / 16;
-    for (int row0 = 0; row0 < n_bucket; row0 += kSmallRows) {
-        if (row0 > 0) __syncthreads();  // everyone is done with the staged rows
-        const int nrows = min(kSmallRows, n_bucket - row0);
-        if (nrows > 16) small_tile<FMT, 2, EPI>(a, lds, e, bucket, row0, nrows, tile, active, lds_bytes);
-        else small_tile<FMT, 1, EPI>(a, lds, e, bucket, row0, nrows, tile, active, lds_bytes);
-    }
+    small_rows<FMT, EPI, false>(a, lds, e, [&](int i) { return bucket[i]; }, n_bucket, rb, max_rows, lds_bytes);
+}
+
+// The same for the entries that keep the reference's data flow: queue entries (expert, row_offset, row_count), fp32 rows by
+// slot.  grid = entries x row blocks.
+template <int FMT, int EPI>
+__global__ __launch_bounds__(64 * kSmallWaves, 4) void expert_small_queue_kernel(ExpertGemmArgs a, int max_rows, int lds_bytes) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int item = blockIdx.x / a.row_blocks;
+    const int rb = blockIdx.x - item * a.row_blocks;
+    const int* entry = a.work_queue + 3 * (size_t)(a.work_start + item);
+    const int off = entry[1];
+    small_rows<FMT, EPI, true>(a, lds, entry[0], [&](int i) { return off + i; }, entry[2], rb, max_rows, lds_bytes);
 }
 
 }  // namespace
@@ -323,32 +371,41 @@ bool expert_small_fits(int n_assign, int rows, int K, int format) {
 }
 
 int launch_expert_small(const ExpertGemmArgs& a, int epi, hipStream_t stream) {
-    if (!a.topk_i || a.rows % 64 != 0 || a.K % 64 != 0) return MOE_ERR_SHAPE;
-    if (!expert_small_fits(a.n_assign, a.rows, a.K, a.format) || a.assign_div <= 0 || a.assign_div > 8 || a.n_experts > 1024)
-        return MOE_ERR_LIMIT;
+    const bool queue = a.work_queue != nullptr;
+    if (a.rows % 64 != 0 || a.K % (a.format == FMT_BF16 ? 64 : 32) != 0 || (!queue && !a.topk_i)) return MOE_ERR_SHAPE;
+    if (!expert_small_fits(queue ? 0 : a.n_assign, a.rows, a.K, a.format)) return MOE_ERR_LIMIT;
+    if (!queue && (a.assign_div <= 0 || a.assign_div > 8 || a.n_experts > 1024)) return MOE_ERR_LIMIT;
     ExpertGemmArgs b = a;
-    const int items = min(a.n_assign, a.n_experts);
+    const int items = queue ? a.work_count : min(a.n_assign, a.n_experts);
+    if (items <= 0) return MOE_OK;
     const int tiles = a.rows / 16;
     // half-sized blocks while whole ones would not give every compute unit one
     const int waves = items * ceil_div(tiles, kSmallWaves) < a.n_cus ? kSmallWaves / 2 : kSmallWaves;
     b.row_blocks = ceil_div(tiles, waves);
-    // a bucket has at most one row per token; what a smaller batch does not stage leaves room for more blocks
-    const int max_rows = min(kSmallRows, (ceil_div(a.n_assign, a.assign_div) + 3) & ~3);
+    // a bucket has at most one row per token (an entry as many as its caller says, or more passes); what smaller ones do not
+    // stage leaves room for more blocks
+    const int rows = queue ? a.max_rows_hint : ceil_div(a.n_assign, a.assign_div);
+    const int max_rows = min(kSmallRows, (max(rows, 1) + 3) & ~3);
     const int n_stages = ceil_div(a.K, kStageElems);
     const int lds_bytes = (int)min((long long)kSmallLds, (long long)ceil_div(n_stages, kSmallGroup) * kSmallGroup * max_rows * 256);
-    const dim3 grid(items * b.row_blocks), block(64 * waves);
-    auto launch = [&](auto fmt, auto e) {
-        hipLaunchKernelGGL((expert_small_kernel<decltype(fmt)::value, decltype(e)::value>), grid, block, lds_bytes, stream, b,
-                           lds_bytes);
-        return launch_status();
-    };
-    auto by_epi = [&](auto fmt) {
-        if (epi == EPI_SWIGLU_BF16) return launch(fmt, std::integral_constant<int, EPI_SWIGLU_BF16>{});
-        if (epi == EPI_ROWS_F32) return launch(fmt, std::integral_constant<int, EPI_ROWS_F32>{});
-        return (int)MOE_ERR_FORMAT;
-    };
-    if (a.format == FMT_BF16) return by_epi(std::integral_constant<int, FMT_BF16>{});
-    if (a.format == FMT_MXFP4) return by_epi(std::integral_constant<int, FMT_MXFP4>{});
+    const dim3 grid((unsigned)items * b.row_blocks), block(64 * waves);
+#define MOE_SMALL(KERNEL, FMT, EPI)                                                                           \
+    if (a.format == FMT && epi == EPI) {                                                                      \
+        hipLaunchKernelGGL((KERNEL<FMT, EPI>), grid, block, lds_bytes, stream, b, max_rows, lds_bytes);       \
+        return launch_status();                                                                               \
+    }
+    if (queue) {
+        MOE_SMALL(expert_small_queue_kernel, FMT_BF16, EPI_SWIGLU_F32)
+        MOE_SMALL(expert_small_queue_kernel, FMT_BF16, EPI_SCATTER)
+        MOE_SMALL(expert_small_queue_kernel, FMT_MXFP4, EPI_SWIGLU_F32)
+        MOE_SMALL(expert_small_queue_kernel, FMT_MXFP4, EPI_SCATTER)
+    } else {
+        MOE_SMALL(expert_small_kernel, FMT_BF16, EPI_SWIGLU_BF16)
+        MOE_SMALL(expert_small_kernel, FMT_BF16, EPI_ROWS_F32)
+        MOE_SMALL(expert_small_kernel, FMT_MXFP4, EPI_SWIGLU_BF16)
+        MOE_SMALL(expert_small_kernel, FMT_MXFP4, EPI_ROWS_F32)
+    }
+#undef MOE_SMALL
     return MOE_ERR_FORMAT;
 }
 

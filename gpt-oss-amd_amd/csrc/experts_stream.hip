@@ -13,17 +13,15 @@
 // The contraction index is a dummy index, so lanes are free to pick which k each of their eight
 // operand elements stands for as long as A and B agree.  Inside a stage, k-step j (0..3) and lane
 // group g = lane/16 take
-//   bf16, uniform-wave kernel    : elements 32j + 8g .. +8
-//   bf16, producer/consumer      : elements 64(j/2) + 16g + 8(j%2) .. +8  (a lane's two loads of a
-//                                  pair of steps are adjacent: whole 128-byte lines per row)
-//   MXFP4                        : elements 32g + 8j .. +8  (lane group g owns MX block g of the
-//                                  stage: one 128-bit load + one scale byte per row tile and stage,
-//                                  dequantised in registers to four A operands)
+//   bf16  : elements 64(j/2) + 16g + 8(j%2) .. +8  (a lane's two loads of a pair of steps are adjacent: whole
+//           128-byte lines per row)
+//   MXFP4 : elements 32g + 8j .. +8  (lane group g owns MX block g of the stage: one 128-bit load + one scale byte
+//           per row tile and stage, dequantised in registers to four A operands)
 //
-// Kernels: expert_stream_ws_kernel (decode-sized buckets, producer and consumer waves) and
+// Kernels: expert_stream_direct_kernel and expert_stream_ws_kernel (decode-sized buckets, producer and consumer waves) and
 // expert_prefill_kernel (128-token blocks, 64 x 128 tile per wave) are what the fused block uses;
-// expert_stream_queue_kernel (uniform waves, fp32 activations staged through registers) serves the
-// entries that keep the reference's signatures and work queue.
+// expert_stream_queue_ws_kernel (the same consumers, producers that round fp32 rows) serves the entries that keep the
+// reference's signatures and work queue.
 #include <type_traits>
 
 #include "expert_tiles.h"
@@ -31,243 +29,6 @@
 namespace moe {
 
 namespace {
-
-
-MOE_DEVICE u32x4 pack_f32x8_to_bf16x8(const float4& lo, const float4& hi) {
-    return u32x4{pack_bf16x2(lo.x, lo.y), pack_bf16x2(lo.z, lo.w), pack_bf16x2(hi.x, hi.y), pack_bf16x2(hi.z, hi.w)};
-}
-
-
-// One (row unit, token block) of one expert.  ACT_F32: activations are fp32 rows indexed by slot
-// (the reference's x_by_expert / gate_by_expert buffers) and are rounded to bf16 while staged.
-// `active` is false for the waves of a ragged last block that own no rows: they still stage
-// activations and take part in every barrier.
-template <int FMT, int R, int NT, int EPI, bool ACT_F32, int WAVES>
-MOE_DEVICE void stream_body(const ExpertGemmArgs& a, uint8_t* lds, int e, int row0, int nrows, int unit,
-                            bool active) {
-    static_assert(WAVES == 4 || WAVES == 8, "a block has 4 or 8 waves");
-    constexpr int kStagers = WAVES / 4;                       // waves that stage the same k-step
-    constexpr int TS = (NT + kStagers - 1) / kStagers;        // token tiles staged per wave
-    constexpr int kUnitsPerGroup = 4 / R;
-    constexpr int NTMAX = kNTMax;
-    constexpr int kStageBytes = kStageSteps * NTMAX * 1024;  // one LDS stage buffer
-    static_assert(NT <= NTMAX && TS * kStagers <= NTMAX, "token tiles must fit the LDS stage");
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int q = lane & 15;
-    const int g = lane >> 4;
-    const int group = unit / kUnitsPerGroup;
-    const int r0 = (unit % kUnitsPerGroup) * R;
-    const int K = a.K;
-    const int n_stages = ceil_div(K, kStageElems);
-
-    // ---- A operand addressing ----
-    const uint8_t* a_ptr[R];
-    const uint8_t* s_ptr[R];
-    if constexpr (FMT == FMT_BF16) {
-        const uint16_t* wbase = reinterpret_cast<const uint16_t*>(a.w) + (size_t)e * a.w_expert_stride;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int row = active ? group * 64 + tile_row_in_group(r0 + r, q) : 0;
-            a_ptr[r] = reinterpret_cast<const uint8_t*>(wbase + (size_t)row * K + 8 * g);
-            s_ptr[r] = nullptr;
-        }
-    } else {
-        const int G = K / 32;
-        const size_t tile_bytes = (size_t)G * 256;
-        const size_t stile_bytes = (size_t)ceil_div(ceil_div(G, 4), 4) * 256;
-        const uint8_t* wbase = reinterpret_cast<const uint8_t*>(a.w) + (size_t)e * a.w_expert_stride;
-        const uint8_t* sbase = a.w_scales + (size_t)e * a.s_expert_stride;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const size_t tile = active ? (size_t)group * 4 + (r0 + r) : 0;
-            a_ptr[r] = wbase + tile * tile_bytes + (size_t)lane * 16;
-            s_ptr[r] = sbase + tile * stile_bytes + (size_t)lane * 4;
-        }
-    }
-
-    // ---- B staging: wave w stages k-step w%4 of every stage, for token tiles w/4, w/4 + WAVES/4, ...
-    // (a tile index past NT-1 stages a clamped copy into an LDS slot nobody reads) ----
-    const int step_w = wave & 3;
-    const int half_w = wave >> 2;
-    // element offset inside an activation row of this lane's eight elements at stage 0
-    const int k_lane = (FMT == FMT_BF16) ? (32 * step_w + 8 * g) : (32 * g + 8 * step_w);
-    const uint8_t* b_src[TS];
-#pragma unroll
-    for (int i = 0; i < TS; ++i) {
-        const int t = half_w + kStagers * i;
-        const int idx = min(t * 16 + q, nrows - 1);
-        if constexpr (ACT_F32) {
-            b_src[i] = reinterpret_cast<const uint8_t*>(a.act_f32 + (size_t)(row0 + idx) * K + k_lane);
-        } else {
-            const int src = a.gather ? a.tokens_flat[row0 + idx] : row0 + idx;
-            b_src[i] = reinterpret_cast<const uint8_t*>(a.act + (size_t)src * K + k_lane);
-        }
-    }
-    uint8_t* const lds_wr = lds + (size_t)(step_w * NTMAX + half_w) * 1024 + (size_t)lane * 16;
-    const uint8_t* const lds_rd = lds + (size_t)lane * 16;
-
-    // Everything inside the stage loops is branch-free (clamped addresses + selects instead of
-    // guards), so the compiler can count outstanding loads exactly and keep the prefetches in flight.
-    u32x4 stg[TS];
-    auto stage_load = [&](int s) {
-        // s may point past the last stage (prefetch of a stage that does not exist): stage zeros
-        const bool live = (s * kStageElems + k_lane) < K;  // false in a ragged or non-existent stage
-        const size_t off = live ? (size_t)s * kStageElems : 0;
-#pragma unroll
-        for (int t = 0; t < TS; ++t) {
-            u32x4 v;
-            if constexpr (ACT_F32) {
-                const float4* p = reinterpret_cast<const float4*>(b_src[t] + off * 4 - (live ? 0 : k_lane * 4));
-                v = pack_f32x8_to_bf16x8(p[0], p[1]);
-            } else {
-                v = *reinterpret_cast<const u32x4*>(b_src[t] + off * 2 - (live ? 0 : k_lane * 2));
-            }
-            stg[t] = live ? v : u32x4{0u, 0u, 0u, 0u};
-        }
-    };
-    auto stage_store = [&](int buf) {
-#pragma unroll
-        for (int t = 0; t < TS; ++t)
-            *reinterpret_cast<u32x4*>(lds_wr + (size_t)buf * kStageBytes + t * kStagers * 1024) = stg[t];
-    };
-    auto b_frag = [&](int buf, int j, int t) {
-        return *reinterpret_cast<const u32x4*>(lds_rd + (size_t)buf * kStageBytes + (j * NTMAX + t) * 1024);
-    };
-
-    if (!active) {
-        // no rows to compute: keep the block's staging and barrier sequence going
-        const int n_iter = (FMT == FMT_BF16) ? n_stages : ceil_div(n_stages, 4) * 4;
-        stage_load(0);
-        stage_store(0);
-        __syncthreads();
-        for (int s = 0; s < n_iter; ++s) {
-            stage_load(s + 1);
-            stage_store((s & 1) ^ 1);
-            __syncthreads();
-        }
-        return;
-    }
-
-    f32x4 acc[R][NT];
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    if constexpr (FMT == FMT_BF16) {
-        // A ring of four k-steps, loads issued three steps ahead of their use
-        const int n_steps = K / 32;
-        const int n_full = K / kStageElems;  // stages with all four k-steps
-        u32x4 ar[4][R];
-        auto load_a = [&](int slot, int n) {
-            const size_t off = (size_t)min(n, n_steps - 1) * 64;  // past the end: reload the last step
-#pragma unroll
-            for (int r = 0; r < R; ++r) ar[slot][r] = *reinterpret_cast<const u32x4*>(a_ptr[r] + off);
-        };
-        auto step = [&](int buf, int j) {
-#pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                const u32x4 b = b_frag(buf, j, t);
-#pragma unroll
-                for (int r = 0; r < R; ++r) acc[r][t] = mfma_16x16x32(ar[j][r], b, acc[r][t]);
-            }
-        };
-        stage_load(0);
-        load_a(0, 0);
-        load_a(1, 1);
-        load_a(2, 2);
-        stage_store(0);
-        __syncthreads();
-        for (int s = 0; s < n_full; ++s) {
-            const int buf = s & 1;
-            stage_load(s + 1);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                load_a((j + 3) & 3, 4 * s + j + 3);
-                step(buf, j);
-            }
-            stage_store(buf ^ 1);
-            __syncthreads();
-        }
-        if (n_full < n_stages) {  // ragged last stage: K % 128 in {32, 64, 96}
-            const int buf = n_full & 1;
-            const int left = n_steps - 4 * n_full;
-            step(buf, 0);
-            if (left > 1) step(buf, 1);
-            if (left > 2) step(buf, 2);
-            __syncthreads();
-        }
-    } else {
-        // A ring of D stages (one 128-bit load per row tile and stage), loads issued D-1 stages ahead
-        // of their use; one scale word per row tile covers four stages and is fetched one quad
-        // ahead.  The stage count is padded to a multiple of four with all-zero stages (zero
-        // weights against zero activations) to keep the loop uniform.
-        constexpr int D = (R >= 4) ? 2 : 4;
-        const int rem_groups = (K / 32) & 3;  // MX blocks in a ragged last stage (0 = none)
-        const int n_quads = ceil_div(n_stages, 4);
-        u32x4 araw[D][R];
-        uint32_t sw_cur[R], sw_nxt[R];
-        auto load_a = [&](int slot, int s) {
-            const bool live = s < n_stages && !(rem_groups != 0 && s == n_stages - 1 && g >= rem_groups);
-            // a dead lane group re-reads a block that exists and drops it
-            const size_t off = live ? (size_t)s * 1024 : 0;
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const u32x4 v = *reinterpret_cast<const u32x4*>(a_ptr[r] + off);
-                araw[slot][r] = live ? v : u32x4{0u, 0u, 0u, 0u};
-            }
-        };
-        auto load_scales = [&](uint32_t (&dst)[R], int quad) {
-            const size_t off = (size_t)min(quad, n_quads - 1) * 256;
-#pragma unroll
-            for (int r = 0; r < R; ++r) dst[r] = *reinterpret_cast<const uint32_t*>(s_ptr[r] + off);
-        };
-        auto do_stage = [&](int slot, int qpos, int s) {
-            const int buf = s & 1;
-            stage_load(s + 1);
-            load_a((slot + D - 1) % D, s + D - 1);
-            float sc[R];
-#pragma unroll
-            for (int r = 0; r < R; ++r) sc[r] = mxfp4_scale_to_f32((sw_cur[r] >> (8 * qpos)) & 0xFFu);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                u32x4 av[R];
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    uint32_t d[4];
-                    mxfp4_dword_to_bf16x8(araw[slot][r][j], sc[r], d);
-                    av[r] = u32x4{d[0], d[1], d[2], d[3]};
-                }
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    const u32x4 b = b_frag(buf, j, t);
-#pragma unroll
-                    for (int r = 0; r < R; ++r) acc[r][t] = mfma_16x16x32(av[r], b, acc[r][t]);
-                }
-            }
-            stage_store(buf ^ 1);
-            __syncthreads();
-        };
-        stage_load(0);
-        load_scales(sw_cur, 0);
-#pragma unroll
-        for (int i = 0; i < D - 1; ++i) load_a(i, i);
-        stage_store(0);
-        __syncthreads();
-        for (int qd = 0; qd < n_quads; ++qd) {
-            load_scales(sw_nxt, qd + 1);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) do_stage(i % D, i, 4 * qd + i);
-#pragma unroll
-            for (int r = 0; r < R; ++r) sw_cur[r] = sw_nxt[r];
-        }
-    }
-
-    uint2 bias_raw[R];
-    load_bias<R>(a, e, group, r0, bias_raw);
-    stream_epilogue<R, NT, EPI>(a, acc, e, [&](int i) { return row0 + i; }, nrows, group, r0, bias_raw);
-}
 
 // ---------------------------------------------------------------------------------------------
 // Producer/consumer variant used by the fused block: a block has CONS consumer waves (R = 2 row
@@ -365,6 +126,60 @@ MOE_DEVICE void ws_producer(const ExpertGemmArgs& a, uint8_t* lds, RowFn act_row
         __builtin_amdgcn_s_barrier();
     }
     wait_vmcnt<0>();  // nothing may still be writing this block's LDS when the wave ends
+}
+
+// The producer for fp32 activations (the entries that keep the reference's data flow): rows first_row .. first_row + nrows of
+// a.act_f32, rounded to bf16 on their way into the same LDS image.  An instruction takes two rows of 512 contiguous bytes; the
+// loads of a stage are issued one stage before it is written, i.e. four before it is read.
+template <int FMT, int NT, int PROD>
+MOE_DEVICE void ws_producer_f32(const ExpertGemmArgs& a, uint8_t* lds, int first_row, int nrows, int p, int passes) {
+    static_assert(PROD == 4, "eight rows of a token tile per step of the loops below");
+    constexpr int Q = 2 * NT;  // loads per stage of this wave
+    const int lane = threadIdx.x & 63;
+    const int col = lane & 31;  // float4 of the row's 128 elements
+    const int K = a.K;
+    const int n_stages = ceil_div(K, kStageElems);
+    const uint8_t* const base = reinterpret_cast<const uint8_t*>(a.act_f32 + (size_t)first_row * K);
+    const int r0 = 2 * p + (lane >> 5);  // this lane's rows are r0, r0 + 8, ..
+    uint32_t src[Q];
+#pragma unroll
+    for (int i = 0; i < Q; ++i)  // places past the bucket's end hold its last row, never stored
+        src[i] = ((uint32_t)min(r0 + 8 * i, nrows - 1) * (uint32_t)K + 4u * (uint32_t)col) * 4u;
+    uint8_t* const dst = lds + r0 * 256 + ((ws_pos<FMT>(col >> 1) ^ r0) << 4) + (col & 1) * 8;
+    const int swap = (ws_pos<FMT>(col >> 1) ^ r0) & 8 ? -128 : 128;  // row r0 + 8 has bit 3 of the position flipped
+    float4 v[Q];
+    auto load = [&](int st) {
+        // a position past the row re-reads its start
+        const uint32_t off = st * kStageElems + 4 * col < K ? (uint32_t)st * (kStageElems * 4u) : 0u - 16u * (uint32_t)col;
+#pragma unroll
+        for (int i = 0; i < Q; ++i) v[i] = *reinterpret_cast<const float4*>(base + (src[i] + off));
+    };
+    auto store = [&](int gs) {
+        uint8_t* at[2];
+        at[0] = dst + (size_t)(gs & (kWsRing - 1)) * kLdsStageBytes;
+        at[1] = at[0] + 2048 + swap;
+#pragma unroll
+        for (int i = 0; i < Q; ++i)
+            *reinterpret_cast<u32x2*>(at[i & 1] + (i >> 1) * 4096) =
+                u32x2{pack_bf16x2(v[i].x, v[i].y), pack_bf16x2(v[i].z, v[i].w)};
+    };
+    int st = 0;  // stage (inside a pass) loaded next
+    auto next_stage = [&]() { st = (st + 1 == n_stages) ? 0 : st + 1; };
+    load(st);
+    next_stage();
+    for (int gs = 0; gs < 3; ++gs) {
+        store(gs);
+        load(st);
+        next_stage();
+    }
+    __syncthreads();  // stages 0 .. 2 are written
+    const int total = passes * n_stages;
+    for (int i = 0; i < total; ++i) {
+        store(i + 3);  // past the last stage of the last pass: a re-read nobody consumes
+        load(st);
+        next_stage();
+        __syncthreads();
+    }
 }
 
 // slot_of_row(i): output row of bucket row i.  PRE: one more barrier comes first, right after the
@@ -804,8 +619,8 @@ MOE_DEVICE void ws_consume_tiles(const ExpertGemmArgs& a, const uint8_t* lds, in
 // One token block: the producer or consumer role of this wave, for the block's token-tile count.
 // u0, u1: the block's row units [u0, u1), walked in passes of CONS units; with TILES its row tiles [u0, u1)
 // (one pass, see ws_consume_tiles).
-template <int FMT, int EPI, int CONS, int PROD, bool PRE = false, bool TWO = false, bool TILES = false, class RowFn,
-          class SlotFn>
+template <int FMT, int EPI, int CONS, int PROD, bool PRE = false, bool TWO = false, bool TILES = false, bool ACT_F32 = false,
+          class RowFn, class SlotFn>
 MOE_DEVICE void ws_token_block(const ExpertGemmArgs& a, uint8_t* lds, int wave, int u0, int u1, int e, RowFn act_row,
                                SlotFn slot_of_row, int nrows) {
     const int nt = (nrows + 15) >> 4;  // block-uniform
@@ -813,7 +628,13 @@ MOE_DEVICE void ws_token_block(const ExpertGemmArgs& a, uint8_t* lds, int wave, 
     if (wave >= CONS) {
         const int p = wave - CONS;
         if constexpr (PRE) __syncthreads();  // no direct-to-LDS load is in flight yet
-        if (nt == 4) ws_producer<FMT, 4, PROD>(a, lds, act_row, nrows, p, passes);
+        if constexpr (ACT_F32) {
+            const int r0 = act_row(0);
+            if (nt == 4) ws_producer_f32<FMT, 4, PROD>(a, lds, r0, nrows, p, passes);
+            else if (nt == 3) ws_producer_f32<FMT, 3, PROD>(a, lds, r0, nrows, p, passes);
+            else if (nt == 2) ws_producer_f32<FMT, 2, PROD>(a, lds, r0, nrows, p, passes);
+            else ws_producer_f32<FMT, 1, PROD>(a, lds, r0, nrows, p, passes);
+        } else if (nt == 4) ws_producer<FMT, 4, PROD>(a, lds, act_row, nrows, p, passes);
         else if (nt == 3) ws_producer<FMT, 3, PROD>(a, lds, act_row, nrows, p, passes);
         else if (nt == 2) ws_producer<FMT, 2, PROD>(a, lds, act_row, nrows, p, passes);
         else ws_producer<FMT, 1, PROD>(a, lds, act_row, nrows, p, passes);
@@ -980,34 +801,40 @@ __global__ __launch_bounds__((CONS + PROD) * 64, (CONS + PROD > 12) ? 4 : 3) voi
     }
 }
 
-template <int FMT, int R, int EPI, bool ACT_F32, int WAVES>
-MOE_DEVICE void stream_dispatch(const ExpertGemmArgs& a, uint8_t* lds, int e, int row0, int nrows, int unit,
-                                bool active) {
-    const int nt = (nrows + 15) >> 4;  // block-uniform
-    if (nt == 4) {
-        stream_body<FMT, R, 4, EPI, ACT_F32, WAVES>(a, lds, e, row0, nrows, unit, active);
-    } else if (nt == 3) {
-        stream_body<FMT, R, 3, EPI, ACT_F32, WAVES>(a, lds, e, row0, nrows, unit, active);
-    } else if (nt == 2) {
-        stream_body<FMT, R, 2, EPI, ACT_F32, WAVES>(a, lds, e, row0, nrows, unit, active);
-    } else if (nt == 1) {
-        stream_body<FMT, R, 1, EPI, ACT_F32, WAVES>(a, lds, e, row0, nrows, unit, active);
-    }
-}
-
-// Token blocks from a queue of (expert, row_offset, row_count) triples (entry format of
-// src/hip/scheduler.hip:163-166).  grid = (ceil(row units / 4), token blocks per entry, entries).
-template <int FMT, int R, int EPI>
-__global__ __launch_bounds__(256) void expert_stream_queue_kernel(ExpertGemmArgs a) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kLdsStageBytes];
+// ---------------------------------------------------------------------------------------------
+// The entries that keep the reference's data flow (work queue of (expert, row_offset, row_count) triples, entry format of
+// src/hip/scheduler.hip:163-166; fp32 rows by slot in, fp32 rows or an atomic scatter out) on the same main loop.  Bound by the
+// weights like the kernels above.  Block (item, rb) takes the item's token blocks blockIdx.y, + gridDim.y, ...; block 0 is the
+// remainder (see expert_stream_direct_kernel).
+// grid = (row blocks x queue entries, padded to a multiple of 8 entries; token-block shares), block = 64 (CONS + PROD).
+// ---------------------------------------------------------------------------------------------
+template <int FMT, int EPI, int CONS, int PROD, bool TWO>
+__global__ __launch_bounds__((CONS + PROD) * 64, (CONS + PROD > 12) ? 4 : 3) void expert_stream_queue_ws_kernel(ExpertGemmArgs a) {
+    __shared__ __attribute__((aligned(16))) uint8_t lds[kWsRing * kLdsStageBytes];
+    int item, rb;
+    ws_block_coords(a, item, rb);
+    if (item >= a.work_count) return;  // block-uniform
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int unit = blockIdx.x * 4 + wave;
-    const bool active = unit < (a.rows / 64) * (4 / R);
-    const int* entry = a.work_queue + 3 * (a.work_start + blockIdx.z);
+    const int* entry = a.work_queue + 3 * (size_t)(a.work_start + item);
     const int e = entry[0], off = entry[1], n = entry[2];
-    for (int tb = blockIdx.y; tb * 64 < n; tb += gridDim.y) {
-        stream_dispatch<FMT, R, EPI, true, 4>(a, lds, e, off + tb * 64, min(64, n - tb * 64), unit, active);
-        __syncthreads();  // the next token block restages both LDS buffers
+    const int tb0 = blockIdx.y;
+    if (tb0 * 64 >= n) return;  // block-uniform; also an empty entry
+    constexpr bool TILES = !TWO && FMT == FMT_BF16;
+    int u0, u1;
+    if constexpr (TILES) ws_row_tiles<CONS>(a, rb, u0, u1);
+    else ws_row_units(a, rb, u0, u1);
+    const int passes = TWO ? min(2, max(1, ceil_div(u1 - u0, CONS))) : 1;
+    const int first = n - ((n - 1) & ~63);
+    if (tb0 == 0) {
+        auto row = [&](int i) { return off + i; };
+        ws_token_block<FMT, EPI, CONS, PROD, false, TWO, TILES, true>(a, lds, wave, u0, u1, e, row, row, first);
+    }
+    for (int tb = tb0 == 0 ? (int)gridDim.y : tb0; first + (tb - 1) * 64 < n; tb += gridDim.y) {
+        const int row0 = off + first + (tb - 1) * 64;
+        auto row = [&](int i) { return row0 + i; };
+        if (wave >= CONS) ws_producer_f32<FMT, 4, PROD>(a, lds, row0, 64, wave - CONS, passes);
+        else if constexpr (TILES) ws_consume_tiles<FMT, 4, EPI, false>(a, lds, e, row, 64, u0, u1, wave);
+        else ws_consume_units<FMT, 4, EPI, false, TWO>(a, lds, e, row, 64, u0 + wave, u1, CONS, passes);
     }
 }
 
@@ -1209,13 +1036,29 @@ __global__ __launch_bounds__(WAVES * 64, 2) void expert_prefill_kernel(ExpertGem
 
 template <int FMT, int EPI>
 int launch_cfg(const ExpertGemmArgs& a, hipStream_t stream) {
-    constexpr int R = 2;
-    const int units = (a.rows / 64) * (4 / R);
     if (a.work_queue) {
         if (a.work_count <= 0) return MOE_OK;
-        dim3 grid(ceil_div(units, 4), max(1, ceil_div(a.max_rows_hint, 64)), a.work_count);
-        hipLaunchKernelGGL((expert_stream_queue_kernel<FMT, R, EPI>), grid, dim3(256), 0, stream, a);
-    } else if constexpr (EPI == EPI_SWIGLU_BF16 || EPI == EPI_ROWS_F32) {
+        if constexpr (EPI == EPI_SWIGLU_F32 || EPI == EPI_SCATTER) {
+            ExpertGemmArgs b = a;
+            const int cons = a.waves_per_block == 1 ? 12 : 10;
+            const int units = a.rows / 32;
+            b.row_blocks = max(a.row_blocks, ceil_div(units, (FMT == FMT_MXFP4 ? 2 : 1) * cons));
+            // token-block shares only where the items alone would leave compute units idle
+            const int items = ceil_div(a.work_count, 8) * 8;
+            const int shares = max(1, min(min(ceil_div(a.max_rows_hint, 64), 65535), ceil_div(2 * a.n_cus, a.work_count * b.row_blocks)));
+            const dim3 grid(items * b.row_blocks, shares), block((cons + 4) * 64);
+            const bool two = ceil_div(units, b.row_blocks) > cons;
+            if constexpr (FMT == FMT_MXFP4) {
+                if (two && cons == 12) hipLaunchKernelGGL((expert_stream_queue_ws_kernel<FMT, EPI, 12, 4, true>), grid, block, 0, stream, b);
+                else if (two) hipLaunchKernelGGL((expert_stream_queue_ws_kernel<FMT, EPI, 10, 4, true>), grid, block, 0, stream, b);
+                if (two) return launch_status();
+            }
+            if (cons == 12) hipLaunchKernelGGL((expert_stream_queue_ws_kernel<FMT, EPI, 12, 4, false>), grid, block, 0, stream, b);
+            else hipLaunchKernelGGL((expert_stream_queue_ws_kernel<FMT, EPI, 10, 4, false>), grid, block, 0, stream, b);
+            return launch_status();
+        }
+    }
+    if constexpr (EPI == EPI_SWIGLU_BF16 || EPI == EPI_ROWS_F32) {
         if (a.topk_i) {  // bucketing inside the expert kernel
             if (a.n_assign > kDirectMaxAssign || a.assign_div <= 0 || a.assign_div > 8 || a.n_experts <= 0) return MOE_ERR_LIMIT;
             ExpertGemmArgs b = a;
@@ -1290,9 +1133,9 @@ int expert_direct_max_assignments() { return kDirectMaxAssign; }
 // in/out, 3 down with fp32 in and atomic scatter.  Token blocks hold at most 64 rows.
 int launch_expert_stream(const ExpertGemmArgs& a, int epi, hipStream_t stream) {
     if (a.rows % 64 != 0 || a.K % 32 != 0) return MOE_ERR_SHAPE;
-    if (a.waves_per_block == 18) return launch_expert_small(a, epi, stream);
     const bool queue = a.work_queue != nullptr;
     if (queue != (epi == EPI_SWIGLU_F32 || epi == EPI_SCATTER)) return MOE_ERR_FORMAT;
+    if (a.waves_per_block == 18) return launch_expert_small(a, epi, stream);
     if (a.format == FMT_BF16) {
         // the streaming consumers address an expert's matrix through a buffer descriptor: 32-bit byte offsets
         if ((unsigned long long)a.rows * (unsigned long long)a.K * 2ull > 0x7fffffffull) return MOE_ERR_LIMIT;

@@ -101,8 +101,8 @@ struct ExpertGemmArgs {
                                 // consumer waves (+ 2 producers), 64-token blocks; 16 prefill kernel (4 waves,
                                 // 128-token blocks, two blocks a CU; MXFP4 weights only); 17 tile kernel
                                 // (256-token blocks; bf16 weights only); 18 a 16-row tile per wave, buckets of a
-                                // handful of rows.  Ignored by the work-queue entries.
-    int n_cus;                  // compute units to fill (18 only)
+                                // handful of rows.  The work-queue entries take 0, 1 and 18.
+    int n_cus;                  // compute units to fill (18 and the work-queue entries)
 };
 int launch_expert_stream(const ExpertGemmArgs& a, int epi, hipStream_t stream);
 

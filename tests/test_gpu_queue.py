@@ -1,0 +1,73 @@
+"""The work-queue entries (moe_mlp1_swiglu, moe_mlp2_scatter and their MXFP4 forms) over entries of every token-tile count, of
+no rows and of many token blocks, few and many of them, against the same sums in 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# rows per entry; up to 16 a tile of weight rows per wave; the last leaves compute units to shares of an entry's token blocks
+ROWS = [[1, 0, 15, 16, 17, 33, 48, 63, 64, 65, 129, 200], [1, 0, 3, 4, 5, 8, 13, 16], [3], [700, 0]]
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "mxfp4"])
+@pytest.mark.parametrize("H,I", [(64, 64), (320, 192), (576, 832)])
+@pytest.mark.parametrize("rows", ROWS, ids=["mixed", "short", "few", "long"])
+def test_queue_entries(pkg, wl, dev, H, I, rows, fmt):
+    E, A = len(rows) + 1, sum(rows)
+    shape = wl.MoeShape("queue", T=A, H=H, I=I, E=E, K=1, fmt=fmt, seed=H + I)
+    blk, raw = wl.make_device_layer(shape, pkg.normal_table(), dev, keep_canonical=True)
+    x = wl.make_device_input(shape, pkg.normal_table(), dev)
+    w = blk.tensors
+    if fmt == "bf16":
+        w1, w2 = w["w_mlp1"].double().view(E, 2 * I, H), w["w_mlp2"].double().view(E, H, I)
+    else:
+        w1, w2 = (pkg.dequant_mxfp4(raw[n + "_blocks"], raw[n + "_scales"]).double().view(E, r, k)
+                  for n, r, k in (("w_mlp1", 2 * I, H), ("w_mlp2", H, I)))
+    b1, b2 = w["b_mlp1"].double().view(E, 2 * I), w["b_mlp2"].double().view(E, H)
+    tokens = torch.randperm(A, device=dev).to(torch.int32)
+    weights = torch.rand(A, device=dev)
+    queue, off = [7, 7, 7], 0  # one triple in front that work_start leaves out
+    gate_want = torch.zeros(A, I, dtype=torch.float64, device=dev)
+    out_want = torch.zeros(A, H, dtype=torch.float64, device=dev)
+    for i, n in enumerate(rows):
+        e = E - 1 - i
+        queue += [e, off, n]
+        y = x[off:off + n].bfloat16().double() @ w1[e].T + b1[e]
+        g, u = y[:, 0::2].clamp(max=7.0), y[:, 1::2].clamp(-7.0, 7.0)
+        gate_want[off:off + n] = g * torch.sigmoid(1.702 * g) * (u + 1)
+        off += n
+    queue = torch.tensor(queue, dtype=torch.int32, device=dev)
+    gate = torch.empty(A, I, device=dev)
+    out = torch.zeros(A, H, device=dev)
+    print("queue", H, I, rows, fmt, flush=True)
+    n = len(rows)
+    if fmt == "bf16":
+        pkg.moe_mlp1_swiglu(queue, 1, n, x, gate, w["w_mlp1"], w["b_mlp1"], H, I, 2 * I * H, 2 * I, 1.702, 7.0, max(rows), 0)
+        pkg.moe_mlp2_scatter(queue, 1, n, gate, tokens, weights, out, w["w_mlp2"], w["b_mlp2"], I, H, I * H, H, max(rows), 0)
+    else:
+        pkg.moe_mlp1_swiglu_mxfp4(queue, 1, n, x, gate, w["w_mlp1"], w["w_mlp1_scales"], w["b_mlp1"], H, I, 2 * I, 1.702, 7.0,
+                                  max(rows), 0)
+        pkg.moe_mlp2_scatter_mxfp4(queue, 1, n, gate, tokens, weights, out, w["w_mlp2"], w["w_mlp2_scales"], w["b_mlp2"], I, H,
+                                   H, max(rows), 0)
+    off = 0
+    for i, n in enumerate(rows):
+        e = E - 1 - i
+        h = gate[off:off + n].bfloat16().double()
+        out_want[tokens[off:off + n].long()] = (h @ w2[e].T + b2[e]) * weights[off:off + n, None].double()
+        off += n
+    # fp32 sums of at most 832 exact products: K / 2 roundings of 2^-24 on average, and 1e-6 of the fast exponential
+    for got, want in ((gate, gate_want), (out, out_want)):
+        assert ((got.double() - want).norm() / want.norm()).item() < 5e-5
+
+
+def test_queue_rows_beyond_the_hint(pkg, wl, dev):
+    """max rows is a hint: entries with more rows than it says take further passes."""
+    shape = wl.MoeShape("queue", T=70, H=128, I=64, E=1, K=1, fmt="bf16", seed=1)
+    blk, _ = wl.make_device_layer(shape, pkg.normal_table(), dev)
+    x = wl.make_device_input(shape, pkg.normal_table(), dev)
+    w = blk.tensors
+    queue = torch.tensor([0, 0, 70], dtype=torch.int32, device=dev)
+    got = [torch.empty(70, 64, device=dev) for _ in range(2)]
+    for hint, gate in zip((5, 70), got):
+        pkg.moe_mlp1_swiglu(queue, 0, 1, x, gate, w["w_mlp1"], w["b_mlp1"], 128, 64, 2 * 64 * 128, 128, 1.702, 7.0, hint, 0)
+    assert torch.equal(*got)
