@@ -32,6 +32,25 @@ MOE_DEVICE void load_bias(const ExpertGemmArgs& a, int e, int group, int r0, uin
     for (int r = 0; r < R; ++r) raw[r] = *reinterpret_cast<const uint2*>(bias + 4 * r);
 }
 
+// Values a and b trade places between the lanes whose ids differ in bit BIT (of 0..2): lanes with the bit set give their a and
+// take the partner's b there, the others give b and take a.
+template <int BIT>
+MOE_DEVICE void lane_bit_swap(uint32_t& a, uint32_t& b, bool set) {
+    uint32_t na, nb;
+    if constexpr (BIT == 2) {  // four lanes up or down inside the row of 16, the other bank keeps its value
+        na = (uint32_t)__builtin_amdgcn_update_dpp((int)a, (int)b, 0x114, 0xF, 0xA, false);
+        nb = (uint32_t)__builtin_amdgcn_update_dpp((int)b, (int)a, 0x104, 0xF, 0x5, false);
+    } else {
+        constexpr int kPerm = BIT == 0 ? 0xB1 : 0x4E;  // quad_perm [1,0,3,2] / [2,3,0,1]
+        const uint32_t pa = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)a, kPerm, 0xF, 0xF, false);
+        const uint32_t pb = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b, kPerm, 0xF, 0xF, false);
+        na = set ? pb : a;
+        nb = set ? b : pa;
+    }
+    a = na;
+    b = nb;
+}
+
 // slot_of_row(i): output row (slot) of bucket row i of the token block.
 template <int R, int NT, int EPI, class SlotFn>
 MOE_DEVICE void stream_epilogue(const ExpertGemmArgs& a, const f32x4 (&acc)[R][NT], int e, SlotFn slot_of_row, int nrows,
@@ -87,6 +106,43 @@ MOE_DEVICE void stream_epilogue(const ExpertGemmArgs& a, const f32x4 (&acc)[R][N
         }
         return;
     }
+    if constexpr (EPI == EPI_SCATTER) {
+        // The atomics are carried out beyond the XCD's L2, one request per piece that an instruction leaves contiguous, and a
+        // lane's 4 R consecutive output values would be 4 R instructions of 64 single words.  The low bits of the lane id (the
+        // token) trade places with the value index, so an instruction adds runs of 4 R words: down launch of 256 tokens,
+        // E = 32, bf16, 247 -> 107 us.
+        static_assert(R <= 2, "4 R values to a run of at most eight lanes");
+        constexpr int V = 4 * R;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const float wgt = a.weights_flat[slot_of_row(min(t * 16 + q, nrows - 1))];
+            uint32_t v[V];
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[4 * r + j] = __float_as_uint((acc[r][t][j] + bv[r][j]) * wgt);
+#pragma unroll
+            for (int i = 0; i < V; i += 2) lane_bit_swap<0>(v[i], v[i + 1], q & 1);
+#pragma unroll
+            for (int i = 0; i < V; ++i)
+                if (!(i & 2)) lane_bit_swap<1>(v[i], v[i + 2], q & 2);
+            if constexpr (R == 2) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) lane_bit_swap<2>(v[i], v[i + 4], q & 4);
+            }
+            // v[i]: token t*16 + (q without its low bits) + i, output row row_base + (the low bits of q)
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+                const int idx = t * 16 + (q & ~(V - 1)) + i;
+                if (idx < nrows) {
+                    const int tok = a.tokens_flat[slot_of_row(idx)];
+                    atomicAdd(reinterpret_cast<float*>(a.out) + (size_t)tok * a.rows + row_base + (q & (V - 1)),
+                              __uint_as_float(v[i]));
+                }
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
         const int idx = t * 16 + q;
@@ -127,14 +183,6 @@ MOE_DEVICE void stream_epilogue(const ExpertGemmArgs& a, const f32x4 (&acc)[R][N
                 v[3] += bv[r][3];
                 *reinterpret_cast<f32x4*>(dst + 4 * r) = v;
             }
-        } else {
-            const int tok = a.tokens_flat[slot];
-            const float wgt = a.weights_flat[slot];
-            float* dst = reinterpret_cast<float*>(a.out) + (size_t)tok * a.rows + row_base;
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) atomicAdd(dst + 4 * r + j, (acc[r][t][j] + bv[r][j]) * wgt);
         }
     }
 }
