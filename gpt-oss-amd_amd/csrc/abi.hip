@@ -581,6 +581,11 @@ struct ExpertPlan {
             a.s_expert_stride = (long long)sb;
         }
     }
+    // MXFP4 prefill launches of at most two and a half rounds of blocks (two to a compute unit): what counts is how evenly they
+    // end, so the largest token blocks come first in both GEMMs and the XCDs get equal shares (two parts to a token block).
+    // Block of 32 experts, us, otherwise : so: 416 tokens skewed 186 : 164, 1000 tokens 279 : 252, skewed 272 : 265, 1600 tokens
+    // skewed 361 : 347, 2500 tokens 493 : 496, skewed 500 : 487; 4096 tokens 746 : 759; 128 experts, 1700 tokens skewed 582 : 586.
+    bool few_blocks() const { return (long long)est_tiles * ceil_div(p->hidden_dim, 256) < 5LL * n_cus; }
     void use_second_map(ExpertGemmArgs& a) const {
         a.tile_expert += second_map;
         a.tile_row0 += second_map;
@@ -598,6 +603,7 @@ struct ExpertPlan {
         // row blocks on one XCD takes 1 % off the bf16 launch (its token rows enter one L2 instead of eight) and
         // leaves the MXFP4 launch as it is; with token blocks from the tile map it cost up to 2 %
         a.xcd_tiles = direct ? 1 : 0;
+        if (a.waves_per_block == 16) a.xcd_tiles = few_blocks() ? 2 : 1;
         if (a.waves_per_block == 17) use_second_map(a);  // places an expert's blocks by where its tiles begin
         return a;
     }
@@ -613,10 +619,11 @@ struct ExpertPlan {
         // (largest first: the launch's tail is made of short blocks); the down GEMM is 2 % faster in bucket
         // order, where a partial block runs next to full blocks of its expert and finds the expert's weights
         // on their way through the caches.
-        if (!direct) use_second_map(a);
+        const bool few = a.waves_per_block == 16 && few_blocks();
+        if (!direct && !few) use_second_map(a);
         // measured: the down GEMM gains 4-10 % from keeping a token block on one XCD (its input rows were
         // written by the gate/up launch just before)
-        a.xcd_tiles = 1;
+        a.xcd_tiles = few ? 2 : 1;
         return a;
     }
 };

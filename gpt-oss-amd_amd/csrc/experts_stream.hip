@@ -1009,12 +1009,16 @@ __global__ __launch_bounds__(WAVES * 64, 2) void expert_prefill_kernel(ExpertGem
     // All row blocks of a token block run on ONE XCD, back to back in that XCD's sequence, so the
     // block's activations are fetched into that L2 once instead of once per XCD (measured: 40 %
     // less traffic into the L2s, -3 % time; sharing the weights between neighbouring token blocks
-    // as well cut the traffic further but ran slower).
-    const int n_rb = a.row_blocks;
-    const int xcd = blockIdx.x & 7;
+    // as well cut the traffic further but ran slower).  A launch of few blocks deals each token block's
+    // row blocks out in two parts instead: with seven token blocks on one XCD and six on another the
+    // launch would end with the one's third round of blocks (see ExpertPlan::few_blocks).
+    const int n_rb = a.row_blocks, parts = a.xcd_tiles;
+    const int per_part = ceil_div(n_rb, parts);
     const int m = blockIdx.x >> 3;
-    const int tile = (m / n_rb) * 8 + xcd;
-    const int row_block = m % n_rb;
+    const int share = (m / per_part) * 8 + (blockIdx.x & 7);  // (tile, part of its row blocks)
+    const int tile = share / parts;
+    const int row_block = (share - tile * parts) * per_part + m % per_part;
+    if (row_block >= n_rb) return;  // block-uniform
     if (tile >= *a.n_tiles) return;  // block-uniform
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int unit = row_block * WAVES + wave;
@@ -1088,7 +1092,8 @@ int launch_cfg(const ExpertGemmArgs& a, hipStream_t stream) {
             if constexpr (FMT == FMT_MXFP4) {
                 ExpertGemmArgs b = a;
                 b.row_blocks = ceil_div(a.rows / 64, 4);
-                dim3 grid(ceil_div(a.max_tiles, 8) * 8 * b.row_blocks);  // every XCD gets whole token blocks
+                // every XCD gets whole token blocks, or whole parts of their row blocks
+                dim3 grid(ceil_div(a.max_tiles * a.xcd_tiles, 8) * 8 * ceil_div(b.row_blocks, a.xcd_tiles));
                 hipLaunchKernelGGL((expert_prefill_kernel<FMT, EPI, 4>), grid, dim3(256), 0, stream, b);
             } else {
                 return MOE_ERR_FORMAT;

@@ -1,0 +1,20 @@
+"""The block index -> (token block, row block) map of the MXFP4 prefill kernel, launches of few and of many blocks: every output
+row as the streaming kernels compute it (they add in the same order)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# one to five row blocks of 256 rows in the two launches, an odd last one among them; 1 to 1000 token blocks
+@pytest.mark.parametrize("H,I", [(64, 64), (320, 192), (576, 640), (1088, 128)])
+@pytest.mark.parametrize("T,E,K,zipf_s", [(1, 4, 2, 0.0), (700, 32, 4, 1.2), (1500, 6, 2, 3.0), (900, 130, 8, 0.0), (9000, 130, 8, 0.5)])
+def test_prefill_blocks_cover_every_row(pkg, wl, dev, H, I, T, E, K, zipf_s):
+    table = pkg.normal_table()
+    shape = wl.MoeShape("prefill", T=T, H=H, I=I, E=E, K=K, fmt="mxfp4", zipf_s=zipf_s, seed=T + H)
+    blk, _ = wl.make_device_layer(shape, table, dev)
+    x = wl.make_device_input(shape, table, dev)
+    print("prefill", shape, flush=True)
+    y, ti, _ = blk.forward(x, flags=pkg.MOE_FLAG_FORCE_TILED)
+    want, _, _ = blk.forward(x, flags=pkg.MOE_FLAG_FORCE_STREAM)
+    assert torch.equal(y, want)
