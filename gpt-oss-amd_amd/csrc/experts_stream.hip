@@ -1012,12 +1012,12 @@ __global__ __launch_bounds__(WAVES * 64, 2) void expert_prefill_kernel(ExpertGem
     // as well cut the traffic further but ran slower).  A launch of few blocks deals each token block's
     // row blocks out in two parts instead: with seven token blocks on one XCD and six on another the
     // launch would end with the one's third round of blocks (see ExpertPlan::few_blocks).
-    const int n_rb = a.row_blocks, parts = a.xcd_tiles;
-    const int per_part = ceil_div(n_rb, parts);
-    const int m = blockIdx.x >> 3;
-    const int share = (m / per_part) * 8 + (blockIdx.x & 7);  // (tile, part of its row blocks)
-    const int tile = share / parts;
-    const int row_block = (share - tile * parts) * per_part + m % per_part;
+    const int n_rb = a.row_blocks, halves = a.xcd_tiles - 1;  // one or two parts: shifts instead of divisions
+    const int per_part = (n_rb + halves) >> halves;
+    const int m = blockIdx.x >> 3, round = m / per_part;
+    const int share = round * 8 + (blockIdx.x & 7);  // (tile, part of its row blocks)
+    const int tile = share >> halves;
+    const int row_block = (share & halves) * per_part + m - round * per_part;
     if (row_block >= n_rb) return;  // block-uniform
     if (tile >= *a.n_tiles) return;  // block-uniform
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
