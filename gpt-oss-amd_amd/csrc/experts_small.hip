@@ -59,20 +59,20 @@ MOE_DEVICE void small_tile(const ExpertGemmArgs& a, uint8_t* lds, int e, SlotFn 
                 ++st;
             }
         };
-        // the lane's row and contraction element; a position past the row re-reads its start: its weights count as zero
+        // the lane's row, and the contraction element at its position (of the padding if it lies past the row)
         auto slot = [&]() { return slot_of_row(min(rq * 4 + g, nrows - 1)); };
-        auto elem = [&]() {
-            const int k = (s0 + st) * kStageElems + 8 * ws_chunk_at<FMT>(q ^ ((rq * 4 + g) & 15));
-            return k < K ? k : 0;
-        };
+        auto elem = [&]() { return (s0 + st) * kStageElems + 8 * ws_chunk_at<FMT>(q ^ ((rq * 4 + g) & 15)); };
         if constexpr (ACT_F32) {
             constexpr int B = 4;  // loads of a batch are in flight together
             for (int n = wave; n < n_instr; n += B * waves) {
                 float4 x[B][2];
+                bool live[B];
 #pragma unroll
                 for (int i = 0; i < B; ++i) {
                     if (n + i * waves < n_instr) {  // wave-uniform
-                        const float4* src = reinterpret_cast<const float4*>(a.act_f32 + (size_t)slot() * K + elem());
+                        const int k = elem();
+                        live[i] = k < K;
+                        const float4* src = reinterpret_cast<const float4*>(a.act_f32 + (size_t)slot() * K + (live[i] ? k : 0));
                         x[i][0] = src[0];
                         x[i][1] = src[1];
                     }
@@ -80,16 +80,21 @@ MOE_DEVICE void small_tile(const ExpertGemmArgs& a, uint8_t* lds, int e, SlotFn 
                 }
 #pragma unroll
                 for (int i = 0; i < B; ++i)
-                    if (n + i * waves < n_instr)
-                        *reinterpret_cast<u32x4*>(lds + (size_t)(n + i * waves) * 1024 + lane * 16) =
-                            u32x4{pack_bf16x2(x[i][0].x, x[i][0].y), pack_bf16x2(x[i][0].z, x[i][0].w),
-                                  pack_bf16x2(x[i][1].x, x[i][1].y), pack_bf16x2(x[i][1].z, x[i][1].w)};
+                    if (n + i * waves < n_instr) {
+                        u32x4 v = {pack_bf16x2(x[i][0].x, x[i][0].y), pack_bf16x2(x[i][0].z, x[i][0].w),
+                                   pack_bf16x2(x[i][1].x, x[i][1].y), pack_bf16x2(x[i][1].z, x[i][1].w)};
+                        // zeros past the row: the weights count as zero there, and zero times an infinity or a NaN
+                        // from elsewhere in the row would reach all of its outputs (bf16 never multiplies them)
+                        if (FMT == FMT_MXFP4 && !live[i]) v = u32x4{0u, 0u, 0u, 0u};
+                        *reinterpret_cast<u32x4*>(lds + (size_t)(n + i * waves) * 1024 + lane * 16) = v;
+                    }
             }
         } else {
             for (int n = wave; n < n_instr; n += waves) {
                 const int s = slot();
                 const int src = a.gather ? (int)(((float)s + 0.5f) * inv_div) : s;
-                dma16(reinterpret_cast<const uint8_t*>(a.act + (size_t)src * K + elem()), lds + (size_t)n * 1024);
+                const int k = elem();  // a position past the row re-reads its start: its weights count as zero
+                dma16(reinterpret_cast<const uint8_t*>(a.act + (size_t)src * K + (k < K ? k : 0)), lds + (size_t)n * 1024);
                 next();
             }
         }

@@ -148,9 +148,11 @@ MOE_DEVICE void ws_producer_f32(const ExpertGemmArgs& a, uint8_t* lds, int first
     uint8_t* const dst = lds + r0 * 256 + ((ws_pos<FMT>(col >> 1) ^ r0) << 4) + (col & 1) * 8;
     const int swap = (ws_pos<FMT>(col >> 1) ^ r0) & 8 ? -128 : 128;  // row r0 + 8 has bit 3 of the position flipped
     float4 v[Q];
+    bool live = true;
     auto load = [&](int st) {
         // a position past the row re-reads its start
-        const uint32_t off = st * kStageElems + 4 * col < K ? (uint32_t)st * (kStageElems * 4u) : 0u - 16u * (uint32_t)col;
+        live = st * kStageElems + 4 * col < K;
+        const uint32_t off = live ? (uint32_t)st * (kStageElems * 4u) : 0u - 16u * (uint32_t)col;
 #pragma unroll
         for (int i = 0; i < Q; ++i) v[i] = *reinterpret_cast<const float4*>(base + (src[i] + off));
     };
@@ -158,10 +160,13 @@ MOE_DEVICE void ws_producer_f32(const ExpertGemmArgs& a, uint8_t* lds, int first
         uint8_t* at[2];
         at[0] = dst + (size_t)(gs & (kWsRing - 1)) * kLdsStageBytes;
         at[1] = at[0] + 2048 + swap;
+        // and is written as zeros where its weights count as zero (MXFP4; bf16 never multiplies it): zero times an
+        // infinity or a NaN from elsewhere in the row would reach all of its outputs
+        const uint32_t keep = FMT == FMT_BF16 || live ? 0xffffffffu : 0u;
 #pragma unroll
         for (int i = 0; i < Q; ++i)
             *reinterpret_cast<u32x2*>(at[i & 1] + (i >> 1) * 4096) =
-                u32x2{pack_bf16x2(v[i].x, v[i].y), pack_bf16x2(v[i].z, v[i].w)};
+                u32x2{pack_bf16x2(v[i].x, v[i].y) & keep, pack_bf16x2(v[i].z, v[i].w) & keep};
     };
     int st = 0;  // stage (inside a pass) loaded next
     auto next_stage = [&]() { st = (st + 1 == n_stages) ? 0 : st + 1; };
