@@ -307,7 +307,9 @@ __global__ __launch_bounds__(64 * kSmallWaves, 4) void expert_small_kernel(Exper
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
         const int s = (p * waves + wave) * 64 + lane;
-        ids[p] = s < a.n_assign ? a.topk_i[s] : -1;
+        // an id that names no expert is skipped, as by the other kernels: the down GEMM entry takes the list from its caller
+        const int id = s < a.n_assign ? a.topk_i[s] : -1;
+        ids[p] = (unsigned)id < (unsigned)a.n_experts ? id : -1;
     }
     if (threadIdx.x < 32) present[threadIdx.x] = 0u;
     __syncthreads();

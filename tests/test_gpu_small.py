@@ -1,6 +1,8 @@
 """The kernels for a handful of rows per expert (experts_small.hip) at the sizes where their phases, rings, tails and block
 sizes change: bit-identical to the producer/consumer kernels, which add in the same order (the oracle checks the block in
 test_gpu_parity.py)."""
+import ctypes
+
 import pytest
 import torch
 
@@ -44,3 +46,29 @@ def test_small_kernel_finds_its_experts(pkg, wl, dev, T, E, K):
         assert blk.describe(blk.params(x, y, ti, y))["down"] == "expert_small_kernel<%d, 1>" % (fmt == "mxfp4")
         want, _, _ = blk.forward(x, flags=pkg.MOE_FLAG_FORCE_DIRECT)
         assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "mxfp4"])
+def test_ids_that_name_no_expert_are_skipped(pkg, wl, dev, fmt):
+    """The down GEMM entry takes its assignment list from the caller: ids outside [0, E) write no row and change no other."""
+    T, H, I, E, K = 20, 192, 320, 48, 2
+    shape = wl.MoeShape("small", T=T, H=H, I=I, E=E, K=K, fmt=fmt, seed=7)
+    blk, _ = wl.make_device_layer(shape, pkg.normal_table(), dev)
+    ids = (torch.arange(T * K, dtype=torch.int32) * 7 % E).view(T, K)
+    bad = torch.zeros(T * K, dtype=torch.bool)
+    for i, v in enumerate([-1, E, E + 1, 63, 64, 1000, 1023, 1024, 1 << 20, 0x7FFFFFFF, -(1 << 31)]):
+        ids.view(-1)[3 * i + 1] = v
+        bad[3 * i + 1] = True
+    ids, bad = ids.to(dev), bad.to(dev)
+    h = torch.randn(T * K, I, device=dev).bfloat16()
+    tv = torch.ones(T, K, device=dev)
+    got = []
+    print("ids out of range", fmt, flush=True)
+    for flags in (0, pkg.MOE_FLAG_FORCE_DIRECT):
+        y = torch.full((T * K, H), 123.0, device=dev)
+        p = blk.params(None, None, ids, tv, flags=flags)
+        assert pkg.lib.moe_block_down_gemm(ctypes.byref(p), h.data_ptr(), y.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
+        assert blk.describe(p)["down"].startswith("expert_stream_direct" if flags else "expert_small")
+        assert (y[bad] == 123.0).all() and not (y[~bad] == 123.0).all(dim=1).any()
+        got.append(y)
+    assert torch.equal(*got)
