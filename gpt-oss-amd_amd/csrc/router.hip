@@ -742,14 +742,12 @@ __global__ __launch_bounds__(256, 4) void router_refine_kernel(const float* __re
 #pragma nounroll
     for (int e0 = 0; e0 < E; e0 += 64) {
         const int e = e0 + lane;
-        const bool in = e < E && approx[e] >= thr;
+        // a not-a-number on either side decides nothing: an infinite router weight makes its expert's approximate score one
+        // (the two pieces of an activation may differ in sign) where the exact score is an infinity
+        const bool in = e < E && !(approx[e] < thr);
         const unsigned long long ballot = __ballot(in);
         if (in) cand[n_cand + __popcll(ballot & ((1ull << lane) - 1ull))] = e;
         n_cand += __popcll(ballot);
-    }
-    if (n_cand < K) {  // not-a-number scores: no screening, every expert is scored exactly
-        for (int e = lane; e < E; e += 64) cand[e] = e;
-        n_cand = E;
     }
     if (lane == 0) {
         if (delta_out) delta_out[t] = delta;

@@ -21,3 +21,28 @@ def test_router_kernels_agree(pkg, wl, dev, H, E, tokens):
         assert torch.equal(ti, wi)
         # logits differ, if at all, in the last place of their rounding to fp32: 2^-23 of |logit| < 16
         assert (tv - wv).abs().max().item() <= 4e-6
+
+
+@pytest.mark.parametrize("T", [700, 2100])
+@pytest.mark.parametrize("what", ["inf weight", "nan weight", "nan weight, ties", "nan bias", "inf bias", "inf row", "nan row", "huge row"])
+def test_screening_keeps_non_finite_scores(pkg, wl, dev, T, what):
+    """Scores that are infinite or not a number rank as in the single exact pass: the screening pass drops an expert for a
+    finite approximate score below the bound only."""
+    H, E, K = 320, 32, 4
+    table = pkg.normal_table()
+    shape = wl.MoeShape("router", T=T, H=H, I=64, E=E, K=K, fmt="mxfp4", seed=11)
+    blk, _ = wl.make_device_layer(shape, table, dev)
+    x = wl.make_device_input(shape, table, dev)
+    w, b = blk.tensors["w_router"], blk.tensors["b_router"]
+    if "ties" in what:  # every other expert inside the bound of the K-th best
+        w.copy_(w[:1].expand(E, H).clone())
+        b.fill_(0.5)
+    v = float(what[:3]) if what[:3] in ("inf", "nan") else 3.39e38  # the last rounds to an infinity in bf16
+    {"weight": w[5], "weight, ties": w[5], "bias": b, "row": x[::3]}[what.split(" ", 1)[1]][..., 7] = v
+    print("non-finite router", T, what, flush=True)
+    _, ti, tv = blk.forward(x)
+    assert blk.describe(blk.params(x, x, ti, tv))["router"] == "router_screen_kernel + router_refine_kernel"
+    _, wi, wv = blk.forward(x, flags=pkg.MOE_FLAG_ROUTER_STRICT_ORDER)
+    assert torch.equal(ti, wi)
+    assert torch.equal(tv.isnan(), wv.isnan())
+    assert (tv.nan_to_num(0.0) - wv.nan_to_num(0.0)).abs().max().item() <= 4e-6
