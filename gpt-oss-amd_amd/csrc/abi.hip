@@ -343,7 +343,6 @@ static int queue_gemm(int epi, int format, const int* work_queue, int work_start
     a.weights_flat = weights_flat;
     a.work_queue = work_queue;
     a.work_start = work_start;
-    a.work_count = work_count;
     a.max_rows_hint = std::max(1, maxNe);
     a.out = out;
     a.rows = rows;
@@ -356,18 +355,28 @@ static int queue_gemm(int epi, int format, const int* work_queue, int work_start
     a.format = format;
     a.n_cus = device_cu_count();
     a.xcd_tiles = 1;
-    // Short entries: a tile of weight rows per wave (experts_small.hip).  The layer's calls with at most n rows an entry, us, that
-    // kernel : producers and consumers: E = 32, bf16, n = 1 92 : 158, 4 176 : 227, 16 294 : 288; MXFP4, 4 92 : 98, 16 124 : 120, 32
-    // 134 : 125; E = 128, bf16, 16 440 : 498, 32 675 : 658; MXFP4, 16 164 : 196.
-    if (maxNe <= 16 && expert_small_fits(0, rows, Kdim, format)) {
-        a.waves_per_block = 18;
-    } else if (format == MOE_WEIGHTS_MXFP4_TILED) {
-        pick_stream_two_pass(rows, work_count, a.n_cus, &a.waves_per_block, &a.row_blocks);
-    } else {
-        a.waves_per_block = pick_stream_kernel(rows, work_count, a.n_cus);
-        a.row_blocks = pick_stream_row_blocks(rows, a.waves_per_block, work_count, a.n_cus);
-    }
-    return launch_expert_stream(a, epi, as_stream(stream));
+    // The blocks of a launch scan its entries for their share of the long ones (experts_stream.hip): a longer queue is run
+    // in parts, each of which fills the device many times over.
+    constexpr int kPart = 1024;
+    int rc = MOE_OK, left = work_count;
+    do {
+        a.work_count = std::min(left, kPart);
+        // Short entries: a tile of weight rows per wave (experts_small.hip).  The layer's calls with at most n rows an entry, us,
+        // that kernel : producers and consumers: E = 32, bf16, n = 1 92 : 158, 4 176 : 227, 16 294 : 288; MXFP4, 4 92 : 98, 16
+        // 124 : 120, 32 134 : 125; E = 128, bf16, 16 440 : 498, 32 675 : 658; MXFP4, 16 164 : 196.
+        if (maxNe <= 16 && expert_small_fits(0, rows, Kdim, format)) {
+            a.waves_per_block = 18;
+        } else if (format == MOE_WEIGHTS_MXFP4_TILED) {
+            pick_stream_two_pass(rows, a.work_count, a.n_cus, &a.waves_per_block, &a.row_blocks);
+        } else {
+            a.waves_per_block = pick_stream_kernel(rows, a.work_count, a.n_cus);
+            a.row_blocks = pick_stream_row_blocks(rows, a.waves_per_block, a.work_count, a.n_cus);
+        }
+        rc = launch_expert_stream(a, epi, as_stream(stream));
+        a.work_start += a.work_count;
+        left -= a.work_count;
+    } while (rc == MOE_OK && left > 0);
+    return rc;
 }
 
 int moe_mlp1_swiglu(const int* work_queue, int work_start, int work_count, const float* x_by_expert,

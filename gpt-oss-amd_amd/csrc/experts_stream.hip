@@ -128,6 +128,16 @@ MOE_DEVICE void ws_producer(const ExpertGemmArgs& a, uint8_t* lds, RowFn act_row
     wait_vmcnt<0>();  // nothing may still be writing this block's LDS when the wave ends
 }
 
+// The lane id; for the work-queue entries (epilogue EPI) as a value that the compiler takes to be new at every call: what
+// follows from it is then worked out per token block, not ahead of the loop over an entry list's whole blocks, where it would
+// wait in scratch memory and be fetched in the stage loops (a spill access there waits for every weight load in flight).
+template <int EPI>
+MOE_DEVICE int ws_lane() {
+    int lane = threadIdx.x & 63;
+    if constexpr (EPI == EPI_SWIGLU_F32 || EPI == EPI_SCATTER) asm volatile("" : "+v"(lane));
+    return lane;
+}
+
 // The producer for fp32 activations (the entries that keep the reference's data flow): rows first_row .. first_row + nrows of
 // a.act_f32, rounded to bf16 on their way into the same LDS image.  An instruction takes two rows of 512 contiguous bytes; the
 // loads of a stage are issued one stage before it is written, i.e. four before it is read.
@@ -135,7 +145,7 @@ template <int FMT, int NT, int PROD>
 MOE_DEVICE void ws_producer_f32(const ExpertGemmArgs& a, uint8_t* lds, int first_row, int nrows, int p, int passes) {
     static_assert(PROD == 4, "eight rows of a token tile per step of the loops below");
     constexpr int Q = 2 * NT;  // loads per stage of this wave
-    const int lane = threadIdx.x & 63;
+    const int lane = ws_lane<EPI_SCATTER>();
     const int col = lane & 31;  // float4 of the row's 128 elements
     const int K = a.K;
     const int n_stages = ceil_div(K, kStageElems);
@@ -197,7 +207,7 @@ template <int FMT, int NT, int EPI, bool PRE = false, int R = 2, class SlotFn>
 MOE_DEVICE void ws_consumer(const ExpertGemmArgs& a, const uint8_t* lds, int e, SlotFn slot_of_row, int nrows, int tile0,
                             bool active) {
     static_assert(R == 1 || R == 2, "one or two row tiles per wave");
-    const int lane = threadIdx.x & 63;
+    const int lane = ws_lane<EPI>();
     const int g = lane >> 4;
     const int q = lane & 15;
     const int K = a.K;
@@ -427,7 +437,7 @@ MOE_DEVICE void ws_consumer_two(const ExpertGemmArgs& a, const uint8_t* lds, int
                             int unit_end, int unit_step, int passes) {
     constexpr int R = 2;
     constexpr bool TWO = true;
-    const int lane = threadIdx.x & 63;
+    const int lane = ws_lane<EPI>();
     const int g = lane >> 4;
     const int q = lane & 15;
     const int K = a.K;
@@ -809,38 +819,90 @@ __global__ __launch_bounds__((CONS + PROD) * 64, (CONS + PROD > 12) ? 4 : 3) voi
 // ---------------------------------------------------------------------------------------------
 // The entries that keep the reference's data flow (work queue of (expert, row_offset, row_count) triples, entry format of
 // src/hip/scheduler.hip:163-166; fp32 rows by slot in, fp32 rows or an atomic scatter out) on the same main loop.  Bound by the
-// weights like the kernels above.  Block (item, rb) takes the item's token blocks blockIdx.y, + gridDim.y, ...; block 0 is the
-// remainder (see expert_stream_direct_kernel).
-// grid = (row blocks x queue entries, padded to a multiple of 8 entries; token-block shares), block = 64 (CONS + PROD).
+// weights like the kernels above.  The queue's token blocks form one list: every entry's remainder (1 .. 64 rows, see
+// expert_stream_direct_kernel), every entry's first whole block of 64 rows (where it has one: on the XCD of its remainder,
+// where a short remainder leaves compute units early), then all other whole blocks, entry by entry.  Slot i of the launch
+// takes list items i, i + slots, .., so an entry of many rows among short ones is dealt out over all compute units and XCDs
+// (the row blocks of one slot run on one of them), whatever the caller's row-count hint says.  With a share of the launch to
+// each entry the longest one set the launch's time: gate/up + down of 31 entries of 8 rows and one of 4000, bf16, 8057 us : 1010
+// now (MXFP4 2816 : 395); one entry of 4000 rows alone, on one XCD then, 4639 : 788; 2048 tokens x 4 of 32 entries, skewed, 4380
+// : 1459; evenly spread 1503 : 1412, 256 tokens 279 : 281.
+// grid = row blocks x slots (xcd_tiles: slots a multiple of 8), block = 64 (CONS + PROD); slots >= work_count.
 // ---------------------------------------------------------------------------------------------
+
+// The next whole block of the slot at list item u or after: its expert and first row; false past the end of the list.
+// `items`: the entries, rounded up to whole rounds of XCDs.  Every wave looks for itself, 64 entries at a time: no state lives
+// across a block's main loop.
+MOE_DEVICE bool queue_next_whole(const ExpertGemmArgs& a, int items, int slots, int& u, int& e, int& row0) {
+    const int lane = threadIdx.x & 63;
+    const int* queue = a.work_queue + 3 * (size_t)a.work_start;
+    int n = lane < a.work_count ? queue[3 * lane + 2] : 0;
+    if (u < 2 * items) {
+        const int* entry = queue + 3 * (size_t)min(u - items, a.work_count - 1);
+        if (u - items < a.work_count && entry[2] > 64) {
+            e = entry[0];
+            row0 = entry[1] + entry[2] - ((entry[2] - 1) & ~63);
+            return true;
+        }
+        u += slots;  // >= 2 * items
+    }
+    int f = u - 2 * items;
+    for (int c = 0; c < a.work_count; c += 64) {
+        if (c > 0) n = c + lane < a.work_count ? queue[3 * (c + lane) + 2] : 0;
+        const int whole = max(n - 65, 0) >> 6;  // but the first
+        uint32_t incl = (uint32_t)whole;
+#define MOE_STEP(C, M) incl += dpp_move<C, M>(0u, incl);
+        MOE_DPP_STEPS(MOE_STEP)
+#undef MOE_STEP
+        const int total = (int)__builtin_amdgcn_readlane(incl, 63);
+        if (f < total) {
+            const int j = __popcll(__ballot((int)incl <= f));  // entries whose whole blocks all come before
+            const int before = (int)__builtin_amdgcn_readlane(incl, j) - __builtin_amdgcn_readlane(whole, j);
+            const int rem = __builtin_amdgcn_readlane(n - 64 * whole, j);  // remainder and first whole block
+            e = __builtin_amdgcn_readfirstlane(queue[3 * (c + j)]);
+            row0 = __builtin_amdgcn_readfirstlane(queue[3 * (c + j) + 1]) + rem + 64 * (f - before);
+            return true;
+        }
+        f -= total;
+    }
+    return false;
+}
+
 template <int FMT, int EPI, int CONS, int PROD, bool TWO>
 __global__ __launch_bounds__((CONS + PROD) * 64, (CONS + PROD > 12) ? 4 : 3) void expert_stream_queue_ws_kernel(ExpertGemmArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[kWsRing * kLdsStageBytes];
-    int item, rb;
-    ws_block_coords(a, item, rb);
-    if (item >= a.work_count) return;  // block-uniform
+    int slot, rb;
+    ws_block_coords(a, slot, rb);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int* entry = a.work_queue + 3 * (size_t)(a.work_start + item);
-    const int e = entry[0], off = entry[1], n = entry[2];
-    const int tb0 = blockIdx.y;
-    if (tb0 * 64 >= n) return;  // block-uniform; also an empty entry
     constexpr bool TILES = !TWO && FMT == FMT_BF16;
     int u0, u1;
     if constexpr (TILES) ws_row_tiles<CONS>(a, rb, u0, u1);
     else ws_row_units(a, rb, u0, u1);
     const int passes = TWO ? min(2, max(1, ceil_div(u1 - u0, CONS))) : 1;
-    const int first = n - ((n - 1) & ~63);
-    if (tb0 == 0) {
-        auto row = [&](int i) { return off + i; };
-        ws_token_block<FMT, EPI, CONS, PROD, false, TWO, TILES, true>(a, lds, wave, u0, u1, e, row, row, first);
+    if (slot < a.work_count) {  // block-uniform, as all of the following
+        const int* entry = a.work_queue + 3 * (size_t)(a.work_start + slot);
+        const int off = entry[1], n = entry[2];
+        if (n > 0) {
+            auto row = [&](int i) { return off + i; };
+            ws_token_block<FMT, EPI, CONS, PROD, false, TWO, TILES, true>(a, lds, wave, u0, u1, entry[0], row, row,
+                                                                          n - ((n - 1) & ~63));
+        }
     }
-    for (int tb = tb0 == 0 ? (int)gridDim.y : tb0; first + (tb - 1) * 64 < n; tb += gridDim.y) {
-        const int row0 = off + first + (tb - 1) * 64;
+    const int slots = gridDim.x / a.row_blocks;
+    const int items = a.xcd_tiles && a.work_count >= 32 ? (a.work_count + 7) & ~7 : a.work_count;  // <= slots
+    int u = slot < items ? slot + slots : slot, e, row0;
+    // The exit in front of the loop is written out: with the search as the loop's condition every block paid for what the
+    // compiler computes ahead of the loop and keeps in scratch memory (0.7 MB, 20 us), also without a whole block.
+    if (!queue_next_whole(a, items, slots, u, e, row0)) return;
+    do {
+        ExpertGemmArgs b = a;
+        asm volatile("" : "+s"(b.K));  // new in every round: nothing that depends on it is worked out ahead of the loop (ws_lane)
         auto row = [&](int i) { return row0 + i; };
-        if (wave >= CONS) ws_producer_f32<FMT, 4, PROD>(a, lds, row0, 64, wave - CONS, passes);
-        else if constexpr (TILES) ws_consume_tiles<FMT, 4, EPI, false>(a, lds, e, row, 64, u0, u1, wave);
-        else ws_consume_units<FMT, 4, EPI, false, TWO>(a, lds, e, row, 64, u0 + wave, u1, CONS, passes);
-    }
+        if (wave >= CONS) ws_producer_f32<FMT, 4, PROD>(b, lds, row0, 64, wave - CONS, passes);
+        else if constexpr (TILES) ws_consume_tiles<FMT, 4, EPI, false>(b, lds, e, row, 64, u0, u1, wave);
+        else ws_consume_units<FMT, 4, EPI, false, TWO>(b, lds, e, row, 64, u0 + wave, u1, CONS, passes);
+        u += slots;
+    } while (queue_next_whole(a, items, slots, u, e, row0));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1052,10 +1114,14 @@ int launch_cfg(const ExpertGemmArgs& a, hipStream_t stream) {
             const int cons = a.waves_per_block == 1 ? 12 : 10;
             const int units = a.rows / 32;
             b.row_blocks = max(a.row_blocks, ceil_div(units, (FMT == FMT_MXFP4 ? 2 : 1) * cons));
-            // token-block shares only where the items alone would leave compute units idle
-            const int items = ceil_div(a.work_count, 8) * 8;
-            const int shares = max(1, min(min(ceil_div(a.max_rows_hint, 64), 65535), ceil_div(2 * a.n_cus, a.work_count * b.row_blocks)));
-            const dim3 grid(items * b.row_blocks, shares), block((cons + 4) * 64);
+            // Slots: one per entry, and more where that would leave compute units idle (two blocks to each, while the list may
+            // be that long).  If even one slot per token block leaves some idle, the blocks get shorter.
+            const long long blocks = (long long)a.work_count * ceil_div(a.max_rows_hint, 64);
+            if (blocks * b.row_blocks < a.n_cus) b.row_blocks = min(units, ceil_div(a.n_cus, (int)blocks));
+            int slots = max(a.work_count, (int)min(blocks, (long long)ceil_div(2 * a.n_cus, b.row_blocks)));
+            b.xcd_tiles = slots >= 8;  // fewer slots would leave XCDs without one
+            if (b.xcd_tiles) slots = ceil_div(slots, 8) * 8;
+            const dim3 grid(slots * b.row_blocks), block((cons + 4) * 64);
             const bool two = ceil_div(units, b.row_blocks) > cons;
             if constexpr (FMT == FMT_MXFP4) {
                 if (two && cons == 12) hipLaunchKernelGGL((expert_stream_queue_ws_kernel<FMT, EPI, 12, 4, true>), grid, block, 0, stream, b);

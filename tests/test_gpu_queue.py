@@ -113,3 +113,71 @@ def test_queue_non_finite_rows(pkg, wl, dev, K, fmt):
         # rows rounded to bf16: 2^-9 of each of K terms
         assert ((got[fin] - ref[fin]).norm() / ref[fin].norm()).item() < 2.0 ** -8
         assert ref[~fin].numel() > 0 and ref.isposinf().any() and ref.isneginf().any()
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "mxfp4"])
+@pytest.mark.parametrize("rows", [[8] * 31 + [1000], [700] + [1] * 70 + [65, 64, 400] + [0] * 60 + [129], [300, 5], [500], [100] * 7,
+                                  [3] * 1020 + [0, 200, 1, 64, 90, 7, 130]],
+                         ids=["last", "spread", "two", "one", "seven", "parts"])
+def test_queue_uneven_entries(pkg, wl, dev, rows, fmt):
+    """Long entries among short ones, fewer entries than XCDs, and more of them than one launch takes: whole blocks of 64 rows
+    are dealt out over all blocks of the launch, and every row is computed once."""
+    H, I, E, A = 192, 320, 5, sum(rows)
+    shape = wl.MoeShape("queue", T=1, H=H, I=I, E=E, K=1, fmt=fmt, seed=len(rows))
+    blk, raw = wl.make_device_layer(shape, pkg.normal_table(), dev, keep_canonical=True)
+    w = blk.tensors
+    w2 = w["w_mlp2"].double() if fmt == "bf16" else pkg.dequant_mxfp4(raw["w_mlp2_blocks"], raw["w_mlp2_scales"]).double()
+    w2 = w2.view(E, H, I)
+    gate = torch.randn(A, I, device=dev)
+    tokens = torch.randperm(A, device=dev).int()
+    weights = torch.rand(A, device=dev) + 0.5
+    expert = torch.tensor([i * 3 % E for i in range(len(rows))], device=dev)
+    sizes = torch.tensor(rows, device=dev)
+    queue = torch.stack([expert, sizes.cumsum(0) - sizes, sizes], 1).int().contiguous()
+    want = torch.zeros(A, H, dtype=torch.float64, device=dev)
+    of_row = expert.repeat_interleave(sizes)
+    for e in range(E):
+        m = of_row == e
+        y = gate[m].bfloat16().double() @ w2[e].T + w["b_mlp2"].view(E, H)[e].double()
+        want[tokens[m].long()] = y * weights[m, None].double()
+    print("queue uneven", len(rows), max(rows), fmt, flush=True)
+    for hint in (max(rows), 100):
+        out = torch.zeros(A, H, device=dev)
+        if fmt == "bf16":
+            pkg.moe_mlp2_scatter(queue, 0, len(rows), gate, tokens, weights, out, w["w_mlp2"], w["b_mlp2"], I, H, I * H, H, hint, 0)
+        else:
+            pkg.moe_mlp2_scatter_mxfp4(queue, 0, len(rows), gate, tokens, weights, out, w["w_mlp2"], w["w_mlp2_scales"],
+                                       w["b_mlp2"], I, H, H, hint, 0)
+        # as in test_queue_entries; a row computed twice or not at all is off by its whole norm
+        assert ((out.double() - want).norm(dim=1) / want.norm(dim=1)).max().item() < 5e-5
+
+
+def queue_time(pkg, dev, w, H, I, rows, hint):
+    """us of one gate/up call, the best of five."""
+    queue, off = [], 0
+    for i, n in enumerate(rows):
+        queue += [i, off, n]
+        off += n
+    queue = torch.tensor(queue, dtype=torch.int32, device=dev)
+    x, gate = torch.randn(off, H, device=dev), torch.empty(off, I, device=dev)
+    us = []
+    for _ in range(6):
+        t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        t0.record()
+        pkg.moe_mlp1_swiglu(queue, 0, len(rows), x, gate, w["w_mlp1"], w["b_mlp1"], H, I, 2 * I * H, 2 * I, 1.702, 7.0, hint, 0)
+        t1.record()
+        torch.cuda.synchronize()
+        us.append(t0.elapsed_time(t1) * 1e3)
+    return min(us[1:])
+
+
+def test_queue_time_follows_the_rows_and_not_the_longest_entry(pkg, wl, dev):
+    """The same number of rows and of experts takes about the same time however they are spread over the entries: with a share
+    of the compute units to each entry the uneven queue took ten times as long."""
+    H, I, E = 2880, 2880, 32
+    shape = wl.MoeShape("queue", T=1, H=H, I=I, E=E, K=1, fmt="bf16", seed=1)
+    blk, _ = wl.make_device_layer(shape, pkg.normal_table(), dev)
+    even = queue_time(pkg, dev, blk.tensors, H, I, [128] * E, 128)
+    uneven = queue_time(pkg, dev, blk.tensors, H, I, [8] * (E - 1) + [128 * E - 8 * (E - 1)], 128 * E)
+    print("queue times", even, uneven, flush=True)
+    assert uneven < 3 * even
