@@ -343,7 +343,7 @@ static int queue_gemm(int epi, int format, const int* work_queue, int work_start
     a.weights_flat = weights_flat;
     a.work_queue = work_queue;
     a.work_start = work_start;
-    a.max_rows_hint = std::max(1, maxNe);
+    a.max_rows_hint = maxNe > 0 ? maxNe : 1 << 16;  // not said: enough blocks for long entries
     a.out = out;
     a.rows = rows;
     a.K = Kdim;
@@ -364,7 +364,7 @@ static int queue_gemm(int epi, int format, const int* work_queue, int work_start
         // Short entries: a tile of weight rows per wave (experts_small.hip).  The layer's calls with at most n rows an entry, us,
         // that kernel : producers and consumers: E = 32, bf16, n = 1 92 : 158, 4 176 : 227, 16 294 : 288; MXFP4, 4 92 : 98, 16
         // 124 : 120, 32 134 : 125; E = 128, bf16, 16 440 : 498, 32 675 : 658; MXFP4, 16 164 : 196.
-        if (maxNe <= 16 && expert_small_fits(0, rows, Kdim, format)) {
+        if (a.max_rows_hint <= 16 && expert_small_fits(0, rows, Kdim, format)) {
             a.waves_per_block = 18;
         } else if (format == MOE_WEIGHTS_MXFP4_TILED) {
             pick_stream_two_pass(rows, a.work_count, a.n_cus, &a.waves_per_block, &a.row_blocks);

@@ -206,7 +206,8 @@ MOE_API int moe_build_work_queue(const int* expert_offsets, int E, int* work_que
  * work_start: gate_by_expert[off+r, i] = swiglu(W1_e x_r + b1_e)[i] for the n rows
  * x_by_expert[off .. off+n).  W1 rows are interleaved gate, up, gate, up (src/run.cpp:667-670).
  * weights_base / bias_base point at the layer's first expert; strides are in elements.
- * maxNe is the largest row count in the queue (a smaller value is allowed: blocks then loop);
+ * maxNe is the largest row count in the queue, which chooses the kernel (a smaller value is allowed: blocks then
+ * loop, and <= 0 means that it is not known);
  * grid_cap is accepted for signature compatibility and ignored.  H % 64 == 0, I % 32 == 0. */
 MOE_API int moe_mlp1_swiglu(const int* work_queue, int work_start, int work_count, const float* x_by_expert,
                     float* gate_by_expert, const moe_bf16_t* weights_base, const moe_bf16_t* bias_base,

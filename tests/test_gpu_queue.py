@@ -181,3 +181,15 @@ def test_queue_time_follows_the_rows_and_not_the_longest_entry(pkg, wl, dev):
     uneven = queue_time(pkg, dev, blk.tensors, H, I, [8] * (E - 1) + [128 * E - 8 * (E - 1)], 128 * E)
     print("queue times", even, uneven, flush=True)
     assert uneven < 3 * even
+
+
+@pytest.mark.parametrize("rows,hint,limit", [([40] * 32, 1, 3.5), ([8] * 31 + [2048], 0, 1.5)], ids=["low", "unknown"])
+def test_queue_time_under_a_hint_that_is_too_low(pkg, wl, dev, rows, hint, limit):
+    """A hint below the row counts costs further passes over the weights, 32 rows each (two of them here, where one is enough
+    with the right hint), not a pass per few rows; a hint of 0 says nothing and costs nothing."""
+    shape = wl.MoeShape("queue", T=1, H=2880, I=2880, E=32, K=1, fmt="bf16", seed=1)
+    blk, _ = wl.make_device_layer(shape, pkg.normal_table(), dev)
+    right = queue_time(pkg, dev, blk.tensors, 2880, 2880, rows, max(rows))
+    low = queue_time(pkg, dev, blk.tensors, 2880, 2880, rows, hint)
+    print("queue times", right, low, flush=True)
+    assert low < limit * right
