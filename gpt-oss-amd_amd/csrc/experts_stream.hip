@@ -1117,9 +1117,11 @@ int launch_cfg(const ExpertGemmArgs& a, hipStream_t stream) {
             // Slots: one per entry, and more where that would leave compute units idle (two blocks to each, while the list may
             // be that long).  If even one slot per token block leaves some idle, the blocks get shorter.
             const long long blocks = (long long)a.work_count * ceil_div(a.max_rows_hint, 64);
-            if (blocks * b.row_blocks < a.n_cus) b.row_blocks = min(units, ceil_div(a.n_cus, (int)blocks));
+            if (blocks * b.row_blocks < a.n_cus) b.row_blocks = min(units, a.n_cus / (int)blocks);
             int slots = max(a.work_count, (int)min(blocks, (long long)ceil_div(2 * a.n_cus, b.row_blocks)));
-            b.xcd_tiles = slots >= 8;  // fewer slots would leave XCDs without one
+            // few slots that do not divide by the XCDs are spread over all of them: 12 entries would put twice as many blocks on
+            // four XCDs as on the others (12 short entries, MXFP4, gate/up + down 57 us : 37)
+            b.xcd_tiles = slots % 8 == 0 || slots > 32;
             if (b.xcd_tiles) slots = ceil_div(slots, 8) * 8;
             const dim3 grid(slots * b.row_blocks), block((cons + 4) * 64);
             const bool two = ceil_div(units, b.row_blocks) > cons;
