@@ -361,9 +361,12 @@ static int queue_gemm(int epi, int format, const int* work_queue, int work_start
     int rc = MOE_OK, left = work_count;
     do {
         a.work_count = std::min(left, kPart);
-        // Short entries: a tile of weight rows per wave (experts_small.hip).  The layer's calls with at most n rows an entry, us,
-        // that kernel : producers and consumers: E = 32, bf16, n = 1 92 : 158, 4 176 : 227, 16 294 : 288; MXFP4, 4 92 : 98, 16
-        // 124 : 120, 32 134 : 125; E = 128, bf16, 16 440 : 498, 32 675 : 658; MXFP4, 16 164 : 196.
+        // Short entries: a tile of weight rows per wave (experts_small.hip), up to 16 rows by the caller's hint.  The hint is often
+        // the batch's token count (the entries then hold a row or two, and few experts may have any), which is what the line is
+        // for: gate/up + down, us, that kernel : producers and consumers, entries of one row, MXFP4, 4 of them 19 : 26, 10 31 :
+        // 33, 20 49 : 53, 32 77 : 74, 36 86 : 118, 128 267 : 266; bf16, 4 44 : 42, 10 83 : 86, 20 160 : 181, 32 243 : 245, 36 294 :
+        // 328, 128 952 : 965; 22 entries of 16, 8, 5 .. 1 rows, MXFP4 56 : 60, bf16 173 : 190.  Entries that really hold 16 rows
+        // each are on the wrong side of it: 32 of them, MXFP4 114 : 84, bf16 286 : 257.
         if (a.max_rows_hint <= 16 && expert_small_fits(0, rows, Kdim, format)) {
             a.waves_per_block = 18;
         } else if (format == MOE_WEIGHTS_MXFP4_TILED) {
