@@ -498,7 +498,12 @@ int moe_mxfp4_tiled_to_bf16(const uint8_t* tiled_blocks, const uint8_t* tiled_sc
 size_t moe_block_workspace_bytes(int n_tokens, int hidden_dim, int intermediate_dim, int n_experts,
                                  int experts_per_token) {
     if (check_dims(n_tokens, hidden_dim, intermediate_dim, n_experts, experts_per_token) != MOE_OK) return 0;
-    return BlockWorkspace(nullptr, n_tokens, hidden_dim, intermediate_dim, n_experts, experts_per_token).bytes;
+    // What any batch of up to n_tokens takes: the routers' segment counts fall as tokens grow, at multiples of their tiles of 16
+    // and 64 tokens, so a smaller batch may need more.
+    size_t most = 0;
+    for (int t = n_tokens; t > 0; t = (t - 1) / 16 * 16)
+        most = std::max(most, BlockWorkspace(nullptr, t, hidden_dim, intermediate_dim, n_experts, experts_per_token).bytes);
+    return most;
 }
 
 struct moe_stage_timer {

@@ -50,6 +50,13 @@ def test_workspace_and_tiled_sizes(pkg):
     assert pkg.mxfp4_tiled_bytes(5760, 2881) == (0, 0)
 
 
+@pytest.mark.parametrize("E", [8, 32, 48, 64, 128, 256, 1000])
+def test_workspace_holds_every_smaller_batch(pkg, E):
+    """A workspace sized for n tokens serves batches of up to n: the size never falls as tokens grow."""
+    sizes = [pkg.block_workspace_bytes(T, 2880, 64, E, 4) for T in list(range(1, 1200)) + list(range(1200, 5000, 7))]
+    assert all(a <= b for a, b in zip(sizes, sizes[1:]))
+
+
 def test_entries_reject_bad_arguments_without_a_device(pkg):
     L = pkg.lib
     assert L.moe_topk(None, None, None, 1, 32, 4, None) == -1
