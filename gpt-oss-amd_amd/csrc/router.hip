@@ -813,8 +813,6 @@ int router_segments(int T, int E, int H, bool strict) {
     return S;
 }
 
-size_t router_partial_bytes(int T, int E) { return (size_t)16 * T * E * sizeof(double); }
-
 int launch_router_partial(const float* x, const uint16_t* w, double* partial, uint16_t* x_bf16, int T, int H,
                           int E, int S, hipStream_t stream) {
     int seg_len = ceil_div(ceil_div(H, S), 8) * 8;
@@ -838,18 +836,25 @@ int launch_router_partial(const float* x, const uint16_t* w, double* partial, ui
 
 // ---- two-pass router -----------------------------------------------------------------------------
 // Worth it once the exact pass is throughput bound (three vector instructions per term), or once the fused kernel (a block
-// per token) would need a second round of blocks over the 256 compute units.  Block of tiny experts, us, fused : two-pass:
-// E = 32, 512 tokens 75 : 80, 700 tokens 90 : 87, 1000 tokens 113 : 103, 1500 tokens 136 : 113; E = 96, 256 tokens 80 : 85,
-// 350 tokens 102 : 89; E = 128, 256 tokens 84 : 84, 350 tokens 109 : 90.
+// per token) would need a second round of blocks over the 256 compute units (the lines below are its rounds there, not asked
+// of the device).  With up to 32 experts a block holds a wave per two of them, several blocks share a compute unit, and
+// what counts is scores per batch.  Block of tiny experts, rows of 2880, us, fused : two-pass: E = 8, 900 tokens 80 : 91, 2047
+// 104 : 112; E = 16, 900 tokens 85 : 91, 1400 102 : 103; E = 24, 769 tokens 91 : 90, 1100 102 : 98; E = 32, 513 tokens 81 : 78, 640
+// 89 : 87, 1100 113 : 97; E = 48, 257 tokens 54 : 57, 400 61 : 63, 513 71 : 64; E = 64, 256 tokens 48 : 57, 257 59 : 57, 640 84 : 71;
+// E = 128, 256 tokens 62 : 62, 257 82 : 63.
 bool router_two_pass(int T, int E, int H) {
-    return H % 32 == 0 && ((long long)T * E >= 65536 || T > (E <= 32 ? 640 : 256));
+    if (H % 32 != 0) return false;
+    const long long scores = (long long)T * E;
+    if (scores >= 65536) return true;
+    return E > 48 ? T > 256 : E > 32 ? T > 512 : E > 16 && scores >= 20480;
 }
 
 // Partial sums and finalize in two launches instead of the fused kernel: beyond 32 experts its eight waves score a token's
 // experts in passes of 32, a memory round trip each, while few tokens leave most compute units idle.  The same block, us, fused :
-// two launches: E = 64, 1 token 35 : 31, 128 tokens 63 : 61, 200 tokens 66 : 70; E = 128, 1 token 45 : 33, 33 tokens 65 : 53, 128
-// tokens 79 : 74; E = 1000, 16 tokens 199 : 92.  Up to 32 experts one launch is the faster one (256 tokens 59 : 63).
-bool router_split(int T, int E) { return E > 32 && T <= 128; }
+// two launches: E = 33, 1 token 24 : 24, 32 30 : 31, 128 37 : 38; E = 48, 1 token 29 : 24, 8 29 : 28, 64 32 : 33, 128 38 : 39; E = 64, 1
+// token 28 : 24, 64 36 : 34, 128 40 : 38, 200 46 : 49; E = 128, 1 token 39 : 26, 33 tokens 55 : 44, 128 57 : 53; E = 1000, 16 tokens
+// 199 : 92.  Up to 32 experts one launch is the faster one (1 token 22 : 24, 8 25 : 27, 256 41 : 45).
+bool router_split(int T, int E) { return E > 32 && T <= (E > 48 ? 128 : 16); }
 
 static int screen_tiles(int E) { return E <= 16 ? 1 : E <= 32 ? 2 : 4; }  // 16-expert tiles per wave
 

@@ -5,18 +5,37 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
+FUSED, SPLIT, TWO = "router_fused_kernel", "router_partial_kernel + router_finalize_kernel", "router_screen_kernel + router_refine_kernel"
+# experts -> tokens and the router of rows that the one-launch kernel takes, on both sides of each line
+LINES = {
+    8: [(1, FUSED), (2048, FUSED), (8191, FUSED), (8192, TWO)],
+    16: [(2048, FUSED), (4095, FUSED), (4096, TWO)],
+    17: [(1204, FUSED), (1205, TWO)],
+    32: [(1, FUSED), (639, FUSED), (640, TWO), (641, TWO), (2047, TWO), (2048, TWO)],
+    33: [(1, SPLIT), (16, SPLIT), (17, FUSED), (128, FUSED), (129, FUSED), (512, FUSED), (513, TWO)],
+    48: [(16, SPLIT), (17, FUSED), (512, FUSED), (513, TWO)],
+    49: [(128, SPLIT), (129, FUSED), (256, FUSED), (257, TWO)],
+    250: [(5, SPLIT), (128, SPLIT), (129, FUSED), (256, FUSED), (257, TWO), (263, TWO)],
+    257: [(128, SPLIT), (129, FUSED), (255, FUSED), (256, TWO)],
+    1000: [(1, SPLIT), (65, SPLIT), (66, TWO), (128, TWO), (129, TWO)],
+}
+
 
 @pytest.mark.parametrize("H", [64, 2880, 3136])  # the last is too long for the one-launch kernel
-@pytest.mark.parametrize("E,tokens", [(32, (1, 640, 641, 2047, 2048)), (33, (1, 128, 129, 256, 257)), (250, (5, 128, 129, 256, 263))])
-def test_router_kernels_agree(pkg, wl, dev, H, E, tokens):
+@pytest.mark.parametrize("E", LINES)
+def test_router_kernels_agree(pkg, wl, dev, H, E):
     table = pkg.normal_table()
-    shape = wl.MoeShape("router", T=max(tokens), H=H, I=64, E=E, K=4, fmt="mxfp4", seed=H + E)
+    most = max(T for T, _ in LINES[E])
+    shape = wl.MoeShape("router", T=most, H=H, I=64, E=E, K=4, fmt="mxfp4", seed=H + E)
     blk, _ = wl.make_device_layer(shape, table, dev)
     x = wl.make_device_input(shape, table, dev)
-    for T in tokens:
+    for T, router in LINES[E]:
         print("router", H, E, T, flush=True)
         t = x[:T].contiguous()
         _, ti, tv = blk.forward(t)
+        if H > 3072 and router == FUSED:
+            router = SPLIT
+        assert blk.describe(blk.params(t, x, ti, tv))["router"] == router
         _, wi, wv = blk.forward(t, flags=pkg.MOE_FLAG_ROUTER_STRICT_ORDER)
         assert torch.equal(ti, wi)
         # logits differ, if at all, in the last place of their rounding to fp32: 2^-23 of |logit| < 16
