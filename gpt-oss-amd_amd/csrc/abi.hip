@@ -56,13 +56,21 @@ inline bool use_direct_bucketing(int T, int K, int E, bool prefill, unsigned fla
 
 // The kernels for a handful of rows per expert (experts_small.hip).  They keep every compute unit busy whatever share of the
 // experts has rows; the producer/consumer kernels have the better rate once all blocks of one round have work.  Whole
-// block, 20b / 120b shapes, small : streaming kernels, us.  Where these come in one round of blocks (E = 32, MXFP4), 7 tokens
-// 57 : 65, 10 tokens 62 : 67, 16 tokens 80 : 76; in several rounds, E = 32, bf16: 7 tokens 168 : 210, 24 tokens 255 : 254, 32
-// skewed 255 : 241; E = 128, MXFP4: 33 tokens 199 : 236, 96 tokens 281 : 285; E = 128, bf16: 33 tokens 650 : 808.
+// block, small : streaming kernels, us, weights from HBM (layers in turn), router of no preference, then skewed.  Where these come
+// in one round of blocks: E = 32, MXFP4, 7 tokens 62 : 66, 56 : 63, 10 tokens 74 : 70, 63 : 65, 16 tokens 81 : 76, 68 : 68; in
+// several rounds: E = 32, bf16, 7 tokens 205 : 231, 145 : 208, 16 tokens 243 : 245, 224 : 226, 24 tokens 257 : 255, 229 : 236; E = 128,
+// MXFP4, 48 tokens 233 : 251, 155 : 190, 96 tokens 274 : 276, 216 : 242; E = 128, bf16, weights once a call, 96 tokens 937 : 962, 703 :
+// 872.  A hot expert's further passes over its weights (32 rows each) don't turn that round.
 inline bool use_small_kernels(int T, int H, int I, int K, int E, int format, bool direct, unsigned flags, int n_cus) {
     if (!direct || (flags & (MOE_FLAG_FORCE_STREAM | MOE_FLAG_FORCE_DIRECT | MOE_FLAG_FUSED_GEMM_LAUNCH))) return false;
     if (!expert_small_fits(T * K, 2 * I, H, format) || !expert_small_fits(T * K, H, I, format)) return false;
-    const long long blocks = (long long)E * ceil_div(2 * I / 32, format == MOE_WEIGHTS_MXFP4_TILED ? 24 : 12);
+    const bool mxfp4 = format == MOE_WEIGHTS_MXFP4_TILED;
+    // Many blocks of a stage or two each are mostly their start: E = 512, MXFP4, H = 2880, I = 64, 32 tokens 72 : 78, 64 tokens
+    // 92 : 91, 128 tokens 129 : 103.
+    const int items = std::min(T * K, E);
+    if (mxfp4 && ((I <= 256 && items * ceil_div(H, 128) > 16 * n_cus) || (H <= 256 && items * ceil_div(2 * I, 128) > 16 * n_cus)))
+        return false;
+    const long long blocks = (long long)E * ceil_div(2 * I / 32, mxfp4 ? 24 : 12);
     return 4LL * T * K <= (blocks > n_cus ? 12LL : 5LL) * E;
 }
 

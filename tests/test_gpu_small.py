@@ -48,6 +48,21 @@ def test_small_kernel_finds_its_experts(pkg, wl, dev, T, E, K):
         assert torch.equal(y, want)
 
 
+@pytest.mark.parametrize("T,H,I,small", [(32, 2880, 64, True), (48, 2880, 64, False), (48, 2880, 320, True), (48, 64, 1472, False)])
+def test_many_short_mxfp4_blocks_go_to_the_streaming_kernels(pkg, wl, dev, T, H, I, small):
+    """More than 16 blocks per compute unit of at most two stages of 128."""
+    E, K = 512, 4
+    table = pkg.normal_table()
+    shape = wl.MoeShape("small", T=T, H=H, I=I, E=E, K=K, fmt="mxfp4", seed=T)
+    blk, _ = wl.make_device_layer(shape, table, dev)
+    x = wl.make_device_input(shape, table, dev)
+    print("small kernel", shape, flush=True)
+    y, ti, _ = blk.forward(x)
+    assert blk.describe(blk.params(x, y, ti, y))["down"].startswith("expert_small" if small else "expert_stream_direct")
+    want, _, _ = blk.forward(x, flags=pkg.MOE_FLAG_FORCE_DIRECT)
+    assert torch.equal(y, want)
+
+
 @pytest.mark.parametrize("fmt", ["bf16", "mxfp4"])
 def test_ids_that_name_no_expert_are_skipped(pkg, wl, dev, fmt):
     """The down GEMM entry takes its assignment list from the caller: ids outside [0, E) write no row and change no other."""
