@@ -32,15 +32,18 @@ inline int tile_tokens_of(bool prefill, int format) {
 // Which family runs the expert GEMMs, by average bucket size T*K/E (measured crossovers, 20b
 // shapes, token counts 256..4096).  MXFP4: the 128-token-block kernels win as soon as buckets start
 // to overflow one 64-token block (the streaming kernel then reads an expert's weights once per
-// block of its bucket).  bf16, streaming kernels against 256-token blocks: E = 32, 302 : 340 us at 44 rows per expert,
-// 373 : 343 at 48, 455 : 347 at 56; E = 128, 1199 : 1228 at 44, 1329 : 1246 at 50.
+// block of its bucket).  bf16: past the 48 rows per expert where the streaming kernels bucket in the expert kernels.  Streaming
+// kernels : 256-token blocks, us, at 46 / 48 / 50 / 52 rows per expert: E = 32, router of no preference, 307 : 336, 309 : 337, 330 :
+// 338, 450 : 339 (below the line no bucket has more than 64 rows there; one that has, as one in six layers at 48 rows, takes a
+// second pass: 440), mildly skewed (Zipf 0.4) 435 : 343, 442 : 344, 446 : 346, 455 : 346; E = 64, K = 8, 48 rows 174 : 201, 50 rows
+// 233 : 202; E = 128, 44 rows 1183 : 1224, 46 rows 1295 : 1230.
 inline bool use_prefill_kernels(int T, int H, int I, int K, int E, int format, unsigned flags) {
     if (flags & MOE_FLAG_FORCE_STREAM) return false;
     const long long rows = (long long)T * K;
     // activation tensors past 4 GiB: only the streaming kernels address them
     if (format == MOE_WEIGHTS_BF16 && !(expert_tile_fits(T, 2 * I, H) && expert_tile_fits(rows, H, I))) return false;
     if (flags & MOE_FLAG_FORCE_TILED) return true;
-    return format == MOE_WEIGHTS_MXFP4_TILED ? rows >= 52LL * E : rows >= 46LL * E;
+    return format == MOE_WEIGHTS_MXFP4_TILED ? rows >= 52LL * E : rows > 48LL * E;
 }
 
 // Bucketing inside the expert kernels instead of a launch of its own: for the weight-streaming

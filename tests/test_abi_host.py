@@ -57,6 +57,26 @@ def test_workspace_holds_every_smaller_batch(pkg, E):
     assert all(a <= b for a, b in zip(sizes, sizes[1:]))
 
 
+def kernels_of(pkg, T, H, I, E, K, fmt, flags=0):
+    p = pkg.BlockParams(struct_bytes=ctypes.sizeof(pkg.BlockParams), n_tokens=T, hidden_dim=H, intermediate_dim=I, n_experts=E,
+                        experts_per_token=K, weight_format=fmt, flags=flags)
+    text = ctypes.create_string_buffer(1024)
+    assert pkg.lib.moe_block_describe(ctypes.byref(p), text, len(text)) == 0
+    return dict(part.split("=", 1) for part in text.value.decode().split("; "))
+
+
+@pytest.mark.parametrize("E,K", [(32, 4), (128, 4), (8, 2), (64, 8)])
+def test_expert_kernel_families_by_rows(pkg, E, K):
+    """Both sides of the lines where the token-block kernels start: past 48 rows per expert (bf16), at 52 (MXFP4)."""
+    for fmt, last, stream, tiled in ((pkg.MOE_WEIGHTS_BF16, 48 * E // K, "expert_stream_direct", "expert_tile_bf16"),
+                                     (pkg.MOE_WEIGHTS_MXFP4_TILED, 52 * E // K - 1, "expert_stream_ws", "expert_prefill")):
+        if last * K > 4096:  # past the longest list that the expert kernels scan
+            stream = "expert_stream_ws"
+        for T, name in ((last, stream), (last + 1, tiled)):
+            k = kernels_of(pkg, T, 2880, 2880, E, K, fmt)
+            assert k["gate_up"].startswith(name) and k["down"].startswith(name), (T, k)
+
+
 def test_entries_reject_bad_arguments_without_a_device(pkg):
     L = pkg.lib
     assert L.moe_topk(None, None, None, 1, 32, 4, None) == -1
