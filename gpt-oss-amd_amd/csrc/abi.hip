@@ -609,11 +609,13 @@ struct ExpertPlan {
             a.s_expert_stride = (long long)sb;
         }
     }
-    // MXFP4 prefill launches of at most two and a half rounds of blocks (two to a compute unit): what counts is how evenly they
-    // end, so the largest token blocks come first in both GEMMs and the XCDs get equal shares (two parts to a token block).
-    // Block of 32 experts, us, otherwise : so: 416 tokens skewed 186 : 164, 1000 tokens 279 : 252, skewed 272 : 265, 1600 tokens
-    // skewed 361 : 347, 2500 tokens 493 : 496, skewed 500 : 487; 4096 tokens 746 : 759; 128 experts, 1700 tokens skewed 582 : 586.
-    bool few_blocks() const { return (long long)est_tiles * ceil_div(p->hidden_dim, 256) < 5LL * n_cus; }
+    // MXFP4 prefill launches of at most two and a half rounds of blocks (two to a compute unit), by the launch's own count: what
+    // counts is how evenly they end, so the largest token blocks come first and the XCDs get equal shares (two parts to a token
+    // block).  Block of 32 experts, us, neither launch so : gate/up : down : both.  Router of no preference, 700 tokens 208 : 211 :
+    // 207 : 209, 1000 tokens 282 : 288 : 257 : 262, 2000 tokens 431 : 435 : 423 : 424, 2700 tokens 539 : 540 : 542 : 545; skewed, 416 tokens
+    // 193 : 189 : 174 : 170, 1000 tokens 302 : 301 : 278 : 276, 2000 tokens 427 : 430 : 422 : 426, 2700 tokens 555 : 558 : 542 : 547; 8
+    // experts, 2400 tokens skewed 286 : 283 : 269 : 262, 3200 tokens 360 : 345 : 360 : 346.
+    bool few_blocks(int rows) const { return (long long)est_tiles * ceil_div(rows, 256) < 5LL * n_cus; }
     void use_second_map(ExpertGemmArgs& a) const {
         a.tile_expert += second_map;
         a.tile_row0 += second_map;
@@ -631,7 +633,7 @@ struct ExpertPlan {
         // row blocks on one XCD takes 1 % off the bf16 launch (its token rows enter one L2 instead of eight) and
         // leaves the MXFP4 launch as it is; with token blocks from the tile map it cost up to 2 %
         a.xcd_tiles = direct ? 1 : 0;
-        if (a.waves_per_block == 16) a.xcd_tiles = few_blocks() ? 2 : 1;
+        if (a.waves_per_block == 16) a.xcd_tiles = few_blocks(a.rows) ? 2 : 1;
         if (a.waves_per_block == 17) use_second_map(a);  // places an expert's blocks by where its tiles begin
         return a;
     }
@@ -647,7 +649,7 @@ struct ExpertPlan {
         // (largest first: the launch's tail is made of short blocks); the down GEMM is 2 % faster in bucket
         // order, where a partial block runs next to full blocks of its expert and finds the expert's weights
         // on their way through the caches.
-        const bool few = a.waves_per_block == 16 && few_blocks();
+        const bool few = a.waves_per_block == 16 && few_blocks(a.rows);
         if (!direct && !few) use_second_map(a);
         // measured: the down GEMM gains 4-10 % from keeping a token block on one XCD (its input rows were
         // written by the gate/up launch just before)

@@ -6,8 +6,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-# one to five row blocks of 256 rows in the two launches, an odd last one among them; 1 to 1000 token blocks
-@pytest.mark.parametrize("H,I", [(64, 64), (320, 192), (576, 640), (1088, 128)])
+# one to five row blocks of 256 rows in the two launches, an odd last one among them; 2 to 694 token blocks; with the most of
+# them either launch, both or neither has few blocks
+@pytest.mark.parametrize("H,I", [(64, 64), (320, 192), (576, 640), (1088, 128), (64, 640)])
 @pytest.mark.parametrize("T,E,K,zipf_s", [(1, 4, 2, 0.0), (700, 32, 4, 1.2), (1500, 6, 2, 3.0), (900, 130, 8, 0.0), (9000, 130, 8, 0.5)])
 def test_prefill_blocks_cover_every_row(pkg, wl, dev, H, I, T, E, K, zipf_s):
     table = pkg.normal_table()
