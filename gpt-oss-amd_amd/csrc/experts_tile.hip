@@ -86,7 +86,7 @@ MOE_DEVICE void tile_body(const ExpertGemmArgs& a, uint8_t* lds, int e, int row0
     for (int i = 0; i < PT; ++i) {
         const int row = 8 * (wave + 8 * i) + sub;
         const int idx = min(row, nrows - 1);  // places past the bucket's end hold its last row again, never stored
-        const int src = a.gather ? a.tokens_flat[row0 + idx] : row0 + idx;
+        const int src = a.gather ? a.tokens_flat[row0 + idx] : idx;  // rows by slot: counted from the block's first
         off_t[i] = (uint32_t)src * (uint32_t)K * 2u + (uint32_t)(((lane & 7) ^ tile_swz(row & 15)) * 16);
     }
 #pragma unroll
@@ -95,7 +95,7 @@ MOE_DEVICE void tile_body(const ExpertGemmArgs& a, uint8_t* lds, int e, int row0
         const int w_row = min((group0 + (row >> 6)) * 64 + tile_row_in_group((row >> 4) & 3, row & 15), a.rows - 1);
         off_w[i] = (uint32_t)w_row * (uint32_t)K * 2u + (uint32_t)(((lane & 7) ^ tile_swz(row & 15)) * 16);
     }
-    const uint8_t* const base_t = reinterpret_cast<const uint8_t*>(a.act);
+    const uint8_t* const base_t = reinterpret_cast<const uint8_t*>(a.act + (a.gather ? 0 : (size_t)row0 * K));
     const uint8_t* const base_w =
         reinterpret_cast<const uint8_t*>(reinterpret_cast<const uint16_t*>(a.w) + (size_t)e * a.w_expert_stride);
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
@@ -224,9 +224,9 @@ __global__ __launch_bounds__(512, 2) void expert_tile_bf16_kernel(ExpertGemmArgs
 
 }  // namespace
 
-// The kernel addresses an expert's matrix and the whole activation tensor by 32-bit byte offsets.
-bool expert_tile_fits(long long act_rows, int rows, int K) {
-    return act_rows * K * 2 <= 0xffffffffll && (long long)rows * K * 2 <= 0xffffffffll;
+// The kernel addresses an expert's matrix and gathered activation rows by 32-bit byte offsets (rows by slot: inside a block).
+bool expert_tile_fits(long long gathered_rows, int rows, int K) {
+    return gathered_rows * K * 2 <= 0xffffffffll && (long long)rows * K * 2 <= 0xffffffffll;
 }
 
 int launch_expert_tile_bf16(const ExpertGemmArgs& a, int epi, hipStream_t stream) {

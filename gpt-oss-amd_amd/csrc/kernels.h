@@ -108,7 +108,7 @@ struct ExpertGemmArgs {
 int launch_expert_stream(const ExpertGemmArgs& a, int epi, hipStream_t stream);
 
 // ---- experts_tile.hip: prefill-sized buckets of bf16 experts (token blocks of up to 256 rows) ----
-bool expert_tile_fits(long long act_rows, int rows, int K);
+bool expert_tile_fits(long long gathered_rows, int rows, int K);
 int launch_expert_tile_bf16(const ExpertGemmArgs& a, int epi, hipStream_t stream);
 int expert_direct_max_assignments();
 

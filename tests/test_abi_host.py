@@ -77,6 +77,13 @@ def test_expert_kernel_families_by_rows(pkg, E, K):
             assert k["gate_up"].startswith(name) and k["down"].startswith(name), (T, k)
 
 
+def test_tile_kernel_takes_large_activation_tensors(pkg):
+    """Rows by slot past 4 GiB are no reason to leave the bf16 tile kernel; gathered rows past it are, at the last byte."""
+    for T, H, I, K, name in ((65535, 64, 8192, 8, "expert_tile_bf16"), (65535, 2880, 14336, 8, "expert_tile_bf16"),
+                             (65535, 32768, 64, 1, "expert_tile_bf16"), (65535, 32832, 64, 1, "expert_stream_ws")):
+        assert kernels_of(pkg, T, H, I, 8, K, pkg.MOE_WEIGHTS_BF16)["down"].startswith(name), (T, H, I, K)
+
+
 def test_entries_reject_bad_arguments_without_a_device(pkg):
     L = pkg.lib
     assert L.moe_topk(None, None, None, 1, 32, 4, None) == -1

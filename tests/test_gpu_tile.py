@@ -39,3 +39,18 @@ def test_tile_kernel_uneven_buckets(pkg, wl, dev, T, E, K, zipf_s):
     y, ti, _ = blk.forward(x, flags=pkg.MOE_FLAG_FORCE_TILED)
     want, _, _ = blk.forward(x, flags=pkg.MOE_FLAG_FORCE_STREAM)
     assert torch.equal(y, want)
+
+
+def test_tile_kernel_rows_past_4_gib(pkg, wl, dev):
+    """The down GEMM's activation rows, by slot, end past byte 2^32."""
+    T, H, I, E, K = 32800, 64, 8192, 8, 8
+    assert T * K * I * 2 > 1 << 32
+    table = pkg.normal_table()
+    shape = wl.MoeShape("tile", T=T, H=H, I=I, E=E, K=K, fmt="bf16", seed=3)
+    blk, _ = wl.make_device_layer(shape, table, dev)
+    x = wl.make_device_input(shape, table, dev)
+    print("tile kernel", shape, flush=True)
+    y, ti, _ = blk.forward(x)
+    assert blk.describe(blk.params(x, y, ti, y))["down"] == "expert_tile_bf16_kernel<1>"
+    want, _, _ = blk.forward(x, flags=pkg.MOE_FLAG_FORCE_STREAM)
+    assert torch.equal(y, want)
