@@ -33,15 +33,16 @@ MOE_DEVICE int tile_swz(int q) {
 
 // 64 lanes x 16 bytes from base + the lane's 32-bit offset to 1 KiB of LDS at a wave-uniform address.  In assembly: the
 // compiler puts a wait for every direct-to-LDS load it knows of in front of the wave's next LDS read, so loads that
-// run a stage ahead must be invisible to it.  They count in vmcnt; the caller waits.  Writes M0.
+// run a stage ahead must be invisible to it.  They count in vmcnt; the caller waits.  Writes M0, which the compiler
+// reserves and does not take in a clobber list: nothing else in a kernel that calls this may use it.
 MOE_DEVICE void tile_dma16(const void* base_uniform, uint32_t lane_off, uint32_t lds_addr_uniform) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(base_uniform),
                  "s"(lds_addr_uniform)
                  : "memory");
 }
 
-// All loads of this wave but the YOUNGER last ones have landed and all its LDS reads are back; then the block's barrier.  One statement with a
-// memory clobber, so that no LDS access of the compiler's moves across the barrier.
+// All loads of this wave but the YOUNGER last ones have landed and all its LDS reads are back; then the block's barrier.  One
+// statement with a memory clobber, so that no LDS access of the compiler's moves across the barrier.
 template <int YOUNGER>
 MOE_DEVICE void wait_and_meet() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(YOUNGER) : "memory");

@@ -7,8 +7,8 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# T, H, I, E, K, fmt -> bucketing inside the expert kernels / bucketing launch + 64-token blocks /
-# 128-token blocks (both MXFP4 and the two bf16 kernels) / two-pass router
+# T, H, I, E, K, fmt -> a handful of rows per expert / bucketing inside the expert kernels / bucketing launch + 64-token
+# blocks / 128-token blocks (MXFP4) and 256-token blocks (bf16) / the three routers
 FUSED = 32  # MOE_FLAG_FUSED_GEMM_LAUNCH: both expert GEMMs in one launch (counters cleared by a kernel)
 CASES = [
     (64, 256, 128, 8, 4, "mxfp4"),
@@ -16,12 +16,15 @@ CASES = [
     (64, 256, 128, 8, 4, "mxfp4", FUSED),
     (96, 320, 192, 16, 4, "bf16", FUSED),
     (300, 192, 128, 8, 1, "mxfp4"),
-    (260, 320, 192, 4, 1, "bf16"),      # 65 rows per expert: two blocks a compute unit
-    (700, 320, 192, 8, 4, "bf16"),      # 350 rows per expert: one block a compute unit
+    (260, 320, 192, 4, 1, "bf16"),      # 65 rows per expert: one partial token block each
+    (700, 320, 192, 8, 4, "bf16"),      # 350 rows per expert: a full and a partial token block each
     (700, 320, 192, 8, 4, "mxfp4"),
     (2100, 128, 64, 32, 2, "mxfp4"),    # T x E >= 65536: the two-pass router
     (1200, 128, 64, 128, 4, "mxfp4"),   # 4800 assignments, 37 rows per expert: bucketing launch + 64-token blocks
     (1200, 128, 64, 128, 4, "bf16"),
+    (5, 256, 128, 16, 2, "mxfp4"),      # under one row per expert: a tile of weight rows per wave
+    (5, 256, 128, 16, 2, "bf16"),
+    (20, 320, 192, 64, 4, "mxfp4"),     # the same behind partial sums and finalize
 ]
 
 
@@ -71,12 +74,14 @@ def test_graph_replays_equal_the_eager_call(pkg, wl, oracle, dev, case):
         assert torch.equal(got[0], ref[0])
 
 
-def test_two_streams_do_not_share_state(pkg, wl, oracle, dev):
+@pytest.mark.parametrize("cases", [((256, 256, 128, 8, 4, "mxfp4"), (700, 320, 192, 8, 4, "bf16")),
+                                   ((5, 256, 128, 16, 2, "mxfp4"), (20, 320, 192, 64, 4, "bf16"))], ids=["large", "small"])
+def test_two_streams_do_not_share_state(pkg, wl, oracle, dev, cases):
     """Two calls with their own workspaces on two streams at once (default priority) give the bits each gives
     alone: the library keeps nothing between or across calls."""
     table = oracle.normal_table()
     jobs = []
-    for T, H, I, E, K, fmt in ((256, 256, 128, 8, 4, "mxfp4"), (700, 320, 192, 8, 4, "bf16")):
+    for T, H, I, E, K, fmt in cases:
         shape = wl.MoeShape("streams", T=T, H=H, I=I, E=E, K=K, fmt=fmt, seed=T)
         blk, raw = wl.make_device_layer(shape, table, dev)
         x = wl.make_device_input(shape, table, dev)
@@ -99,3 +104,60 @@ def test_two_streams_do_not_share_state(pkg, wl, oracle, dev):
         torch.cuda.synchronize()
         for blk, raw, x, p, out, alone in jobs:
             assert all(torch.equal(o, a) for o, a in zip(out, alone))
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "mxfp4"])
+@pytest.mark.parametrize("rows", [[3, 0, 1, 2], [100, 0, 17, 300]], ids=["short", "long"])
+def test_graph_replays_of_the_queue_entries(pkg, wl, dev, rows, fmt):
+    """The work-queue entries in a captured graph, one assignment to a token (the atomic sums then have one term): the queue is
+    read on the device, so replays follow what it holds."""
+    H, I, E, A = 320, 192, len(rows), sum(rows)
+    shape = wl.MoeShape("queue", T=A, H=H, I=I, E=E, K=1, fmt=fmt, seed=A)
+    blk, _ = wl.make_device_layer(shape, pkg.normal_table(), dev)
+    w = blk.tensors
+    x = wl.make_device_input(shape, pkg.normal_table(), dev)
+    tokens = torch.randperm(A, device=dev).int()
+    weights = torch.rand(A, device=dev)
+    gate, out = torch.empty(A, I, device=dev), torch.empty(A, H, device=dev)
+    queues = []
+    for order in (rows, rows[::-1]):
+        off, q = 0, []
+        for e, n in enumerate(order):
+            q += [e, off, n]
+            off += n
+        queues.append(torch.tensor(q, dtype=torch.int32, device=dev))
+    queue = queues[0].clone()
+
+    def calls(stream):
+        out.zero_()
+        if fmt == "bf16":
+            pkg.moe_mlp1_swiglu(queue, 0, E, x, gate, w["w_mlp1"], w["b_mlp1"], H, I, 2 * I * H, 2 * I, 1.702, 7.0, max(rows), 0,
+                                stream=stream)
+            pkg.moe_mlp2_scatter(queue, 0, E, gate, tokens, weights, out, w["w_mlp2"], w["b_mlp2"], I, H, I * H, H, max(rows), 0,
+                                 stream=stream)
+        else:
+            pkg.moe_mlp1_swiglu_mxfp4(queue, 0, E, x, gate, w["w_mlp1"], w["w_mlp1_scales"], w["b_mlp1"], H, I, 2 * I, 1.702, 7.0,
+                                      max(rows), 0, stream=stream)
+            pkg.moe_mlp2_scatter_mxfp4(queue, 0, E, gate, tokens, weights, out, w["w_mlp2"], w["w_mlp2_scales"], w["b_mlp2"], I, H,
+                                       H, max(rows), 0, stream=stream)
+
+    def eager(q):
+        queue.copy_(q)
+        calls(None)
+        torch.cuda.synchronize()
+        return gate.clone(), out.clone()
+
+    print("queue graph", rows, fmt, flush=True)
+    want = [eager(q) for q in queues]
+    assert not torch.equal(want[0][1], want[1][1])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        calls(torch.cuda.current_stream())
+    for rep in range(4):
+        queue.copy_(queues[rep % 2])
+        gate.fill_(float("nan"))
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(gate, want[rep % 2][0]) and torch.equal(out, want[rep % 2][1]), rep
+        assert torch.equal(eager(queues[rep % 2])[1], want[rep % 2][1])
