@@ -7,6 +7,7 @@
 // 1077 us).  Here a stage brings 64 KiB for the same work, and an XCD's blocks share it: 1.4 to 2.1 GB, 484 to 525 us,
 // i.e. 1.1 PFLOP/s (down launch 564 -> 287 us).  Of the parts on their own, at that size: matrix instructions and epilogues
 // 366 us, fragment reads from LDS 284, loads into LDS 247 from L2 and 435 from where the data are.
+#include <algorithm>
 #include <type_traits>
 
 #include "expert_tiles.h"
@@ -225,9 +226,10 @@ __global__ __launch_bounds__(512, 2) void expert_tile_bf16_kernel(ExpertGemmArgs
 
 }  // namespace
 
-// The kernel addresses an expert's matrix and gathered activation rows by 32-bit byte offsets (rows by slot: inside a block).
+// The kernel addresses an expert's matrix and gathered activation rows by 32-bit byte offsets (rows by slot: the 256 of a
+// block).
 bool expert_tile_fits(long long gathered_rows, int rows, int K) {
-    return gathered_rows * K * 2 <= 0xffffffffll && (long long)rows * K * 2 <= 0xffffffffll;
+    return std::max(gathered_rows, 256ll) * K * 2 <= 0xffffffffll && (long long)rows * K * 2 <= 0xffffffffll;
 }
 
 int launch_expert_tile_bf16(const ExpertGemmArgs& a, int epi, hipStream_t stream) {

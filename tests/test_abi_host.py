@@ -78,8 +78,10 @@ def test_expert_kernel_families_by_rows(pkg, E, K):
 
 
 def test_tile_kernel_takes_large_activation_tensors(pkg):
-    """Rows by slot past 4 GiB are no reason to leave the bf16 tile kernel; gathered rows past it are, at the last byte."""
+    """Rows by slot past 4 GiB are no reason to leave the bf16 tile kernel, unless the 256 of one block are; gathered rows past it
+    are, at the last byte."""
     for T, H, I, K, name in ((65535, 64, 8192, 8, "expert_tile_bf16"), (65535, 2880, 14336, 8, "expert_tile_bf16"),
+                             (4000, 64, 8388544, 1, "expert_tile_bf16"), (4000, 64, 8388608, 1, "expert_stream_ws"),
                              (65535, 32768, 64, 1, "expert_tile_bf16"), (65535, 32832, 64, 1, "expert_stream_ws")):
         assert kernels_of(pkg, T, H, I, 8, K, pkg.MOE_WEIGHTS_BF16)["down"].startswith(name), (T, H, I, K)
 
