@@ -7,7 +7,7 @@
 // 768 weight rows, one to a compute unit: one token's four experts occupy 32 of 256 compute units, and the 20 experts of
 // seven tokens are 320 blocks, i.e. two rounds for the work of 1.25.  Here the bucket's few rows are staged once, whole,
 // the stage barriers go, and the work is cut by MFMA tile.  Gate/up + down launch, us: one token, E = 32 MXFP4 25 + 15 -> 10 + 7
-// (2.1 TB/s in the larger: ids, rows and weights are a chain of three round trips), bf16 124 + 65 -> 25 + 14; 7 tokens, E = 32
+// (3.4 TB/s in the larger: ids, rows and weights are a chain of three round trips), bf16 124 + 65 -> 25 + 14; 7 tokens, E = 32
 // bf16 138 + 66 -> 105 + 52 (6.2 TB/s); 33 tokens, E = 128 MXFP4 116 + 70 -> 108 + 59 (6.8).  Two tiles a wave, and three
 // blocks a compute unit instead of two: no faster.
 #include <type_traits>

@@ -5,8 +5,8 @@
 // What bounds it: with 128 tokens to a block the launch was bound by the weights on their way to the compute units
 // (96 KiB a CU for every 2048 cycles of matrix work; 5.1 GB into the L2s per gate/up launch at 4096 tokens x 32 experts,
 // 1077 us).  Here a stage brings 64 KiB for the same work, and an XCD's blocks share it: 1.4 to 2.1 GB, 484 to 525 us,
-// i.e. 1.1 PFLOP/s (down launch 564 -> 287 us).  Of the parts on their own, at that size: matrix instructions and epilogues
-// 366 us, fragment reads from LDS 284, loads into LDS 247 from L2 and 435 from where the data are.
+// i.e. 1.1 PFLOP/s (down launch 564 -> 304 us).  Gate/up launch at that size with the other parts taken out: matrix
+// instructions and epilogues 366 us, fragment reads from LDS 284, loads into LDS 247 from L2 and 435 from where the data are.
 #include <algorithm>
 #include <type_traits>
 
