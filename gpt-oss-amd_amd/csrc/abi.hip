@@ -73,8 +73,17 @@ inline bool use_small_kernels(int T, int H, int I, int K, int E, int format, boo
     const int items = std::min(T * K, E);
     if (mxfp4 && ((I <= 256 && items * ceil_div(H, 128) > 16 * n_cus) || (H <= 256 && items * ceil_div(2 * I, 128) > 16 * n_cus)))
         return false;
+    // MXFP4 in several rounds: the figures above hold for contractions of 2560 and more.  Shorter ones have too little to stream
+    // for what a block stages, and rows of a multiple of 1024 put the tiles that a launch's waves walk in step a multiple of 8 KiB
+    // apart.  E = 128, K = 8, small : streaming, router of no preference, then skewed, 20 tokens (1.25 rows per expert) and 32:
+    // H x I = 2816 x 2816 208 : 233, 151 : 183 and 241 : 250, 173 : 220; 2880 x 4096 282 : 308, 218 : 258 and 351 : 362, 260 : 305;
+    // 3584 x 3584 327 : 354, 228 : 283 and 391 : 396, 291 : 339; but 3072 x 3072 285 : 269, 213 : 218 and 348 : 299, 267 : 259; 2048 x
+    // 2880 187 : 185, 128 : 145 and 221 : 201, 159 : 161; 4096 x 1536 at 16 tokens 183 : 188, 149 : 168 and 237 : 224, 188 : 195; 2048 x
+    // 1024 at 16 tokens 90 : 90, 67 : 70 and 113 : 104, 85 : 84.  bf16 blocks stream four times as much: none of these shapes lose.
+    // Up to 1.25 rows the small kernel stays for the skewed routers (1024 x 2880 at 16 tokens 114 : 102, but 66 : 73).
+    const bool far = !mxfp4 || (std::min(H, I) >= 2560 && H % 1024 != 0);
     const long long blocks = (long long)E * ceil_div(2 * I / 32, mxfp4 ? 24 : 12);
-    return 4LL * T * K <= (blocks > n_cus ? 12LL : 5LL) * E;
+    return 4LL * T * K <= (blocks > n_cus && far ? 12LL : 5LL) * E;
 }
 
 // Both expert GEMMs in one launch: on request, when the bucketing is done inside the expert kernels and

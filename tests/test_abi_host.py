@@ -77,6 +77,17 @@ def test_expert_kernel_families_by_rows(pkg, E, K):
             assert k["gate_up"].startswith(name) and k["down"].startswith(name), (T, k)
 
 
+@pytest.mark.parametrize("fmt,H,I,last", [("mxfp4", 2880, 2880, 48), ("mxfp4", 2560, 2560, 48), ("mxfp4", 2880, 2496, 20), ("mxfp4", 2496, 2880, 20), ("mxfp4", 2880, 3072, 48),
+                                          ("mxfp4", 3072, 2880, 20), ("mxfp4", 2048, 1024, 20), ("mxfp4", 4096, 1536, 20),
+                                          ("bf16", 2048, 1024, 48), ("bf16", 3072, 3072, 48)])
+def test_small_kernel_line_of_many_rounds(pkg, fmt, H, I, last):
+    """Several rounds of blocks of 128 experts: up to 3 rows per expert, or 1.25 where MXFP4 rows are short or a multiple of 1024."""
+    code = pkg.MOE_WEIGHTS_BF16 if fmt == "bf16" else pkg.MOE_WEIGHTS_MXFP4_TILED
+    for T, name in ((last, "expert_small"), (last + 1, "expert_stream_direct")):
+        k = kernels_of(pkg, T, H, I, 128, 8, code)
+        assert k["gate_up"].startswith(name) and k["down"].startswith(name), (T, k)
+
+
 def test_tile_kernel_takes_large_activation_tensors(pkg):
     """Rows by slot past 4 GiB are no reason to leave the bf16 tile kernel, unless the 256 of one block are; gathered rows past it
     are, at the last byte."""
