@@ -706,7 +706,7 @@ static int block_forward_impl(const moe_block_params* caller, moe_stream_t strea
     // Large batches without a request for the full score matrix take the two-pass router (same
     // indices and weights); everything else the single exact pass.
     const bool strict = (p->flags & MOE_FLAG_ROUTER_STRICT_ORDER) != 0;
-    if (!strict && !p->router_score && router_two_pass(T, E, H)) {
+    if (!strict && !p->router_score && (router_two_pass(T, E, H) || router_rows(T, E, H))) {
         rc = launch_router_two_pass(p->t, p->w_router, p->b_router, ws.router_partial, ws.t_bf16, p->topk_v, p->topk_i, T,
                                     H, E, K, 1, stream, timer ? timer->ev[stage++] : nullptr);
         if (rc) return rc;

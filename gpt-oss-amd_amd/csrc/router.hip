@@ -511,7 +511,7 @@ __global__ __launch_bounds__(256) void router_screen_kernel(const float* __restr
 // on NE or on which other experts share the call.  The trip count is the same for every lane (a
 // lane past the end multiplies zeros), so that the loads of several iterations can be in flight
 // together.  Every lane returns all NE totals.
-template <int NE>
+template <int NE, int UNROLL>
 MOE_DEVICE void exact_dots(const float* __restrict__ x_row, const uint16_t* __restrict__ w, const int (&e)[NE], int H,
                            int lane, double (&total)[NE]) {
     const int n4 = H >> 2;
@@ -524,7 +524,7 @@ MOE_DEVICE void exact_dots(const float* __restrict__ x_row, const uint16_t* __re
         wrow[i] = reinterpret_cast<const uint2*>(w + (size_t)e[i] * H);
         acc[i] = 0.0;
     }
-#pragma unroll 4
+#pragma unroll UNROLL
     for (int j = 0; j < trips; ++j) {
         const bool live = lane + 64 * j < n4;
         const int i4 = min(lane + 64 * j, n4 - 1);
@@ -786,7 +786,7 @@ __global__ __launch_bounds__(256, 4) void router_refine_kernel(const float* __re
         double total[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) e[i] = __builtin_amdgcn_readfirstlane(cand[min(c0 + i, n_cand - 1)]);
-        exact_dots<4>(x_row, w, e, H, lane, total);
+        exact_dots<4, 4>(x_row, w, e, H, lane, total);
         if (lane == 0) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) exact[e[i]] = (float)total[i] + bf16_bits_to_f32(bias[e[i]]);
@@ -796,6 +796,242 @@ __global__ __launch_bounds__(256, 4) void router_refine_kernel(const float* __re
 
     select_topk(exact, E, K, lane, my_v, my_i);
     write_topk(my_v, my_i, K, lane, do_softmax, topk_v + (size_t)t * K, topk_i + (size_t)t * K);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Both passes of the two-pass router in one launch, for up to 128 experts and rows of up to 3072 values: a block of 16
+// waves takes TPB tokens whole.  Same steps and the same error model as router_screen_kernel and router_refine_kernel; the
+// waves share the k range instead of the tokens while they screen (16 MFMA rows are 16 / TPB copies of each token, the sums of
+// the 16 waves meet in LDS), and the tokens' candidates afterwards.
+// What bounds it: a chain of latencies in a single round of blocks (256 tokens x 32 experts, in cycles: loads and screening 10400,
+// sums 900, candidates 2300, their exact scores 3700, top-k and softmax 1800), and with eight tokens or more to a block the
+// fp64 sums (16 cycles per product and wave) and the router rows through one compute unit's L1.  Screen + refine kernels : this
+// one inside a block, us: E = 32, 512 tokens 23 : 13, 1000 25 : 17, 4096 43 : 40, 16384 149 : 135; E = 128, 1024 tokens 31 : 25.
+// grid = ceil(T / TPB), block = 1024.
+// ---------------------------------------------------------------------------------------------
+constexpr int kRowsWaves = 16;
+constexpr int kRowsPairs = 3;  // pairs of k-steps (64 values) per wave: rows of up to 3072 values
+
+// The lanes of a wave exchange values through its own LDS area: no instruction is needed (a wave's LDS accesses are carried out in
+// order), but the compiler must neither move accesses across nor run the two sides under different lane masks.
+MOE_DEVICE void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+// the area holds pieces of activations, of router rows and sums in turn
+typedef __attribute__((may_alias)) u32x4 lds_u32x4;
+typedef __attribute__((may_alias)) f32x4 lds_f32x4;
+typedef __attribute__((may_alias)) float lds_f32;
+
+template <int NE, int TPB>
+__global__ __launch_bounds__(64 * kRowsWaves) void router_rows_kernel(const float* __restrict__ x, const uint16_t* __restrict__ w,
+                                                                      const uint16_t* __restrict__ bias, float err_coeff,
+                                                                      uint16_t* __restrict__ x_bf16, float* __restrict__ topk_v,
+                                                                      int* __restrict__ topk_i, int T, int H, int E, int K,
+                                                                      int do_softmax, float* __restrict__ approx_out,
+                                                                      float* __restrict__ delta_out, int* __restrict__ n_cand_out) {
+    constexpr int W = kRowsWaves, NP = kRowsPairs;
+    constexpr int DUP = 16 / TPB;           // copies of a token among the 16 MFMA rows, and waves per token afterwards
+    constexpr int EP = 16 * NE;             // experts, padded
+    constexpr int LDP = EP + 4;             // floats from one token's partial row to the next
+    constexpr int XI = TPB > 4 ? TPB / 4 : 1;                                 // loads that take a pair of all tokens
+    constexpr int kStageBytes = 1024 * XI > 2048 ? 1024 * XI : 2048, kPartBytes = TPB * LDP * 4;
+    constexpr int kArea = kStageBytes > kPartBytes ? kStageBytes : kPartBytes;  // LDS of one wave
+    __shared__ __attribute__((aligned(16))) uint8_t area[W][(kArea + 15) & ~15];
+    __shared__ float wsq[W][EP], xsq[W][16];
+    __shared__ float approx[TPB][EP], exact[TPB][EP], w2[EP], x2[16];
+    __shared__ int cand[TPB][EP], n_cands[TPB];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const int t0 = blockIdx.x * TPB;
+    const int pairs = H >> 6;
+    const int per = ceil_div(pairs, W);
+    const int first = wave * per;
+    const int count = min(max(pairs - first, 0), per);  // pairs of this wave, <= NP
+    uint8_t* const mine = area[wave];
+    lds_f32* const part = reinterpret_cast<lds_f32*>(mine);  // [TPB][LDP], once the wave has read all else
+
+    // All loads take whole lines, consecutive lanes consecutive pieces of 16 bytes, and are turned into the MFMA operands'
+    // layout in LDS: a load whose lanes follow the operand's layout (16 rows) runs at a lane a cycle, 16 bytes per compute unit
+    // where these reach 50 to 60 (E = 128, one pass over the router rows from L2 50 thousand cycles against 14).
+    // Buffer loads: the pair is the scalar part of an address, so that a lane keeps one offset per row.  Pairs that do not
+    // exist re-read the last one.
+    auto k_of = [&](int p) { return 64 * min(first + p, pairs - 1); };
+    const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x + (size_t)t0 * H), 0, min(TPB, T - t0) * H * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w), 0, E * H * 2, 0x00020000);
+    u32x4 xf[NP][XI], wf[NP][2];
+    // four tokens x 256 bytes a load
+    const int last_row = min(TPB, T - t0) - 1;
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int i = 0; i < XI; ++i)
+            xf[p][i] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, min(4 * i + g, last_row) * H * 4 + r * 16, k_of(p) * 4, 0);
+    // eight router rows x 128 bytes a load
+    auto load_w = [&](int tile, int p) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            wf[p][i] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, min(16 * tile + 8 * i + (lane >> 3), E - 1) * H * 2 + (lane & 7) * 16,
+                                                             k_of(p) * 2, 0);
+    };
+#pragma unroll
+    for (int p = 0; p < NP; ++p) load_w(0, p);
+    __builtin_amdgcn_sched_barrier(0);
+    // The activations in two bf16 pieces.  In k-step h of a pair a lane holds elements 32 h + 8 g .. + 7 of the 64.  LDS: token
+    // row i at i * 256, its sixteen pieces of four values permuted, piece c at c ^ i.
+    u32x4 hi[NP][2], lo[NP][2];
+    {
+        const int row = r / DUP;
+        f32x4 xn = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+#pragma unroll
+            for (int i = 0; i < XI; ++i) {
+                *reinterpret_cast<lds_u32x4*>(mine + (4 * i + g) * 256 + ((r ^ (4 * i + g)) << 4)) = xf[p][i];
+                if (x_bf16 != nullptr && p < count && 4 * i + g <= last_row)
+                    *reinterpret_cast<u32x2*>(x_bf16 + (size_t)(t0 + 4 * i + g) * H + k_of(p) + 4 * r) =
+                        u32x2{pack_bf16x2(__uint_as_float(xf[p][i][0]), __uint_as_float(xf[p][i][1])),
+                              pack_bf16x2(__uint_as_float(xf[p][i][2]), __uint_as_float(xf[p][i][3]))};
+            }
+            wave_lds_order();
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                float v[8];
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const f32x4 q = *reinterpret_cast<const lds_f32x4*>(mine + row * 256 + (((8 * h + 2 * g + c) ^ row) << 4));
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) v[4 * c + j] = q[j];
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t h2 = pack_bf16x2(v[2 * i], v[2 * i + 1]);
+                    hi[p][h][i] = h2;
+                    lo[p][h][i] = pack_bf16x2(v[2 * i] - __uint_as_float(h2 << 16), v[2 * i + 1] - __uint_as_float(h2 & 0xFFFF0000u));
+                }
+                if (p < count) {  // wave-uniform
+                    xn = mfma_16x16x32(hi[p][h], hi[p][h], xn);
+                }
+            }
+            wave_lds_order();
+        }
+        // element (i, i) of a 16 x 16 product in the accumulator layout: lane (r, g = r / 4), value r % 4
+        if (g == r >> 2) xsq[wave][r] = (r & 2) ? ((r & 1) ? xn[3] : xn[2]) : ((r & 1) ? xn[1] : xn[0]);
+    }
+    f32x4 acc[NE];
+    // LDS: router row i of the tile at i * 128, its eight pieces of eight values permuted, piece c at c ^ (i / 2)
+#pragma unroll
+    for (int n = 0; n < NE; ++n) {
+        f32x4 wn = {0.f, 0.f, 0.f, 0.f};
+        acc[n] = wn;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int row = 8 * i + (lane >> 3);
+                *reinterpret_cast<lds_u32x4*>(mine + row * 128 + (((lane & 7) ^ (row >> 1)) << 4)) = wf[p][i];
+            }
+            wave_lds_order();
+            if (n + 1 < NE) load_w(n + 1, p);
+            if (p < count) {  // wave-uniform
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const u32x4 b = *reinterpret_cast<const lds_u32x4*>(mine + r * 128 + (((4 * h + g) ^ (r >> 1)) << 4));
+                    acc[n] = mfma_16x16x32(hi[p][h], b, acc[n]);
+                    wn = mfma_16x16x32(b, b, wn);
+                    acc[n] = mfma_16x16x32(lo[p][h], b, acc[n]);
+                }
+            }
+            wave_lds_order();
+        }
+        if (g == r >> 2) wsq[wave][16 * n + r] = (r & 2) ? ((r & 1) ? wn[3] : wn[2]) : ((r & 1) ? wn[1] : wn[0]);
+    }
+    // accumulator layout: lane holds MFMA rows 4 g + i (i = 0..3) for expert 16 n + r
+#pragma unroll
+    for (int n = 0; n < NE; ++n)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if ((4 * g + i) % DUP == 0) part[(4 * g + i) / DUP * LDP + 16 * n + r] = acc[n][i];
+    __syncthreads();
+    for (int i = threadIdx.x; i < TPB * EP; i += 64 * W) {
+        const int t = i / EP, e = i % EP;
+        float sum = 0.f;
+#pragma unroll
+        for (int p = 0; p < W; ++p) sum += reinterpret_cast<const lds_f32*>(area[p])[t * LDP + e];
+        approx[t][e] = e < E ? sum + bf16_bits_to_f32(bias[e]) : 0.f;
+    }
+    // from the other end, where the waves have no sum of their own while there are few tokens
+    const int back = 64 * W - 1 - (int)threadIdx.x;
+    if (back < EP + 16) {
+        float q = 0.f;
+        const float* from = back < EP ? &wsq[0][back] : &xsq[0][back - EP];
+        const int stride = back < EP ? EP : 16;
+#pragma unroll
+        for (int p = 0; p < W; ++p) q += from[p * stride];
+        if (back < EP) w2[back] = q;
+        else x2[back - EP] = q;
+    }
+    __syncthreads();
+    const int tl = wave / DUP, sub = wave % DUP;  // the wave's token, and its place among the token's waves
+    const int t = t0 + tl;
+    if (sub == 0) {  // candidates, as in router_refine_kernel
+        const float* my = approx[tl];
+        float amax = 0.f, wmax = 0.f;
+#pragma unroll
+        for (int e = lane; e < EP; e += 64) {
+            amax = fmaxf(amax, fabsf(my[e]));
+            wmax = fmaxf(wmax, w2[e]);
+            if (approx_out && e < E && t < T) approx_out[(size_t)t * E + e] = my[e];
+        }
+        amax = wave_max_nonneg(amax);
+        wmax = wave_max_nonneg(wmax);
+        // the activations' norm is that of their upper pieces, each within 2^-8 of its activation
+        const float delta = err_coeff * (sqrtf(x2[tl * DUP]) * 1.006f) * (sqrtf(wmax) * 1.001f) + amax * 0x1p-20f;
+        float my_v;
+        int my_i;
+        select_topk_of<(EP + 63) / 64>(my, E, K, lane, my_v, my_i);
+        const float thr = lane_value(my_v, K - 1) - 2.f * delta;
+        int n = 0;
+#pragma unroll
+        for (int e0 = 0; e0 < EP; e0 += 64) {
+            const int e = e0 + lane;
+            const bool in = e < E && !(my[e < EP ? e : 0] < thr);  // a not-a-number decides nothing
+            const unsigned long long ballot = __ballot(in);
+            if (in) cand[tl][n + __popcll(ballot & ((1ull << lane) - 1ull))] = e;
+            n += __popcll(ballot);
+        }
+        if (lane == 0) {
+            n_cands[tl] = n;
+            if (delta_out && t < T) delta_out[t] = delta;
+            if (n_cand_out && t < T) n_cand_out[t] = n;
+        }
+    }
+    __syncthreads();
+    const int n_cand = __builtin_amdgcn_readfirstlane(n_cands[tl]);
+    // exact scores: the waves of a token take its candidates in turn, C at a time
+    constexpr int C = TPB == 16 ? 4 : TPB == 8 ? 2 : 1;
+    const float* x_row = x + (size_t)min(t, T - 1) * H;
+#pragma nounroll
+    for (int c0 = C * sub; c0 < n_cand; c0 += C * DUP) {
+        int e[C];
+        double total[C];
+#pragma unroll
+        for (int i = 0; i < C; ++i) e[i] = __builtin_amdgcn_readfirstlane(cand[tl][min(c0 + i, n_cand - 1)]);
+        exact_dots<C, C == 4 ? 4 : 12>(x_row, w, e, H, lane, total);
+        if (lane == 0) {
+#pragma unroll
+            for (int i = 0; i < C; ++i)
+                if (c0 + i < n_cand) exact[tl][c0 + i] = (float)total[i] + bf16_bits_to_f32(bias[e[i]]);
+        }
+    }
+    __syncthreads();
+    if (sub == 0 && t < T) {
+        float my_v;
+        int my_i;
+        select_topk(exact[tl], n_cand, K, lane, my_v, my_i);  // candidates are in ascending order: ties as by expert id
+        write_topk(my_v, cand[tl][my_i], K, lane, do_softmax, topk_v + (size_t)t * K, topk_i + (size_t)t * K);
+    }
 }
 
 // In-place softmax over the last dimension, one thread per row, the reference's order of
@@ -900,10 +1136,55 @@ size_t router_screen_bytes(int T, int E, int H) {
     return ((size_t)S * T * E + (size_t)S * E + (size_t)S * T) * sizeof(float);
 }
 
+static bool router_rows_fits(int E, int H) { return E <= 128 && H % 64 == 0 && H <= 64 * kRowsWaves * kRowsPairs; }
+
+// router_rows_kernel instead of the exact passes as well (it always carries out the two-pass method where it can).  Exact passes :
+// router_rows_kernel inside a block, us, rows of 2880, from HBM: E = 8, 600 tokens 10.6 : 13.2, 2000 tokens 24 : 22; E = 16, 300 tokens
+// 10.5 : 10.7, 4000 tokens 64 : 28; E = 32, 64 tokens 8.9 : 9.4, 256 tokens 10.6 : 11.3, 512 tokens (a second round of blocks) 18 : 13;
+// E = 48, 16 tokens 11.6 : 11.0, 64 tokens 12.5 : 11.4, 300 tokens 24 : 12.6; E = 128, 33 tokens 13.3 : 15.5, 64 tokens 14.3 : 15.2, 128
+// tokens 21 : 16.8, 200 tokens 28 : 16.9.
+bool router_rows(int T, int E, int H) {
+    return router_rows_fits(E, H) && (E > 48 ? T > 64 : E > 32 ? T > 16 : E > 16 ? T > 256 : (long long)T * E > 12000);
+}
+
+static int launch_router_rows(const float* x, const uint16_t* w, const uint16_t* bias, uint16_t* x_bf16, float* topk_v,
+                              int* topk_i, int T, int H, int E, int K, int do_softmax, hipStream_t stream, float* approx_out,
+                              float* delta_out, int* n_cand_out) {
+    const int per_wave = 2 * ceil_div(H / 64, kRowsWaves);
+    // per wave and segment as in launch_router_two_pass, and 16 additions of the waves' sums
+    const float err_coeff = ((float)(33 + 2 * per_wave + 16) * 0x1p-23f + 0x1p-16f + 8 * 0x1p-24f) * 1.01f;
+    // as few tokens to a block as one round of blocks over 256 compute units allows; more than 64 experts leave LDS for eight
+    const int tpb = T <= 256 ? 1 : T <= 512 ? 2 : T <= 1024 ? 4 : T <= 2048 || E > 64 ? 8 : 16;
+#define MOE_ROWS(NE_, TPB_)                                                                                             \
+    if (tpb == TPB_) {                                                                                                  \
+        hipLaunchKernelGGL((router_rows_kernel<NE_, TPB_>), dim3(ceil_div(T, TPB_)), dim3(64 * kRowsWaves), 0, stream, x, w, \
+                           bias, err_coeff, x_bf16, topk_v, topk_i, T, H, E, K, do_softmax, approx_out, delta_out, n_cand_out); \
+        return launch_status();                                                                                         \
+    }
+#define MOE_ROWS_NE(NE_) MOE_ROWS(NE_, 1) MOE_ROWS(NE_, 2) MOE_ROWS(NE_, 4) MOE_ROWS(NE_, 8)
+    if (E <= 32) {
+        MOE_ROWS_NE(2) MOE_ROWS(2, 16)
+    } else if (E <= 64) {
+        MOE_ROWS_NE(4) MOE_ROWS(4, 16)
+    } else {
+        MOE_ROWS_NE(8)
+    }
+#undef MOE_ROWS_NE
+#undef MOE_ROWS
+    return MOE_ERR_LIMIT;
+}
+
 int launch_router_two_pass(const float* x, const uint16_t* w, const uint16_t* bias, void* scratch, uint16_t* x_bf16,
                            float* topk_v, int* topk_i, int T, int H, int E, int K, int do_softmax,
                            hipStream_t stream, hipEvent_t between, float* approx_out, float* delta_out,
                            int* n_cand_out) {
+    if (router_rows_fits(E, H)) {
+        int rc = launch_router_rows(x, w, bias, x_bf16, topk_v, topk_i, T, H, E, K, do_softmax, stream, approx_out, delta_out,
+                                    n_cand_out);
+        if (rc) return rc;
+        if (between) MOE_RETURN_IF_HIP(hipEventRecord(between, stream));
+        return MOE_OK;
+    }
     int seg_len, S;
     screen_plan(T, E, H, &seg_len, &S);
     float* partial = static_cast<float*>(scratch);
