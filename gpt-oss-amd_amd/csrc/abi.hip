@@ -706,7 +706,17 @@ static int block_forward_impl(const moe_block_params* caller, moe_stream_t strea
     // Large batches without a request for the full score matrix take the two-pass router (same
     // indices and weights); everything else the single exact pass.
     const bool strict = (p->flags & MOE_FLAG_ROUTER_STRICT_ORDER) != 0;
-    if (!strict && !p->router_score && (router_two_pass(T, E, H) || router_rows(T, E, H))) {
+    const bool prefill = use_prefill_kernels(T, H, I, K, E, p->weight_format, p->flags);
+    const bool direct = use_direct_bucketing(T, K, E, prefill, p->flags);
+    // a handful of tokens: the scores only, top-k and softmax are the gate/up kernel's
+    const bool scores_only = !strict && expert_small_takes_scores(T, T * K) &&
+                             use_small_kernels(T, H, I, K, E, p->weight_format, direct, p->flags, device_cu_count());
+    float* const scores = p->router_score ? p->router_score : reinterpret_cast<float*>(ws.router_partial);
+    if (scores_only) {
+        rc = launch_router_scores(p->t, p->w_router, p->b_router, ws.t_bf16, scores, T, H, E, stream);
+        if (rc) return rc;
+        if ((rc = mark())) return rc;
+    } else if (!strict && !p->router_score && (router_two_pass(T, E, H) || router_rows(T, E, H))) {
         rc = launch_router_two_pass(p->t, p->w_router, p->b_router, ws.router_partial, ws.t_bf16, p->topk_v, p->topk_i, T,
                                     H, E, K, 1, stream, timer ? timer->ev[stage++] : nullptr);
         if (rc) return rc;
@@ -730,8 +740,6 @@ static int block_forward_impl(const moe_block_params* caller, moe_stream_t strea
     // 2. bucketing + token-block map  (src/forward.cpp:329-376)
     // Small batches need no bucketing launch: each block of the expert kernels finds its expert's
     // bucket in topk_i itself and rows are addressed by assignment id (token * K + k).
-    const bool prefill = use_prefill_kernels(T, H, I, K, E, p->weight_format, p->flags);
-    const bool direct = use_direct_bucketing(T, K, E, prefill, p->flags);
     const int tile_tokens = tile_tokens_of(prefill, fmt);
     const int max_tiles = tile_map_capacity(T * K, E, tile_tokens);  // <= ws.max_tiles (sized for 64)
     if (!direct) {
@@ -745,8 +753,19 @@ static int block_forward_impl(const moe_block_params* caller, moe_stream_t strea
     // 3. gate/up GEMM + SwiGLU  (src/forward.cpp:474-479; src/run.cpp:657-689)
     // 4. down GEMM  (src/forward.cpp:481-487; src/run.cpp:691-700)
     const ExpertPlan plan(p, ws, prefill, direct, tile_tokens, max_tiles);
-    const ExpertGemmArgs a1 = plan.gate_up(ws.t_bf16, ws.h_by_slot);
-    const ExpertGemmArgs a2 = plan.down(ws.h_by_slot, ws.y_by_slot);
+    ExpertGemmArgs a1 = plan.gate_up(ws.t_bf16, ws.h_by_slot);
+    ExpertGemmArgs a2 = plan.down(ws.h_by_slot, ws.y_by_slot);
+    if (scores_only) {
+        a1.scores = scores;
+        a1.topk_v_out = p->topk_v;
+        a1.topk_i_out = p->topk_i;
+    }
+    const bool combined = scores_only && !p->next_norm_out && expert_small_combines(T * K, I, fmt);
+    if (combined) {
+        a2.combine_v = p->topk_v;
+        a2.e_agg = p->e_agg;
+        a2.residual_x = p->residual_x;
+    }
     if (use_fused_experts(E, direct, p->flags)) {
         // one launch for both (its stage time is reported as the gate/up stage, the down stage is empty)
         ExpertFusedArgs f{};
@@ -770,6 +789,7 @@ static int block_forward_impl(const moe_block_params* caller, moe_stream_t strea
     if ((rc = mark())) return rc;
 
     // 5. weighted combine in ascending expert id (+ residual)  (src/run.cpp:702-712)
+    if (combined) return mark();
     const int* slot_of = direct ? nullptr : ws.slot_of;  // direct: the row of assignment (t, k) is t * K + k
     if (p->next_norm_out) {
         rc = launch_combine_norm(ws.y_by_slot, slot_of, p->topk_i, p->topk_v, p->e_agg, p->residual_x,

@@ -13,6 +13,7 @@
 #include <type_traits>
 
 #include "expert_tiles.h"
+#include "topk.h"
 
 namespace moe {
 
@@ -302,13 +303,29 @@ __global__ __launch_bounds__(64 * kSmallWaves, 4) void expert_small_kernel(Exper
     const int waves = blockDim.x >> 6;
     const int ordinal = blockIdx.x / a.row_blocks;
     const int rb = blockIdx.x - ordinal * a.row_blocks;
+    if constexpr (EPI == EPI_SWIGLU_BF16) {
+        if (a.scores) {  // at most 64 assignments: the list goes through bucket[]
+            const int T = a.n_assign / a.assign_div;
+            for (int t = wave; t < T; t += waves) {
+                float my_v;
+                int my_i;
+                select_topk(a.scores + (size_t)t * a.n_experts, a.n_experts, a.assign_div, lane, my_v, my_i);
+                if (lane < a.assign_div) bucket[t * a.assign_div + lane] = my_i;
+                if (blockIdx.x == 0)
+                    write_topk(my_v, my_i, a.assign_div, lane, 1, a.topk_v_out + (size_t)t * a.assign_div,
+                               a.topk_i_out + (size_t)t * a.assign_div);
+            }
+            __syncthreads();
+        }
+    }
+    const int* const list = EPI == EPI_SWIGLU_BF16 && a.scores ? bucket : a.topk_i;
     // chunk c of 64 assignments: wave c % waves (a block of four waves takes two chunks each)
     int ids[kSmallMaxAssign / 64 / 4];
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
         const int s = (p * waves + wave) * 64 + lane;
         // an id that names no expert is skipped, as by the other kernels: the down GEMM entry takes the list from its caller
-        const int id = s < a.n_assign ? a.topk_i[s] : -1;
+        const int id = s < a.n_assign ? list[s] : -1;
         ids[p] = (unsigned)id < (unsigned)a.n_experts ? id : -1;
     }
     if (threadIdx.x < 32) present[threadIdx.x] = 0u;
@@ -368,6 +385,172 @@ __global__ __launch_bounds__(64 * kSmallWaves, 4) void expert_small_queue_kernel
     small_rows<FMT, EPI, true>(a, lds, entry[0], [&](int i) { return off + i; }, entry[2], rb, max_rows, lds_bytes);
 }
 
+// ---- down GEMM of a token or two: a wave per (assignment, tile of 16 weight rows); the waves of a block share the tile ------------
+// What bounds it: round trips (ids and rows, then weights, then the stores).  The block that holds all of a token's rows of its
+// tile also combines them, which takes the combine's launch away; a wave needs nobody else's row until then.  MXFP4, us, down
+// + combine, two launches : one: 1 token 7.7 + 3.8 : 8.3, 2 tokens 9.9 + 3.9 : 10.4.  The gate/up GEMM in this form was no faster (1
+// token 12.2 : 11.9), and neither was a whole MXFP4 tile requested at once instead of a ring of eight stages: straight-line code for 24
+// stages is fetched anew by every launch.
+constexpr int kTinyAssign = 16;
+
+// The wave's activation row, as it is (the 16 columns of the product are this one row), zeros past its end.  Loaded ahead of the
+// expert's id, stored to LDS before the weights are requested.
+constexpr int kTinyRowLoads = 6;  // loads of 512 values: rows of up to 3072 values, what is longer in a loop
+MOE_DEVICE void tiny_row_load(u32x4 (&xr)[kTinyRowLoads], const uint16_t* row, int K) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < kTinyRowLoads; ++i) {
+        const int k = 512 * i + 8 * lane;
+        xr[i] = k < K ? *reinterpret_cast<const u32x4*>(row + k) : u32x4{0u, 0u, 0u, 0u};
+    }
+}
+MOE_DEVICE void tiny_row_store(const u32x4 (&xr)[kTinyRowLoads], uint8_t* row_lds, const uint16_t* row, int K) {
+    const int lane = threadIdx.x & 63;
+    const int padded = ceil_div(K, kStageElems) * kStageElems;
+#pragma unroll
+    for (int i = 0; i < kTinyRowLoads; ++i)
+        if (512 * i + 8 * lane < padded) *reinterpret_cast<u32x4*>(row_lds + 1024 * i + 16 * lane) = xr[i];
+    for (int k = 512 * kTinyRowLoads + 8 * lane; k < padded; k += 512)
+        *reinterpret_cast<u32x4*>(row_lds + 2 * k) = k < K ? *reinterpret_cast<const u32x4*>(row + k) : u32x4{0u, 0u, 0u, 0u};
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();  // the wave's own LDS accesses are carried out in order
+}
+
+template <int FMT>
+MOE_DEVICE f32x4 tiny_tile(const ExpertGemmArgs& a, const uint8_t* row_lds, int e, int tile) {
+    const int lane = threadIdx.x & 63;
+    const int q = lane & 15;
+    const int g = lane >> 4;
+    const int K = a.K;
+    auto b_frag = [&](int s, int j) { return *reinterpret_cast<const u32x4*>(row_lds + s * 256 + ws_chunk<FMT>(j, g) * 16); };
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (FMT == FMT_BF16) {
+        constexpr int D = 4;
+        const int n_pairs = K / 64;
+        const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint16_t*>(reinterpret_cast<const uint16_t*>(a.w) + (size_t)e * a.w_expert_stride), 0,
+            (int)((uint32_t)a.rows * (uint32_t)K * 2u), 0x00020000);
+        const uint32_t a_tile = (uint32_t)((tile >> 2) * 64 + tile_row_in_group(tile & 3, 0)) * (uint32_t)K * 2u;
+        const uint32_t a_lane = (uint32_t)(tile_row_in_group(0, q & 7) * K + 8 * (2 * g + (q >> 3))) * 2u;
+        const uint32_t second_half = 32u * (uint32_t)K * 2u;
+        u32x4 ar[D][2];
+        auto load_a = [&](int slot, int pair) {
+            const uint32_t off = a_tile + (uint32_t)(pair < n_pairs ? pair : 0) * 128u;  // past the end: unused
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                ar[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, (int)a_lane, (int)(off + second_half * i), 2 /* nt */);
+        };
+#pragma unroll
+        for (int i = 0; i < D - 1; ++i) load_a(i, i);
+        for (int p0 = 0; p0 < n_pairs; p0 += D) {
+#pragma unroll
+            for (int u = 0; u < D; ++u) {
+                load_a((u + D - 1) % D, p0 + u + D - 1);
+                __builtin_amdgcn_sched_barrier(0);
+                if (p0 + u < n_pairs) {  // wave-uniform
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        u32x4 av;
+#pragma unroll
+                        for (int d = 0; d < 4; ++d)
+                            av[d] = h == 0 ? (uint32_t)__builtin_amdgcn_update_dpp((int)ar[u][0][d], (int)ar[u][1][d], 0x128, 0xF, 0xC, false)
+                                           : (uint32_t)__builtin_amdgcn_update_dpp((int)ar[u][1][d], (int)ar[u][0][d], 0x128, 0xF, 0x3, false);
+                        acc = mfma_16x16x32(av, b_frag((p0 + u) >> 1, 2 * (u & 1) + h), acc);
+                    }
+                }
+            }
+        }
+    } else {
+        const int G = K / 32;
+        const int n_stages = ceil_div(K, kStageElems);
+        const uint32_t wtile = (uint32_t)tile * (uint32_t)G * 256u;
+        const uint32_t stile = (uint32_t)tile * (uint32_t)ceil_div(ceil_div(G, 4), 4) * 256u;
+        const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint8_t*>(reinterpret_cast<const uint8_t*>(a.w) + (size_t)e * a.w_expert_stride), 0,
+            (int)a.w_expert_stride, 0x00020000);
+        const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint8_t*>(a.w_scales + (size_t)e * a.s_expert_stride), 0, (int)a.s_expert_stride, 0x00020000);
+        constexpr int D = kSmallGroup;
+        u32x4 araw[D];
+        uint32_t sw_cur[2], sw_nxt[2];
+        auto load_a = [&](int slot, int s) {
+            araw[slot] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, lane * 16, (int)(wtile + (uint32_t)s * 1024u), 2 /* nt */);
+        };
+        auto load_scales = [&](uint32_t (&dst)[2], int grp) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                dst[i] = __builtin_amdgcn_raw_buffer_load_b32(s_rsrc, lane * 4, (int)(stile + (uint32_t)(2 * grp + i) * 256u), 0);
+        };
+        load_scales(sw_cur, 0);
+#pragma unroll
+        for (int i = 0; i < D; ++i) load_a(i, i);
+        for (int s0 = 0; s0 < n_stages; s0 += D) {
+            load_scales(sw_nxt, s0 / D + 1);
+#pragma unroll
+            for (int i = 0; i < D; ++i) {
+                if (s0 + i < n_stages) {  // wave-uniform
+                    const float sc = mxfp4_scale_to_f32((sw_cur[i >> 2] >> (8 * (i & 3))) & 0xFFu);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        uint32_t d[4];
+                        mxfp4_dword_to_bf16x8(araw[i][j], sc, d);
+                        acc = mfma_16x16x32(u32x4{d[0], d[1], d[2], d[3]}, b_frag(s0 + i, j), acc);
+                    }
+                }
+                // reads past the tile only where the scale byte is 0 or nobody looks, as in small_tile
+                load_a(i, s0 + i + D);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            sw_cur[0] = sw_nxt[0];
+            sw_cur[1] = sw_nxt[1];
+        }
+    }
+    return acc;
+}
+
+// grid = tiles, block = 64 x assignments, dynamic LDS = assignments x padded row.
+template <int FMT>
+__global__ __launch_bounds__(64 * kTinyAssign, 4) void expert_tiny_down_kernel(ExpertGemmArgs a, int row_bytes) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    __shared__ float y[kTinyAssign][16];  // by token, then by rank of the expert id among the token's
+    __shared__ float weight[kTinyAssign];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // the assignment
+    const int g = lane >> 4;
+    const int top = a.assign_div;
+    const int t = wave / top, k = wave - t * top;
+    const int tile = blockIdx.x;
+    uint8_t* const row_lds = lds + (size_t)wave * row_bytes;
+    const uint16_t* const row = a.act + (size_t)wave * a.K;
+    u32x4 xr[kTinyRowLoads];
+    tiny_row_load(xr, row, a.K);
+    const int id = lane < top ? a.topk_i[t * top + lane] : 0x7FFFFFFF;
+    const int e = __builtin_amdgcn_readlane(id, k);
+    const int at = t * top + __popcll(__ballot(id < e || (id == e && lane < k)));
+    if (lane == 0) weight[at] = a.combine_v[wave];
+    tiny_row_store(xr, row_lds, row, a.K);
+    uint2 bias_raw[1];
+    const int group = tile >> 2, r0 = tile & 3;
+    load_bias<1>(a, e, group, r0, bias_raw);
+    const f32x4 acc = tiny_tile<FMT>(a, row_lds, e, tile);
+    if ((lane & 15) == 0)  // all columns are the same row
+        *reinterpret_cast<f32x4*>(&y[at][4 * g]) =
+            f32x4{acc[0] + bf16_bits_to_f32(bias_raw[0].x & 0xFFFFu), acc[1] + bf16_bits_to_f32(bias_raw[0].x >> 16),
+                  acc[2] + bf16_bits_to_f32(bias_raw[0].y & 0xFFFFu), acc[3] + bf16_bits_to_f32(bias_raw[0].y >> 16)};
+    __syncthreads();
+    // the weighted sum in ascending expert id, each step one fused multiply-add (combine_kernel)
+    const int ct = threadIdx.x >> 4, r = threadIdx.x & 15;
+    if (ct < a.n_assign / top) {
+        // tile row 4 g + j is weight row g * 16 + r0 * 4 + j of the group (stream_epilogue)
+        const size_t out = (size_t)ct * a.rows + group * 64 + (r >> 2) * 16 + r0 * 4 + (r & 3);
+        const float before = a.residual_x ? a.residual_x[out] : 0.f;
+        float sum = 0.f;
+        for (int i = 0; i < top; ++i) sum = fmaf(y[ct * top + i][r], weight[ct * top + i], sum);
+        a.e_agg[out] = sum;
+        if (a.residual_x) a.residual_x[out] = before + sum;
+    }
+}
+
 }  // namespace
 
 // Assignments, and buffer descriptors that reach an expert's whole matrix (31-bit byte offsets).
@@ -377,12 +560,31 @@ bool expert_small_fits(int n_assign, int rows, int K, int format) {
     return n_assign <= kSmallMaxAssign && bytes <= 0x7fffffffull;
 }
 
+// Every block of the gate/up launch finds the top-k of all tokens itself, a token to a wave: worth the router's second half while that
+// is one token each.  Whole block, us, router and small kernels : this, MXFP4, E = 32, 1 token 30 : 24, 4 tokens 50 : 47, 8 tokens 61.5 : 59, 10
+// tokens 68 : 69; E = 128, 1 token 34 : 25, 4 tokens 60 : 50, 8 tokens 87 : 80, 10 tokens 100 : 100, 16 tokens 131 : 134.
+bool expert_small_takes_scores(int n_tokens, int n_assign) { return n_tokens <= kSmallWaves && n_assign <= 64; }
+
+// bf16 weights of 16 assignments load a compute unit longer than the combine's launch takes (4 tokens, E = 32, two launches : one, us,
+// MXFP4 18.7 : 17.3, bf16 49.0 : 49.9; 3 tokens 16.2 : 13.7 and 40.3 : 38.5).
+bool expert_small_combines(int n_assign, int K, int format) {
+    return n_assign <= (format == FMT_BF16 ? 12 : kTinyAssign) && (long long)n_assign * K <= 64 * 1024 - kTinyAssign * kStageElems;
+}
+
 int launch_expert_small(const ExpertGemmArgs& a, int epi, hipStream_t stream) {
     const bool queue = a.work_queue != nullptr;
     if (a.rows % 64 != 0 || a.K % (a.format == FMT_BF16 ? 64 : 32) != 0 || (!queue && !a.topk_i)) return MOE_ERR_SHAPE;
     if (!expert_small_fits(queue ? 0 : a.n_assign, a.rows, a.K, a.format)) return MOE_ERR_LIMIT;
     if (!queue && (a.assign_div <= 0 || a.assign_div > 8 || a.n_experts > 1024)) return MOE_ERR_LIMIT;
     ExpertGemmArgs b = a;
+    if (!queue && a.combine_v && epi == EPI_ROWS_F32 && expert_small_combines(a.n_assign, a.K, a.format)) {
+        const int row_bytes = ceil_div(a.K, kStageElems) * kStageElems * 2;
+        const dim3 grid(a.rows / 16), block(64 * a.n_assign);
+        if (a.format == FMT_BF16) hipLaunchKernelGGL(expert_tiny_down_kernel<FMT_BF16>, grid, block, row_bytes * a.n_assign, stream, b, row_bytes);
+        else hipLaunchKernelGGL(expert_tiny_down_kernel<FMT_MXFP4>, grid, block, row_bytes * a.n_assign, stream, b, row_bytes);
+        return launch_status();
+    }
+    if (a.combine_v || (a.scores && !expert_small_takes_scores(a.n_assign / a.assign_div, a.n_assign))) return MOE_ERR_LIMIT;
     const int items = queue ? a.work_count : min(a.n_assign, a.n_experts);
     if (items <= 0) return MOE_OK;
     const int tiles = a.rows / 16;

@@ -16,6 +16,9 @@ int launch_router_finalize(const double* partial, int S, const float* scores_in,
                            float* scores_out, float* topk_v, int* topk_i, int T, int E, int K, int do_topk,
                            int do_softmax, hipStream_t stream);
 int launch_softmax_rows(float* x, int B, int size, hipStream_t stream);
+// Scores only ([T, E]) and the bf16 activation copy; top-k and softmax are the gate/up kernel's then (ExpertGemmArgs::scores).
+int launch_router_scores(const float* x, const uint16_t* w, const uint16_t* bias, uint16_t* x_bf16, float* scores, int T, int H,
+                         int E, hipStream_t stream);
 // Whole router in one launch (block per token): logits as the exact pass of the two-pass router,
 // top-k, softmax, the bf16 activation copy and, if scores_out is not NULL, the score matrix.
 bool router_fused_fits(int H);
@@ -105,6 +108,15 @@ struct ExpertGemmArgs {
                                 // (256-token blocks; bf16 weights only); 18 a 16-row tile per wave, buckets of a
                                 // handful of rows.  The work-queue entries take 0, 1 and 18.
     int n_cus;                  // compute units to fill (18 and the work-queue entries)
+    // experts_small.hip.  Gate/up: with scores (router logits [T, n_experts]) topk_i is not read; the kernel finds it and
+    // the softmax weights itself and leaves both for the launches after it.
+    const float* scores;
+    float* topk_v_out;
+    int* topk_i_out;
+    // Down: with combine_v (the softmax weights) the launch combines the tokens' rows too, into e_agg and, if not NULL, residual_x.
+    const float* combine_v;
+    float* e_agg;
+    float* residual_x;
 };
 int launch_expert_stream(const ExpertGemmArgs& a, int epi, hipStream_t stream);
 
@@ -115,6 +127,8 @@ int expert_direct_max_assignments();
 
 // ---- experts_small.hip: a handful of rows per expert (bucketing inside the kernel) ---------------
 bool expert_small_fits(int n_assign, int rows, int K, int format);
+bool expert_small_takes_scores(int n_tokens, int n_assign);  // ExpertGemmArgs::scores
+bool expert_small_combines(int n_assign, int K, int format);  // ExpertGemmArgs::combine_v
 int launch_expert_small(const ExpertGemmArgs& a, int epi, hipStream_t stream);
 
 // ---- experts_fused.hip: both expert GEMMs of a block in one launch (bucketing inside the kernel) --

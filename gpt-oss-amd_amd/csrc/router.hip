@@ -4,6 +4,7 @@
 // (src/hip/gemms/gemm_router.hip:184), topk (src/hip/topk.hip:59) and softmax (src/hip/softmax.hip:46).
 #include "common.h"
 #include "kernels.h"
+#include "topk.h"
 
 namespace moe {
 
@@ -229,105 +230,6 @@ __global__ __launch_bounds__(256) void router_partial_small_kernel(const float* 
 // grid = ceil(T/4), block = 256, dynamic LDS = 4*E floats.
 // ---------------------------------------------------------------------------------------------
 
-// These kernels run their code once per wave, so their time is instruction fetch as much as
-// anything: loops stay rolled (the round and segment counts are wave-uniform anyway).
-//
-// Sort key of a score: larger key = better candidate.  The score's bits mapped to an unsigned integer in score order (-0
-// counts as +0, as in the reference's float comparison); key 0 is "nothing".
-MOE_DEVICE uint32_t rank_key(float v) {
-    const uint32_t u = __float_as_uint(v + 0.f);
-    return max(u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u), 1u);
-}
-MOE_DEVICE float rank_key_value(uint32_t m) { return __uint_as_float((m & 0x80000000u) ? m ^ 0x80000000u : ~m); }
-
-// K rounds of wave-wide argmax over vals[0..E) ordered by (value desc, index asc).  Lane r < K ends up holding the winner of
-// round r in (my_v, my_i).  C > 0: E <= 64 C, the keys stay in registers; C = 0: any E <= 2048, read anew in every round.
-// A round is a chain of dependent instructions and little else: the maximum of the 32-bit keys is one instruction per DPP
-// step, and the lowest index that has it comes from a ballot.  (A 64-bit key with the index in it took five instructions a
-// step: 850 cycles a round, 200 now.)
-template <int C>
-MOE_DEVICE void select_topk_of(const float* vals, int E, int K, int lane, float& my_v, int& my_i) {
-    uint32_t key[C > 0 ? C : 1];
-    uint32_t taken = 0;  // C = 0: bit c set: candidate lane + 64*c already selected
-    if constexpr (C > 0) {
-#pragma unroll
-        for (int c = 0; c < C; ++c) key[c] = lane + 64 * c < E ? rank_key(vals[lane + 64 * c]) : 0u;
-    }
-    auto key_at = [&](int c) { return lane + 64 * c < E && !((taken >> c) & 1u) ? rank_key(vals[lane + 64 * c]) : 0u; };
-    my_v = -INFINITY;
-    my_i = 0;
-#pragma nounroll
-    for (int r = 0; r < K; ++r) {
-        uint32_t best = 0;
-        if constexpr (C > 0) {
-#pragma unroll
-            for (int c = 0; c < C; ++c) best = max(best, key[c]);
-        } else {
-#pragma nounroll
-            for (int c = 0; 64 * c < E; ++c) best = max(best, key_at(c));
-        }
-#define MOE_STEP(CTRL, M) best = max(best, dpp_move<CTRL, M>(0u, best));
-        MOE_DPP_STEPS(MOE_STEP)
-#undef MOE_STEP
-        best = __builtin_amdgcn_readlane(best, 63);
-        int bi = 0;
-        if constexpr (C > 0) {
-#pragma unroll
-            for (int c = C - 1; c >= 0; --c) {
-                const unsigned long long has = __ballot(key[c] == best);
-                if (has) bi = 64 * c + (int)__builtin_ctzll(has);
-            }
-#pragma unroll
-            for (int c = 0; c < C; ++c) key[c] = bi == lane + 64 * c ? 0u : key[c];
-        } else {
-#pragma nounroll
-            for (int c = 0; 64 * c < E; ++c) {
-                const unsigned long long has = __ballot(key_at(c) == best);
-                if (has) {
-                    bi = 64 * c + (int)__builtin_ctzll(has);
-                    break;
-                }
-            }
-            if ((bi & 63) == lane) taken |= 1u << (bi >> 6);
-        }
-        if (lane == r) {
-            my_v = rank_key_value(best);
-            my_i = bi;
-        }
-    }
-}
-
-MOE_DEVICE void select_topk(const float* vals, int E, int K, int lane, float& my_v, int& my_i) {
-    if (E <= 64) select_topk_of<1>(vals, E, K, lane, my_v, my_i);  // wave-uniform
-    else if (E <= 128) select_topk_of<2>(vals, E, K, lane, my_v, my_i);
-    else select_topk_of<0>(vals, E, K, lane, my_v, my_i);
-}
-
-MOE_DEVICE float lane_value(float v, int src_lane) {
-    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), src_lane));
-}
-
-// Softmax of src/run.cpp:321-339 over the K selected values in its own order of operations (max,
-// then exponentials, then their fp64 sum in index order), or the values themselves; lane r < K
-// stores entry r.
-MOE_DEVICE void write_topk(float my_v, int my_i, int K, int lane, int do_softmax, float* __restrict__ out_v,
-                           int* __restrict__ out_i) {
-    float o = my_v;
-    if (do_softmax) {
-        // the first of the selected values is the largest (or not a number, which no other compares greater than)
-        const double max_val = lane_value(my_v, 0);
-        const float ex = expf((float)((double)my_v - max_val));
-        double sum = 0.0;
-#pragma nounroll
-        for (int r = 0; r < K; ++r) sum += (double)lane_value(ex, r);
-        o = (float)((double)ex / sum);
-    }
-    if (lane < K) {
-        out_v[lane] = o;
-        out_i[lane] = my_i;
-    }
-}
-
 __global__ __launch_bounds__(256) void router_finalize_kernel(const double* __restrict__ partial, int S,
                                                               const float* __restrict__ scores_in,
                                                               const uint16_t* __restrict__ bias,
@@ -543,6 +445,32 @@ MOE_DEVICE void exact_dots(const float* __restrict__ x_row, const uint16_t* __re
     }
 #pragma unroll
     for (int i = 0; i < NE; ++i) total[i] = wave_sum(acc[i]);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Scores only, for a handful of tokens whose top-k is left to the gate/up kernel (experts_small.hip): a wave per (token, expert), so
+// that the router rows come through many compute units instead of one.  Block of 1 token, E = 32, us, whole router before : this
+// kernel 7.9 : 4.4; E = 128 11.8 : 4.4.
+// grid = (ceil(E / 4), T), block = 256.
+// ---------------------------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void router_scores_kernel(const float* __restrict__ x, const uint16_t* __restrict__ w,
+                                                            const uint16_t* __restrict__ bias, uint16_t* __restrict__ x_bf16,
+                                                            float* __restrict__ scores, int H, int E) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t = blockIdx.y;
+    const int n4 = H >> 2;
+    const float4* xr = reinterpret_cast<const float4*>(x + (size_t)t * H);
+    if (blockIdx.x == 0)
+        for (int c = threadIdx.x; c < n4; c += 256) {
+            const float4 v = xr[c];
+            reinterpret_cast<uint2*>(x_bf16 + (size_t)t * H)[c] = make_uint2(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w));
+        }
+    const int e[1] = {(int)blockIdx.x * 4 + wave};
+    if (e[0] >= E) return;
+    double total[1];
+    exact_dots<1, 12>(x + (size_t)t * H, w, e, H, lane, total);
+    if (lane == 0) scores[(size_t)t * E + e[0]] = (float)total[0] + bf16_bits_to_f32(bias[e[0]]);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1254,6 +1182,12 @@ int launch_router_fused(const float* x, const uint16_t* w, const uint16_t* bias,
         hipLaunchKernelGGL(router_fused_kernel<4>, dim3(T), dim3(64 * min(8, ceil_div(E, 4))), lds, stream, x, w, bias,
                            x_bf16, scores_out, topk_v, topk_i, H, E, K, do_softmax);
     }
+    return launch_status();
+}
+
+int launch_router_scores(const float* x, const uint16_t* w, const uint16_t* bias, uint16_t* x_bf16, float* scores, int T, int H,
+                         int E, hipStream_t stream) {
+    hipLaunchKernelGGL(router_scores_kernel, dim3(ceil_div(E, 4), T), dim3(256), 0, stream, x, w, bias, x_bf16, scores, H, E);
     return launch_status();
 }
 
