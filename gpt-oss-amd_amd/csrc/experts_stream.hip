@@ -1024,16 +1024,17 @@ MOE_DEVICE void prefill_body_mxfp4(const ExpertGemmArgs& a, uint8_t* lds, int e,
                 av[r] = u32x4{d[0], d[1], d[2], d[3]};
             }
             // activation operands are read from LDS two token tiles ahead of the MFMAs that use
-            // them, across the k-steps of the stage (NT is even, so the buffer parity carries over)
+            // them, across the k-steps of the stage
             if (j == 0) {
                 bq[0] = b_frag(s, 0, 0);
                 bq[1] = b_frag(s, 0, 1);
             }
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                const u32x4 b = bq[t & 1];
-                if (t + 2 < NT) bq[t & 1] = b_frag(s, j, t + 2);
-                else if (j + 1 < 4) bq[t & 1] = b_frag(s, j + 1, t + 2 - NT);
+                const int slot_b = (j * NT + t) & 1;
+                const u32x4 b = bq[slot_b];
+                if (t + 2 < NT) bq[slot_b] = b_frag(s, j, t + 2);
+                else if (j + 1 < 4) bq[slot_b] = b_frag(s, j + 1, t + 2 - NT);
                 __builtin_amdgcn_sched_barrier(0);  // keep the read above ahead of the MFMAs below
 #pragma unroll
                 for (int r = 0; r < R; ++r) acc[r][t] = mfma_16x16x32(av[r], b, acc[r][t]);
@@ -1094,14 +1095,14 @@ __global__ __launch_bounds__(WAVES * 64, 2) void expert_prefill_kernel(ExpertGem
     const int row0 = a.tile_row0[tile];
     const int nrows = a.tile_rows[tile];
     const int nt = (nrows + 15) >> 4;  // block-uniform
-    if (nt > 6) {
-        prefill_body_mxfp4<8, EPI, WAVES>(a, lds, e, row0, nrows, unit, active);
-    } else if (nt > 4) {
-        prefill_body_mxfp4<6, EPI, WAVES>(a, lds, e, row0, nrows, unit, active);
-    } else if (nt > 2) {
-        prefill_body_mxfp4<4, EPI, WAVES>(a, lds, e, row0, nrows, unit, active);
-    } else {
-        prefill_body_mxfp4<2, EPI, WAVES>(a, lds, e, row0, nrows, unit, active);
+    switch (nt) {
+        case 8: prefill_body_mxfp4<8, EPI, WAVES>(a, lds, e, row0, nrows, unit, active); break;
+        case 7: prefill_body_mxfp4<7, EPI, WAVES>(a, lds, e, row0, nrows, unit, active); break;
+        case 6: prefill_body_mxfp4<6, EPI, WAVES>(a, lds, e, row0, nrows, unit, active); break;
+        case 5: prefill_body_mxfp4<5, EPI, WAVES>(a, lds, e, row0, nrows, unit, active); break;
+        case 4: prefill_body_mxfp4<4, EPI, WAVES>(a, lds, e, row0, nrows, unit, active); break;
+        case 3: prefill_body_mxfp4<3, EPI, WAVES>(a, lds, e, row0, nrows, unit, active); break;
+        default: prefill_body_mxfp4<2, EPI, WAVES>(a, lds, e, row0, nrows, unit, active); break;
     }
 }
 
