@@ -600,9 +600,9 @@ struct ExpertPlan {
         a.rows = rows;
         a.K = Kdim;
         a.bias_expert_stride = rows;
+        a.n_cus = n_cus;
         if (small) {
             a.waves_per_block = 18;
-            a.n_cus = n_cus;
         } else if (direct && p->weight_format == MOE_WEIGHTS_MXFP4_TILED) {
             pick_two_pass(rows, &a.waves_per_block, &a.row_blocks);
         } else {

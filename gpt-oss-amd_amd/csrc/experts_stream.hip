@@ -131,7 +131,7 @@ MOE_DEVICE void ws_producer(const ExpertGemmArgs& a, uint8_t* lds, RowFn act_row
 // The lane id; for the work-queue entries (epilogue EPI) as a value that the compiler takes to be new at every call: what
 // follows from it is then worked out per token block, not ahead of the loop over an entry list's whole blocks, where it would
 // wait in scratch memory and be fetched in the stage loops (a spill access there waits for every weight load in flight).
-template <int EPI>
+template <int EPI, bool PRE = true>
 MOE_DEVICE int ws_lane() {
     int lane = threadIdx.x & 63;
     if constexpr (EPI == EPI_SWIGLU_F32 || EPI == EPI_SCATTER) asm volatile("" : "+v"(lane));
@@ -207,7 +207,7 @@ template <int FMT, int NT, int EPI, bool PRE = false, int R = 2, class SlotFn>
 MOE_DEVICE void ws_consumer(const ExpertGemmArgs& a, const uint8_t* lds, int e, SlotFn slot_of_row, int nrows, int tile0,
                             bool active) {
     static_assert(R == 1 || R == 2, "one or two row tiles per wave");
-    const int lane = ws_lane<EPI>();
+    const int lane = ws_lane<EPI, PRE>();
     const int g = lane >> 4;
     const int q = lane & 15;
     const int K = a.K;
@@ -437,7 +437,7 @@ MOE_DEVICE void ws_consumer_two(const ExpertGemmArgs& a, const uint8_t* lds, int
                             int unit_end, int unit_step, int passes) {
     constexpr int R = 2;
     constexpr bool TWO = true;
-    const int lane = ws_lane<EPI>();
+    const int lane = ws_lane<EPI, PRE>();
     const int g = lane >> 4;
     const int q = lane & 15;
     const int K = a.K;
@@ -733,7 +733,7 @@ __global__ __launch_bounds__((CONS + PROD) * 64, (CONS + PROD > 12) ? 4 : 3) voi
 // chunks of 64 consecutive assignments of topk_i with the expert id, the per-chunk match counts go
 // through LDS, one wave-wide prefix sum gives every chunk its offset, and the matching assignment
 // ids (token * experts_per_token + k, ascending: the bucket order of bucket_kernel) land in an LDS
-// list.  The block then runs the bucket's token blocks of up to 64 rows one after the other.
+// list.
 // Rows are addressed by assignment id: the activation row of assignment s is s / assign_div (gate/up
 // launch: the token's row) or s itself (down launch), and the output row is s.
 // grid = row blocks x experts (padded to a multiple of 8), block = 64 (CONS + PROD).
@@ -741,73 +741,148 @@ __global__ __launch_bounds__((CONS + PROD) * 64, (CONS + PROD > 12) ? 4 : 3) voi
 constexpr int kDirectMaxAssign = 4096;  // 64 chunks of 64: one lane per chunk in the prefix sum
 constexpr int kDirectMaxRows = 2048;    // longest bucket the LDS list holds
 
+// Item f of the list of the buckets' whole blocks of 64 rows but each one's first, expert by expert: its expert and first
+// row; false past the end of the list.
+MOE_DEVICE bool direct_whole_block(const int* hist, int n_experts, int f, int& e, int& row0) {
+    const int lane = threadIdx.x & 63;
+    for (int c = 0; c < n_experts; c += 64) {
+        const int n = c + lane < n_experts ? hist[c + lane] : 0;
+        const int whole = max(n - 65, 0) >> 6;
+        uint32_t incl = (uint32_t)whole;
+#define MOE_STEP(C, M) incl += dpp_move<C, M>(0u, incl);
+        MOE_DPP_STEPS(MOE_STEP)
+#undef MOE_STEP
+        const int total = (int)__builtin_amdgcn_readlane(incl, 63);
+        if (f < total) {
+            const int j = __popcll(__ballot((int)incl <= f));  // experts whose whole blocks all come before
+            const int before = (int)__builtin_amdgcn_readlane(incl, j) - __builtin_amdgcn_readlane(whole, j);
+            e = c + j;
+            row0 = __builtin_amdgcn_readlane(n - 64 * whole, j) + 64 * (f - before);
+            return true;
+        }
+        f -= total;
+    }
+    return false;
+}
+
+// This wave's chunks (p * WAVES + wave) of the assignment list.
+template <int WAVES, int P>
+MOE_DEVICE void direct_load_ids(const ExpertGemmArgs& a, int wave, int (&ids)[P]) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int s = (p * WAVES + wave) * 64 + (threadIdx.x & 63);
+        ids[p] = s < a.n_assign ? a.topk_i[s] : -1;
+    }
+}
+
+// Lists the expert's bucket (complete behind the next barrier) and returns its rows.
+template <int WAVES, int P>
+MOE_DEVICE int direct_list_bucket(const ExpertGemmArgs& a, int wave, const int (&ids)[P], int e, int* bucket, int* chunk_cnt) {
+    const int lane = threadIdx.x & 63;
+    const int n_chunks = (a.n_assign + 63) >> 6;
+    unsigned long long match[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int c = p * WAVES + wave;
+        match[p] = __ballot(ids[p] == e);
+        if (lane == 0 && c < n_chunks) chunk_cnt[c] = __popcll(match[p]);
+    }
+    __syncthreads();
+    // inclusive prefix sum of the chunk counts over the wave's lanes
+    uint32_t incl = lane < n_chunks ? (uint32_t)chunk_cnt[lane] : 0u;
+#define MOE_STEP(C, M) incl += dpp_move<C, M>(0u, incl);
+    MOE_DPP_STEPS(MOE_STEP)
+#undef MOE_STEP
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int c = p * WAVES + wave;
+        if (c < n_chunks) {  // wave-uniform
+            const int base = (int)__builtin_amdgcn_readlane(incl, c) - __popcll(match[p]);
+            const int dst = base + __popcll(match[p] & ((1ull << lane) - 1ull));
+            if (ids[p] == e && dst < kDirectMaxRows) bucket[dst] = c * 64 + lane;
+        }
+    }
+    return min((int)__builtin_amdgcn_readlane(incl, 63), kDirectMaxRows);
+}
+
 // TWO: blocks cover up to 2 CONS row units, in two passes over the bucket's activations.
+// MXFP4: the first a.main_blocks blocks of the launch take their bucket's remainder (1 .. 64 rows) and its first whole block of 64
+// rows.  What a skewed router leaves beyond that is dealt out over the other blocks, which come last and leave at once where
+// there is nothing.  With all of a bucket's token blocks run by its expert's own compute units, one after the other, the
+// hottest expert set the launch's time.  Whole block, us, so : dealt out, E = 32, router of no preference, 256 tokens 109 : 109, 384
+// tokens 147 : 146; Zipf 1.0, 256 tokens 187 : 182, 384 tokens 267 : 198; Zipf 1.5 245 : 174 and 375 : 189; E = 128, Zipf 1.0, 512 tokens
+// 548 : 446, 1024 tokens 859 : 540.
+// bf16 blocks keep to that: the second way into the stage loops costs the first its registers (256 tokens 280 : 287).
 template <int FMT, int EPI, int CONS, int PROD, bool TWO>
 __global__ __launch_bounds__((CONS + PROD) * 64, (CONS + PROD > 12) ? 4 : 3) void expert_stream_direct_kernel(ExpertGemmArgs a) {
     constexpr int WAVES = CONS + PROD;
     constexpr int P = (64 + WAVES - 1) / WAVES;  // chunks per wave
+    constexpr bool DEAL = FMT == FMT_MXFP4;
     __shared__ __attribute__((aligned(16))) uint8_t lds[kWsRing * kLdsStageBytes];
     __shared__ int bucket[kDirectMaxRows];
     __shared__ int chunk_cnt[64];
-    int e, rb;
-    ws_block_coords(a, e, rb);
-    if (e >= a.n_experts) return;  // block-uniform (grid padding)
-    const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n_chunks = (a.n_assign + 63) >> 6;
     // bf16 blocks make one pass over their rows and take them as a range of row tiles; MXFP4 blocks make up to two
     // passes of CONS units each, whose time does not depend on how many units a pass holds
     constexpr bool TILES = !TWO && FMT == FMT_BF16;
-    int u0, u1;
-    if constexpr (TILES) ws_row_tiles<CONS>(a, rb, u0, u1);
-    else ws_row_units(a, rb, u0, u1);
-    int n_bucket;
-    {
-        // this wave's chunks of the assignment list
-        int ids[P];
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            const int s = (p * WAVES + wave) * 64 + lane;
-            ids[p] = s < a.n_assign ? a.topk_i[s] : -1;
-        }
-        unsigned long long match[P];
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            const int c = p * WAVES + wave;
-            match[p] = __ballot(ids[p] == e);
-            if (lane == 0 && c < n_chunks) chunk_cnt[c] = __popcll(match[p]);
-        }
-        __syncthreads();
-        // inclusive prefix sum of the chunk counts over the wave's lanes
-        uint32_t incl = lane < n_chunks ? (uint32_t)chunk_cnt[lane] : 0u;
-#define MOE_STEP(C, M) incl += dpp_move<C, M>(0u, incl);
-        MOE_DPP_STEPS(MOE_STEP)
-#undef MOE_STEP
-        n_bucket = min((int)__builtin_amdgcn_readlane(incl, 63), kDirectMaxRows);
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            const int c = p * WAVES + wave;
-            if (c < n_chunks) {  // wave-uniform
-                const int base = (int)__builtin_amdgcn_readlane(incl, c) - __popcll(match[p]);
-                const int dst = base + __popcll(match[p] & ((1ull << lane) - 1ull));
-                if (ids[p] == e && dst < kDirectMaxRows) bucket[dst] = c * 64 + lane;
-            }
-        }
-        // the barrier that completes the list is the first one of the token block below
-    }
-    if (n_bucket == 0) return;
     // token of assignment s = s / assign_div, as a float multiplication (exact for s < 4096, assign_div <= 8)
     const float inv_div = 1.0f / (float)a.assign_div;
     auto token_of = [&](int s) { return (int)(((float)s + 0.5f) * inv_div); };
+    int ids[P];
+    if constexpr (DEAL) {
+        if ((int)blockIdx.x >= a.main_blocks) {  // block-uniform, as all of the following
+            __shared__ int hist[1024];  // rows per expert
+            const int slot = ((int)blockIdx.x - a.main_blocks) / a.row_blocks;
+            const int rb = (int)blockIdx.x - a.main_blocks - slot * a.row_blocks;
+            const int slots = ((int)gridDim.x - a.main_blocks) / a.row_blocks;
+            direct_load_ids<WAVES, P>(a, wave, ids);
+            for (int i = threadIdx.x; i < a.n_experts; i += 64 * WAVES) hist[i] = 0;
+            __syncthreads();
+#pragma unroll
+            for (int p = 0; p < P; ++p)
+                if ((unsigned)ids[p] < (unsigned)a.n_experts) atomicAdd(&hist[ids[p]], 1);
+            __syncthreads();
+            int f = slot, e, row0;
+            if (!direct_whole_block(hist, a.n_experts, f, e, row0)) return;
+            int u0, u1;
+            ws_row_units(a, rb, u0, u1);
+            const int passes = TWO ? min(2, max(1, ceil_div(u1 - u0, CONS))) : 1;
+            do {
+                direct_load_ids<WAVES, P>(a, wave, ids);
+                direct_list_bucket<WAVES, P>(a, wave, ids, e, bucket, chunk_cnt);
+                __syncthreads();
+                ExpertGemmArgs b = a;
+                asm volatile("" : "+s"(b.K));  // new in every round: nothing that depends on it is worked out ahead of the loop
+                auto act_row = [&](int i) { return a.gather ? token_of(bucket[row0 + i]) : bucket[row0 + i]; };
+                auto slot_of_row = [&](int i) { return bucket[row0 + i]; };
+                if (wave >= CONS) ws_producer<FMT, 4, PROD>(b, lds, act_row, 64, wave - CONS, passes);
+                else ws_consume_units<FMT, 4, EPI, false, TWO>(b, lds, e, slot_of_row, 64, u0 + wave, u1, CONS, passes);
+                __syncthreads();  // everyone is done with the list and the stages
+                f += slots;
+            } while (direct_whole_block(hist, a.n_experts, f, e, row0));
+            return;
+        }
+    }
+    int e, rb;
+    ws_block_coords(a, e, rb);
+    if (e >= a.n_experts) return;  // block-uniform (grid padding)
+    int u0, u1;
+    if constexpr (TILES) ws_row_tiles<CONS>(a, rb, u0, u1);
+    else ws_row_units(a, rb, u0, u1);
+    direct_load_ids<WAVES, P>(a, wave, ids);
+    const int n_bucket = direct_list_bucket<WAVES, P>(a, wave, ids, e, bucket, chunk_cnt);
+    if (n_bucket == 0) return;
     // The first token block takes the bucket's remainder (1..64 rows, any tile count) in straight-line
     // code; what is left are whole blocks of 64 rows, run by a loop that holds the four-tile variant
     // only (a loop around all tile-count variants costs every variant 30 registers per lane).
+    // The barrier that completes the list is the first one of the token block.
     const int first = n_bucket - ((n_bucket - 1) & ~63);
     ws_token_block<FMT, EPI, CONS, PROD, true, TWO, TILES>(
         a, lds, wave, u0, u1, e, [&](int i) { return a.gather ? token_of(bucket[i]) : bucket[i]; },
         [&](int i) { return bucket[i]; }, first);
     const int passes = TWO ? min(2, max(1, ceil_div(u1 - u0, CONS))) : 1;
-    for (int row0 = first; row0 < n_bucket; row0 += 64) {
+    const int end = DEAL ? min(n_bucket, first + 64) : n_bucket;
+    for (int row0 = first; row0 < end; row0 += 64) {
         auto act_row = [&](int i) { return a.gather ? token_of(bucket[row0 + i]) : bucket[row0 + i]; };
         auto slot_of_row = [&](int i) { return bucket[row0 + i]; };
         if (wave >= CONS) ws_producer<FMT, 4, PROD>(a, lds, act_row, 64, wave - CONS, passes);
@@ -1138,7 +1213,7 @@ int launch_cfg(const ExpertGemmArgs& a, hipStream_t stream) {
     }
     if constexpr (EPI == EPI_SWIGLU_BF16 || EPI == EPI_ROWS_F32) {
         if (a.topk_i) {  // bucketing inside the expert kernel
-            if (a.n_assign > kDirectMaxAssign || a.assign_div <= 0 || a.assign_div > 8 || a.n_experts <= 0) return MOE_ERR_LIMIT;
+            if (a.n_assign > kDirectMaxAssign || a.assign_div <= 0 || a.assign_div > 8 || a.n_experts <= 0 || a.n_experts > 1024) return MOE_ERR_LIMIT;
             ExpertGemmArgs b = a;
             const int cons = a.waves_per_block == 1 ? 12 : 10;
             // a block covers at most `cons` row units per pass; MXFP4 blocks may make two passes (the
@@ -1146,7 +1221,10 @@ int launch_cfg(const ExpertGemmArgs& a, hipStream_t stream) {
             const int units = a.rows / 32;
             b.row_blocks = max(a.row_blocks, ceil_div(units, (FMT == FMT_MXFP4 ? 2 : 1) * cons));
             const bool two = ceil_div(units, b.row_blocks) > cons;
-            dim3 grid(ceil_div(a.n_experts, 8) * 8 * b.row_blocks);
+            b.main_blocks = ceil_div(a.n_experts, 8) * 8 * b.row_blocks;
+            // and blocks for the token blocks from a bucket's third on: at most so many, one round of them
+            const int more = FMT == FMT_MXFP4 ? min((a.n_assign - 1) / 128, ceil_div(a.n_cus, b.row_blocks)) : 0;
+            dim3 grid(b.main_blocks + more * b.row_blocks);
             if constexpr (FMT == FMT_MXFP4) {
                 if (two && cons == 12) {
                     hipLaunchKernelGGL((expert_stream_direct_kernel<FMT, EPI, 12, 2, true>), grid, dim3(896), 0, stream, b);

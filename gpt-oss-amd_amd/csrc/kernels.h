@@ -98,6 +98,7 @@ struct ExpertGemmArgs {
     float alpha, limit;
     int max_tiles;
     int format;
+    int main_blocks;            // bucketing inside the streaming kernel: blocks of (expert, row block), set by the launcher
     int row_blocks;             // row blocks per token block (producer-consumer kernel: 0 = as few as fit;
                                 // prefill kernel: set by the launcher)
     int xcd_tiles;              // producer-consumer kernel: all row blocks of a token block on one XCD; prefill kernel
@@ -107,7 +108,7 @@ struct ExpertGemmArgs {
                                 // 128-token blocks, two blocks a CU; MXFP4 weights only); 17 tile kernel
                                 // (256-token blocks; bf16 weights only); 18 a 16-row tile per wave, buckets of a
                                 // handful of rows.  The work-queue entries take 0, 1 and 18.
-    int n_cus;                  // compute units to fill (18 and the work-queue entries)
+    int n_cus;                  // compute units to fill (bucketing inside the kernel, 18 and the work-queue entries)
     // experts_small.hip.  Gate/up: with scores (router logits [T, n_experts]) topk_i is not read; the kernel finds it and
     // the softmax weights itself and leaves both for the launches after it.
     const float* scores;
