@@ -15,12 +15,18 @@ namespace moe {
 constexpr int kHistCopies = 32;
 static int hist_copies(int E) { return E <= 256 ? kHistCopies : E <= 512 ? 16 : 8; }
 
+// V4: four experts per token and ids at 16-byte boundaries, up to kHeldTokens tokens: a thread holds the ids of its tokens in
+// registers from one 16-byte load each, for the histogram and for the compaction (the general form reads them twice, word by word, a
+// round trip per 8192 ids and per 4096 tokens).  32 experts, us, general : V4: 1000 tokens 9.2 : 8.6, 4096 tokens 12.6 : 9.8, 16384 tokens 35 : 20.
+constexpr int kHeldTokens = 16 * 1024;
+
 // grid = E blocks (one expert each), block = 1024 threads, dynamic LDS = (E * copies + E + 32) ints.
 // Tile map order: every full tile first (ascending expert), then the experts' partial last tiles from
 // the largest to the smallest (equal sizes: ascending expert).  An expert kernel that takes tiles in
 // this order runs its shortest blocks last, next to compute units that have already run out of work.
 // With map.second > 0 the same tiles are listed a second time, from index map.second of the three
 // arrays, in bucket order (an expert's tiles together, the partial one last).
+template <bool V4>
 __global__ __launch_bounds__(1024) void bucket_kernel(const int* __restrict__ topk_i,
                                                       const float* __restrict__ topk_v, int T, int K, int E,
                                                       int copies, int* __restrict__ expert_offsets,
@@ -39,19 +45,42 @@ __global__ __launch_bounds__(1024) void bucket_kernel(const int* __restrict__ to
     const int lane = tid & 63;
     const int wave = tid >> 6;
     const int A = T * K;
+    constexpr int HELD = V4 ? kHeldTokens / 1024 : 1;
+    int4 held[HELD];
+    if constexpr (V4) {
+#pragma unroll
+        for (int u = 0; u < HELD; ++u) {
+            const int t = u * 1024 + tid;
+            held[u] = make_int4(-1, -1, -1, -1);
+            if (u * 1024 < T && t < T) held[u] = reinterpret_cast<const int4*>(topk_i)[t];
+        }
+    }
 
     for (int i = tid; i < E * copies; i += blockDim.x) hist_c[i] = 0;
     if (tid < 8) scal[tid] = 0;
     __syncthreads();
     const int my_copy = tid & (copies - 1);
+    auto count = [&](int id) {
+        if ((unsigned)id < (unsigned)E) atomicAdd(&hist_c[id * copies + my_copy], 1);
+    };
+    if constexpr (V4) {
+#pragma unroll
+        for (int u = 0; u < HELD; ++u)
+            if (u * 1024 < T) {
+                count(held[u].x);
+                count(held[u].y);
+                count(held[u].z);
+                count(held[u].w);
+            }
+    }
     // eight loads per thread in flight: the pass costs memory round trips, not adds
-    for (int a0 = tid; a0 < A; a0 += 8 * 1024) {
+    for (int a0 = V4 ? A : tid; a0 < A; a0 += 8 * 1024) {
         int id[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) id[u] = a0 + u * 1024 < A ? topk_i[a0 + u * 1024] : -1;
 #pragma unroll
         for (int u = 0; u < 8; ++u)
-            if ((unsigned)id[u] < (unsigned)E) atomicAdd(&hist_c[id[u] * copies + my_copy], 1);
+            count(id[u]);
     }
     __syncthreads();
     for (int i = tid; i < E; i += blockDim.x) {
@@ -124,15 +153,13 @@ __global__ __launch_bounds__(1024) void bucket_kernel(const int* __restrict__ to
     // ordered compaction: tokens visited in ascending id, 1024 tokens per step; the ids of four steps
     // are fetched together (K <= 8 per token)
     int base = my_off;
-    for (int t00 = 0; t00 < T; t00 += 4 * 1024) {
+    auto steps = [&](int t00, auto ids_of) {  // tokens t00 .. t00 + 4095
         int mk4[4];
         float wv4[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const int t = t00 + u * 1024 + tid;
             int ids[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) ids[k] = (t < T && k < K) ? topk_i[(size_t)t * K + k] : -1;
+            ids_of(u, t00 + u * 1024 + tid, ids);
             int mk = -1;
 #pragma unroll
             for (int k = 7; k >= 0; --k) mk = ids[k] == e ? k : mk;  // the first k that names this expert
@@ -171,14 +198,39 @@ __global__ __launch_bounds__(1024) void bucket_kernel(const int* __restrict__ to
             base += total;
         }
         __syncthreads();
+    };
+    if constexpr (V4) {
+#pragma unroll
+        for (int h = 0; h < HELD / 4; ++h)
+            if (4096 * h < T)  // block-uniform
+                steps(4096 * h, [&](int u, int, int(&ids)[8]) {
+                    const int4 v = held[4 * h + u];
+                    ids[0] = v.x;
+                    ids[1] = v.y;
+                    ids[2] = v.z;
+                    ids[3] = v.w;
+                    ids[4] = ids[5] = ids[6] = ids[7] = -1;
+                });
+    } else {
+        for (int t00 = 0; t00 < T; t00 += 4 * 1024)
+            steps(t00, [&](int, int t, int(&ids)[8]) {
+#pragma unroll
+                for (int k = 0; k < 8; ++k) ids[k] = (t < T && k < K) ? topk_i[(size_t)t * K + k] : -1;
+            });
     }
 }
 
 int launch_bucket(const int* topk_i, const float* topk_v, int T, int K, int E, int* expert_offsets,
                   int* tokens_flat, float* weights_flat, int* slot_of, TileMap map, hipStream_t stream) {
     const int copies = hist_copies(E);
-    hipLaunchKernelGGL(bucket_kernel, dim3(E), dim3(1024), (size_t)(E * copies + E + 32) * sizeof(int), stream, topk_i,
-                       topk_v, T, K, E, copies, expert_offsets, tokens_flat, weights_flat, slot_of, map);
+    const size_t lds = (size_t)(E * copies + E + 32) * sizeof(int);
+    if (K == 4 && T <= kHeldTokens && ((uintptr_t)topk_i & 15u) == 0) {
+        hipLaunchKernelGGL(bucket_kernel<true>, dim3(E), dim3(1024), lds, stream, topk_i, topk_v, T, K, E, copies, expert_offsets,
+                           tokens_flat, weights_flat, slot_of, map);
+    } else {
+        hipLaunchKernelGGL(bucket_kernel<false>, dim3(E), dim3(1024), lds, stream, topk_i, topk_v, T, K, E, copies, expert_offsets,
+                           tokens_flat, weights_flat, slot_of, map);
+    }
     return launch_status();
 }
 
