@@ -963,11 +963,32 @@ __global__ __launch_bounds__(64 * kRowsWaves) void router_rows_kernel(const floa
 }
 
 // In-place softmax over the last dimension, one thread per row, the reference's order of
-// operations (src/run.cpp:321-339).
+// operations (src/run.cpp:321-339).  Up to eight values are loaded together instead of one after the other (256 rows of four, us,
+// 4.6 : 4.5; two rows 2.5 : 2.0).
 __global__ void softmax_rows_kernel(float* __restrict__ x, int B, int size) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= B) return;
     float* r = x + (size_t)b * size;
+    if (size <= 8) {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = r[min(i, size - 1)];
+        double max_val = v[0];
+#pragma unroll
+        for (int i = 1; i < 8; ++i)
+            if (v[i] > max_val) max_val = v[i];  // the last value again past the end
+        double sum = 0.0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (i < size) {
+                v[i] = expf((float)((double)v[i] - max_val));
+                sum += v[i];
+            }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (i < size) r[i] = (float)((double)v[i] / sum);
+        return;
+    }
     double max_val = r[0];
     for (int i = 1; i < size; ++i)
         if (r[i] > max_val) max_val = r[i];
@@ -1192,7 +1213,7 @@ int launch_router_scores(const float* x, const uint16_t* w, const uint16_t* bias
 }
 
 int launch_softmax_rows(float* x, int B, int size, hipStream_t stream) {
-    hipLaunchKernelGGL(softmax_rows_kernel, dim3(ceil_div(B, 256)), dim3(256), 0, stream, x, B, size);
+    hipLaunchKernelGGL(softmax_rows_kernel, dim3(ceil_div(B, 64)), dim3(64), 0, stream, x, B, size);
     return launch_status();
 }
 
