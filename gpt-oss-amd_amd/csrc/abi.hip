@@ -732,6 +732,12 @@ static int block_forward_impl(const moe_block_params* caller, moe_stream_t strea
                                  E, K, 1, stream);
         if (rc) return rc;
         if ((rc = mark())) return rc;
+    } else if (!strict && router_scores(T)) {
+        rc = launch_router_scores(p->t, p->w_router, p->b_router, ws.t_bf16, scores, T, H, E, stream);
+        if (rc) return rc;
+        if ((rc = mark())) return rc;
+        rc = launch_router_finalize(nullptr, 0, scores, nullptr, nullptr, p->topk_v, p->topk_i, T, E, K, 1, 1, stream);
+        if (rc) return rc;
     } else {
         const int S = router_segments(T, E, H, strict);
         rc = launch_router_partial(p->t, p->w_router, ws.router_partial, ws.t_bf16, T, H, E, S, stream);

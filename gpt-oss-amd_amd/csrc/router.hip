@@ -1064,6 +1064,11 @@ bool router_two_pass(int T, int E, int H) {
 // 199 : 92.  Up to 32 experts one launch is the faster one (1 token 22 : 24, 8 25 : 27, 256 41 : 45).
 bool router_split(int T, int E) { return E > 32 && T <= (E > 48 ? 128 : 16); }
 
+// Of those, a wave per (token, expert) for the scores rather than segments and their sums: a router row comes through the compute unit
+// once per token.  Partial + finalize : scores + finalize, us: E = 128, 9 tokens 12.2 : 9.7, 33 tokens 13.1 : 11.9, 48 tokens 13.7 : 13.8, 64 tokens
+// 14.2 : 17.6; E = 250, 20 tokens 22 : 15, 64 tokens 25 : 25; E = 1000, 9 tokens 52 : 31, 30 tokens 54 : 49.
+bool router_scores(int T) { return T <= 40; }
+
 static int screen_tiles(int E) { return E <= 16 ? 1 : E <= 32 ? 2 : 4; }  // 16-expert tiles per wave
 
 // Segment length (multiple of 32) and count of the screening pass: enough segments for about 2048
