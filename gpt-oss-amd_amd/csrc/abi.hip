@@ -32,10 +32,7 @@ inline int tile_tokens_of(bool prefill, int format) {
 // Which family runs the expert GEMMs, by average bucket size T*K/E (measured crossovers, 20b
 // shapes, token counts 256..4096).  MXFP4: the 128-token-block kernels win as soon as buckets start
 // to overflow one 64-token block (the streaming kernel then reads an expert's weights once per
-// block of its bucket), or, where the streaming launch takes four rounds of blocks or more, as soon as half its blocks hold three
-// token tiles.  Streaming : 128-token blocks, us, router of no preference, then skewed (Zipf 0.7): E = 32, 46.5 rows per expert 130 :
-// 147, 48 rows 172 : 151 and 199 : 152; E = 64, 42.5 rows 225 : 245, 47.5 rows 289 : 253, 45 rows 258 : 250 and 323 : 265; E = 128, 28 rows
-// 395 : 398 and 488 : 441, 32 rows 408 : 406, 34.4 rows 424 : 416, 37.5 rows 433 : 427 and 491 : 472; E = 256, 32 rows 829 : 821.  bf16: past the 48 rows per expert where the streaming kernels bucket in the expert kernels.  Streaming
+// block of its bucket).  bf16: past the 48 rows per expert where the streaming kernels bucket in the expert kernels.  Streaming
 // kernels : 256-token blocks, us, at 46 / 48 / 50 / 52 rows per expert: E = 32, router of no preference, 307 : 336, 309 : 337, 330 :
 // 338, 450 : 339 (below the line no bucket has more than 64 rows there; one that has, as one in six layers at 48 rows, takes a
 // second pass: 440), mildly skewed (Zipf 0.4) 435 : 343, 442 : 344, 446 : 346, 455 : 346; E = 64, K = 8, 48 rows 174 : 201, 50 rows
@@ -46,10 +43,7 @@ inline bool use_prefill_kernels(int T, int H, int I, int K, int E, int format, u
     // a block input past 4 GiB in bf16: only the streaming kernels address its rows
     if (format == MOE_WEIGHTS_BF16 && !(expert_tile_fits(T, 2 * I, H) && expert_tile_fits(0, H, I))) return false;
     if (flags & MOE_FLAG_FORCE_TILED) return true;
-    if (format != MOE_WEIGHTS_MXFP4_TILED) return rows > 48LL * E;
-    if (std::min(H, I) < 2560) return rows >= 52LL * E;  // the lines below are measured on contractions of 2880
-    const bool four_rounds = (long long)E * ceil_div(2 * I / 32, 24) >= 4 * 256;
-    return rows >= (four_rounds ? 34LL : 48LL) * E;
+    return format == MOE_WEIGHTS_MXFP4_TILED ? rows >= 52LL * E : rows > 48LL * E;
 }
 
 // Bucketing inside the expert kernels instead of a launch of its own: for the weight-streaming
