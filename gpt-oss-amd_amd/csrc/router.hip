@@ -1043,13 +1043,13 @@ int launch_router_partial(const float* x, const uint16_t* w, double* partial, ui
 }
 
 // ---- two-pass router -----------------------------------------------------------------------------
-// Worth it once the exact pass is throughput bound (three vector instructions per term), or once the fused kernel (a block
+// Worth it once the exact pass is throughput bound (16 cycles per term and wave), or once the fused kernel (a block
 // per token) would need a second round of blocks over the 256 compute units (the lines below are its rounds there, not asked
 // of the device).  With up to 32 experts a block holds a wave per two of them, several blocks share a compute unit, and
-// what counts is scores per batch.  Block of tiny experts, rows of 2880, us, fused : two-pass: E = 8, 900 tokens 80 : 91, 2047
-// 104 : 112; E = 16, 900 tokens 85 : 91, 1400 102 : 103; E = 24, 769 tokens 91 : 90, 1100 102 : 98; E = 32, 513 tokens 81 : 78, 640
-// 89 : 87, 1100 113 : 97; E = 48, 257 tokens 54 : 57, 400 61 : 63, 513 71 : 64; E = 64, 256 tokens 48 : 57, 257 59 : 57, 640 84 : 71;
-// E = 128, 256 tokens 62 : 62, 257 82 : 63.
+// what counts is scores per batch.  Up to 128 experts and rows of 3072 router_rows says when router_rows_kernel runs, and this
+// line only how much scratch the batch is given; beyond, it chooses screen + refine.  Whole block of tiny experts, rows of
+// 2880, before the top-k became shorter in all of them (4 us), us, fused : screen + refine: E = 64, 256 tokens 48 : 57, 640 84 :
+// 71; E = 128, 256 tokens 62 : 62, 257 82 : 63.
 bool router_two_pass(int T, int E, int H) {
     if (H % 32 != 0) return false;
     const long long scores = (long long)T * E;
@@ -1058,8 +1058,8 @@ bool router_two_pass(int T, int E, int H) {
 }
 
 // Partial sums and finalize in two launches instead of the fused kernel: beyond 32 experts its eight waves score a token's
-// experts in passes of 32, a memory round trip each, while few tokens leave most compute units idle.  The same block, us, fused :
-// two launches: E = 33, 1 token 24 : 24, 32 30 : 31, 128 37 : 38; E = 48, 1 token 29 : 24, 8 29 : 28, 64 32 : 33, 128 38 : 39; E = 64, 1
+// experts in passes of 32, a memory round trip each, while few tokens leave most compute units idle.  The same block at that time, us,
+// fused : two launches: E = 33, 1 token 24 : 24, 32 30 : 31, 128 37 : 38; E = 48, 1 token 29 : 24, 8 29 : 28, 64 32 : 33, 128 38 : 39; E = 64, 1
 // token 28 : 24, 64 36 : 34, 128 40 : 38, 200 46 : 49; E = 128, 1 token 39 : 26, 33 tokens 55 : 44, 128 57 : 53; E = 1000, 16 tokens
 // 199 : 92.  Up to 32 experts one launch is the faster one (1 token 22 : 24, 8 25 : 27, 256 41 : 45).
 bool router_split(int T, int E) { return E > 32 && T <= (E > 48 ? 128 : 16); }
