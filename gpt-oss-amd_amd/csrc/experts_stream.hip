@@ -742,11 +742,12 @@ constexpr int kDirectMaxAssign = 4096;  // 64 chunks of 64: one lane per chunk i
 constexpr int kDirectMaxRows = 2048;    // longest bucket the LDS list holds
 
 // Item f of the list of the buckets' whole blocks of 64 rows but each one's first, expert by expert: its expert and first
-// row; false past the end of the list.
+// row; false past the end of the list.  A bucket ends at kDirectMaxRows rows here as in direct_list_bucket: a caller's list may name
+// an expert more often, and bucket[] holds no more.
 MOE_DEVICE bool direct_whole_block(const int* hist, int n_experts, int f, int& e, int& row0) {
     const int lane = threadIdx.x & 63;
     for (int c = 0; c < n_experts; c += 64) {
-        const int n = c + lane < n_experts ? hist[c + lane] : 0;
+        const int n = c + lane < n_experts ? min(hist[c + lane], kDirectMaxRows) : 0;
         const int whole = max(n - 65, 0) >> 6;
         uint32_t incl = (uint32_t)whole;
 #define MOE_STEP(C, M) incl += dpp_move<C, M>(0u, incl);

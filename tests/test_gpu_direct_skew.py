@@ -60,3 +60,38 @@ def test_dealt_out_blocks_of_a_callers_list(pkg, wl, dev):
         assert torch.equal(got[named], yp[named])
         assert got[~named].isnan().all()
     assert (flat == 0).sum().item() > 128
+
+
+@pytest.mark.parametrize("fmt", ["mxfp4", "bf16"])
+@pytest.mark.parametrize("H,I", [(64, 64), (1088, 960)])
+@pytest.mark.parametrize("often", [2047, 2049, 3000, 4096])
+def test_an_expert_named_more_often_than_a_list_holds(pkg, wl, dev, H, I, fmt, often):
+    """A caller's list with one expert in more than 2048 assignments: the first 2048 of them get their rows, the others' rows and
+    what lies around the output stay as they are, and the other experts' rows are right."""
+    E, K, T = 128, 4, 1024
+    shape = wl.MoeShape("skew", T=T, H=H, I=I, E=E, K=K, fmt=fmt, seed=often)
+    blk, _ = wl.make_device_layer(shape, pkg.normal_table(), dev)
+    A = T * K
+    ids = (torch.arange(A, dtype=torch.int32) % (E - 1)) + 1
+    ids[torch.randperm(A, generator=torch.Generator().manual_seed(often))[:often]] = 0
+    ids = ids.view(T, K).to(dev)
+    h = torch.randn(A, I, device=dev).bfloat16()
+    tv = torch.zeros(T, K, device=dev)
+    st = torch.cuda.current_stream().cuda_stream
+    guarded = torch.full((3 * A, H), 123.0, device=dev)
+    y = guarded[A:2 * A]
+    p = blk.params(None, None, ids, tv)
+    assert blk.describe(p)["down"].startswith("expert_stream_direct")
+    print("long list", H, I, fmt, often, flush=True)
+    assert pkg.lib.moe_block_down_gemm(ctypes.byref(p), h.data_ptr(), y.data_ptr(), st) == 0
+    want = torch.empty_like(y)
+    for a in range(0, A, 512):  # the same rows, no expert named more than 512 times
+        part = ids.view(-1)[a:a + 512].view(-1, K).contiguous()
+        q = blk.params(None, None, part, tv[:part.shape[0]].contiguous(), flags=pkg.MOE_FLAG_FORCE_STREAM | pkg.MOE_FLAG_FORCE_DIRECT)
+        assert pkg.lib.moe_block_down_gemm(ctypes.byref(q), h[a:].data_ptr(), want[a:].data_ptr(), st) == 0
+    flat = ids.view(-1)
+    past = (flat == 0) & ((flat == 0).cumsum(0) > 2048)
+    assert int(past.sum()) == max(0, often - 2048)
+    want[past] = 123.0
+    assert torch.equal(y, want)
+    assert (guarded[:A] == 123.0).all() and (guarded[2 * A:] == 123.0).all()
