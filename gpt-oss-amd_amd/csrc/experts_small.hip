@@ -292,8 +292,9 @@ MOE_DEVICE void small_rows(const ExpertGemmArgs& a, uint8_t* lds, int e, SlotFn 
 // Block index -> (i-th expert that has a row, row block).  Experts are counted off in the assignment list itself, so blocks
 // of experts without rows (most of them at one token) are neither launched nor scheduled between the others.
 // grid = min(E, assignments) x row blocks, block = 64 waves, one tile of 16 weight rows per wave.
+// Three blocks to a compute unit (with 84 registers two, 7 tokens, 32 and 128 MXFP4 experts, us, 50.7 and 71.2 instead of 49.4 and 68.8).
 template <int FMT, int EPI>
-__global__ __launch_bounds__(64 * kSmallWaves, 4) void expert_small_kernel(ExpertGemmArgs a, int max_rows, int lds_bytes) {
+__global__ __launch_bounds__(64 * kSmallWaves, 6) void expert_small_kernel(ExpertGemmArgs a, int max_rows, int lds_bytes) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ uint32_t present[32];
     __shared__ int counts[8];
@@ -562,7 +563,9 @@ bool expert_small_fits(int n_assign, int rows, int K, int format) {
 
 // Every block of the gate/up launch finds the top-k of all tokens itself, a token to a wave: worth the router's second half while that
 // is one token each.  Whole block, us, router and small kernels : this, MXFP4, E = 32, 1 token 30 : 24, 4 tokens 50 : 47, 8 tokens 61.5 : 59, 10
-// tokens 68 : 69; E = 128, 1 token 34 : 25, 4 tokens 60 : 50, 8 tokens 87 : 80, 10 tokens 100 : 100, 16 tokens 131 : 134.
+// tokens 68 : 69; E = 128, 1 token 34 : 25, 4 tokens 60 : 50, 8 tokens 87 : 80, 10 tokens 100 : 100, 16 tokens 131 : 134.  More experts, K = 8:
+// blocks of 1024 x 1024, scores + finalize and small kernels : this, MXFP4, E = 256, 1 token 28 : 18, 8 tokens 50 : 44; E = 1000, 1 token 47 :
+// 21, 8 tokens 73 : 52; bf16, E = 1000, 8 tokens 108 : 90.
 bool expert_small_takes_scores(int n_tokens, int n_assign) { return n_tokens <= kSmallWaves && n_assign <= 64; }
 
 // bf16 weights of 16 assignments load a compute unit longer than the combine's launch takes (4 tokens, E = 32, two launches : one, us,

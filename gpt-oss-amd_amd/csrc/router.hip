@@ -957,7 +957,9 @@ __global__ __launch_bounds__(64 * kRowsWaves) void router_rows_kernel(const floa
     if (sub == 0 && t < T) {
         float my_v;
         int my_i;
-        select_topk(exact[tl], n_cand, K, lane, my_v, my_i);  // candidates are in ascending order: ties as by expert id
+        // candidates are in ascending order: ties as by expert id
+        if (EP <= 64 || n_cand <= 64) select_topk_of<1>(exact[tl], n_cand, K, lane, my_v, my_i);  // wave-uniform
+        else select_topk_of<2>(exact[tl], n_cand, K, lane, my_v, my_i);
         write_topk(my_v, cand[tl][my_i], K, lane, do_softmax, topk_v + (size_t)t * K, topk_i + (size_t)t * K);
     }
 }

@@ -16,56 +16,46 @@ MOE_DEVICE uint32_t rank_key(float v) {
 }
 MOE_DEVICE float rank_key_value(uint32_t m) { return __uint_as_float((m & 0x80000000u) ? m ^ 0x80000000u : ~m); }
 
-// K rounds of wave-wide argmax over vals[0..E) ordered by (value desc, index asc).  Lane r < K ends up holding the winner of
-// round r in (my_v, my_i).  C > 0: E <= 64 C, the keys stay in registers; C = 0: any E <= 2048, read anew in every round.
+// K rounds of wave-wide argmax over vals[0..E), E <= 64 C, ordered by (value desc, index asc).  Lane r < K ends up holding the
+// winner of round r in (my_v, my_i).  The keys stay in registers (read anew in every round, for more than 128 experts : so, 64
+// tokens, us: 256 experts, K = 8 10.2 : 5.2; 512, K = 4 10.8 : 5.5; 1000, K = 8 29 : 9.0).
 // A round is a chain of dependent instructions and little else: the maximum of the 32-bit keys is one instruction per DPP
 // step, and the lowest index that has it comes from a ballot.  (A 64-bit key with the index in it took five instructions a
 // step: 850 cycles a round, 200 now.)
 template <int C>
 MOE_DEVICE void select_topk_of(const float* vals, int E, int K, int lane, float& my_v, int& my_i) {
-    uint32_t key[C > 0 ? C : 1];
-    uint32_t taken = 0;  // C = 0: bit c set: candidate lane + 64*c already selected
-    if constexpr (C > 0) {
+    uint32_t key[C];
 #pragma unroll
-        for (int c = 0; c < C; ++c) key[c] = lane + 64 * c < E ? rank_key(vals[lane + 64 * c]) : 0u;
-    }
-    auto key_at = [&](int c) { return lane + 64 * c < E && !((taken >> c) & 1u) ? rank_key(vals[lane + 64 * c]) : 0u; };
+    for (int c = 0; c < C; ++c) key[c] = lane + 64 * c < E ? rank_key(vals[lane + 64 * c]) : 0u;
     my_v = -INFINITY;
     my_i = 0;
 #pragma nounroll
     for (int r = 0; r < K; ++r) {
         uint32_t best = 0;
-        if constexpr (C > 0) {
 #pragma unroll
-            for (int c = 0; c < C; ++c) best = max(best, key[c]);
-        } else {
-#pragma nounroll
-            for (int c = 0; 64 * c < E; ++c) best = max(best, key_at(c));
-        }
+        for (int c = 0; c < C; ++c) best = max(best, key[c]);
 #define MOE_STEP(CTRL, M) best = max(best, dpp_move<CTRL, M>(0u, best));
         MOE_DPP_STEPS(MOE_STEP)
 #undef MOE_STEP
         best = __builtin_amdgcn_readlane(best, 63);
         int bi = 0;
-        if constexpr (C > 0) {
+        if constexpr (C <= 2) {
 #pragma unroll
             for (int c = C - 1; c >= 0; --c) {
                 const unsigned long long has = __ballot(key[c] == best);
                 if (has) bi = 64 * c + (int)__builtin_ctzll(has);
             }
+        } else {  // as many ballots would fill the scalar registers
+            uint32_t miss = 0;  // ~index, or 0
 #pragma unroll
-            for (int c = 0; c < C; ++c) key[c] = bi == lane + 64 * c ? 0u : key[c];
-        } else {
-#pragma nounroll
-            for (int c = 0; 64 * c < E; ++c) {
-                const unsigned long long has = __ballot(key_at(c) == best);
-                if (has) {
-                    bi = 64 * c + (int)__builtin_ctzll(has);
-                    break;
-                }
-            }
-            if ((bi & 63) == lane) taken |= 1u << (bi >> 6);
+            for (int c = C - 1; c >= 0; --c) miss = key[c] == best ? ~(uint32_t)(64 * c + lane) : miss;
+#define MOE_STEP(CTRL, M) miss = max(miss, dpp_move<CTRL, M>(0u, miss));
+            MOE_DPP_STEPS(MOE_STEP)
+#undef MOE_STEP
+            bi = (int)~(uint32_t)__builtin_amdgcn_readlane(miss, 63);
         }
+#pragma unroll
+        for (int c = 0; c < C; ++c) key[c] = bi == lane + 64 * c ? 0u : key[c];
         if (lane == r) {
             my_v = rank_key_value(best);
             my_i = bi;
@@ -73,10 +63,13 @@ MOE_DEVICE void select_topk_of(const float* vals, int E, int K, int lane, float&
     }
 }
 
+// E <= 1024
 MOE_DEVICE void select_topk(const float* vals, int E, int K, int lane, float& my_v, int& my_i) {
     if (E <= 64) select_topk_of<1>(vals, E, K, lane, my_v, my_i);  // wave-uniform
     else if (E <= 128) select_topk_of<2>(vals, E, K, lane, my_v, my_i);
-    else select_topk_of<0>(vals, E, K, lane, my_v, my_i);
+    else if (E <= 256) select_topk_of<4>(vals, E, K, lane, my_v, my_i);
+    else if (E <= 512) select_topk_of<8>(vals, E, K, lane, my_v, my_i);
+    else select_topk_of<16>(vals, E, K, lane, my_v, my_i);
 }
 
 MOE_DEVICE float lane_value(float v, int src_lane) {

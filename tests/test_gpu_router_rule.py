@@ -65,3 +65,27 @@ def test_screening_keeps_non_finite_scores(pkg, wl, dev, T, what):
     assert torch.equal(ti, wi)
     assert torch.equal(tv.isnan(), wv.isnan())
     assert (tv.nan_to_num(0.0) - wv.nan_to_num(0.0)).abs().max().item() <= 4e-6
+
+
+@pytest.mark.parametrize("E", [1, 63, 64, 65, 128, 129, 192, 256, 257, 512, 513, 1000, 1024])
+def test_topk_register_forms(pkg, dev, E):
+    """Every number of keys per lane, at its edges: ties to the lower index, infinities and signed zeros in the order of the values,
+    rows that are one value throughout."""
+    g = torch.Generator().manual_seed(E)
+    rows = torch.randn(41, E, generator=g)
+    rows[1] = 0.25
+    rows[2] = float("-inf")
+    rows[3] = torch.where(torch.rand(E, generator=g) < 0.5, -0.0, 0.0)
+    rows[4::3] = rows[4::3].mul(2).round()  # few values, many ties
+    rows[5, E // 2], rows[5, E - 1], rows[5, 0] = float("inf"), float("inf"), float("-inf")
+    rows[6] = torch.arange(E)
+    rows[7] = -torch.arange(E).float()
+    for K in (1, 3, 8):
+        if K > E:
+            continue
+        v = torch.empty(41, K, device=dev)
+        i = torch.empty(41, K, dtype=torch.int32, device=dev)
+        print("top-k", E, K, flush=True)
+        pkg.topk(v, i, rows.to(dev), 41, E, K)
+        want_v, want_i = rows.sort(dim=1, descending=True, stable=True)
+        assert torch.equal(i.cpu().long(), want_i[:, :K]) and torch.equal(v.cpu(), want_v[:, :K])
