@@ -95,6 +95,34 @@ inline bool use_fused_experts(int E, bool direct, unsigned flags) {
     return direct && (flags & MOE_FLAG_FUSED_GEMM_LAUNCH) && E <= expert_fused_max_experts();
 }
 
+// Which kernels a block runs: block_forward_impl carries it out, moe_block_describe reports it.  The shapes are checked.
+enum class Router { kScores, kRows, kScreenRefine, kFused, kScoresFinalize, kPartialFinalize };
+struct BlockRoute {
+    bool prefill, direct;
+    Router router;
+    bool combined;  // the down kernel combines the tokens' rows as well
+
+    BlockRoute(const moe_block_params* p, int n_cus) {
+        const int T = p->n_tokens, H = p->hidden_dim, I = p->intermediate_dim, E = p->n_experts, K = p->experts_per_token;
+        const int fmt = p->weight_format;
+        prefill = use_prefill_kernels(T, H, I, K, E, fmt, p->flags);
+        direct = use_direct_bucketing(T, K, E, prefill, p->flags);
+        if (p->flags & MOE_FLAG_ROUTER_STRICT_ORDER) {
+            router = Router::kPartialFinalize;
+        } else if (expert_small_takes_scores(T, T * K) && use_small_kernels(T, H, I, K, E, fmt, direct, p->flags, n_cus)) {
+            router = Router::kScores;  // a handful of tokens: top-k and softmax are the gate/up kernel's
+        } else if (!p->router_score && (router_two_pass(T, E, H) || router_rows(T, E, H))) {
+            // same indices and weights, but no full score matrix
+            router = router_one_launch(T, E, H) ? Router::kRows : Router::kScreenRefine;
+        } else if (router_fused_fits(H) && !router_split(T, E)) {
+            router = Router::kFused;  // block per token: the exact pass of the two-pass router applied to every expert
+        } else {
+            router = router_scores(T) ? Router::kScoresFinalize : Router::kPartialFinalize;
+        }
+        combined = router == Router::kScores && !p->next_norm_out && expert_small_combines(T * K, I, fmt);
+    }
+};
+
 // Carves the caller's workspace for moe_block_forward; with base == nullptr only sizes it.
 struct BlockWorkspace {
     double* router_partial;
@@ -703,44 +731,41 @@ static int block_forward_impl(const moe_block_params* caller, moe_stream_t strea
     if ((rc = mark())) return rc;
 
     // 1. router logits -> top-k -> softmax  (src/forward.cpp:318-327; src/run.cpp:630-642)
-    // Large batches without a request for the full score matrix take the two-pass router (same
-    // indices and weights); everything else the single exact pass.
-    const bool strict = (p->flags & MOE_FLAG_ROUTER_STRICT_ORDER) != 0;
-    const bool prefill = use_prefill_kernels(T, H, I, K, E, p->weight_format, p->flags);
-    const bool direct = use_direct_bucketing(T, K, E, prefill, p->flags);
-    // a handful of tokens: the scores only, top-k and softmax are the gate/up kernel's
-    const bool scores_only = !strict && expert_small_takes_scores(T, T * K) &&
-                             use_small_kernels(T, H, I, K, E, p->weight_format, direct, p->flags, device_cu_count());
+    const BlockRoute route(p, device_cu_count());
+    const bool prefill = route.prefill, direct = route.direct;
     float* const scores = p->router_score ? p->router_score : reinterpret_cast<float*>(ws.router_partial);
-    if (scores_only) {
-        rc = launch_router_scores(p->t, p->w_router, p->b_router, ws.t_bf16, scores, T, H, E, stream);
-        if (rc) return rc;
-        if ((rc = mark())) return rc;
-    } else if (!strict && !p->router_score && (router_two_pass(T, E, H) || router_rows(T, E, H))) {
-        rc = launch_router_two_pass(p->t, p->w_router, p->b_router, ws.router_partial, ws.t_bf16, p->topk_v, p->topk_i, T,
-                                    H, E, K, 1, stream, timer ? timer->ev[stage++] : nullptr);
-        if (rc) return rc;
-    } else if (!strict && router_fused_fits(H) && !router_split(T, E)) {
-        // one launch, block per token: the exact pass of the two-pass router applied to every expert
-        rc = launch_router_fused(p->t, p->w_router, p->b_router, ws.t_bf16, p->router_score, p->topk_v, p->topk_i, T, H,
-                                 E, K, 1, stream);
-        if (rc) return rc;
-        if ((rc = mark())) return rc;
-    } else if (!strict && router_scores(T)) {
-        rc = launch_router_scores(p->t, p->w_router, p->b_router, ws.t_bf16, scores, T, H, E, stream);
-        if (rc) return rc;
-        if ((rc = mark())) return rc;
-        rc = launch_router_finalize(nullptr, 0, scores, nullptr, nullptr, p->topk_v, p->topk_i, T, E, K, 1, 1, stream);
-        if (rc) return rc;
-    } else {
-        const int S = router_segments(T, E, H, strict);
-        rc = launch_router_partial(p->t, p->w_router, ws.router_partial, ws.t_bf16, T, H, E, S, stream);
-        if (rc) return rc;
-        if ((rc = mark())) return rc;
-        rc = launch_router_finalize(ws.router_partial, S, nullptr, p->b_router, p->router_score, p->topk_v, p->topk_i, T,
-                                    E, K, 1, 1, stream);
-        if (rc) return rc;
+    switch (route.router) {
+        case Router::kScores:
+            rc = launch_router_scores(p->t, p->w_router, p->b_router, ws.t_bf16, scores, T, H, E, stream);
+            if (!rc) rc = mark();
+            break;
+        case Router::kRows:
+        case Router::kScreenRefine:
+            rc = launch_router_two_pass(p->t, p->w_router, p->b_router, ws.router_partial, ws.t_bf16, p->topk_v, p->topk_i, T,
+                                        H, E, K, 1, stream, timer ? timer->ev[stage++] : nullptr);
+            break;
+        case Router::kFused:
+            rc = launch_router_fused(p->t, p->w_router, p->b_router, ws.t_bf16, p->router_score, p->topk_v, p->topk_i, T, H,
+                                     E, K, 1, stream);
+            if (!rc) rc = mark();
+            break;
+        case Router::kScoresFinalize:
+            rc = launch_router_scores(p->t, p->w_router, p->b_router, ws.t_bf16, scores, T, H, E, stream);
+            if (rc) return rc;
+            if ((rc = mark())) return rc;
+            rc = launch_router_finalize(nullptr, 0, scores, nullptr, nullptr, p->topk_v, p->topk_i, T, E, K, 1, 1, stream);
+            break;
+        case Router::kPartialFinalize: {
+            const int S = router_segments(T, E, H, (p->flags & MOE_FLAG_ROUTER_STRICT_ORDER) != 0);
+            rc = launch_router_partial(p->t, p->w_router, ws.router_partial, ws.t_bf16, T, H, E, S, stream);
+            if (rc) return rc;
+            if ((rc = mark())) return rc;
+            rc = launch_router_finalize(ws.router_partial, S, nullptr, p->b_router, p->router_score, p->topk_v, p->topk_i, T,
+                                        E, K, 1, 1, stream);
+            break;
+        }
     }
+    if (rc) return rc;
     if ((rc = mark())) return rc;
 
     // 2. bucketing + token-block map  (src/forward.cpp:329-376)
@@ -761,13 +786,12 @@ static int block_forward_impl(const moe_block_params* caller, moe_stream_t strea
     const ExpertPlan plan(p, ws, prefill, direct, tile_tokens, max_tiles);
     ExpertGemmArgs a1 = plan.gate_up(ws.t_bf16, ws.h_by_slot);
     ExpertGemmArgs a2 = plan.down(ws.h_by_slot, ws.y_by_slot);
-    if (scores_only) {
+    if (route.router == Router::kScores) {
         a1.scores = scores;
         a1.topk_v_out = p->topk_v;
         a1.topk_i_out = p->topk_i;
     }
-    const bool combined = scores_only && !p->next_norm_out && expert_small_combines(T * K, I, fmt);
-    if (combined) {
+    if (route.combined) {
         a2.combine_v = p->topk_v;
         a2.e_agg = p->e_agg;
         a2.residual_x = p->residual_x;
@@ -795,7 +819,7 @@ static int block_forward_impl(const moe_block_params* caller, moe_stream_t strea
     if ((rc = mark())) return rc;
 
     // 5. weighted combine in ascending expert id (+ residual)  (src/run.cpp:702-712)
-    if (combined) return mark();
+    if (route.combined) return mark();
     const int* slot_of = direct ? nullptr : ws.slot_of;  // direct: the row of assignment (t, k) is t * K + k
     if (p->next_norm_out) {
         rc = launch_combine_norm(ws.y_by_slot, slot_of, p->topk_i, p->topk_v, p->e_agg, p->residual_x,
@@ -828,26 +852,31 @@ int moe_block_forward_layers(const moe_block_params* params, int n_layers, moe_s
     return MOE_OK;
 }
 
-int moe_block_describe(const moe_block_params* p, char* text, size_t text_bytes) {
-    if (!p || !text) return MOE_ERR_NULL;
+int moe_block_describe(const moe_block_params* caller, char* text, size_t text_bytes) {
+    if (!caller || !text) return MOE_ERR_NULL;
     if (text_bytes < 64) return MOE_ERR_LIMIT;
-    if (p->struct_bytes != sizeof(moe_block_params) && p->struct_bytes != offsetof(moe_block_params, next_norm_weight))
-        return MOE_ERR_FORMAT;
+    constexpr size_t kOldBytes = offsetof(moe_block_params, next_norm_weight);
+    if (caller->struct_bytes != sizeof(moe_block_params) && caller->struct_bytes != kOldBytes) return MOE_ERR_FORMAT;
+    moe_block_params local{};
+    memcpy(&local, caller, caller->struct_bytes);
+    const moe_block_params* p = &local;
     const int T = p->n_tokens, H = p->hidden_dim, I = p->intermediate_dim, E = p->n_experts,
               K = p->experts_per_token;
     int rc = check_dims(T, H, I, E, K);
     if (rc) return rc;
     const int fmt = p->weight_format;
     if (fmt != MOE_WEIGHTS_BF16 && fmt != MOE_WEIGHTS_MXFP4_TILED) return MOE_ERR_FORMAT;
-    // the same decisions, in the same order, as block_forward_impl
-    const bool strict = (p->flags & MOE_FLAG_ROUTER_STRICT_ORDER) != 0;
-    const char* router = (!strict && !p->router_score && router_two_pass(T, E, H))
-                             ? "router_screen_kernel + router_refine_kernel"
-                             : (!strict && router_fused_fits(H) && !router_split(T, E))
-                                 ? "router_fused_kernel"
-                                                                 : "router_partial_kernel + router_finalize_kernel";
-    const bool prefill = use_prefill_kernels(T, H, I, K, E, fmt, p->flags);
-    const bool direct = use_direct_bucketing(T, K, E, prefill, p->flags);
+    const BlockRoute route(p, device_cu_count());
+    const bool prefill = route.prefill, direct = route.direct;
+    const char* router = "";
+    switch (route.router) {
+        case Router::kScores: router = "router_scores_kernel"; break;
+        case Router::kRows: router = "router_rows_kernel"; break;
+        case Router::kScreenRefine: router = "router_screen_kernel + router_refine_kernel"; break;
+        case Router::kFused: router = "router_fused_kernel"; break;
+        case Router::kScoresFinalize: router = "router_scores_kernel + router_finalize_kernel"; break;
+        case Router::kPartialFinalize: router = "router_partial_kernel + router_finalize_kernel"; break;
+    }
     const int tile_tokens = tile_tokens_of(prefill, fmt);
     BlockWorkspace ws(nullptr, T, H, I, E, K);
     const ExpertPlan plan(p, ws, prefill, direct, tile_tokens, tile_map_capacity(T * K, E, tile_tokens));
@@ -859,6 +888,8 @@ int moe_block_describe(const moe_block_params* p, char* text, size_t text_bytes)
             snprintf(out, n, "expert_tile_bf16_kernel<%d>", epi);
         } else if (prefill) {
             snprintf(out, n, "expert_prefill_kernel<%d, %d, 4>", fmt, epi);
+        } else if (epi == 1 && route.combined) {
+            snprintf(out, n, "expert_tiny_down_kernel<%d>", fmt);
         } else if (plan.small) {
             snprintf(out, n, "expert_small_kernel<%d, %d>", fmt, epi);
         } else if (direct) {
@@ -881,7 +912,11 @@ int moe_block_describe(const moe_block_params* p, char* text, size_t text_bytes)
     }
     const int n = snprintf(text, text_bytes, "router=%s; bucketing=%s; gate_up=%s; down=%s; combine=%s; compute_units=%d",
                            router, direct ? "in the expert kernels" : "bucket_kernel", g1, g2,
-                           p->next_norm_out ? "combine_norm_kernel" : "combine_kernel", plan.n_cus);
+                           route.combined                 ? "in the down kernel"
+                           : !p->next_norm_out            ? "combine_kernel"
+                           : combine_norm_fits(H)         ? "combine_norm_kernel"
+                                                          : "combine_kernel + rmsnorm_kernel",
+                           plan.n_cus);
     return (n < 0 || (size_t)n >= text_bytes) ? MOE_ERR_LIMIT : MOE_OK;
 }
 

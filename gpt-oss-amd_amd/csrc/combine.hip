@@ -271,9 +271,12 @@ __global__ __launch_bounds__(256) void combine_norm_kernel(const float4* __restr
 
 // Returns MOE_ERR_LIMIT when the row is too long for the fused kernel (the caller then runs the two
 // kernels one after the other).
+bool combine_norm_fits(int H) { return H <= 4 * 1024; }
+
 int launch_combine_norm(const float* y_by_slot, const int* slot_of, const int* topk_i, const float* topk_v,
                         float* e_agg, float* residual_x, const uint16_t* norm_weight, float* norm_out, int T, int K,
                         int H, hipStream_t stream) {
+    if (!combine_norm_fits(H)) return MOE_ERR_LIMIT;
     const int H4 = H / 4;
     const int ni = ceil_div(H4, 256);
     auto y = reinterpret_cast<const float4*>(y_by_slot);
@@ -289,11 +292,9 @@ int launch_combine_norm(const float* y_by_slot, const int* slot_of, const int* t
     } else if (ni <= 3) {
         hipLaunchKernelGGL((combine_norm_kernel<3>), dim3(T), dim3(256), 0, stream, y, slot_of, topk_i, topk_v, e, r,
                            norm_weight, o, K, H4);
-    } else if (ni <= 4) {
+    } else {
         hipLaunchKernelGGL((combine_norm_kernel<4>), dim3(T), dim3(256), 0, stream, y, slot_of, topk_i, topk_v, e, r,
                            norm_weight, o, K, H4);
-    } else {
-        return MOE_ERR_LIMIT;
     }
     return launch_status();
 }

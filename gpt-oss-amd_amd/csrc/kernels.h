@@ -31,6 +31,7 @@ int launch_router_fused(const float* x, const uint16_t* w, const uint16_t* bias,
 // recorded after the first pass.
 bool router_two_pass(int T, int E, int H);
 bool router_rows(int T, int E, int H);  // launch_router_two_pass is the faster one for smaller batches too: needs no scratch there
+bool router_one_launch(int T, int E, int H);  // launch_router_two_pass is router_rows_kernel, not screen + refine
 size_t router_screen_bytes(int T, int E, int H);
 int launch_router_two_pass(const float* x, const uint16_t* w, const uint16_t* bias, void* scratch, uint16_t* x_bf16,
                            float* topk_v, int* topk_i, int T, int H, int E, int K, int do_softmax,
@@ -153,6 +154,7 @@ int launch_expert_fused(const ExpertFusedArgs& f, int n_blocks, hipStream_t stre
 int launch_combine(const float* y_by_slot, const int* slot_of, const int* topk_i, const float* topk_v,
                    float* e_agg, float* residual_x, int T, int K, int H, hipStream_t stream);
 // combine + residual add + the RMSNorm that follows; MOE_ERR_LIMIT if H is too long for one pass
+bool combine_norm_fits(int H);
 int launch_combine_norm(const float* y_by_slot, const int* slot_of, const int* topk_i, const float* topk_v,
                         float* e_agg, float* residual_x, const uint16_t* norm_weight, float* norm_out, int T, int K,
                         int H, hipStream_t stream);

@@ -1121,6 +1121,8 @@ bool router_rows(int T, int E, int H) {
     return router_rows_fits(E, H) && (E > 48 ? T > 64 : E > 32 ? T > 16 : E > 16 ? T > 256 : (long long)T * E > 12000);
 }
 
+bool router_one_launch(int, int E, int H) { return router_rows_fits(E, H); }
+
 static int launch_router_rows(const float* x, const uint16_t* w, const uint16_t* bias, uint16_t* x_bf16, float* topk_v,
                               int* topk_i, int T, int H, int E, int K, int do_softmax, hipStream_t stream, float* approx_out,
                               float* delta_out, int* n_cand_out) {
@@ -1152,7 +1154,7 @@ int launch_router_two_pass(const float* x, const uint16_t* w, const uint16_t* bi
                            float* topk_v, int* topk_i, int T, int H, int E, int K, int do_softmax,
                            hipStream_t stream, hipEvent_t between, float* approx_out, float* delta_out,
                            int* n_cand_out) {
-    if (router_rows_fits(E, H)) {
+    if (router_one_launch(T, E, H)) {
         int rc = launch_router_rows(x, w, bias, x_bf16, topk_v, topk_i, T, H, E, K, do_softmax, stream, approx_out, delta_out,
                                     n_cand_out);
         if (rc) return rc;

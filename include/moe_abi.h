@@ -352,12 +352,7 @@ MOE_API int moe_block_forward_layers(const moe_block_params* params, int n_layer
  * whether router_score / next_norm_out are set; pointers are not dereferenced and may be NULL), as
  * one line of text: "router=...; bucketing=...; gate_up=<kernel name as a profiler shows it>;
  * down=...; combine=...; compute_units=N".  For benchmarks and profile summaries that have to name
- * the kernel they measured.  "router=" names the method, by the kernels that carry it out for any sizes:
- * with up to 128 experts and rows of up to 3072 values, one launch of router_rows_kernel takes their place
- * in all but the smallest batches.  Up to 8 tokens of expert_small_kernel have their scores from
- * router_scores_kernel and their top-k from the gate/up kernel, up to 40 tokens that kernel stands in for
- * router_partial_kernel; the down GEMM of up to 16 assignments combines them as well
- * (expert_tiny_down_kernel).  text_bytes >= 64; MOE_ERR_LIMIT if the line does not fit. */
+ * the kernel they measured.  text_bytes >= 64; MOE_ERR_LIMIT if the line does not fit. */
 MOE_API int moe_block_describe(const moe_block_params* params, char* text, size_t text_bytes);
 
 /* The down-projection GEMM of moe_block_forward on its own, on rows the caller provides (the

@@ -88,6 +88,36 @@ def test_small_kernel_line_of_many_rounds(pkg, fmt, H, I, last):
         assert k["gate_up"].startswith(name) and k["down"].startswith(name), (T, k)
 
 
+def test_describe_names_the_kernels_that_run(pkg):
+    """Router, down GEMM and combine as they are launched, for each way through a block; the struct without the norm's members."""
+    def names(T, E, K=4, H=2880, fmt=pkg.MOE_WEIGHTS_MXFP4_TILED, **kw):
+        return kernels_of(pkg, T, H, 2880, E, K, fmt, **kw)
+    tiny = names(1, 32)
+    assert (tiny["router"], tiny["gate_up"], tiny["down"], tiny["combine"]) == (
+        "router_scores_kernel", "expert_small_kernel<1, 0>", "expert_tiny_down_kernel<1>", "in the down kernel")
+    few = names(8, 32)
+    assert (few["router"], few["down"], few["combine"]) == ("router_scores_kernel", "expert_small_kernel<1, 1>", "combine_kernel")
+    assert names(3, 32, fmt=pkg.MOE_WEIGHTS_BF16)["down"] == "expert_tiny_down_kernel<0>"
+    assert names(4, 32, fmt=pkg.MOE_WEIGHTS_BF16)["down"] == "expert_small_kernel<0, 1>"
+    assert names(9, 128)["router"] == "router_scores_kernel + router_finalize_kernel"
+    assert names(41, 128)["router"] == "router_partial_kernel + router_finalize_kernel"
+    assert names(256, 32)["router"] == "router_fused_kernel"
+    assert names(1000, 32)["router"] == names(100, 128)["router"] == "router_rows_kernel"
+    assert names(1000, 200)["router"] == names(1000, 32, H=3136)["router"] == "router_screen_kernel + router_refine_kernel"
+    strict = names(1, 32, flags=pkg.MOE_FLAG_ROUTER_STRICT_ORDER)
+    assert (strict["router"], strict["combine"]) == ("router_partial_kernel + router_finalize_kernel", "combine_kernel")
+    # a norm to follow: the down kernel leaves the combine to the kernel that has the whole row
+    for H, combine in ((2880, "combine_norm_kernel"), (4096, "combine_norm_kernel"), (4160, "combine_kernel + rmsnorm_kernel")):
+        p = pkg.BlockParams(struct_bytes=ctypes.sizeof(pkg.BlockParams), n_tokens=1, hidden_dim=H, intermediate_dim=2880, n_experts=32,
+                            experts_per_token=4, weight_format=pkg.MOE_WEIGHTS_MXFP4_TILED, next_norm_weight=16, next_norm_out=16)
+        text = ctypes.create_string_buffer(1024)
+        assert pkg.lib.moe_block_describe(ctypes.byref(p), text, len(text)) == 0
+        assert "; combine=%s; " % combine in text.value.decode()
+        p.struct_bytes = pkg.BlockParams.next_norm_weight.offset  # what lies past the older struct is not looked at
+        assert pkg.lib.moe_block_describe(ctypes.byref(p), text, len(text)) == 0
+        assert "; combine=in the down kernel; " in text.value.decode()
+
+
 def test_tile_kernel_takes_large_activation_tensors(pkg):
     """Rows by slot past 4 GiB are no reason to leave the bf16 tile kernel, unless the 256 of one block are; gathered rows past it
     are, at the last byte."""

@@ -6,19 +6,28 @@ import torch
 pytestmark = pytest.mark.gpu
 
 FUSED, SPLIT, TWO = "router_fused_kernel", "router_partial_kernel + router_finalize_kernel", "router_screen_kernel + router_refine_kernel"
-# experts -> tokens and the router of rows that the one-launch kernel takes, on both sides of each line
+ROWS, SCORES, TOPK_LATER = "router_rows_kernel", "router_scores_kernel + router_finalize_kernel", "router_scores_kernel"
+# experts -> tokens and the router of rows that the one-launch kernels take, on both sides of each line
 LINES = {
-    8: [(1, FUSED), (2048, FUSED), (8191, FUSED), (8192, TWO)],
-    16: [(2048, FUSED), (4095, FUSED), (4096, TWO)],
-    17: [(1204, FUSED), (1205, TWO)],
-    32: [(1, FUSED), (639, FUSED), (640, TWO), (641, TWO), (2047, TWO), (2048, TWO)],
-    33: [(1, SPLIT), (16, SPLIT), (17, FUSED), (128, FUSED), (129, FUSED), (512, FUSED), (513, TWO)],
-    48: [(16, SPLIT), (17, FUSED), (512, FUSED), (513, TWO)],
-    49: [(128, SPLIT), (129, FUSED), (256, FUSED), (257, TWO)],
-    250: [(5, SPLIT), (128, SPLIT), (129, FUSED), (256, FUSED), (257, TWO), (263, TWO)],
+    8: [(2, TOPK_LATER), (3, FUSED), (1500, FUSED), (1501, ROWS), (2048, ROWS), (8191, ROWS), (8192, ROWS)],
+    16: [(750, FUSED), (751, ROWS), (2048, ROWS), (4096, ROWS)],
+    17: [(256, FUSED), (257, ROWS), (1204, ROWS), (1205, ROWS)],
+    32: [(1, TOPK_LATER), (8, TOPK_LATER), (9, FUSED), (256, FUSED), (257, ROWS), (640, ROWS), (2047, ROWS), (2048, ROWS)],
+    33: [(1, TOPK_LATER), (16, SCORES), (17, ROWS), (128, ROWS), (513, ROWS)],
+    48: [(16, SCORES), (17, ROWS), (513, ROWS)],
+    49: [(40, SCORES), (41, SPLIT), (64, SPLIT), (65, ROWS), (257, ROWS)],
+    128: [(8, TOPK_LATER), (9, SCORES), (64, SPLIT), (65, ROWS), (257, ROWS), (2049, ROWS)],
+    250: [(5, TOPK_LATER), (9, SCORES), (40, SCORES), (41, SPLIT), (128, SPLIT), (129, FUSED), (256, FUSED), (257, TWO), (263, TWO)],
     257: [(128, SPLIT), (129, FUSED), (255, FUSED), (256, TWO)],
-    1000: [(1, SPLIT), (65, SPLIT), (66, TWO), (128, TWO), (129, TWO)],
+    1000: [(1, TOPK_LATER), (40, SCORES), (41, SPLIT), (65, SPLIT), (66, TWO), (128, TWO), (129, TWO)],
 }
+
+
+def long_rows(T, E, router):
+    """The router of rows past 3072 values."""
+    if router == ROWS:
+        router = TWO if T * E >= (20480 if 16 < E <= 32 else 65536) or T > (256 if E > 48 else 512) and E > 32 else FUSED
+    return (SCORES if T <= 40 else SPLIT) if router == FUSED else router
 
 
 @pytest.mark.parametrize("H", [64, 2880, 3136])  # the last is too long for the one-launch kernel
@@ -33,9 +42,7 @@ def test_router_kernels_agree(pkg, wl, dev, H, E):
         print("router", H, E, T, flush=True)
         t = x[:T].contiguous()
         _, ti, tv = blk.forward(t)
-        if H > 3072 and router == FUSED:
-            router = SPLIT
-        assert blk.describe(blk.params(t, x, ti, tv))["router"] == router
+        assert blk.describe(blk.params(t, x, ti, tv))["router"] == (long_rows(T, E, router) if H > 3072 else router)
         _, wi, wv = blk.forward(t, flags=pkg.MOE_FLAG_ROUTER_STRICT_ORDER)
         assert torch.equal(ti, wi)
         # logits differ, if at all, in the last place of their rounding to fp32: 2^-23 of |logit| < 16
@@ -43,11 +50,12 @@ def test_router_kernels_agree(pkg, wl, dev, H, E):
 
 
 @pytest.mark.parametrize("T", [700, 2100])
+@pytest.mark.parametrize("H,E,router", [(320, 32, ROWS), (320, 160, TWO), (3136, 32, TWO)])
 @pytest.mark.parametrize("what", ["inf weight", "nan weight", "nan weight, ties", "nan bias", "inf bias", "inf row", "nan row", "huge row"])
-def test_screening_keeps_non_finite_scores(pkg, wl, dev, T, what):
+def test_screening_keeps_non_finite_scores(pkg, wl, dev, T, H, E, router, what):
     """Scores that are infinite or not a number rank as in the single exact pass: the screening pass drops an expert for a
     finite approximate score below the bound only."""
-    H, E, K = 320, 32, 4
+    K = 4
     table = pkg.normal_table()
     shape = wl.MoeShape("router", T=T, H=H, I=64, E=E, K=K, fmt="mxfp4", seed=11)
     blk, _ = wl.make_device_layer(shape, table, dev)
@@ -58,9 +66,9 @@ def test_screening_keeps_non_finite_scores(pkg, wl, dev, T, what):
         b.fill_(0.5)
     v = float(what[:3]) if what[:3] in ("inf", "nan") else 3.39e38  # the last rounds to an infinity in bf16
     {"weight": w[5], "weight, ties": w[5], "bias": b, "row": x[::3]}[what.split(" ", 1)[1]][..., 7] = v
-    print("non-finite router", T, what, flush=True)
+    print("non-finite router", T, H, E, what, flush=True)
     _, ti, tv = blk.forward(x)
-    assert blk.describe(blk.params(x, x, ti, tv))["router"] == "router_screen_kernel + router_refine_kernel"
+    assert blk.describe(blk.params(x, x, ti, tv))["router"] == router
     _, wi, wv = blk.forward(x, flags=pkg.MOE_FLAG_ROUTER_STRICT_ORDER)
     assert torch.equal(ti, wi)
     assert torch.equal(tv.isnan(), wv.isnan())

@@ -43,7 +43,9 @@ def test_small_kernel_finds_its_experts(pkg, wl, dev, T, E, K):
         x = wl.make_device_input(shape, table, dev)
         print("small kernel", shape, flush=True)
         y, ti, _ = blk.forward(x)
-        assert blk.describe(blk.params(x, y, ti, y))["down"] == "expert_small_kernel<%d, 1>" % (fmt == "mxfp4")
+        tiny = T * K <= (16 if fmt == "mxfp4" else 12)
+        assert blk.describe(blk.params(x, y, ti, y))["gate_up"] == "expert_small_kernel<%d, 0>" % (fmt == "mxfp4")
+        assert blk.describe(blk.params(x, y, ti, y))["down"] == ("expert_tiny_down_kernel<%d>" if tiny else "expert_small_kernel<%d, 1>") % (fmt == "mxfp4")
         want, _, _ = blk.forward(x, flags=pkg.MOE_FLAG_FORCE_DIRECT)
         assert torch.equal(y, want)
 
