@@ -30,7 +30,7 @@ int launch_router_fused(const float* x, const uint16_t* w, const uint16_t* bias,
 // softmax as partial + finalize.  `scratch` holds router_screen_bytes(); `between`, if not NULL, is
 // recorded after the first pass.
 bool router_two_pass(int T, int E, int H);
-bool router_rows(int T, int E, int H);  // launch_router_two_pass is the faster one for smaller batches too: needs no scratch there
+bool router_rows(int T, int E, int H);  // router_rows_kernel is the fastest, for smaller batches than those too; it needs no scratch
 bool router_one_launch(int T, int E, int H);  // launch_router_two_pass is router_rows_kernel, not screen + refine
 size_t router_screen_bytes(int T, int E, int H);
 int launch_router_two_pass(const float* x, const uint16_t* w, const uint16_t* bias, void* scratch, uint16_t* x_bf16,

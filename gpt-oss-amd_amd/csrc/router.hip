@@ -1066,8 +1066,8 @@ int launch_router_partial(const float* x, const uint16_t* w, double* partial, ui
 // Worth it once the exact pass is throughput bound (16 cycles per term and wave), or once the fused kernel (a block
 // per token) would need a second round of blocks over the 256 compute units (the lines below are its rounds there, not asked
 // of the device).  With up to 32 experts a block holds a wave per two of them, several blocks share a compute unit, and
-// what counts is scores per batch.  Up to 128 experts and rows of 3072 router_rows says when router_rows_kernel runs, and this
-// line only how much scratch the batch is given; beyond, it chooses screen + refine.  Whole block of tiny experts, rows of
+// what counts is scores per batch.  Up to 128 experts and rows of 3072 router_rows says when router_rows_kernel runs instead of
+// these or the exact passes.  Whole block of tiny experts, rows of
 // 2880, before the top-k became shorter in all of them (4 us), us, fused : screen + refine: E = 64, 256 tokens 48 : 57, 640 84 :
 // 71; E = 128, 256 tokens 62 : 62, 257 82 : 63.
 bool router_two_pass(int T, int E, int H) {
@@ -1112,16 +1112,38 @@ size_t router_screen_bytes(int T, int E, int H) {
 
 static bool router_rows_fits(int E, int H) { return E <= 128 && H % 64 == 0 && H <= 64 * kRowsWaves * kRowsPairs; }
 
-// router_rows_kernel instead of the exact passes as well (it always carries out the two-pass method where it can).  Exact passes :
-// router_rows_kernel inside a block, us, rows of 2880, from HBM: E = 8, 600 tokens 10.6 : 13.2, 2000 tokens 24 : 22; E = 16, 300 tokens
-// 10.5 : 10.7, 4000 tokens 64 : 28; E = 32, 64 tokens 8.9 : 9.4, 256 tokens 10.6 : 11.3, 512 tokens (a second round of blocks) 18 : 13;
-// E = 48, 16 tokens 11.6 : 11.0, 64 tokens 12.5 : 11.4, 300 tokens 24 : 12.6; E = 128, 33 tokens 13.3 : 15.5, 64 tokens 14.3 : 15.2, 128
-// tokens 21 : 16.8, 200 tokens 28 : 16.9.
-bool router_rows(int T, int E, int H) {
-    return router_rows_fits(E, H) && (E > 48 ? T > 64 : E > 32 ? T > 16 : E > 16 ? T > 256 : (long long)T * E > 12000);
+// As few tokens to a block as one round of blocks over 256 compute units allows; more than 64 experts leave LDS for eight.
+static int router_rows_tokens(int T, int E) {
+    return T <= 256 ? 1 : T <= 512 ? 2 : T <= 1024 ? 4 : T <= 2048 || E > 64 ? 8 : 16;
 }
 
-bool router_one_launch(int, int E, int H) { return router_rows_fits(E, H); }
+// Whether router_rows_kernel runs, instead of the exact passes or, where router_two_pass holds, instead of screen + refine.
+// Blocks of tiny experts, rows as said, us.
+//   Exact passes : this, rows of 2880: E = 16, 1000 tokens 69 : 61; E = 32, 257 tokens 48 : 42 (64 tokens 8.9 : 9.4 for the router
+// alone); E = 48, 17 tokens 31.4 : 30.2; E = 64, 65 tokens 34.4 : 31.9; E = 128, 65 tokens 49 : 43, but 33 tokens 13.3 : 15.5 alone, and
+// with rows of 320 65 tokens 25.1 : 25.9, 128 25.1 : 26.0.  Up to eight experts a block of sixteen tokens does little more than load
+// them, so its rounds have to be full: E = 8, 3300 tokens 107 : 105, 4200 (half of two rounds) 121 : 131, 7400 177 : 168, rows of 320, 4200
+// 61 : 59; E = 6, 4000 tokens 112 : 112, 4500 120 : 133; E = 4 loses everywhere (5000 tokens 121 : 138, rows of 320 56 : 61).
+//   Screen + refine : this: E = 16, 4097 tokens 125 : 129, 8192 189 : 181, rows of 320 8194 tokens 72 : 77; E = 64, 4096 tokens 214 : 204 and
+// 65535, rows of 64, 381 : 419; E = 128, 2048 tokens 137 : 123, 2049 (a second round) rows of 1024 73 : 77, of 2048 106 : 109, of 2880 137 : 137;
+// 4096 tokens, rows of 640 93 : 97, of 1024 101 : 97, of 2880 242 : 214; 30000 tokens, rows of 1024 591 : 636, of 1536 830 : 837.
+bool router_rows(int T, int E, int H) {
+    if (!router_rows_fits(E, H)) return false;
+    const int blocks = ceil_div(T, router_rows_tokens(T, E));
+    const int full = 100 * blocks / (ceil_div(blocks, 256) * 256);  // percent of the places in its rounds
+    if (router_two_pass(T, E, H))
+        return E > 64   ? T <= 2048 || H >= 2560 || (H >= 1024 && T > 3072 && T <= 16384)
+               : E > 16 ? T <= 16384 || H >= 640
+                        : H >= 1024 && full >= 70;
+    return E > 64   ? T > (H < 1024 ? 128 : 64)
+           : E > 48 ? T > 64
+           : E > 32 ? T > 16
+           : E > 16 ? T > 256
+                    : (long long)T * E > 12000 && (E > 8 || (E > 4 && full >= (H >= 2048 ? 80 : E > 6 ? 0 : 60)));
+}
+
+// moe_router_two_pass_report takes it for all batches that moe_block_forward would not screen in a launch of its own.
+bool router_one_launch(int T, int E, int H) { return router_rows(T, E, H) || (router_rows_fits(E, H) && !router_two_pass(T, E, H)); }
 
 static int launch_router_rows(const float* x, const uint16_t* w, const uint16_t* bias, uint16_t* x_bf16, float* topk_v,
                               int* topk_i, int T, int H, int E, int K, int do_softmax, hipStream_t stream, float* approx_out,
@@ -1129,8 +1151,7 @@ static int launch_router_rows(const float* x, const uint16_t* w, const uint16_t*
     const int per_wave = 2 * ceil_div(H / 64, kRowsWaves);
     // per wave and segment as in launch_router_two_pass, and 16 additions of the waves' sums
     const float err_coeff = ((float)(33 + 2 * per_wave + 16) * 0x1p-23f + 0x1p-16f + 8 * 0x1p-24f) * 1.01f;
-    // as few tokens to a block as one round of blocks over 256 compute units allows; more than 64 experts leave LDS for eight
-    const int tpb = T <= 256 ? 1 : T <= 512 ? 2 : T <= 1024 ? 4 : T <= 2048 || E > 64 ? 8 : 16;
+    const int tpb = router_rows_tokens(T, E);
 #define MOE_ROWS(NE_, TPB_)                                                                                             \
     if (tpb == TPB_) {                                                                                                  \
         hipLaunchKernelGGL((router_rows_kernel<NE_, TPB_>), dim3(ceil_div(T, TPB_)), dim3(64 * kRowsWaves), 0, stream, x, w, \

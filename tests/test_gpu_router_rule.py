@@ -9,25 +9,30 @@ FUSED, SPLIT, TWO = "router_fused_kernel", "router_partial_kernel + router_final
 ROWS, SCORES, TOPK_LATER = "router_rows_kernel", "router_scores_kernel + router_finalize_kernel", "router_scores_kernel"
 # experts -> tokens and the router of rows that the one-launch kernels take, on both sides of each line
 LINES = {
-    8: [(2, TOPK_LATER), (3, FUSED), (1500, FUSED), (1501, ROWS), (2048, ROWS), (8191, ROWS), (8192, ROWS)],
-    16: [(750, FUSED), (751, ROWS), (2048, ROWS), (4096, ROWS)],
+    4: [(1, TOPK_LATER), (8000, FUSED), (16383, FUSED), (16384, ROWS)],
+    6: [(2000, FUSED), (3300, ROWS), (4096, ROWS), (4200, FUSED)],
+    8: [(2, TOPK_LATER), (3, FUSED), (1500, FUSED), (2048, ROWS), (4096, ROWS), (8191, ROWS), (8192, ROWS)],
+    16: [(750, FUSED), (751, ROWS), (2048, ROWS), (4095, ROWS), (4096, ROWS), (4097, TWO)],
     17: [(256, FUSED), (257, ROWS), (1204, ROWS), (1205, ROWS)],
-    32: [(1, TOPK_LATER), (8, TOPK_LATER), (9, FUSED), (256, FUSED), (257, ROWS), (640, ROWS), (2047, ROWS), (2048, ROWS)],
+    32: [(8, TOPK_LATER), (9, FUSED), (256, FUSED), (257, ROWS), (640, ROWS), (2047, ROWS), (2048, ROWS)],
     33: [(1, TOPK_LATER), (16, SCORES), (17, ROWS), (128, ROWS), (513, ROWS)],
     48: [(16, SCORES), (17, ROWS), (513, ROWS)],
     49: [(40, SCORES), (41, SPLIT), (64, SPLIT), (65, ROWS), (257, ROWS)],
-    128: [(8, TOPK_LATER), (9, SCORES), (64, SPLIT), (65, ROWS), (257, ROWS), (2049, ROWS)],
+    128: [(8, TOPK_LATER), (9, SCORES), (64, SPLIT), (65, ROWS), (128, ROWS), (129, ROWS), (2048, ROWS), (2049, ROWS)],
     250: [(5, TOPK_LATER), (9, SCORES), (40, SCORES), (41, SPLIT), (128, SPLIT), (129, FUSED), (256, FUSED), (257, TWO), (263, TWO)],
     257: [(128, SPLIT), (129, FUSED), (255, FUSED), (256, TWO)],
     1000: [(1, TOPK_LATER), (40, SCORES), (41, SPLIT), (65, SPLIT), (66, TWO), (128, TWO), (129, TWO)],
 }
 
 
-def long_rows(T, E, router):
-    """The router of rows past 3072 values."""
-    if router == ROWS:
-        router = TWO if T * E >= (20480 if 16 < E <= 32 else 65536) or T > (256 if E > 48 else 512) and E > 32 else FUSED
-    return (SCORES if T <= 40 else SPLIT) if router == FUSED else router
+def other_rows(H, T, E, router):
+    """The router of rows of 64, which the one-launch kernel leaves to the others more often, and of rows past its 3072 values."""
+    if H == 2880 or router != ROWS:
+        return (SCORES if T <= 40 else SPLIT) if router == FUSED and H > 3072 else router
+    two = T * E >= (20480 if 16 < E <= 32 else 65536) or T > (256 if E > 48 else 512) and E > 32
+    if H == 64:
+        return TWO if two and (E <= 16 or E > 64 and T > 2048) else SPLIT if E > 64 and T <= 128 else ROWS
+    return TWO if two else SCORES if T <= 40 else SPLIT
 
 
 @pytest.mark.parametrize("H", [64, 2880, 3136])  # the last is too long for the one-launch kernel
@@ -42,7 +47,7 @@ def test_router_kernels_agree(pkg, wl, dev, H, E):
         print("router", H, E, T, flush=True)
         t = x[:T].contiguous()
         _, ti, tv = blk.forward(t)
-        assert blk.describe(blk.params(t, x, ti, tv))["router"] == (long_rows(T, E, router) if H > 3072 else router)
+        assert blk.describe(blk.params(t, x, ti, tv))["router"] == other_rows(H, T, E, router)
         _, wi, wv = blk.forward(t, flags=pkg.MOE_FLAG_ROUTER_STRICT_ORDER)
         assert torch.equal(ti, wi)
         # logits differ, if at all, in the last place of their rounding to fp32: 2^-23 of |logit| < 16
