@@ -117,7 +117,7 @@ struct BlockRoute {
         } else if (router_fused_fits(H) && !router_split(T, E)) {
             router = Router::kFused;  // block per token: the exact pass of the two-pass router applied to every expert
         } else {
-            router = router_scores(T) ? Router::kScoresFinalize : Router::kPartialFinalize;
+            router = router_scores(T, E) ? Router::kScoresFinalize : Router::kPartialFinalize;
         }
         combined = router == Router::kScores && !p->next_norm_out && expert_small_combines(T * K, I, fmt);
     }

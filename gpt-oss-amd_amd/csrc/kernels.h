@@ -16,8 +16,9 @@ int launch_router_finalize(const double* partial, int S, const float* scores_in,
                            float* scores_out, float* topk_v, int* topk_i, int T, int E, int K, int do_topk,
                            int do_softmax, hipStream_t stream);
 int launch_softmax_rows(float* x, int B, int size, hipStream_t stream);
-// Scores only ([T, E]) and the bf16 activation copy; top-k and softmax are the gate/up kernel's then (ExpertGemmArgs::scores).
-bool router_scores(int T);  // scores and finalize rather than partial and finalize
+bool router_scores(int T, int E);  // scores and finalize rather than partial and finalize
+// Scores only ([T, E]) and the bf16 activation copy; top-k and softmax are the finalize kernel's, or for a handful of tokens the
+// gate/up kernel's (ExpertGemmArgs::scores).
 int launch_router_scores(const float* x, const uint16_t* w, const uint16_t* bias, uint16_t* x_bf16, float* scores, int T, int H,
                          int E, hipStream_t stream);
 // Whole router in one launch (block per token): logits as the exact pass of the two-pass router,

@@ -1085,9 +1085,11 @@ bool router_two_pass(int T, int E, int H) {
 bool router_split(int T, int E) { return E > 32 && T <= (E > 48 ? 128 : 16); }
 
 // Of those, a wave per (token, expert) for the scores rather than segments and their sums: a router row comes through the compute unit
-// once per token.  Partial + finalize : scores + finalize, us: E = 128, 9 tokens 12.2 : 9.7, 33 tokens 13.1 : 11.9, 48 tokens 13.7 : 13.8, 64 tokens
-// 14.2 : 17.6; E = 250, 20 tokens 22 : 15, 64 tokens 25 : 25; E = 1000, 9 tokens 52 : 31, 30 tokens 54 : 49.
-bool router_scores(int T) { return T <= 40; }
+// once per token.  Block of tiny experts, partial + finalize : scores + finalize, us: E = 49, rows of 64, 40 tokens 22.8 : 20.9; E = 128, rows
+// of 2880, 9 tokens 31.4 : 28.3, 40 tokens 44.8 : 42.3 (48 and 64 tokens of the router alone 13.7 : 13.8 and 14.2 : 17.6); E = 512, rows of 320, 9
+// tokens 25.8 : 23.0, 40 tokens 28.0 : 27.1; E = 1000, rows of 2880, 9 tokens 61 : 40, 32 tokens 78 : 75, 40 tokens 85 : 87, rows of 64, 32
+// tokens 27.8 : 27.9, 40 tokens 28.2 : 29.5.
+bool router_scores(int T, int E) { return T <= 40 && T * E <= 32000; }
 
 static int screen_tiles(int E) { return E <= 16 ? 1 : E <= 32 ? 2 : 4; }  // 16-expert tiles per wave
 

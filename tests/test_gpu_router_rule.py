@@ -21,7 +21,8 @@ LINES = {
     128: [(8, TOPK_LATER), (9, SCORES), (64, SPLIT), (65, ROWS), (128, ROWS), (129, ROWS), (2048, ROWS), (2049, ROWS)],
     250: [(5, TOPK_LATER), (9, SCORES), (40, SCORES), (41, SPLIT), (128, SPLIT), (129, FUSED), (256, FUSED), (257, TWO), (263, TWO)],
     257: [(128, SPLIT), (129, FUSED), (255, FUSED), (256, TWO)],
-    1000: [(1, TOPK_LATER), (40, SCORES), (41, SPLIT), (65, SPLIT), (66, TWO), (128, TWO), (129, TWO)],
+    800: [(40, SCORES), (41, SPLIT)],
+    1000: [(1, TOPK_LATER), (32, SCORES), (33, SPLIT), (65, SPLIT), (66, TWO), (128, TWO), (129, TWO)],
 }
 
 
@@ -56,7 +57,7 @@ def test_router_kernels_agree(pkg, wl, dev, H, E):
 
 @pytest.mark.parametrize("T", [700, 2100])
 @pytest.mark.parametrize("H,E,router", [(320, 32, ROWS), (320, 160, TWO), (3136, 32, TWO)])
-@pytest.mark.parametrize("what", ["inf weight", "nan weight", "nan weight, ties", "nan bias", "inf bias", "inf row", "nan row", "huge row"])
+@pytest.mark.parametrize("what", ["inf weight", "nan weight", "neg nan weight", "nan weight, ties", "nan bias", "inf bias", "inf row", "nan row", "huge row"])
 def test_screening_keeps_non_finite_scores(pkg, wl, dev, T, H, E, router, what):
     """Scores that are infinite or not a number rank as in the single exact pass: the screening pass drops an expert for a
     finite approximate score below the bound only."""
@@ -69,8 +70,11 @@ def test_screening_keeps_non_finite_scores(pkg, wl, dev, T, H, E, router, what):
     if "ties" in what:  # every other expert inside the bound of the K-th best
         w.copy_(w[:1].expand(E, H).clone())
         b.fill_(0.5)
+    if what == "neg nan weight":  # ranks last
+        w.view(torch.int16)[5, 7] = -64
+        w.view(torch.int16)[E - 1, 9] = -64
     v = float(what[:3]) if what[:3] in ("inf", "nan") else 3.39e38  # the last rounds to an infinity in bf16
-    {"weight": w[5], "weight, ties": w[5], "bias": b, "row": x[::3]}[what.split(" ", 1)[1]][..., 7] = v
+    {"nan weight": w[6:6], "weight": w[5], "weight, ties": w[5], "bias": b, "row": x[::3]}[what.split(" ", 1)[1]][..., 7] = v
     print("non-finite router", T, H, E, what, flush=True)
     _, ti, tv = blk.forward(x)
     assert blk.describe(blk.params(x, x, ti, tv))["router"] == router
