@@ -455,6 +455,23 @@ def test_block_extreme_routing_skew(pkg, wl, oracle, dev, T, zipf_s, fmt):
         (T, fmt, counts.max(), (counts == 0).sum(), err))
 
 
+@pytest.mark.parametrize("size", [4, 64, 252, 256, 260, 512, 768, 1020, 1024, 1028, 3072, 3076, 4096])
+def test_rmsnorm_register_forms(pkg, oracle, dev, size):
+    """Row lengths on both sides of a wave, of each number of values held per thread and of the form that reads a row twice; in place."""
+    rng = np.random.default_rng(size)
+    x = rng.standard_normal((7, size)).astype(np.float32)
+    x[3] *= 1e-6
+    x[4, :] = 0.0
+    x[5, 0] = 4e4
+    w = oracle.f32_to_bf16(rng.standard_normal(size))
+    xd, wd = torch.from_numpy(x).to(dev), torch.from_numpy(w).view(torch.int16).view(torch.bfloat16).to(dev)
+    print("rmsnorm", size, flush=True)
+    pkg.rmsnorm(xd, xd, wd, 7, size)
+    # fp64 sums of fp32 squares in another order: the scale rounds to fp32 the other way at most, and the value after it: 2^-23 each
+    ref = np.stack([oracle.rmsnorm(r, oracle.bf16_to_f32(w)) for r in x])
+    np.testing.assert_allclose(xd.cpu().numpy(), ref, rtol=2.4e-7)
+
+
 def test_block_residual_and_rmsnorm_glue(pkg, wl, oracle, dev):
     shape = wl.MoeShape("glue", T=40, H=256, I=128, E=8, K=4, fmt="bf16", seed=3)
     table = oracle.normal_table()
