@@ -608,6 +608,15 @@ __global__ __launch_bounds__(NE == 2 ? 1024 : 512) void router_fused_kernel(cons
     write_topk(my_v, my_i, K, lane, do_softmax, topk_v + (size_t)t * K, topk_i + (size_t)t * K);
 }
 
+// Bound of a token's approximate scores, from the squared norms of its row and of the longest router row.  Squares of small values are
+// lost from the sums, up to 2^-126 each: a sum is taken to be at least 2^-95, which covers those and the bits that the lower pieces of
+// such values lack.  Not a number stays one.
+MOE_DEVICE float screen_bound(float err_coeff, float x2, float x2_margin, float w2, float amax) {
+    if (x2 < 0x1p-95f) x2 = 0x1p-95f;
+    if (w2 < 0x1p-95f) w2 = 0x1p-95f;
+    return err_coeff * (sqrtf(x2) * x2_margin) * (sqrtf(w2) * 1.001f) + amax * 0x1p-20f;
+}
+
 // ---------------------------------------------------------------------------------------------
 // Second pass of the two-pass router: one wave per token.
 //   1. approximate scores a[e] = float(sum_s partial[s][t][e]) + bias[e] from the screening pass,
@@ -699,7 +708,7 @@ __global__ __launch_bounds__(256, 4) void router_refine_kernel(const float* __re
     amax = wave_max_nonneg(amax);
     // upper bound of |approx - exact| for every expert of this token; the 1.001 factors cover the
     // rounding of the two norms themselves, the last term the final roundings of both scores
-    const float delta = err_coeff * (sqrtf(x2) * 1.001f) * (sqrtf(w2max) * 1.001f) + amax * 0x1p-20f;
+    const float delta = screen_bound(err_coeff, x2, 1.001f, w2max, amax);
     __builtin_amdgcn_wave_barrier();
 
     float my_v;
@@ -933,7 +942,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void router_rows_kernel(const floa
         amax = wave_max_nonneg(amax);
         wmax = wave_max_nonneg(wmax);
         // the activations' norm is that of their upper pieces, each within 2^-8 of its activation
-        const float delta = err_coeff * (sqrtf(x2[tl * DUP]) * 1.006f) * (sqrtf(wmax) * 1.001f) + amax * 0x1p-20f;
+        const float delta = screen_bound(err_coeff, x2[tl * DUP], 1.006f, wmax, amax);
         float my_v;
         int my_i;
         select_topk_of<(EP + 63) / 64>(my, E, K, lane, my_v, my_i);

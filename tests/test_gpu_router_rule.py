@@ -84,6 +84,28 @@ def test_screening_keeps_non_finite_scores(pkg, wl, dev, T, H, E, router, what):
     assert (tv.nan_to_num(0.0) - wv.nan_to_num(0.0)).abs().max().item() <= 4e-6
 
 
+@pytest.mark.parametrize("T,H,E,router", [(300, 2880, 32, ROWS), (300, 320, 128, ROWS), (1000, 2880, 200, TWO), (700, 3136, 32, TWO)])
+@pytest.mark.parametrize("x_scale,w_scale", [(1e-38, 1.0), (1e-30, 1.0), (1e-20, 1.0), (1.0, 1e-25), (1e-12, 1e-12), (1e30, 1.0)])
+def test_screening_at_the_ends_of_the_float_range(pkg, wl, dev, T, H, E, router, x_scale, w_scale):
+    """Norms whose squares are no longer floats: near ties of such rows are decided by exact scores, rows of zeros by the biases."""
+    shape = wl.MoeShape("router", T=T, H=H, I=64, E=E, K=4, fmt="mxfp4", seed=5)
+    blk, _ = wl.make_device_layer(shape, pkg.normal_table(), dev)
+    x = wl.make_device_input(shape, pkg.normal_table(), dev) * x_scale
+    w, b = blk.tensors["w_router"], blk.tensors["b_router"]
+    b.zero_()
+    for e in range(1, E // 2):  # bf16 steps apart
+        w[e] = w[0]
+        w[e, (7 * e) % H] *= 1.01
+    w *= w_scale
+    x[5:9] = 0.0
+    b[E - 3:] = 1e-30
+    print("router, float range", T, H, E, x_scale, w_scale, flush=True)
+    _, ti, tv = blk.forward(x)
+    assert blk.describe(blk.params(x, x, ti, tv))["router"] == router
+    _, wi, wv = blk.forward(x, flags=pkg.MOE_FLAG_ROUTER_STRICT_ORDER)
+    assert torch.equal(ti, wi) and (tv - wv).nan_to_num(0.0).abs().max().item() <= 4e-6
+
+
 @pytest.mark.parametrize("E", [1, 63, 64, 65, 128, 129, 192, 256, 257, 512, 513, 1000, 1024])
 def test_topk_register_forms(pkg, dev, E):
     """Every number of keys per lane, at its edges: ties to the lower index, infinities and signed zeros in the order of the values,
