@@ -48,7 +48,7 @@ inline bool use_prefill_kernels(int T, int H, int I, int K, int E, int format, u
 
 // Bucketing inside the expert kernels instead of a launch of its own: for the weight-streaming
 // kernels, while the assignment list is short enough for one block to scan and buckets mostly fit one
-// 64-token block (a block runs its bucket's token blocks one after the other).
+// 64-token block (a bf16 block runs its bucket's token blocks one after the other, an MXFP4 block the first two of them).
 inline bool use_direct_bucketing(int T, int K, int E, bool prefill, unsigned flags) {
     if (prefill || (flags & MOE_FLAG_FORCE_BUCKET_LAUNCH)) return false;
     const long long A = (long long)T * K;

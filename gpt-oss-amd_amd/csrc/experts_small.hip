@@ -386,7 +386,7 @@ __global__ __launch_bounds__(64 * kSmallWaves, 4) void expert_small_queue_kernel
     small_rows<FMT, EPI, true>(a, lds, entry[0], [&](int i) { return off + i; }, entry[2], rb, max_rows, lds_bytes);
 }
 
-// ---- down GEMM of a token or two: a wave per (assignment, tile of 16 weight rows); the waves of a block share the tile ------------
+// ---- down GEMM of up to 16 assignments: a wave per (assignment, tile of 16 weight rows); the waves of a block share the tile --------
 // What bounds it: round trips (ids and rows, then weights, then the stores).  The block that holds all of a token's rows of its
 // tile also combines them, which takes the combine's launch away; a wave needs nobody else's row until then.  MXFP4, us, down
 // + combine, two launches : one: 1 token 7.7 + 3.8 : 8.3, 2 tokens 9.9 + 3.9 : 10.4.  The gate/up GEMM in this form was no faster (1

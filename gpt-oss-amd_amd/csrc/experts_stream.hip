@@ -131,7 +131,7 @@ MOE_DEVICE void ws_producer(const ExpertGemmArgs& a, uint8_t* lds, RowFn act_row
 // The lane id; for the work-queue entries (epilogue EPI) as a value that the compiler takes to be new at every call: what
 // follows from it is then worked out per token block, not ahead of the loop over an entry list's whole blocks, where it would
 // wait in scratch memory and be fetched in the stage loops (a spill access there waits for every weight load in flight).
-template <int EPI, bool PRE = true>
+template <int EPI>
 MOE_DEVICE int ws_lane() {
     int lane = threadIdx.x & 63;
     if constexpr (EPI == EPI_SWIGLU_F32 || EPI == EPI_SCATTER) asm volatile("" : "+v"(lane));
@@ -207,7 +207,7 @@ template <int FMT, int NT, int EPI, bool PRE = false, int R = 2, class SlotFn>
 MOE_DEVICE void ws_consumer(const ExpertGemmArgs& a, const uint8_t* lds, int e, SlotFn slot_of_row, int nrows, int tile0,
                             bool active) {
     static_assert(R == 1 || R == 2, "one or two row tiles per wave");
-    const int lane = ws_lane<EPI, PRE>();
+    const int lane = ws_lane<EPI>();
     const int g = lane >> 4;
     const int q = lane & 15;
     const int K = a.K;
@@ -437,7 +437,7 @@ MOE_DEVICE void ws_consumer_two(const ExpertGemmArgs& a, const uint8_t* lds, int
                             int unit_end, int unit_step, int passes) {
     constexpr int R = 2;
     constexpr bool TWO = true;
-    const int lane = ws_lane<EPI, PRE>();
+    const int lane = ws_lane<EPI>();
     const int g = lane >> 4;
     const int q = lane & 15;
     const int K = a.K;
@@ -813,7 +813,9 @@ MOE_DEVICE int direct_list_bucket(const ExpertGemmArgs& a, int wave, const int (
 // hottest expert set the launch's time.  Whole block, us, so : dealt out, E = 32, router of no preference, 256 tokens 109 : 109, 384
 // tokens 147 : 146; Zipf 1.0, 256 tokens 187 : 182, 384 tokens 267 : 198; Zipf 1.5 245 : 174 and 375 : 189; E = 128, Zipf 1.0, 512 tokens
 // 548 : 446, 1024 tokens 859 : 540.
-// bf16 blocks keep to that: the second way into the stage loops costs the first its registers (256 tokens 280 : 287).
+// bf16 blocks keep to that: the second way into the stage loops costs the first its registers (256 tokens 280 : 287).  It costs the
+// MXFP4 loops over whole blocks a few more spill accesses as well (gate/up 36 : 57 in the kernel, most of them around the stage loops),
+// which no launch shows: 8 to 1000 tokens of 8 to 128 experts, blocks of 1024 to 4096, router of no preference, as fast or faster.
 template <int FMT, int EPI, int CONS, int PROD, bool TWO>
 __global__ __launch_bounds__((CONS + PROD) * 64, (CONS + PROD > 12) ? 4 : 3) void expert_stream_direct_kernel(ExpertGemmArgs a) {
     constexpr int WAVES = CONS + PROD;
