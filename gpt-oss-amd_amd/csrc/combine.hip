@@ -270,10 +270,10 @@ __global__ __launch_bounds__(256) void combine_norm_kernel(const float4* __restr
     }
 }
 
-// Returns MOE_ERR_LIMIT when the row is too long for the fused kernel (the caller then runs the two
-// kernels one after the other).
 bool combine_norm_fits(int H) { return H <= 4 * 1024; }
 
+// Returns MOE_ERR_LIMIT when the row is too long for the fused kernel (the caller then runs the two
+// kernels one after the other).
 int launch_combine_norm(const float* y_by_slot, const int* slot_of, const int* topk_i, const float* topk_v,
                         float* e_agg, float* residual_x, const uint16_t* norm_weight, float* norm_out, int T, int K,
                         int H, hipStream_t stream) {

@@ -1140,8 +1140,8 @@ static int router_rows_tokens(int T, int E) {
 // 4096 tokens, rows of 640 93 : 97, of 1024 101 : 97, of 2880 242 : 214; 30000 tokens, rows of 1024 591 : 636, of 1536 830 : 837.
 bool router_rows(int T, int E, int H) {
     if (!router_rows_fits(E, H)) return false;
-    const int blocks = ceil_div(T, router_rows_tokens(T, E));
-    const int full = 100 * blocks / (ceil_div(blocks, 256) * 256);  // percent of the places in its rounds
+    const long long blocks = ceil_div(T, router_rows_tokens(T, E));
+    const int full = (int)(100 * blocks / (ceil_div(blocks, 256LL) * 256));  // percent of the places in its rounds
     if (router_two_pass(T, E, H))
         return E > 64   ? T <= 2048 || H >= 2560 || (H >= 1024 && T > 3072 && T <= 16384)
                : E > 16 ? T <= 16384 || H >= 640
