@@ -20,6 +20,14 @@ static int hist_copies(int E) { return E <= 256 ? kHistCopies : E <= 512 ? 16 : 
 // round trip per 8192 ids and per 4096 tokens).  32 experts, us, general : V4: 1000 tokens 9.2 : 8.6, 4096 tokens 12.6 : 9.8, 16384 tokens 35 : 20.
 constexpr int kHeldTokens = 16 * 1024;
 
+// Rows of an expert's token blocks: the map's tile_tokens, or with `even` as many blocks as that gives, cut evenly into whole
+// MFMA tiles.  A remainder of a few rows streams the expert's weights once more for next to no matrix work, and takes more than half
+// of a whole block's time for it.  Whole block, us, whole blocks and a remainder : even ones, 32 experts: bf16, 4096 tokens (half the
+// buckets a few rows past 512) 891 : 867; MXFP4, skewed, 1000 tokens 240 : 235, 4096 tokens 729 : 728.
+MOE_DEVICE int tile_rows_of(const TileMap& map, int count) {
+    return map.even ? even_tile_rows(count, map.tile_tokens) : map.tile_tokens;
+}
+
 // grid = E blocks (one expert each), block = 1024 threads, dynamic LDS = (E * copies + E + 32) ints.
 // Tile map order: every full tile first (ascending expert), then the experts' partial last tiles from
 // the largest to the smallest (equal sizes: ascending expert).  An expert kernel that takes tiles in
@@ -89,8 +97,8 @@ __global__ __launch_bounds__(1024) void bucket_kernel(const int* __restrict__ to
         hist[i] = c;
     }
     __syncthreads();
-    const int nb = map.tile_tokens;
     const int my_cnt = hist[e];
+    const int nb = tile_rows_of(map, my_cnt);
     {
         const int my_rem = nb > 0 ? my_cnt % nb : 0;
         int rows_before = 0, full_before = 0, full_all = 0, part_ahead = 0, part_all = 0, part_before = 0;
@@ -98,7 +106,7 @@ __global__ __launch_bounds__(1024) void bucket_kernel(const int* __restrict__ to
             const int c = hist[i];
             if (i < e) rows_before += c;
             if (nb > 0) {
-                const int full = c / nb, rem = c - full * nb;
+                const int nb_i = tile_rows_of(map, c), full = c / nb_i, rem = c - full * nb_i;
                 full_all += full;
                 if (i < e) full_before += full;
                 if (rem > 0) {

@@ -19,3 +19,20 @@ def test_prefill_blocks_cover_every_row(pkg, wl, dev, H, I, T, E, K, zipf_s):
     y, ti, _ = blk.forward(x, flags=pkg.MOE_FLAG_FORCE_TILED)
     want, _, _ = blk.forward(x, flags=pkg.MOE_FLAG_FORCE_STREAM)
     assert torch.equal(y, want)
+
+
+# buckets of one row more and less than whole token blocks, of 16, 17 and 18 of them
+@pytest.mark.parametrize("fmt,block", [("mxfp4", 128), ("bf16", 256)])
+@pytest.mark.parametrize("blocks", [2, 17])
+def test_evenly_cut_buckets(pkg, wl, dev, fmt, block, blocks):
+    table = pkg.normal_table()
+    T = blocks * block + 1
+    shape = wl.MoeShape("prefill", T=T, H=64, I=128, E=2, K=2, fmt=fmt, seed=T)  # every token uses both experts
+    blk, _ = wl.make_device_layer(shape, table, dev)
+    x = wl.make_device_input(shape, table, dev)
+    for n in (T, T - 1, T - 2, T - block + 15):
+        print("evenly cut", fmt, n, flush=True)
+        t = x[:n].contiguous()
+        y, ti, _ = blk.forward(t, flags=pkg.MOE_FLAG_FORCE_TILED)
+        want, _, _ = blk.forward(t, flags=pkg.MOE_FLAG_FORCE_STREAM)
+        assert torch.equal(y, want), n
