@@ -1017,19 +1017,20 @@ MOE_DEVICE void prefill_body_mxfp4(const ExpertGemmArgs& a, uint8_t* lds, int e,
     const int half_w = wave >> 2;
     const int q_dma = 4 * blk_w + (lane >> 4);     // row of the token tile this lane moves
     const int chunk_dma = ws_chunk_at<FMT_MXFP4>((lane & 15) ^ q_dma);  // chunk of the stage it fetches
-    const uint8_t* b_row[TS];
+    uint32_t b_row[TS];  // byte offsets: 32 bits, nine registers fewer than pointers (launcher: expert_rows_fit)
 #pragma unroll
     for (int i = 0; i < TS; ++i) {
         const int idx = min((half_w + kStagers * i) * 16 + q_dma, nrows - 1);
-        const int src = a.gather ? a.tokens_flat[row0 + idx] : row0 + idx;
-        b_row[i] = reinterpret_cast<const uint8_t*>(a.act + (size_t)src * K);
+        const int src = a.gather ? a.tokens_flat[row0 + idx] : idx;  // rows by slot: counted from the block's first
+        b_row[i] = (uint32_t)src * (uint32_t)K * 2u;
     }
+    const uint8_t* const b_base = reinterpret_cast<const uint8_t*>(a.act + (a.gather ? 0 : (size_t)row0 * K));
     auto issue_b = [&](int s) {
         const int k = s * kStageElems + 8 * chunk_dma;
-        const size_t off = (k < K) ? (size_t)k * 2 : 0;  // past the row: re-read its start (weights are 0 there)
+        const uint32_t off = (k < K) ? (uint32_t)k * 2u : 0u;  // past the row: re-read its start (weights are 0 there)
         uint8_t* dst = lds + (size_t)(s & 1) * kStageBytes + (size_t)half_w * 4096 + blk_w * 1024;
 #pragma unroll
-        for (int i = 0; i < TS; ++i) dma16(b_row[i] + off, dst + i * kStagers * 4096);
+        for (int i = 0; i < TS; ++i) dma16(b_base + (size_t)(b_row[i] + off), dst + i * kStagers * 4096);
     };
     const uint8_t* const lds_rd = lds + (size_t)q * 256;
     auto b_frag = [&](int s, int j, int t) {  // lane group g owns MX block g of a stage: chunk 4g + j
@@ -1115,7 +1116,13 @@ MOE_DEVICE void prefill_body_mxfp4(const ExpertGemmArgs& a, uint8_t* lds, int e,
                 else if (j + 1 < 4) bq[slot_b] = b_frag(s, j + 1, t + 2 - NT);
                 __builtin_amdgcn_sched_barrier(0);  // keep the read above ahead of the MFMAs below
 #pragma unroll
-                for (int r = 0; r < R; ++r) acc[r][t] = mfma_16x16x32(av[r], b, acc[r][t]);
+                for (int i = 0; i < R; ++i) {
+                    // there and back over the row tiles: every product has an operand of the one before it.  The launch's clock
+                    // hangs on the power that changing operands take: 16384 tokens, 32 experts, whole block 2707 : 2688 us, and with 32-bit
+                    // row offsets 2736 : 2709 on another box; 1000 tokens 248 : 246.
+                    const int r = (t & 1) ? R - 1 - i : i;
+                    acc[r][t] = mfma_16x16x32(av[r], b, acc[r][t]);
+                }
             }
         }
         wait_vmcnt<0>();  // next stage's activations (direct-to-LDS) and weights have landed

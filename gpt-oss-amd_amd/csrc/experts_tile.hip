@@ -7,7 +7,6 @@
 // 1077 us).  Here a stage brings 64 KiB for the same work, and an XCD's blocks share it: 1.4 to 2.1 GB, 484 to 525 us,
 // i.e. 1.1 PFLOP/s (down launch 564 -> 304 us).  Gate/up launch at that size with the other parts taken out: matrix
 // instructions and epilogues 366 us, fragment reads from LDS 284, loads into LDS 247 from L2 and 435 from where the data are.
-#include <algorithm>
 #include <type_traits>
 
 #include "expert_tiles.h"
@@ -183,7 +182,10 @@ MOE_DEVICE void tile_body(const ExpertGemmArgs& a, uint8_t* lds, int e, int row0
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int r = 0; r < R; ++r) acc[r][t] = mfma_16x16x32(aw[j][r], bt[j][t], acc[r][t]);
+            for (int i = 0; i < R; ++i) {
+                const int r = (t & 1) ? R - 1 - i : i;  // there and back: each product has an operand of the one before it (less power)
+                acc[r][t] = mfma_16x16x32(aw[j][r], bt[j][t], acc[r][t]);
+            }
         }
     };
     int ts = 0, ws = 0;
@@ -244,10 +246,9 @@ __global__ __launch_bounds__(512, 2) void expert_tile_bf16_kernel(ExpertGemmArgs
 
 }  // namespace
 
-// The kernel addresses an expert's matrix and gathered activation rows by 32-bit byte offsets (rows by slot: the 256 of a
-// block).
+// The kernel addresses an expert's matrix by 32-bit byte offsets too.
 bool expert_tile_fits(long long gathered_rows, int rows, int K) {
-    return std::max(gathered_rows, 256ll) * K * 2 <= 0xffffffffll && (long long)rows * K * 2 <= 0xffffffffll;
+    return expert_rows_fit(gathered_rows, K) && (long long)rows * K * 2 <= 0xffffffffll;
 }
 
 int launch_expert_tile_bf16(const ExpertGemmArgs& a, int epi, hipStream_t stream) {

@@ -118,6 +118,15 @@ def test_describe_names_the_kernels_that_run(pkg):
         assert "; combine=in the down kernel; " in text.value.decode()
 
 
+@pytest.mark.parametrize("T,H,I,K,name", [(65535, 32704, 64, 8, "expert_prefill"), (65535, 32832, 64, 8, "expert_stream_ws"),
+                                          (65535, 64, 8192, 8, "expert_prefill"), (65535, 2880, 2880, 4, "expert_prefill")])
+def test_mxfp4_prefill_kernel_takes_inputs_of_4_gib(pkg, T, H, I, K, name):
+    """Gathered rows past 4 GiB go to the streaming kernels; rows by slot do not matter."""
+    for flags in (0, pkg.MOE_FLAG_FORCE_TILED):
+        k = kernels_of(pkg, T, H, I, 32, K, pkg.MOE_WEIGHTS_MXFP4_TILED, flags=flags)
+        assert k["gate_up"].startswith(name) and k["down"].startswith(name), k
+
+
 def test_tile_kernel_takes_large_activation_tensors(pkg):
     """Rows by slot past 4 GiB are no reason to leave the bf16 tile kernel, unless the 256 of one block are; gathered rows past it
     are, at the last byte."""
