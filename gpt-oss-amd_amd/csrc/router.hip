@@ -465,6 +465,32 @@ MOE_DEVICE void exact_dots(const float* __restrict__ x_row, const uint16_t* __re
     for (int i = 0; i < NE; ++i) total[i] = wave_sum(acc[i]);
 }
 
+// The same for one expert and a row of up to 256 TRIPS values that the wave holds in registers (row_load): all of the router row's
+// loads are in flight together.
+template <int TRIPS>
+MOE_DEVICE void row_load(const float* __restrict__ x_row, int H, int lane, float4 (&xv)[TRIPS]) {
+#pragma unroll
+    for (int j = 0; j < TRIPS; ++j) xv[j] = reinterpret_cast<const float4*>(x_row)[min(lane + 64 * j, (H >> 2) - 1)];
+}
+template <int TRIPS>
+MOE_DEVICE double exact_dot_held(const float4 (&xv)[TRIPS], const uint16_t* __restrict__ w_row, int H, int lane) {
+    const int n4 = H >> 2;
+    uint2 wb[TRIPS];
+#pragma unroll
+    for (int j = 0; j < TRIPS; ++j) wb[j] = reinterpret_cast<const uint2*>(w_row)[min(lane + 64 * j, n4 - 1)];
+    double acc = 0.0;
+#pragma unroll
+    for (int j = 0; j < TRIPS; ++j) {
+        if (64 * j >= n4) break;  // wave-uniform; the trips of exact_dots and no more: zero times an infinity is none
+        if (lane + 64 * j >= n4) wb[j] = make_uint2(0u, 0u);  // zero products leave the sum unchanged
+        acc += (double)__fmul_rn(__uint_as_float(wb[j].x << 16), xv[j].x);
+        acc += (double)__fmul_rn(__uint_as_float(wb[j].x & 0xFFFF0000u), xv[j].y);
+        acc += (double)__fmul_rn(__uint_as_float(wb[j].y << 16), xv[j].z);
+        acc += (double)__fmul_rn(__uint_as_float(wb[j].y & 0xFFFF0000u), xv[j].w);
+    }
+    return wave_sum(acc);
+}
+
 // ---------------------------------------------------------------------------------------------
 // Scores only, for a handful of tokens whose top-k is left to the gate/up kernel (experts_small.hip): a wave per (token, expert), so
 // that the router rows come through many compute units instead of one.  Block of 1 token, E = 32, us, whole router before : this
@@ -766,6 +792,7 @@ __global__ __launch_bounds__(256, 4) void router_refine_kernel(const float* __re
 // ---------------------------------------------------------------------------------------------
 constexpr int kRowsWaves = 16;
 constexpr int kRowsPairs = 3;  // pairs of k-steps (64 values) per wave: rows of up to 3072 values
+constexpr int kHeldTrips = 64 * kRowsWaves * kRowsPairs / 256;  // float4s of a row per lane
 
 // The lanes of a wave exchange values through its own LDS area: no instruction is needed (a wave's LDS accesses are carried out in
 // order), but the compiler must neither move accesses across nor run the two sides under different lane masks.
@@ -908,13 +935,22 @@ __global__ __launch_bounds__(64 * kRowsWaves) void router_rows_kernel(const floa
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             if ((4 * g + i) % DUP == 0) part[(4 * g + i) / DUP * LDP + 16 * n + r] = acc[n][i];
+    const int tl = wave / DUP, sub = wave % DUP;  // the wave's token, and its place among the token's waves
+    const int t = t0 + tl;
+    const float* x_row = x + (size_t)min(t, T - 1) * H;
+    // Up to four tokens to a block the wave's row comes while the candidates are found (us, so : with them, E = 32, 300 tokens 11.1 : 10.6,
+    // 1000 tokens 17.0 : 15.0; E = 128, 1024 tokens 24.2 : 22.8).  From eight on the waves take several candidates at a time, and a
+    // held row costs them registers (2000 tokens 23.2 : 27.7, 4096 tokens 35.7 : 35.4).
+    constexpr bool HELD = TPB <= 4;
+    float4 x_held[HELD ? kHeldTrips : 1];
+    if constexpr (HELD) row_load<kHeldTrips>(x_row, H, lane, x_held);
     __syncthreads();
     for (int i = threadIdx.x; i < TPB * EP; i += 64 * W) {
-        const int t = i / EP, e = i % EP;
+        const int ti = i / EP, e = i % EP;
         float sum = 0.f;
 #pragma unroll
-        for (int p = 0; p < W; ++p) sum += reinterpret_cast<const lds_f32*>(area[p])[t * LDP + e];
-        approx[t][e] = e < E ? sum + bf16_bits_to_f32(bias[e]) : 0.f;
+        for (int p = 0; p < W; ++p) sum += reinterpret_cast<const lds_f32*>(area[p])[ti * LDP + e];
+        approx[ti][e] = e < E ? sum + bf16_bits_to_f32(bias[e]) : 0.f;
     }
     // from the other end, where the waves have no sum of their own while there are few tokens
     const int back = 64 * W - 1 - (int)threadIdx.x;
@@ -928,8 +964,6 @@ __global__ __launch_bounds__(64 * kRowsWaves) void router_rows_kernel(const floa
         else x2[back - EP] = q;
     }
     __syncthreads();
-    const int tl = wave / DUP, sub = wave % DUP;  // the wave's token, and its place among the token's waves
-    const int t = t0 + tl;
     if (sub == 0) {  // candidates, as in router_refine_kernel
         const float* my = approx[tl];
         float amax = 0.f, wmax = 0.f;
@@ -966,14 +1000,14 @@ __global__ __launch_bounds__(64 * kRowsWaves) void router_rows_kernel(const floa
     const int n_cand = __builtin_amdgcn_readfirstlane(n_cands[tl]);
     // exact scores: the waves of a token take its candidates in turn, C at a time
     constexpr int C = TPB == 16 ? 4 : TPB == 8 ? 2 : 1;
-    const float* x_row = x + (size_t)min(t, T - 1) * H;
 #pragma nounroll
     for (int c0 = C * sub; c0 < n_cand; c0 += C * DUP) {
         int e[C];
         double total[C];
 #pragma unroll
         for (int i = 0; i < C; ++i) e[i] = __builtin_amdgcn_readfirstlane(cand[tl][min(c0 + i, n_cand - 1)]);
-        exact_dots<C, C == 4 ? 4 : 12>(x_row, w, e, H, lane, total);
+        if constexpr (HELD) total[0] = exact_dot_held<kHeldTrips>(x_held, w + (size_t)e[0] * H, H, lane);
+        else exact_dots<C, C == 4 ? 4 : 12>(x_row, w, e, H, lane, total);
         if (lane == 0) {
 #pragma unroll
             for (int i = 0; i < C; ++i)

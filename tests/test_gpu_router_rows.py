@@ -32,3 +32,24 @@ def test_one_launch_router(pkg, wl, dev, H, E, K):
         y, ti, tv = blk.forward(t)  # whichever router the batch takes: the bf16 rows it leaves are the same
         assert torch.equal(ti, wi) and (tv - wv).abs().max().item() <= 4e-6
         assert (y - wy).abs().max().item() <= 1e-5 * max(1.0, wy.abs().max().item())
+
+
+@pytest.mark.parametrize("H", [256, 1024, 1088, 3072])
+def test_one_launch_router_infinite_last_activation(pkg, wl, dev, H):
+    """A wave that holds a row in registers has places past the row's end: they take no part, whatever the last value is."""
+    T, E, K = 300, 32, 4
+    shape = wl.MoeShape("rows", T=T, H=H, I=64, E=E, K=K, fmt="mxfp4", seed=H)
+    blk, raw = wl.make_device_layer(shape, pkg.normal_table(), dev)
+    x = wl.make_device_input(shape, pkg.normal_table(), dev)
+    w = raw["w_router"]
+    w[:, H - 1] = 0.0
+    w[3, H - 1] = 0.5
+    if H % 256 == 0:  # other lengths leave lanes without a value in the last trip, which multiply the row's last by zero
+        x[::7, H - 1] = float("inf")
+        w[:, H - 1] = 0.25
+        w[4:, H - 1] = -0.25
+    print("one-launch router, infinite value", H, flush=True)
+    _, ti, tv = blk.forward(x)
+    assert blk.describe(blk.params(x, x, ti, tv))["router"] == "router_rows_kernel"
+    _, wi, wv = blk.forward(x, flags=pkg.MOE_FLAG_ROUTER_STRICT_ORDER)
+    assert torch.equal(ti, wi) and (tv.nan_to_num(0.0) - wv.nan_to_num(0.0)).abs().max().item() <= 4e-6
