@@ -20,12 +20,26 @@ static int hist_copies(int E) { return E <= 256 ? kHistCopies : E <= 512 ? 16 : 
 // round trip per 8192 ids and per 4096 tokens).  32 experts, us, general : V4: 1000 tokens 9.2 : 8.6, 4096 tokens 12.6 : 9.8, 16384 tokens 35 : 20.
 constexpr int kHeldTokens = 16 * 1024;
 
-// Rows of an expert's token blocks: the map's tile_tokens, or with `even` as many blocks as that gives, cut evenly into whole
-// MFMA tiles.  A remainder of a few rows streams the expert's weights once more for next to no matrix work, and takes more than half
-// of a whole block's time for it.  Whole block, us, whole blocks and a remainder : even ones, 32 experts: bf16, 4096 tokens (half the
-// buckets a few rows past 512) 891 : 867; MXFP4, skewed, 1000 tokens 240 : 235, 4096 tokens 729 : 728.
-MOE_DEVICE int tile_rows_of(const TileMap& map, int count) {
-    return map.even ? even_tile_rows(count, map.tile_tokens) : map.tile_tokens;
+// An expert's token blocks: `full` ones of `rows` rows and a last one of `rem` (none if 0).  EVEN: as many blocks as map.tile_tokens
+// gives, cut evenly into whole MFMA tiles.  A remainder of a few rows streams the expert's weights once more for next to no matrix
+// work, and takes more than half of a whole block's time for it.  Whole block, us, whole blocks and a remainder : even ones, 32
+// experts: bf16, 4096 tokens (half the buckets a few rows past 512) 891 : 867; MXFP4, skewed, 1000 tokens 240 : 235, 4096 tokens
+// 729 : 728.
+struct TokenBlocks {
+    int rows, full, rem;
+};
+template <bool EVEN>
+MOE_DEVICE TokenBlocks token_blocks(const TileMap& map, int count) {
+    TokenBlocks b;
+    b.rows = EVEN ? even_tile_rows(count, map.tile_tokens) : map.tile_tokens;
+    if constexpr (EVEN) {  // all of ceil(count / tile_tokens) but perhaps the last are full: no second division
+        const int n = (count + map.tile_tokens - 1) / map.tile_tokens;
+        b.full = n > 0 && n * b.rows != count ? n - 1 : n;
+    } else {
+        b.full = count / b.rows;
+    }
+    b.rem = count - b.full * b.rows;
+    return b;
 }
 
 // grid = E blocks (one expert each), block = 1024 threads, dynamic LDS = (E * copies + E + 32) ints.
@@ -34,7 +48,8 @@ MOE_DEVICE int tile_rows_of(const TileMap& map, int count) {
 // this order runs its shortest blocks last, next to compute units that have already run out of work.
 // With map.second > 0 the same tiles are listed a second time, from index map.second of the three
 // arrays, in bucket order (an expert's tiles together, the partial one last).
-template <bool V4>
+// EVEN is a constant: as a runtime choice it cost the launches without a map 0.35 of 5.8 us.
+template <bool V4, bool EVEN>
 __global__ __launch_bounds__(1024) void bucket_kernel(const int* __restrict__ topk_i,
                                                       const float* __restrict__ topk_v, int T, int K, int E,
                                                       int copies, int* __restrict__ expert_offsets,
@@ -98,15 +113,17 @@ __global__ __launch_bounds__(1024) void bucket_kernel(const int* __restrict__ to
     }
     __syncthreads();
     const int my_cnt = hist[e];
-    const int nb = tile_rows_of(map, my_cnt);
+    const bool mapped = map.tile_tokens > 0;
+    const TokenBlocks mine = mapped ? token_blocks<EVEN>(map, my_cnt) : TokenBlocks{};
     {
-        const int my_rem = nb > 0 ? my_cnt % nb : 0;
+        const int my_rem = mine.rem;
         int rows_before = 0, full_before = 0, full_all = 0, part_ahead = 0, part_all = 0, part_before = 0;
         for (int i = tid; i < E; i += blockDim.x) {
             const int c = hist[i];
             if (i < e) rows_before += c;
-            if (nb > 0) {
-                const int nb_i = tile_rows_of(map, c), full = c / nb_i, rem = c - full * nb_i;
+            if (mapped) {
+                const TokenBlocks b = token_blocks<EVEN>(map, c);
+                const int full = b.full, rem = b.rem;
                 full_all += full;
                 if (i < e) full_before += full;
                 if (rem > 0) {
@@ -133,9 +150,8 @@ __global__ __launch_bounds__(1024) void bucket_kernel(const int* __restrict__ to
         expert_offsets[e] = my_off;
         if (e == E - 1) expert_offsets[E] = my_off + my_cnt;
     }
-    if (nb > 0) {
-        const int my_full = my_cnt / nb;
-        const int my_rem = my_cnt - my_full * nb;
+    if (mapped) {
+        const int nb = mine.rows, my_full = mine.full, my_rem = mine.rem;
         for (int j = tid; j < my_full; j += blockDim.x) {
             map.tile_expert[scal[1] + j] = e;
             map.tile_row0[scal[1] + j] = my_off + j * nb;
@@ -232,13 +248,13 @@ int launch_bucket(const int* topk_i, const float* topk_v, int T, int K, int E, i
                   int* tokens_flat, float* weights_flat, int* slot_of, TileMap map, hipStream_t stream) {
     const int copies = hist_copies(E);
     const size_t lds = (size_t)(E * copies + E + 32) * sizeof(int);
-    if (K == 4 && T <= kHeldTokens && ((uintptr_t)topk_i & 15u) == 0) {
-        hipLaunchKernelGGL(bucket_kernel<true>, dim3(E), dim3(1024), lds, stream, topk_i, topk_v, T, K, E, copies, expert_offsets,
-                           tokens_flat, weights_flat, slot_of, map);
-    } else {
-        hipLaunchKernelGGL(bucket_kernel<false>, dim3(E), dim3(1024), lds, stream, topk_i, topk_v, T, K, E, copies, expert_offsets,
-                           tokens_flat, weights_flat, slot_of, map);
-    }
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(E), dim3(1024), lds, stream, topk_i, topk_v, T, K, E, copies, expert_offsets, tokens_flat,
+                           weights_flat, slot_of, map);
+    };
+    const bool v4 = K == 4 && T <= kHeldTokens && ((uintptr_t)topk_i & 15u) == 0;
+    if (map.even) launch(v4 ? bucket_kernel<true, true> : bucket_kernel<false, true>);
+    else launch(v4 ? bucket_kernel<true, false> : bucket_kernel<false, false>);
     return launch_status();
 }
 
