@@ -1025,12 +1025,22 @@ MOE_DEVICE void prefill_body_mxfp4(const ExpertGemmArgs& a, uint8_t* lds, int e,
         b_row[i] = (uint32_t)src * (uint32_t)K * 2u;
     }
     const uint8_t* const b_base = reinterpret_cast<const uint8_t*>(a.act + (a.gather ? 0 : (size_t)row0 * K));
+    // Rows of the last token tile past the block's end are cleared once and never loaded: products of zeros take the least power
+    // (up to 15 such rows to a bucket; whole block, the last row again : zeros, 1000 tokens 243.8 : 241.4 us, 4096 tokens 718 : 716).
+    static_assert(kStagers == 1, "this wave's last tile is the block's");
+    const bool last_live = (NT - 1) * 16 + q_dma < nrows;
+    if (!last_live) {
+#pragma unroll
+        for (int slot = 0; slot < 2; ++slot)
+            *reinterpret_cast<u32x4*>(lds + (size_t)slot * kStageBytes + (NT - 1) * 4096 + blk_w * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+    }
     auto issue_b = [&](int s) {
         const int k = s * kStageElems + 8 * chunk_dma;
         const uint32_t off = (k < K) ? (uint32_t)k * 2u : 0u;  // past the row: re-read its start (weights are 0 there)
         uint8_t* dst = lds + (size_t)(s & 1) * kStageBytes + (size_t)half_w * 4096 + blk_w * 1024;
 #pragma unroll
-        for (int i = 0; i < TS; ++i) dma16(b_base + (size_t)(b_row[i] + off), dst + i * kStagers * 4096);
+        for (int i = 0; i < TS - 1; ++i) dma16(b_base + (size_t)(b_row[i] + off), dst + i * kStagers * 4096);
+        if (last_live) dma16(b_base + (size_t)(b_row[TS - 1] + off), dst + (TS - 1) * kStagers * 4096);
     };
     const uint8_t* const lds_rd = lds + (size_t)q * 256;
     auto b_frag = [&](int s, int j, int t) {  // lane group g owns MX block g of a stage: chunk 4g + j
