@@ -428,9 +428,10 @@ __global__ __launch_bounds__(256) void router_screen_kernel(const float* __restr
 // Exact logits of NE experts for one token, by one wave: fp32 products, fp64 sums
 // (src/run.cpp:341-354).  Lane l takes float4 number l, l + 64, ... of the token's activations in
 // ascending order; the lanes' sums are combined by wave_sum's fixed tree, so a logit does not depend
-// on NE or on which other experts share the call.  The trip count is the same for every lane (a
-// lane past the end multiplies zeros), so that the loads of several iterations can be in flight
-// together.  Every lane returns all NE totals.
+// on NE or on which other experts share the call.  The trip count is the same for every lane, so that
+// the loads of several iterations can be in flight together: a lane past the end re-reads the row's last
+// values and multiplies zeros in place of both (either may be an infinity), which leave its sum unchanged.
+// Every lane returns all NE totals.
 template <int NE, int UNROLL>
 MOE_DEVICE void exact_dots(const float* __restrict__ x_row, const uint16_t* __restrict__ w, const int (&e)[NE], int H,
                            int lane, double (&total)[NE]) {
@@ -448,13 +449,14 @@ MOE_DEVICE void exact_dots(const float* __restrict__ x_row, const uint16_t* __re
     for (int j = 0; j < trips; ++j) {
         const bool live = lane + 64 * j < n4;
         const int i4 = min(lane + 64 * j, n4 - 1);
-        const float4 xv = xrow[i4];
+        float4 xv = xrow[i4];
         uint2 wb[NE];
 #pragma unroll
         for (int i = 0; i < NE; ++i) wb[i] = wrow[i][i4];
+        if (!live) xv = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int i = 0; i < NE; ++i) {
-            if (!live) wb[i] = make_uint2(0u, 0u);  // zero products leave the sum unchanged
+            if (!live) wb[i] = make_uint2(0u, 0u);
             acc[i] += (double)__fmul_rn(__uint_as_float(wb[i].x << 16), xv.x);
             acc[i] += (double)__fmul_rn(__uint_as_float(wb[i].x & 0xFFFF0000u), xv.y);
             acc[i] += (double)__fmul_rn(__uint_as_float(wb[i].y << 16), xv.z);
@@ -481,12 +483,16 @@ MOE_DEVICE double exact_dot_held(const float4 (&xv)[TRIPS], const uint16_t* __re
     double acc = 0.0;
 #pragma unroll
     for (int j = 0; j < TRIPS; ++j) {
-        if (64 * j >= n4) break;  // wave-uniform; the trips of exact_dots and no more: zero times an infinity is none
-        if (lane + 64 * j >= n4) wb[j] = make_uint2(0u, 0u);  // zero products leave the sum unchanged
-        acc += (double)__fmul_rn(__uint_as_float(wb[j].x << 16), xv[j].x);
-        acc += (double)__fmul_rn(__uint_as_float(wb[j].x & 0xFFFF0000u), xv[j].y);
-        acc += (double)__fmul_rn(__uint_as_float(wb[j].y << 16), xv[j].z);
-        acc += (double)__fmul_rn(__uint_as_float(wb[j].y & 0xFFFF0000u), xv[j].w);
+        if (64 * j >= n4) break;  // wave-uniform
+        float4 v = xv[j];
+        if (lane + 64 * j >= n4) {
+            v = make_float4(0.f, 0.f, 0.f, 0.f);
+            wb[j] = make_uint2(0u, 0u);
+        }
+        acc += (double)__fmul_rn(__uint_as_float(wb[j].x << 16), v.x);
+        acc += (double)__fmul_rn(__uint_as_float(wb[j].x & 0xFFFF0000u), v.y);
+        acc += (double)__fmul_rn(__uint_as_float(wb[j].y << 16), v.z);
+        acc += (double)__fmul_rn(__uint_as_float(wb[j].y & 0xFFFF0000u), v.w);
     }
     return wave_sum(acc);
 }
@@ -526,7 +532,7 @@ __global__ __launch_bounds__(256) void router_scores_kernel(const float* __restr
 // softmax and writes the score row if the caller wants it.
 // All loads of a wave's first pass (the activation piece it stages, its two router rows) are issued
 // before anything waits, so a block costs one memory round trip plus the arithmetic.
-// grid = T, block = 64 * waves, dynamic LDS = (H + E) floats; H <= 256 * kFusedTrips.  NE experts per
+// grid = T, block = 64 * waves, dynamic LDS = (256 * kFusedTrips + E) floats; H <= 256 * kFusedTrips.  NE experts per
 // wave and pass: two with up to 16 waves (128 registers per lane hold the loads of two rows), four
 // with up to 8 waves.
 // ---------------------------------------------------------------------------------------------
@@ -540,8 +546,8 @@ __global__ __launch_bounds__(NE == 2 ? 1024 : 512) void router_fused_kernel(cons
                                                             int* __restrict__ topk_i, int H, int E, int K,
                                                             int do_softmax) {
     extern __shared__ __attribute__((aligned(16))) float fused_lds[];
-    float4* xs = reinterpret_cast<float4*>(fused_lds);  // [H / 4]
-    float* sc = fused_lds + H;                           // [E]
+    float4* xs = reinterpret_cast<float4*>(fused_lds);  // [64 * kFusedTrips], zeros past the row
+    float* sc = fused_lds + 256 * kFusedTrips;           // [E]
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n_waves = blockDim.x >> 6;
@@ -573,6 +579,7 @@ __global__ __launch_bounds__(NE == 2 ? 1024 : 512) void router_fused_kernel(cons
         }
     };
     if (wave < n_groups) load_rows(wave);
+    for (int c = n4 + threadIdx.x; c < 64 * kFusedTrips; c += blockDim.x) xs[c] = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int c = threadIdx.x + STG * blockDim.x; c < n4; c += blockDim.x) xs[c] = xr[c];  // blocks with few waves
 #pragma unroll
     for (int i = 0; i < STG; ++i) {
@@ -597,10 +604,10 @@ __global__ __launch_bounds__(NE == 2 ? 1024 : 512) void router_fused_kernel(cons
 #pragma unroll
         for (int j = 0; j < kFusedTrips; ++j) {
             const bool live = lane + 64 * j < n4;
-            const float4 xv = xs[idx[j]];
+            const float4 xv = xs[lane + 64 * j];
 #pragma unroll
             for (int i = 0; i < NE; ++i) {
-                const uint2 wv = live ? wb[j][i] : make_uint2(0u, 0u);  // zero products leave the sum unchanged
+                const uint2 wv = live ? wb[j][i] : make_uint2(0u, 0u);  // zeros on both sides: the sum stays
                 acc[i] += (double)__fmul_rn(__uint_as_float(wv.x << 16), xv.x);
                 acc[i] += (double)__fmul_rn(__uint_as_float(wv.x & 0xFFFF0000u), xv.y);
                 acc[i] += (double)__fmul_rn(__uint_as_float(wv.y << 16), xv.z);
@@ -1288,7 +1295,7 @@ bool router_fused_fits(int H) { return H % 4 == 0 && H <= 256 * kFusedTrips; }
 int launch_router_fused(const float* x, const uint16_t* w, const uint16_t* bias, uint16_t* x_bf16, float* scores_out,
                         float* topk_v, int* topk_i, int T, int H, int E, int K, int do_softmax, hipStream_t stream) {
     if (!router_fused_fits(H)) return MOE_ERR_LIMIT;
-    const size_t lds = (size_t)(H + E) * sizeof(float);
+    const size_t lds = (size_t)(256 * kFusedTrips + E) * sizeof(float);
     if (E <= 32) {
         hipLaunchKernelGGL(router_fused_kernel<2>, dim3(T), dim3(64 * min(16, ceil_div(E, 2))), lds, stream, x, w, bias,
                            x_bf16, scores_out, topk_v, topk_i, H, E, K, do_softmax);

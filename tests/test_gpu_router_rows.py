@@ -34,22 +34,34 @@ def test_one_launch_router(pkg, wl, dev, H, E, K):
         assert (y - wy).abs().max().item() <= 1e-5 * max(1.0, wy.abs().max().item())
 
 
-@pytest.mark.parametrize("H", [256, 1024, 1088, 3072])
-def test_one_launch_router_infinite_last_activation(pkg, wl, dev, H):
-    """A wave that holds a row in registers has places past the row's end: they take no part, whatever the last value is."""
-    T, E, K = 300, 32, 4
+# every kernel with lanes past the row's end, and 300, 600 and 2050 tokens for the forms of the one-launch kernel
+ROUTES = [(3, 32, "router_scores_kernel"), (30, 128, "router_scores_kernel + router_finalize_kernel"), (100, 32, "router_fused_kernel"),
+          (150, 200, "router_fused_kernel"), (300, 32, "router_rows_kernel"), (600, 32, "router_rows_kernel"), (2050, 32, "router_rows_kernel"),
+          (300, 200, "router_screen_kernel + router_refine_kernel")]
+
+
+@pytest.mark.parametrize("H", [256, 1024, 1088, 2880, 3072])  # 1088 and 2880 leave lanes without a value in a wave's last 256
+@pytest.mark.parametrize("T,E,router", ROUTES)
+def test_infinite_last_value(pkg, wl, dev, T, E, router, H):
+    """Lanes past the row's end take no part, whatever the last value of the row, or of a router row, is."""
+    K = 4
     shape = wl.MoeShape("rows", T=T, H=H, I=64, E=E, K=K, fmt="mxfp4", seed=H)
     blk, raw = wl.make_device_layer(shape, pkg.normal_table(), dev)
-    x = wl.make_device_input(shape, pkg.normal_table(), dev)
+    x0 = wl.make_device_input(shape, pkg.normal_table(), dev)
     w = raw["w_router"]
-    w[:, H - 1] = 0.0
-    w[3, H - 1] = 0.5
-    if H % 256 == 0:  # other lengths leave lanes without a value in the last trip, which multiply the row's last by zero
-        x[::7, H - 1] = float("inf")
-        w[:, H - 1] = 0.25
-        w[4:, H - 1] = -0.25
-    print("one-launch router, infinite value", H, flush=True)
-    _, ti, tv = blk.forward(x)
-    assert blk.describe(blk.params(x, x, ti, tv))["router"] == "router_rows_kernel"
-    _, wi, wv = blk.forward(x, flags=pkg.MOE_FLAG_ROUTER_STRICT_ORDER)
-    assert torch.equal(ti, wi) and (tv.nan_to_num(0.0) - wv.nan_to_num(0.0)).abs().max().item() <= 4e-6
+    w[:, H - 1] = -0.25
+    w[[5, 9, 20, E - 1], H - 1] = 0.25
+    for what in ("activation", "weight"):
+        x = x0.clone()
+        if what == "activation":
+            x[::7, H - 1] = float("inf")
+        else:
+            w[11, H - 1] = float("inf")
+        print("infinite last", what, T, E, H, flush=True)
+        _, ti, tv = blk.forward(x)
+        assert blk.describe(blk.params(x, x, ti, tv))["router"] == router
+        _, wi, wv = blk.forward(x, flags=pkg.MOE_FLAG_ROUTER_STRICT_ORDER)
+        if what == "activation":
+            assert (wi[::7] == torch.tensor([5, 9, 20, E - 1], dtype=torch.int32, device=dev)).all()
+        assert torch.equal(ti, wi) and torch.equal(tv.isnan(), wv.isnan())
+        assert (tv.nan_to_num(0.0) - wv.nan_to_num(0.0)).abs().max().item() <= 4e-6  # as above
