@@ -28,6 +28,8 @@ constexpr int kPrefillTileTokensBf16 = 256;
 inline int tile_tokens_of(bool prefill, int format) {
     return !prefill ? kStreamTileTokens : format == MOE_WEIGHTS_BF16 ? kPrefillTileTokensBf16 : kPrefillTileTokens;
 }
+inline int tile_even_of(bool prefill, int format) { return !prefill ? 0 : format == MOE_WEIGHTS_BF16 ? kPrefillStepBf16 : kPrefillStep; }
+
 // Which family runs the expert GEMMs, by average bucket size T*K/E (measured crossovers, 20b
 // shapes, token counts 256..4096).  MXFP4: the 128-token-block kernels win as soon as buckets start
 // to overflow one 64-token block (the streaming kernel then reads an expert's weights once per
@@ -774,7 +776,7 @@ static int block_forward_impl(const moe_block_params* caller, moe_stream_t strea
     const int tile_tokens = tile_tokens_of(prefill, fmt);
     const int max_tiles = tile_map_capacity(T * K, E, tile_tokens);  // <= ws.max_tiles (sized for 64)
     if (!direct) {
-        TileMap map{ws.tile_expert, ws.tile_row0, ws.tile_rows, ws.n_tiles, tile_tokens, max_tiles, ws.max_tiles, prefill};
+        TileMap map{ws.tile_expert, ws.tile_row0, ws.tile_rows, ws.n_tiles, tile_tokens, max_tiles, ws.max_tiles, tile_even_of(prefill, fmt)};
         rc = launch_bucket(p->topk_i, p->topk_v, T, K, E, ws.expert_offsets, ws.tokens_flat, ws.weights_flat,
                            ws.slot_of, map, stream);
         if (rc) return rc;
@@ -955,7 +957,7 @@ int moe_block_down_gemm(const moe_block_params* caller, const moe_bf16_t* h_by_a
     const ExpertPlan plan(p, ws, prefill, direct, tile_tokens, max_tiles);
     if (direct) return launch_expert_stream(plan.down(h_by_assignment, y_by_assignment), 1, stream);
     // rows by slot: bucket, bring the caller's rows into slot order, multiply, bring the result back
-    TileMap map{ws.tile_expert, ws.tile_row0, ws.tile_rows, ws.n_tiles, tile_tokens, max_tiles, ws.max_tiles, prefill};
+    TileMap map{ws.tile_expert, ws.tile_row0, ws.tile_rows, ws.n_tiles, tile_tokens, max_tiles, ws.max_tiles, tile_even_of(prefill, fmt)};
     rc = launch_bucket(p->topk_i, p->topk_v, T, K, E, ws.expert_offsets, ws.tokens_flat, ws.weights_flat, ws.slot_of,
                        map, stream);
     if (rc) return rc;

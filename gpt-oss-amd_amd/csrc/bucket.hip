@@ -20,19 +20,21 @@ static int hist_copies(int E) { return E <= 256 ? kHistCopies : E <= 512 ? 16 : 
 // round trip per 8192 ids and per 4096 tokens).  32 experts, us, general : V4: 1000 tokens 9.2 : 8.6, 4096 tokens 12.6 : 9.8, 16384 tokens 35 : 20.
 constexpr int kHeldTokens = 16 * 1024;
 
-// An expert's token blocks: `full` ones of `rows` rows and a last one of `rem` (none if 0).  EVEN: as many blocks as map.tile_tokens
-// gives, cut evenly into whole MFMA tiles.  A remainder of a few rows streams the expert's weights once more for next to no matrix
-// work, and takes more than half of a whole block's time for it.  Whole block, us, whole blocks and a remainder : even ones, 32
-// experts: bf16, 4096 tokens (half the buckets a few rows past 512) 891 : 867; MXFP4, skewed, 1000 tokens 240 : 235, 4096 tokens
-// 729 : 728.
+// An expert's token blocks: `full` ones of `rows` rows and a last one of `rem` (none if 0).  EVEN > 0: as many blocks as
+// map.tile_tokens gives, cut evenly in steps of EVEN rows (even_tile_rows).  A remainder of a few rows streams the expert's weights once
+// more for next to no matrix work, and takes more than half of a whole block's time for it.
+// bf16, whole MoE block, us, whole token blocks and a remainder : even ones, 32 experts: 1500 tokens 433 : 434, 2048 tokens 599 : 575,
+// 2400 tokens 667 : 591, 3400 tokens 726 : 727, 4096 tokens 868 : 855, 4864 tokens 1025 : 1017, 6656 tokens 1323 : 1327, 8192 tokens 1548 :
+// 1548; 8 experts, 1100 tokens 335 : 309.  In steps of 16 rows, which the bf16 kernel rounds up to 64: 2400 tokens 600, 4096 tokens 859
+// (skewed 878 against 869), 4864 tokens 1022 (1028), 6656 tokens 1363 (1357).
 struct TokenBlocks {
     int rows, full, rem;
 };
-template <bool EVEN>
+template <int EVEN>
 MOE_DEVICE TokenBlocks token_blocks(const TileMap& map, int count) {
     TokenBlocks b;
-    b.rows = EVEN ? even_tile_rows(count, map.tile_tokens) : map.tile_tokens;
-    if constexpr (EVEN) {  // all of ceil(count / tile_tokens) but perhaps the last are full: no second division
+    b.rows = EVEN ? even_tile_rows(count, map.tile_tokens, EVEN) : map.tile_tokens;
+    if constexpr (EVEN > 0) {  // all of ceil(count / tile_tokens) but perhaps the last are full: no division by rows
         const int n = (count + map.tile_tokens - 1) / map.tile_tokens;
         b.full = n > 0 && n * b.rows != count ? n - 1 : n;
     } else {
@@ -49,7 +51,7 @@ MOE_DEVICE TokenBlocks token_blocks(const TileMap& map, int count) {
 // With map.second > 0 the same tiles are listed a second time, from index map.second of the three
 // arrays, in bucket order (an expert's tiles together, the partial one last).
 // EVEN is a constant: as a runtime choice it cost the launches without a map 0.35 of 5.8 us.
-template <bool V4, bool EVEN>
+template <bool V4, int EVEN>
 __global__ __launch_bounds__(1024) void bucket_kernel(const int* __restrict__ topk_i,
                                                       const float* __restrict__ topk_v, int T, int K, int E,
                                                       int copies, int* __restrict__ expert_offsets,
@@ -253,8 +255,9 @@ int launch_bucket(const int* topk_i, const float* topk_v, int T, int K, int E, i
                            weights_flat, slot_of, map);
     };
     const bool v4 = K == 4 && T <= kHeldTokens && ((uintptr_t)topk_i & 15u) == 0;
-    if (map.even) launch(v4 ? bucket_kernel<true, true> : bucket_kernel<false, true>);
-    else launch(v4 ? bucket_kernel<true, false> : bucket_kernel<false, false>);
+    if (map.even == kPrefillStep) launch(v4 ? bucket_kernel<true, kPrefillStep> : bucket_kernel<false, kPrefillStep>);
+    else if (map.even == kPrefillStepBf16) launch(v4 ? bucket_kernel<true, kPrefillStepBf16> : bucket_kernel<false, kPrefillStepBf16>);
+    else launch(v4 ? bucket_kernel<true, 0> : bucket_kernel<false, 0>);
     return launch_status();
 }
 

@@ -223,7 +223,7 @@ __global__ __launch_bounds__(512, 2) void expert_tile_bf16_kernel(ExpertGemmArgs
     const int begin = a.expert_offsets[e];
     const int count = a.expert_offsets[e + 1] - begin;
     const int n_et = (count + 255) >> 8;                                             // the expert's tiles,
-    const int first = any - (a.tile_row0[any] - begin) / even_tile_rows(count, 256);  // the first of them
+    const int first = any - (a.tile_row0[any] - begin) / even_tile_rows(count, 256, kPrefillStepBf16);  // the first of them
     const int local = seq - first * n_rb;
     const int rb = local / n_et;
     const int tile = first + local - rb * n_et;

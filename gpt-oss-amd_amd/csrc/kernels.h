@@ -50,13 +50,17 @@ struct TileMap {
     int tile_tokens;  // rows per tile (NB); 0 = no map requested
     int max_tiles;    // capacity = upper bound used as grid dimension
     int second;       // the same tiles in bucket order start at this index of the three arrays (0: not wanted)
-    int even;         // an expert's tiles are cut to the same number of MFMA tiles of 16 rows (the last may have less)
+    int even;         // an expert's tiles are cut evenly, in steps of 16 or 64 rows (even_tile_rows); 0: whole tiles and a remainder
 };
-// Rows of each but the last of an expert's tiles, cut evenly; as many tiles as tile_tokens (a multiple of 16) would give.
-__host__ __device__ inline int even_tile_rows(int count, int tile_tokens) {
+// Rows of each but the last of an expert's tiles, cut evenly; as many tiles as tile_tokens (a multiple of step) would give.  step is
+// what the kernel that takes the tiles rounds their rows up to: all but the last are multiples of it, so that a bucket's matrix work is
+// ceil(count / step) steps, as few as there can be.
+__host__ __device__ inline int even_tile_rows(int count, int tile_tokens, int step) {
     const int n = (count + tile_tokens - 1) / tile_tokens;
-    return n <= 1 ? tile_tokens : ((count + n - 1) / n + 15) / 16 * 16;
+    return n <= 1 ? tile_tokens : ((count + n - 1) / n + step - 1) / step * step;
 }
+constexpr int kPrefillStep = 16;      // the MXFP4 kernel runs any number of MFMA tiles,
+constexpr int kPrefillStepBf16 = 64;  // the bf16 kernel (full row blocks) multiples of four
 inline int tile_map_capacity(int A, int E, int tile_tokens) { return (A + tile_tokens - 1) / tile_tokens + E; }
 
 int launch_bucket(const int* topk_i, const float* topk_v, int T, int K, int E, int* expert_offsets,

@@ -21,18 +21,21 @@ def test_prefill_blocks_cover_every_row(pkg, wl, dev, H, I, T, E, K, zipf_s):
     assert torch.equal(y, want)
 
 
-# buckets of one row more and less than whole token blocks, of 16, 17 and 18 of them
-@pytest.mark.parametrize("fmt,block", [("mxfp4", 128), ("bf16", 256)])
-@pytest.mark.parametrize("blocks", [2, 17])
-def test_evenly_cut_buckets(pkg, wl, dev, fmt, block, blocks):
+# MXFP4 blocks of up to 128 rows, bf16 of up to 256: buckets of up to 8 blocks, among them the first and the last length that is cut into
+# two and into three equal ones, and one row past whole blocks
+@pytest.mark.parametrize("fmt,rows", [("mxfp4", [128, 129, 144, 145, 224, 225, 256, 257, 300, 336, 337, 385, 513, 769, 897]),
+                                      ("bf16", [256, 257, 320, 384, 385, 512, 513, 576, 577, 769, 1025])])
+def test_evenly_cut_buckets(pkg, wl, dev, fmt, rows):
     table = pkg.normal_table()
-    T = blocks * block + 1
-    shape = wl.MoeShape("prefill", T=T, H=64, I=128, E=2, K=2, fmt=fmt, seed=T)  # every token uses both experts
+    # two row blocks and more in both launches; every token uses both experts
+    shape = wl.MoeShape("prefill", T=max(rows), H=320, I=448, E=2, K=2, fmt=fmt, seed=len(rows))
     blk, _ = wl.make_device_layer(shape, table, dev)
     x = wl.make_device_input(shape, table, dev)
-    for n in (T, T - 1, T - 2, T - block + 15):
+    for n in rows:
         print("evenly cut", fmt, n, flush=True)
         t = x[:n].contiguous()
-        y, ti, _ = blk.forward(t, flags=pkg.MOE_FLAG_FORCE_TILED)
+        y, ti, tv = blk.forward(t, flags=pkg.MOE_FLAG_FORCE_TILED)
+        p = blk.params(t, y, ti, tv, flags=pkg.MOE_FLAG_FORCE_TILED)
+        assert blk.describe(p)["gate_up"].startswith("expert_tile" if fmt == "bf16" else "expert_prefill")
         want, _, _ = blk.forward(t, flags=pkg.MOE_FLAG_FORCE_STREAM)
         assert torch.equal(y, want), n
