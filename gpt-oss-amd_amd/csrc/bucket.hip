@@ -22,7 +22,7 @@ constexpr int kHeldTokens = 16 * 1024;
 
 // An expert's token blocks: `full` ones of `rows` rows and a last one of `rem` (none if 0).  EVEN > 0: as many blocks as
 // map.tile_tokens gives, cut evenly in steps of EVEN rows (even_tile_rows).  A remainder of a few rows streams the expert's weights once
-// more for next to no matrix work, and takes more than half of a whole block's time for it.
+// more for next to no matrix work, and takes more than half of a whole block's time for it.  (MXFP4: figures at even_tile_rows.)
 // bf16, whole MoE block, us, whole token blocks and a remainder : even ones, 32 experts: 1500 tokens 433 : 434, 2048 tokens 599 : 575,
 // 2400 tokens 667 : 591, 3400 tokens 726 : 727, 4096 tokens 868 : 855, 4864 tokens 1025 : 1017, 6656 tokens 1323 : 1327, 8192 tokens 1548 :
 // 1548; 8 experts, 1100 tokens 335 : 309.  In steps of 16 rows, which the bf16 kernel rounds up to 64: 2400 tokens 600, 4096 tokens 859

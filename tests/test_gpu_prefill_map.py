@@ -21,8 +21,8 @@ def test_prefill_blocks_cover_every_row(pkg, wl, dev, H, I, T, E, K, zipf_s):
     assert torch.equal(y, want)
 
 
-# MXFP4 blocks of up to 128 rows, bf16 of up to 256: buckets of up to 8 blocks, among them the first and the last length that is cut into
-# two and into three equal ones, and one row past whole blocks
+# MXFP4 blocks of up to 128 rows, bf16 of up to 256: buckets of up to 8 blocks, among them the first and the last length that is cut (into
+# two equal ones, bf16 into three as well), and one row past whole blocks
 @pytest.mark.parametrize("fmt,rows", [("mxfp4", [128, 129, 144, 145, 224, 225, 256, 257, 300, 336, 337, 385, 513, 769, 897]),
                                       ("bf16", [256, 257, 320, 384, 385, 512, 513, 576, 577, 769, 1025])])
 def test_evenly_cut_buckets(pkg, wl, dev, fmt, rows):
