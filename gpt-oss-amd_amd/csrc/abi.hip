@@ -265,7 +265,7 @@ int moe_bucket_by_expert(const int* topk_i, const float* topk_v, int B, int K, i
     if (!topk_i || !topk_v || !expert_offsets || !tokens_flat || !weights_flat) return MOE_ERR_NULL;
     if (B <= 0 || K <= 0 || E <= 0) return MOE_ERR_SHAPE;
     if (E > 1024 || K > 8 || (long long)B * K > 0x7FFFFFFFll / 4) return MOE_ERR_LIMIT;
-    TileMap none{nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0};
+    TileMap none{nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
     return launch_bucket(topk_i, topk_v, B, K, E, expert_offsets, tokens_flat, weights_flat, slot_of, none,
                          as_stream(stream));
 }
@@ -560,6 +560,22 @@ struct moe_stage_timer {
     hipEvent_t ev[MOE_N_STAGES + 1];
 };
 
+// Token blocks of a launch, as far as the host can tell: at least so many, and not many more with a router of no preference.
+static int expected_tiles(int A, int E, int tile_tokens) { return std::max(ceil_div(A, tile_tokens), std::min(E, A)); }
+
+// The token-block map of a block whose expert kernels do not bucket.  MXFP4 prefill: where the gate/up launch has more than two rounds of
+// blocks (two to a compute unit) the largest come first, so that it ends with its shortest.  With fewer that starts all long blocks
+// together and is the slower order.  Whole block, us, every expert's last token block after all the others : by size, 32 experts: 700 tokens
+// skewed 189 : 193, 850 tokens 208 : 213, 1000 tokens 237 : 240, 1500 tokens 307 : 302, 2000 tokens 383 : 380, skewed 394 : 391, 3600 tokens
+// 646 : 644, 6000 tokens 1037 : 1034; 16 experts, 500 tokens 136 : 143; 128 experts, 4500 tokens 971 : 949, 6000 tokens 1193 : 1165.  The
+// down launch reads this order only where it has few blocks; bf16 launches never do.
+static TileMap block_tile_map(const moe_block_params* p, const BlockWorkspace& ws, bool prefill) {
+    const int A = p->n_tokens * p->experts_per_token, tokens = tile_tokens_of(prefill, p->weight_format);
+    const long long blocks = (long long)expected_tiles(A, p->n_experts, tokens) * ceil_div(2 * p->intermediate_dim, 256);
+    return {ws.tile_expert, ws.tile_row0, ws.tile_rows, ws.n_tiles, tokens, tile_map_capacity(A, p->n_experts, tokens), ws.max_tiles,
+            tile_even_of(prefill, p->weight_format), blocks > 4LL * device_cu_count()};
+}
+
 // Launch parameters of the two expert GEMMs of one block.
 struct ExpertPlan {
     const moe_block_params* p;
@@ -588,7 +604,7 @@ struct ExpertPlan {
             g.assign_div = K;
             g.n_experts = E;
         }
-        est_tiles = direct ? E : std::max(ceil_div(T * K, tile_tokens), std::min(E, T * K));
+        est_tiles = direct ? E : expected_tiles(T * K, E, tile_tokens);
         n_cus = device_cu_count();
         small = use_small_kernels(T, p->hidden_dim, p->intermediate_dim, K, E, p->weight_format, direct, p->flags, n_cus);
         second_map = ws.max_tiles;
@@ -649,11 +665,12 @@ struct ExpertPlan {
         }
     }
     // MXFP4 prefill launches of at most two and a half rounds of blocks (two to a compute unit), by the launch's own count: what
-    // counts is how evenly they end, so the largest token blocks come first and the XCDs get equal shares (two parts to a token
-    // block).  Block of 32 experts, us, neither launch so : gate/up : down : both.  Router of no preference, 700 tokens 208 : 211 :
-    // 207 : 209, 1000 tokens 282 : 288 : 257 : 262, 2000 tokens 431 : 435 : 423 : 424, 2700 tokens 539 : 540 : 542 : 545; skewed, 416 tokens
-    // 193 : 189 : 174 : 170, 1000 tokens 302 : 301 : 278 : 276, 2000 tokens 427 : 430 : 422 : 426, 2700 tokens 555 : 558 : 542 : 547; 8
-    // experts, 2400 tokens skewed 286 : 283 : 269 : 262, 3200 tokens 360 : 345 : 360 : 346.
+    // counts is how evenly they end, so the XCDs get equal shares (two parts to a token block) and the down launch too takes the map's
+    // first order (block_tile_map).  Whole block of 32 experts, us, neither launch so : gate/up : down : both.  Router of no preference,
+    // 700 tokens 185 : 189 : 185 : 189, 1000 tokens 251 : 251 : 237 : 237, 1400 tokens 296 : 293 : 295 : 292, 2000 tokens 397 : 404 : 386 : 391,
+    // 2700 tokens 508 : 507 : 506 : 508, 3600 tokens 647 : 653 : 648 : 652; skewed, 416 tokens 164 : 160 : 157 : 152, 1000 tokens 257 : 255 :
+    // 243 : 238, 1700 tokens 356 : 354 : 345 : 345, 2700 tokens 509 : 508 : 505 : 506; 8 experts, 2400 tokens skewed 435 : 430 : 434 : 429,
+    // 3200 tokens 550 : 544 : 549 : 545.
     bool few_blocks(int rows) const { return (long long)est_tiles * ceil_div(rows, 256) < 5LL * n_cus; }
     void use_second_map(ExpertGemmArgs& a) const {
         a.tile_expert += second_map;
@@ -684,10 +701,10 @@ struct ExpertPlan {
         a.act = act;
         a.gather = 0;
         a.out = out;
-        // Measured at 4096 tokens: the gate/up GEMM is up to 9 % faster with the partial token blocks last
-        // (largest first: the launch's tail is made of short blocks); the down GEMM is 2 % faster in bucket
-        // order, where a partial block runs next to full blocks of its expert and finds the expert's weights
-        // on their way through the caches.
+        // MXFP4 launches of many blocks, us: the gate/up GEMM with the largest token blocks first : in bucket order, 2000 tokens 211 :
+        // 238, 4096 tokens 397 : 412, skewed 397 : 408.  The down GEMM does as well in bucket order, where a block runs next to the others
+        // of its expert and finds the expert's weights on their way through the caches: whole block, largest first : so, 4096 tokens
+        // 718 : 721, 9000 tokens 1531 : 1517, 128 experts, 4500 tokens 957 : 949.
         const bool few = a.waves_per_block == 16 && few_blocks(a.rows);
         if (!direct && !few) use_second_map(a);
         // measured: the down GEMM gains 4-10 % from keeping a token block on one XCD (its input rows were
@@ -776,7 +793,7 @@ static int block_forward_impl(const moe_block_params* caller, moe_stream_t strea
     const int tile_tokens = tile_tokens_of(prefill, fmt);
     const int max_tiles = tile_map_capacity(T * K, E, tile_tokens);  // <= ws.max_tiles (sized for 64)
     if (!direct) {
-        TileMap map{ws.tile_expert, ws.tile_row0, ws.tile_rows, ws.n_tiles, tile_tokens, max_tiles, ws.max_tiles, tile_even_of(prefill, fmt)};
+        const TileMap map = block_tile_map(p, ws, prefill);
         rc = launch_bucket(p->topk_i, p->topk_v, T, K, E, ws.expert_offsets, ws.tokens_flat, ws.weights_flat,
                            ws.slot_of, map, stream);
         if (rc) return rc;
@@ -957,7 +974,7 @@ int moe_block_down_gemm(const moe_block_params* caller, const moe_bf16_t* h_by_a
     const ExpertPlan plan(p, ws, prefill, direct, tile_tokens, max_tiles);
     if (direct) return launch_expert_stream(plan.down(h_by_assignment, y_by_assignment), 1, stream);
     // rows by slot: bucket, bring the caller's rows into slot order, multiply, bring the result back
-    TileMap map{ws.tile_expert, ws.tile_row0, ws.tile_rows, ws.n_tiles, tile_tokens, max_tiles, ws.max_tiles, tile_even_of(prefill, fmt)};
+    const TileMap map = block_tile_map(p, ws, prefill);
     rc = launch_bucket(p->topk_i, p->topk_v, T, K, E, ws.expert_offsets, ws.tokens_flat, ws.weights_flat, ws.slot_of,
                        map, stream);
     if (rc) return rc;

@@ -20,36 +20,9 @@ static int hist_copies(int E) { return E <= 256 ? kHistCopies : E <= 512 ? 16 : 
 // round trip per 8192 ids and per 4096 tokens).  32 experts, us, general : V4: 1000 tokens 9.2 : 8.6, 4096 tokens 12.6 : 9.8, 16384 tokens 35 : 20.
 constexpr int kHeldTokens = 16 * 1024;
 
-// An expert's token blocks: `full` ones of `rows` rows and a last one of `rem` (none if 0).  EVEN > 0: as many blocks as
-// map.tile_tokens gives, cut evenly in steps of EVEN rows (even_tile_rows).  A remainder of a few rows streams the expert's weights once
-// more for next to no matrix work, and takes more than half of a whole block's time for it.  (MXFP4: figures at even_tile_rows.)
-// bf16, whole MoE block, us, whole token blocks and a remainder : even ones, 32 experts: 1500 tokens 433 : 434, 2048 tokens 599 : 575,
-// 2400 tokens 667 : 591, 3400 tokens 726 : 727, 4096 tokens 868 : 855, 4864 tokens 1025 : 1017, 6656 tokens 1323 : 1327, 8192 tokens 1548 :
-// 1548; 8 experts, 1100 tokens 335 : 309.  In steps of 16 rows, which the bf16 kernel rounds up to 64: 2400 tokens 600, 4096 tokens 859
-// (skewed 878 against 869), 4864 tokens 1022 (1028), 6656 tokens 1363 (1357).
-struct TokenBlocks {
-    int rows, full, rem;
-};
-template <int EVEN>
-MOE_DEVICE TokenBlocks token_blocks(const TileMap& map, int count) {
-    TokenBlocks b;
-    b.rows = EVEN ? even_tile_rows(count, map.tile_tokens, EVEN) : map.tile_tokens;
-    if constexpr (EVEN > 0) {  // all of ceil(count / tile_tokens) but perhaps the last are full: no division by rows
-        const int n = (count + map.tile_tokens - 1) / map.tile_tokens;
-        b.full = n > 0 && n * b.rows != count ? n - 1 : n;
-    } else {
-        b.full = count / b.rows;
-    }
-    b.rem = count - b.full * b.rows;
-    return b;
-}
-
 // grid = E blocks (one expert each), block = 1024 threads, dynamic LDS = (E * copies + E + 32) ints.
-// Tile map order: every full tile first (ascending expert), then the experts' partial last tiles from
-// the largest to the smallest (equal sizes: ascending expert).  An expert kernel that takes tiles in
-// this order runs its shortest blocks last, next to compute units that have already run out of work.
-// With map.second > 0 the same tiles are listed a second time, from index map.second of the three
-// arrays, in bucket order (an expert's tiles together, the partial one last).
+// The tile map lists the tiles of token_blocks in the order of TileOrder.  With map.second > 0 the same tiles are listed a second time,
+// from index map.second of the three arrays, in bucket order (an expert's tiles together, the shortest one last).
 // EVEN is a constant: as a runtime choice it cost the launches without a map 0.35 of 5.8 us.
 template <bool V4, int EVEN>
 __global__ __launch_bounds__(1024) void bucket_kernel(const int* __restrict__ topk_i,
@@ -61,9 +34,8 @@ __global__ __launch_bounds__(1024) void bucket_kernel(const int* __restrict__ to
     extern __shared__ int lds[];
     __shared__ int wave_cnt[4 * 16];  // matches per wave of the four compaction steps in flight
     int* hist = lds;                  // [E]
-    int* scal = lds + E + 16;         // [0] rows before this expert, [1] full tiles before it, [2] full tiles in all,
-                                      // [3] partial tiles ahead of this expert's (by size), [4] partial tiles in all,
-                                      // [5] partial tiles of the experts before this one
+    int* scal = lds + E + 16;         // [0] rows before this expert, [1] tiles before it, [2] tiles in all,
+                                      // [3] tiles ahead of this expert's full ones in the map's order, [4] ahead of its last one
     int* hist_c = lds + E + 32;       // [E][copies]
     const int e = blockIdx.x;
     const int tid = threadIdx.x;
@@ -116,31 +88,28 @@ __global__ __launch_bounds__(1024) void bucket_kernel(const int* __restrict__ to
     __syncthreads();
     const int my_cnt = hist[e];
     const bool mapped = map.tile_tokens > 0;
-    const TokenBlocks mine = mapped ? token_blocks<EVEN>(map, my_cnt) : TokenBlocks{};
+    const TokenBlocks mine = mapped ? token_blocks<EVEN>(map.tile_tokens, my_cnt) : TokenBlocks{};
     {
-        const int my_rem = mine.rem;
-        int rows_before = 0, full_before = 0, full_all = 0, part_ahead = 0, part_all = 0, part_before = 0;
+        int rows_before = 0, tiles_before = 0, tiles_all = 0, ahead_of_full = 0, ahead_of_last = 0;
+        const TileOrder<EVEN> order{map.tile_tokens, map.by_size};
         for (int i = tid; i < E; i += blockDim.x) {
             const int c = hist[i];
             if (i < e) rows_before += c;
             if (mapped) {
-                const TokenBlocks b = token_blocks<EVEN>(map, c);
-                const int full = b.full, rem = b.rem;
-                full_all += full;
-                if (i < e) full_before += full;
-                if (rem > 0) {
-                    part_all += 1;
-                    if (i < e) part_before += 1;
-                    if (rem > my_rem || (rem == my_rem && i < e)) part_ahead += 1;
-                }
+                const TokenBlocks b = token_blocks<EVEN>(map.tile_tokens, c);
+                const int tiles = b.full + (b.rem > 0);
+                tiles_all += tiles;
+                if (i < e) tiles_before += tiles;
+                ahead_of_full += order.ahead_of_full(b, i, mine, e);
+                ahead_of_last += order.ahead_of_last(b, i, mine, e);
             }
         }
         // wave sums first, one add per wave and quantity (an atomic add of a different value per lane
         // is carried out lane by lane)
-        int sums[6] = {rows_before, full_before, full_all, part_ahead, part_all, part_before};
+        int sums[5] = {rows_before, tiles_before, tiles_all, ahead_of_full, ahead_of_last};
         if (wave * 64 < E) {  // wave-uniform: later waves hold zeros
 #pragma unroll
-            for (int i = 0; i < 6; ++i) {
+            for (int i = 0; i < 5; ++i) {
                 const int total = wave_sum(sums[i]);
                 if (lane == 0 && total) atomicAdd(&scal[i], total);
             }
@@ -155,25 +124,25 @@ __global__ __launch_bounds__(1024) void bucket_kernel(const int* __restrict__ to
     if (mapped) {
         const int nb = mine.rows, my_full = mine.full, my_rem = mine.rem;
         for (int j = tid; j < my_full; j += blockDim.x) {
-            map.tile_expert[scal[1] + j] = e;
-            map.tile_row0[scal[1] + j] = my_off + j * nb;
-            map.tile_rows[scal[1] + j] = nb;
+            map.tile_expert[scal[3] + j] = e;
+            map.tile_row0[scal[3] + j] = my_off + j * nb;
+            map.tile_rows[scal[3] + j] = nb;
         }
         if (my_rem > 0 && tid == 0) {
-            const int at = scal[2] + scal[3];
+            const int at = scal[4];
             map.tile_expert[at] = e;
             map.tile_row0[at] = my_off + my_full * nb;
             map.tile_rows[at] = my_rem;
         }
         if (map.second > 0) {  // the same tiles in bucket order: an expert's tiles together, its partial one last
-            const int first = map.second + scal[1] + scal[5];
+            const int first = map.second + scal[1];
             for (int j = tid; j < my_full + (my_rem > 0); j += blockDim.x) {
                 map.tile_expert[first + j] = e;
                 map.tile_row0[first + j] = my_off + j * nb;
                 map.tile_rows[first + j] = min(nb, my_cnt - j * nb);
             }
         }
-        if (e == E - 1 && tid == 0) *map.n_tiles = scal[2] + scal[4];
+        if (e == E - 1 && tid == 0) *map.n_tiles = scal[2];
     }
 
     // ordered compaction: tokens visited in ascending id, 1024 tokens per step; the ids of four steps

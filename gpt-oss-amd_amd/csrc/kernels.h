@@ -4,6 +4,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "token_blocks.h"
+
 struct moe_queue_stats;  // include/moe_abi.h
 
 namespace moe {
@@ -50,23 +52,9 @@ struct TileMap {
     int tile_tokens;  // rows per tile (NB); 0 = no map requested
     int max_tiles;    // capacity = upper bound used as grid dimension
     int second;       // the same tiles in bucket order start at this index of the three arrays (0: not wanted)
-    int even;         // an expert's tiles are cut evenly, in steps of 16 or 64 rows (even_tile_rows); 0: whole tiles and a remainder
+    int even;         // how buckets are cut and in which order their tiles are listed (token_blocks.h)
+    int by_size;
 };
-constexpr int kPrefillStep = 16;      // the MXFP4 kernel runs any number of MFMA tiles,
-constexpr int kPrefillStepBf16 = 64;  // the bf16 kernel (full row blocks) multiples of four
-// Rows of each but the last of an expert's tiles, cut evenly; as many tiles as tile_tokens (a multiple of step) would give.  step is
-// what the kernel that takes the tiles rounds their rows up to: all but the last are multiples of it, so that a bucket's matrix work is
-// ceil(count / step) steps, as few as there can be.  Of MXFP4 buckets only those of two tiles are cut evenly: from three on a remainder
-// is a smaller part of the bucket, and short blocks at the end of a launch even out how its compute units finish.  Whole MoE block, us,
-// 128-row tiles and a remainder : all cut evenly : those of two tiles, 32 experts: 1000 tokens 238 : 233 : 231, 1500 tokens 306 : 304 : 304, 1800
-// tokens 349 : 365 : 348, 2000 tokens 382 : 394 : 380, 3000 tokens 542 : 551 : 541, 4096 tokens 712 : 707 : 713; skewed, 900 tokens 210 : 221 :
-// 209, 1000 tokens 236 : 233 : 233, 4096 tokens 713 : 711 : 711; 8 experts, 600 tokens 145 : 155 : 145, 800 tokens 189 : 182 : 188; 128 experts,
-// 6000 tokens 1233 : 1174 : 1172.  169 sizes together 1 : 1.001 : 0.997.
-__host__ __device__ inline int even_tile_rows(int count, int tile_tokens, int step) {
-    const int n = (count + tile_tokens - 1) / tile_tokens;
-    if (n <= 1 || (n > 2 && step == kPrefillStep)) return tile_tokens;
-    return ((count + n - 1) / n + step - 1) / step * step;
-}
 inline int tile_map_capacity(int A, int E, int tile_tokens) { return (A + tile_tokens - 1) / tile_tokens + E; }
 
 int launch_bucket(const int* topk_i, const float* topk_v, int T, int K, int E, int* expert_offsets,
