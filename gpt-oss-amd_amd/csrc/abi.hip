@@ -41,8 +41,7 @@ inline int tile_even_of(bool prefill, int format) { return !prefill ? 0 : format
 inline bool use_prefill_kernels(int T, int H, int I, int K, int E, int format, unsigned flags) {
     if (flags & MOE_FLAG_FORCE_STREAM) return false;
     const long long rows = (long long)T * K;
-    // a block input past 4 GiB in bf16: only the streaming kernels address its rows
-    if (!expert_rows_fit(T, H) || !expert_rows_fit(0, I)) return false;
+    // a block input past 4 GiB in bf16: only the streaming kernels address its rows for bf16 experts
     if (format == MOE_WEIGHTS_BF16 && !(expert_tile_fits(T, 2 * I, H) && expert_tile_fits(0, H, I))) return false;
     if (flags & MOE_FLAG_FORCE_TILED) return true;
     return format == MOE_WEIGHTS_MXFP4_TILED ? rows >= 52LL * E : rows > 48LL * E;

@@ -1017,12 +1017,15 @@ MOE_DEVICE void prefill_body_mxfp4(const ExpertGemmArgs& a, uint8_t* lds, int e,
     const int half_w = wave >> 2;
     const int q_dma = 4 * blk_w + (lane >> 4);     // row of the token tile this lane moves
     const int chunk_dma = ws_chunk_at<FMT_MXFP4>((lane & 15) ^ q_dma);  // chunk of the stage it fetches
-    uint32_t b_row[TS];  // byte offsets: 32 bits, nine registers fewer than pointers (launcher: expert_rows_fit)
+    // Rows in units of 64 bytes (32 values): a register each, where a pointer takes two, and they reach 256 GiB.  Whole block, us,
+    // pointers : bytes, which reach 4 GiB : so, 32 experts: 1000 tokens 232.2 : 232.3 : 230.9, 16384 tokens 2653.6 : 2654.2 : 2651.7, which two
+    // runs of one build differ by as well.
+    uint32_t b_row[TS];
 #pragma unroll
     for (int i = 0; i < TS; ++i) {
         const int idx = min((half_w + kStagers * i) * 16 + q_dma, nrows - 1);
         const int src = a.gather ? a.tokens_flat[row0 + idx] : idx;  // rows by slot: counted from the block's first
-        b_row[i] = (uint32_t)src * (uint32_t)K * 2u;
+        b_row[i] = (uint32_t)src * ((uint32_t)K / 32u);
     }
     const uint8_t* const b_base = reinterpret_cast<const uint8_t*>(a.act + (a.gather ? 0 : (size_t)row0 * K));
     // Rows of the last token tile past the block's end are cleared once and never loaded: products of zeros take the least power
@@ -1036,11 +1039,11 @@ MOE_DEVICE void prefill_body_mxfp4(const ExpertGemmArgs& a, uint8_t* lds, int e,
     }
     auto issue_b = [&](int s) {
         const int k = s * kStageElems + 8 * chunk_dma;
-        const uint32_t off = (k < K) ? (uint32_t)k * 2u : 0u;  // past the row: re-read its start (weights are 0 there)
+        const uint8_t* const b_at = b_base + ((k < K) ? (size_t)k * 2 : 0);  // past the row: re-read its start (weights are 0 there)
         uint8_t* dst = lds + (size_t)(s & 1) * kStageBytes + (size_t)half_w * 4096 + blk_w * 1024;
 #pragma unroll
-        for (int i = 0; i < TS - 1; ++i) dma16(b_base + (size_t)(b_row[i] + off), dst + i * kStagers * 4096);
-        if (last_live) dma16(b_base + (size_t)(b_row[TS - 1] + off), dst + (TS - 1) * kStagers * 4096);
+        for (int i = 0; i < TS - 1; ++i) dma16(b_at + (size_t)b_row[i] * 64, dst + i * kStagers * 4096);
+        if (last_live) dma16(b_at + (size_t)b_row[TS - 1] * 64, dst + (TS - 1) * kStagers * 4096);
     };
     const uint8_t* const lds_rd = lds + (size_t)q * 256;
     auto b_frag = [&](int s, int j, int t) {  // lane group g owns MX block g of a stage: chunk 4g + j
@@ -1128,8 +1131,8 @@ MOE_DEVICE void prefill_body_mxfp4(const ExpertGemmArgs& a, uint8_t* lds, int e,
 #pragma unroll
                 for (int i = 0; i < R; ++i) {
                     // there and back over the row tiles: every product has an operand of the one before it.  The launch's clock
-                    // hangs on the power that changing operands take: 16384 tokens, 32 experts, whole block 2707 : 2688 us, and with 32-bit
-                    // row offsets 2736 : 2709 on another box; 1000 tokens 248 : 246.
+                    // hangs on the power that changing operands take: whole block, us, one way : so, 32 experts, 1000 tokens 233.5 : 232.3, 4096
+                    // tokens 706 : 704, skewed 712 : 708, 8192 tokens 1359 : 1352, 16384 tokens 2667 : 2654.
                     const int r = (t & 1) ? R - 1 - i : i;
                     acc[r][t] = mfma_16x16x32(av[r], b, acc[r][t]);
                 }

@@ -127,8 +127,6 @@ struct ExpertGemmArgs {
     float* residual_x;
 };
 int launch_expert_stream(const ExpertGemmArgs& a, int epi, hipStream_t stream);
-// The token-block kernels address gathered activation rows, and the rows by slot of one block, by 32-bit byte offsets.
-inline bool expert_rows_fit(long long gathered_rows, int K) { return (gathered_rows > 256 ? gathered_rows : 256) * K * 2 <= 0xffffffffll; }
 
 // ---- experts_tile.hip: prefill-sized buckets of bf16 experts (token blocks of up to 256 rows) ----
 bool expert_tile_fits(long long gathered_rows, int rows, int K);

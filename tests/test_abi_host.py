@@ -118,10 +118,11 @@ def test_describe_names_the_kernels_that_run(pkg):
         assert "; combine=in the down kernel; " in text.value.decode()
 
 
-@pytest.mark.parametrize("T,H,I,K,name", [(65535, 32704, 64, 8, "expert_prefill"), (65535, 32832, 64, 8, "expert_stream_ws"),
-                                          (65535, 64, 8192, 8, "expert_prefill"), (65535, 2880, 2880, 4, "expert_prefill")])
+@pytest.mark.parametrize("T,H,I,K,name", [(65535, 32704, 64, 8, "expert_prefill"), (65535, 32832, 64, 8, "expert_prefill"),
+                                          (65535, 64, 8192, 8, "expert_prefill"), (65535, 2880, 2880, 4, "expert_prefill"),
+                                          (4000, 64, 8388608, 1, "expert_prefill")])
 def test_mxfp4_prefill_kernel_takes_inputs_of_4_gib(pkg, T, H, I, K, name):
-    """Gathered rows past 4 GiB go to the streaming kernels; rows by slot do not matter."""
+    """Gathered rows past 4 GiB, and rows by slot, are no reason to leave the prefill kernel."""
     for flags in (0, pkg.MOE_FLAG_FORCE_TILED):
         k = kernels_of(pkg, T, H, I, 32, K, pkg.MOE_WEIGHTS_MXFP4_TILED, flags=flags)
         assert k["gate_up"].startswith(name) and k["down"].startswith(name), k
