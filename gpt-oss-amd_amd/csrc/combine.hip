@@ -8,8 +8,9 @@ namespace moe {
 
 // K, the experts per token, is a constant of these kernels (combine_of picks the instance): with a runtime K every step was a branch,
 // the routing was loaded a value at a time, a scalar round trip each, and a row's loads waited for the branch in front of them.
-// Rows of 2880, K = 4, us, so : now: by assignment 256 tokens 5.2 : 5.2, by slot 1000 tokens 12.7 : 10.1, 4096 tokens 48.4 : 35.6 (6.6 TB/s),
-// 16384 tokens 184.7 : 175.2 (5.4); with the norm, 100 tokens 8.7 : 5.1, 1024 tokens 17.6 : 14.9.
+// Rows of 2880, K = 4, us, so : now: by assignment 256 tokens 5.2 : 5.2, by slot 1000 tokens 12.7 : 10.1, 4096 tokens 48.4 : 35.6 (6.6 TB/s);
+// with the norm, 100 tokens 8.7 : 5.1, 1024 tokens 17.6 : 14.9.  Other K, stage of the block, 2048 tokens: K = 1 18.3 : 10.7, K = 2 18.7 : 13.8,
+// K = 6 27.7 : 27.3, K = 8 35.0 : 34.6; with the norm, K = 2 25.3 : 23.5, K = 6 41.1 : 38.3, K = 8 58.9 : 48.0.
 
 // The token's K (slot, weight) pairs in ascending expert id (block-uniform: scalar loads and a
 // fully unrolled insertion sort on K register entries).
@@ -44,11 +45,22 @@ MOE_DEVICE float4 fma4(const float4& v, float w, const float4& acc) {
     return make_float4(fmaf(v.x, w, acc.x), fmaf(v.y, w, acc.y), fmaf(v.z, w, acc.z), fmaf(v.w, w, acc.w));
 }
 
+// NT: the rows by slot are more than the last-level cache holds and not in it any more; they are read past it.
+template <bool NT>
+MOE_DEVICE float4 load_value(const float4* p) {
+    if constexpr (NT) {
+        const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+        return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
+    } else {
+        return *p;
+    }
+}
+
 // NI float4 columns (from c0, `step` apart, those below H4) of the token's combined row: K fused multiply-adds in ascending expert id.
 // slot_of == NULL: rows are stored by assignment, the row of (t, k) is t * K + k, known without looking at the routing, so
 // their loads go out together with the loads of the routing itself (one memory round trip instead of two).  The order of the
 // additions is fixed afterwards: the rank of each k by expert id is block-uniform, and rank r is added in step r.
-template <int K, int NI>
+template <int K, int NI, bool NT>
 MOE_DEVICE void combine_columns(const float4* __restrict__ y, const int* __restrict__ slot_of, const int* __restrict__ topk_i,
                                 const float* __restrict__ topk_v, int t, int H4, int c0, int step, float4 (&acc)[NI]) {
     float4 v[NI][K];
@@ -57,14 +69,22 @@ MOE_DEVICE void combine_columns(const float4* __restrict__ y, const int* __restr
         int sl[K];
         sorted_slots<K>(slot_of, topk_i, topk_v, t, sl, wt);
 #pragma unroll
-        for (int i = 0; i < NI; ++i)
+        for (int i = 0; i < NI; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        // Rows whose loads are in flight together.  Eight rows of a multiple of 4096 meet in the same L2 sets (stage of the block, 1024 tokens of
+        // 4096 values, a runtime K : eight rows : two, 26.4 : 30.3 : 28.7; with the norm 34.1 : 35.3 : 33.6; of 2880 values 19.6 : 19.3 : 19.2).
+        constexpr int AT_ONCE = K < 8 ? K : 2;
 #pragma unroll
-            for (int k = 0; k < K; ++k) v[i][k] = y[(size_t)sl[k] * H4 + min(c0 + i * step, H4 - 1)];
+        for (int k0 = 0; k0 < K; k0 += AT_ONCE) {
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            for (int i = 0; i < NI; ++i)
 #pragma unroll
-            for (int k = 0; k < K; ++k) acc[i] = fma4(v[i][k], wt[k], acc[i]);
+                for (int k = k0; k < min(k0 + AT_ONCE, K); ++k)
+                    v[i][k] = load_value<NT>(y + (size_t)sl[k] * H4 + min(c0 + i * step, H4 - 1));
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+                for (int k = k0; k < min(k0 + AT_ONCE, K); ++k) acc[i] = fma4(v[i][k], wt[k], acc[i]);
+            if (AT_ONCE < K) __builtin_amdgcn_sched_barrier(0);
         }
         return;
     }
@@ -105,18 +125,25 @@ MOE_DEVICE void combine_columns(const float4* __restrict__ y, const int* __restr
     }
 }
 
-// f(integral_constant<int, K>) for the runtime K of 1 .. 8
+// Whether the rows by slot are more than the 256 MiB of the last-level cache (NT).  Stage of the block, us, a runtime K : this without NT : with
+// it, 8192 tokens: K = 4 of 2880 values 106 : 95 : 74 (6.4 TB/s), K = 6 of 5120 253 : 260 : 188, K = 8 of 8192 492 : 510 : 417; with the norm, K = 4 of 2880
+// 166 : 153 : 116; 16384 tokens, K = 4 of 2880, 213 : 209 : 147.  Rows that the cache does hold are read from there: 2048 tokens, K = 7 of 4096 (235 MB)
+// without : with 41.4 : 44.5, K = 5 of 5120 (210 MB) 38.3 : 39.2, and just past it K = 7 of 5120 (294 MB) 59.6 : 56.0, K = 8 of 4096 (268 MB) 54.8 : 50.8.
+static bool rows_past_cache(const int* slot_of, int T, int K, int H) { return slot_of && (long long)T * K * H * 4 > (256ll << 20); }
+
+// f(integral_constant<int, K>, bool_constant<NT>) for the runtime K of 1 .. 8
 template <class Fn>
-static int combine_of(int K, Fn&& f) {
+static int combine_of(int K, bool nt, Fn&& f) {
+    auto with = [&](auto k) { return nt ? f(k, std::true_type{}) : f(k, std::false_type{}); };
     switch (K) {
-        case 1: return f(std::integral_constant<int, 1>{});
-        case 2: return f(std::integral_constant<int, 2>{});
-        case 3: return f(std::integral_constant<int, 3>{});
-        case 4: return f(std::integral_constant<int, 4>{});
-        case 5: return f(std::integral_constant<int, 5>{});
-        case 6: return f(std::integral_constant<int, 6>{});
-        case 7: return f(std::integral_constant<int, 7>{});
-        case 8: return f(std::integral_constant<int, 8>{});
+        case 1: return with(std::integral_constant<int, 1>{});
+        case 2: return with(std::integral_constant<int, 2>{});
+        case 3: return with(std::integral_constant<int, 3>{});
+        case 4: return with(std::integral_constant<int, 4>{});
+        case 5: return with(std::integral_constant<int, 5>{});
+        case 6: return with(std::integral_constant<int, 6>{});
+        case 7: return with(std::integral_constant<int, 7>{});
+        case 8: return with(std::integral_constant<int, 8>{});
     }
     return MOE_ERR_LIMIT;
 }
@@ -127,7 +154,7 @@ static int combine_of(int K, Fn&& f) {
 // moe_mlp2_scatter_mfma_kernel (src/hip/moe.hip:464-492), whose order is not fixed.
 // Optionally also residual_x += e_agg (src/forward.cpp:514).
 // grid = (ceil(H/4/256), T), block = 256.
-template <int K>
+template <int K, bool NT>
 __global__ __launch_bounds__(256) void combine_kernel(const float4* __restrict__ y, const int* __restrict__ slot_of,
                                                       const int* __restrict__ topk_i,
                                                       const float* __restrict__ topk_v, float4* __restrict__ e_agg,
@@ -137,7 +164,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const float4* __restrict__
     if (c >= H4) return;
     float4 before, acc[1];
     if (residual_x) before = residual_x[(size_t)t * H4 + c];  // uniform
-    combine_columns<K, 1>(y, slot_of, topk_i, topk_v, t, H4, c, 0, acc);
+    combine_columns<K, 1, NT>(y, slot_of, topk_i, topk_v, t, H4, c, 0, acc);
     e_agg[(size_t)t * H4 + c] = acc[0];
     if (residual_x)
         residual_x[(size_t)t * H4 + c] =
@@ -147,8 +174,8 @@ __global__ __launch_bounds__(256) void combine_kernel(const float4* __restrict__
 int launch_combine(const float* y_by_slot, const int* slot_of, const int* topk_i, const float* topk_v,
                    float* e_agg, float* residual_x, int T, int K, int H, hipStream_t stream) {
     const int H4 = H / 4;
-    return combine_of(K, [&](auto k) {
-        hipLaunchKernelGGL((combine_kernel<decltype(k)::value>), dim3(ceil_div(H4, 256), T), dim3(256), 0, stream,
+    return combine_of(K, rows_past_cache(slot_of, T, K, H), [&](auto k, auto nt) {
+        hipLaunchKernelGGL((combine_kernel<decltype(k)::value, decltype(nt)::value>), dim3(ceil_div(H4, 256), T), dim3(256), 0, stream,
                            reinterpret_cast<const float4*>(y_by_slot), slot_of, topk_i, topk_v,
                            reinterpret_cast<float4*>(e_agg), reinterpret_cast<float4*>(residual_x), T, H4);
         return launch_status();
@@ -251,7 +278,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(float* __restrict__ o, con
 //   e_agg = combine;  residual_x += e_agg;  norm_out = rmsnorm(residual_x, norm_weight).
 // Same arithmetic as combine_kernel followed by rmsnorm_kernel.  A thread keeps its NI float4 columns
 // of the updated residual in registers.  grid = T, block = 256, H/4 <= 256 * NI.
-template <int NI, int K>
+template <int NI, int K, bool NT>
 __global__ __launch_bounds__(256) void combine_norm_kernel(const float4* __restrict__ y, const int* __restrict__ slot_of,
                                                            const int* __restrict__ topk_i,
                                                            const float* __restrict__ topk_v, float4* __restrict__ e_agg,
@@ -263,7 +290,7 @@ __global__ __launch_bounds__(256) void combine_norm_kernel(const float4* __restr
     float4 r[NI], acc[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) r[i] = residual_x[(size_t)t * H4 + min((int)threadIdx.x + 256 * i, H4 - 1)];
-    combine_columns<K, NI>(y, slot_of, topk_i, topk_v, t, H4, threadIdx.x, 256, acc);
+    combine_columns<K, NI, NT>(y, slot_of, topk_i, topk_v, t, H4, threadIdx.x, 256, acc);
     double ss = 0.0;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
@@ -300,16 +327,17 @@ int launch_combine_norm(const float* y_by_slot, const int* slot_of, const int* t
     auto e = reinterpret_cast<float4*>(e_agg);
     auto r = reinterpret_cast<float4*>(residual_x);
     auto o = reinterpret_cast<float4*>(norm_out);
-    return combine_of(K, [&](auto k) {
+    return combine_of(K, rows_past_cache(slot_of, T, K, H), [&](auto k, auto nt) {
         constexpr int KC = decltype(k)::value;
+        constexpr bool NT = decltype(nt)::value;
         auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(T), dim3(256), 0, stream, y, slot_of, topk_i, topk_v, e, r, norm_weight, o, H4);
             return launch_status();
         };
-        if (ni <= 1) return launch(combine_norm_kernel<1, KC>);
-        if (ni <= 2) return launch(combine_norm_kernel<2, KC>);
-        if (ni <= 3) return launch(combine_norm_kernel<3, KC>);
-        return launch(combine_norm_kernel<4, KC>);
+        if (ni <= 1) return launch(combine_norm_kernel<1, KC, NT>);
+        if (ni <= 2) return launch(combine_norm_kernel<2, KC, NT>);
+        if (ni <= 3) return launch(combine_norm_kernel<3, KC, NT>);
+        return launch(combine_norm_kernel<4, KC, NT>);
     });
 }
 
