@@ -13,7 +13,6 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
@@ -85,13 +84,6 @@ MOE_DEVICE void mxfp4_dword_to_bf16x8(uint32_t codes, float scale, uint32_t out[
 // D[rows 4*(l/16) .. +4][col l%16].
 MOE_DEVICE f32x4 mfma_16x16x32(const u32x4& a, const u32x4& b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
-// D(32x32) += A(32x16) * B(16x32); lane l holds A[row l%32][8*(l/32) .. +8), B[..][col l%32],
-// D[rows 8*(i/4) + 4*(l/32) + i%4 for i in 0..15][col l%32].
-MOE_DEVICE f32x16 mfma_32x32x16(const u32x4& a, const u32x4& b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
