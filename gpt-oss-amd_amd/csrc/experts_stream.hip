@@ -1029,7 +1029,8 @@ MOE_DEVICE void prefill_body_mxfp4(const ExpertGemmArgs& a, uint8_t* lds, int e,
     }
     const uint8_t* const b_base = reinterpret_cast<const uint8_t*>(a.act + (a.gather ? 0 : (size_t)row0 * K));
     // Rows of the last token tile past the block's end are cleared once and never loaded: products of zeros take the least power
-    // (up to 15 such rows to a bucket; whole block, the last row again : zeros, 1000 tokens 243.8 : 241.4 us, 4096 tokens 718 : 716).
+    // (up to 15 such rows to a bucket; whole block, the last row again : zeros, 1000 tokens 243.8 : 241.4 us, from 4096 tokens on
+    // within two runs of one build).
     static_assert(kStagers == 1, "this wave's last tile is the block's");
     const bool last_live = (NT - 1) * 16 + q_dma < nrows;
     if (!last_live) {

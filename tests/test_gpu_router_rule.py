@@ -103,7 +103,7 @@ def test_screening_at_the_ends_of_the_float_range(pkg, wl, dev, T, H, E, router,
     _, ti, tv = blk.forward(x)
     assert blk.describe(blk.params(x, x, ti, tv))["router"] == router
     _, wi, wv = blk.forward(x, flags=pkg.MOE_FLAG_ROUTER_STRICT_ORDER)
-    assert torch.equal(ti, wi) and (tv - wv).nan_to_num(0.0).abs().max().item() <= 4e-6
+    assert torch.equal(ti, wi) and torch.equal(tv.isnan(), wv.isnan()) and (tv - wv).nan_to_num(0.0).abs().max().item() <= 4e-6
 
 
 @pytest.mark.parametrize("E", [1, 63, 64, 65, 128, 129, 192, 256, 257, 512, 513, 1000, 1024])
